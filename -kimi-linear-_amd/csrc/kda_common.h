@@ -170,6 +170,45 @@ __device__ __forceinline__ float rowgroup_sum(float x) {
     return x;
 }
 
+// Sum of x over the 16 lanes of a DPP row (all-reduce).
+__device__ __forceinline__ float row16_sum(float x) {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xF, 0xF, true));  // row_ror:8
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xF, 0xF, true));  // row_ror:4
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xF, 0xF, true));  // row_ror:2
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xF, 0xF, true));  // row_ror:1
+    return x;
+}
+
+// Sum of x over each run of N lanes (N-aligned; all-reduce).
+template <int N>
+__device__ __forceinline__ float lanes_sum(float x) {
+    static_assert(N == 4 || N == 8 || N == 16 || N == 32, "runs of 4, 8, 16 or 32 lanes");
+    if constexpr (N >= 16) {
+        x = row16_sum(x);
+        if constexpr (N == 32) {
+            const unsigned u = __float_as_uint(x);
+            const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+            x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+    } else {
+        x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0xB1, 0xF, 0xF, true));   // quad [1,0,3,2]
+        x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x4E, 0xF, 0xF, true));   // quad [2,3,0,1]
+        if constexpr (N == 8)
+            x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x141, 0xF, 0xF, true));   // row_half_mirror
+    }
+    return x;
+}
+
+// x of lane J of each DPP row, to all 16 lanes of the row.
+template <int J>
+__device__ __forceinline__ float row16_bcast(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + J, 0xF, 0xF, true));   // row_newbcast
+}
+// x of the lane four further on in the DPP row (cyclic).
+__device__ __forceinline__ float row16_down4(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x12C, 0xF, 0xF, true));   // row_ror:12
+}
+
 // Sum of x over the 4 lanes that share l & 15 (all-reduce): the permlane
 // swaps of bits 4 and 5.
 __device__ __forceinline__ float lanegroup4_sum(float x) {
