@@ -660,15 +660,20 @@ int launch_k(const kda_fwd_args& a, hipStream_t stream, const kda_gate_args& gat
     const int64_t cols = a.B * a.H * a.V;
     const bool wide = cols > 64 * 512;
     if (ckpt != nullptr || (a.T > 1 && (a.T >= 8 || !wide))) return launch_seq<K>(a, stream, gate, ckpt);
-    // K 128 with V % 64 == 0: one wave of 64 columns (32 rows x 4 columns a
-    // lane, 239 VGPRs: the 2048 waves of a B=64 H=16 V=128 step are all
-    // resident at once); other K <= 128: one wave of 32 columns (K / 8 rows x
-    // 4 columns a lane); K 256: 16 columns a wave (K / 16 rows a lane).
-    if constexpr (K == 128) {
-        if (a.V % 64 == 0) return launch_k_nw<K, 1, 16>(a, stream, gate);
-    }
+    // K <= 128: one wave a workgroup, of 64 columns (K = 128: 32 rows x 4
+    // columns a lane, 2 waves a SIMD: the 2048 waves of a B=64 H=16 V=128 step
+    // are all resident at once), 32 or 16.  A narrower wave's chain is
+    // shorter, a wider one has more of the state in flight.  us a step at
+    // H=16 K=V=128, 64 / 32 / 16 columns: B=1 5.3 / 4.3 / 4.0, B=8 6.0 / 5.3 /
+    // 5.2, B=16 8.9 / 8.6 / 10.6, B=32 14.2 / 13.1 / 23.0, B=48 18.8 / 19.5 /
+    // 33.1, B=64 22.9 / 27.8 / 44.0; K=V=64, 32 / 16: B=1 3.5 / 3.4, B=16 4.1 /
+    // 4.1, B=64 7.8 / 11.1.  K 256: 16 columns a wave (K / 16 rows a lane).
     if constexpr (K <= 128) {
-        if (a.V % 32 == 0) return launch_k_nw<K, 1, 8>(a, stream, gate);
+        if (cols <= 64 * 256 || a.V % 32 != 0) return launch_k_nw<K, 1, 4>(a, stream, gate);
+        if constexpr (K == 128) {
+            if (cols > 64 * 1024 && a.V % 64 == 0) return launch_k_nw<K, 1, 16>(a, stream, gate);
+        }
+        return launch_k_nw<K, 1, 8>(a, stream, gate);
     }
     if (a.V % 64 == 0) return launch_k_nw<K, 4, 4>(a, stream, gate);
     if (a.V % 32 == 0) return launch_k_nw<K, 2, 4>(a, stream, gate);
