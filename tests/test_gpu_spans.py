@@ -140,3 +140,22 @@ def test_fp32_checkpoints_hold_the_states(kda_pkg, T):
                 want = kda_pkg.kda_recurrent(*(x[:, :32 * c] for x in args), state=dev["state"])[1]
             got = ck[:, :, c, :K * V].reshape(B, H, K, V)
             assert torch.equal(got, want)
+
+
+def test_bf16_rounding_is_nearest_even(kda_pkg):
+    """Stored bf16 values (here the state of a call without tokens) are torch's
+    rounding of the fp32 ones bit for bit: any exponent, ties, denormals,
+    infinities; a NaN stays one."""
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randint(-2 ** 31, 2 ** 31 - 1, (4, 1, 128, 128), generator=gen).to(torch.int32)
+    edge = [0x7f800000, 0x7f7fffff, 0x7f7f8000, 1, 0x7fffff, 0x8000, 0x18000, 0x3f808000, 0x3f818000, 0x7f800001,
+            0x7fc00000, 0x7fffffff]
+    x.view(-1)[:len(edge)] = torch.tensor(edge, dtype=torch.int64).to(torch.int32)
+    f = x.view(torch.float32).to(DEV)
+    e = torch.zeros(4, 0, 1, 128, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        _, s = kda_pkg.kda_recurrent(e, e, e, e.float(), torch.zeros(4, 0, 1, device=DEV), state=f,
+                                     state_dtype=torch.bfloat16)
+    nan = torch.isnan(f)
+    assert torch.isnan(s[nan]).all()
+    assert torch.equal(s[~nan].view(torch.int16), f[~nan].to(torch.bfloat16).view(torch.int16))
