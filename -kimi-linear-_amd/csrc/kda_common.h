@@ -184,12 +184,17 @@ __device__ __forceinline__ float row16_sum(float x) {
 // Sum of x over each run of N lanes (N-aligned; all-reduce).
 template <int N>
 __device__ __forceinline__ float lanes_sum(float x) {
-    static_assert(N == 4 || N == 8 || N == 16 || N == 32, "runs of 4, 8, 16 or 32 lanes");
+    static_assert(N == 4 || N == 8 || N == 16 || N == 32 || N == 64, "runs of 4, 8, 16, 32 or 64 lanes");
     if constexpr (N >= 16) {
         x = row16_sum(x);
-        if constexpr (N == 32) {
+        if constexpr (N >= 32) {
             const unsigned u = __float_as_uint(x);
             const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+            x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+        if constexpr (N == 64) {
+            const unsigned u = __float_as_uint(x);
+            const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
             x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
         }
     } else {

@@ -16,21 +16,27 @@
 // _output (kda.py:258-279, 464-470): one read of the core output and of the
 // gate projection, one write of the o_proj input.
 //
-// Both are HBM-streaming kernels: one wave per unit of work (a 16-token tile
-// of one head of one tensor, or an 8-token tile of one output head), lanes
-// across the head's channels (K / 64 consecutive channels per lane, one
-// vector access per row), cross-lane sums on DPP and permlane swaps.  Every
-// load of a unit is issued unconditionally before its first use (rows past
-// the data re-read a valid row and are masked), so a wave keeps all of its
-// rows in flight at once instead of waiting on each.
+// Both are streaming kernels with the lanes across channels, eight adjacent
+// ones a lane (16 bytes of a 16-bit row), so a wave takes 512 channels of a
+// row: the heads' sums of squares are DPP sums over K / 8 lanes, and the
+// per-row work (addresses, the sum's exchange, the row's rsqrt) is shared by
+// eight channels.  Every load of a unit is issued unconditionally before its
+// first use (rows past the data re-read a valid row and are masked), so a
+// wave keeps all of its rows in flight at once instead of waiting on each.
+#include <type_traits>
+
 #include "kda_common.h"
 
 namespace kda {
 
 namespace {
 
-constexpr int kTile = 16;      // tokens per prep unit (a single-token call uses units of one token)
+constexpr int kTile = 16;      // tokens per prep unit at most; an in-place conv cache needs T <= this
 constexpr int kMaxConv = 4;    // largest conv_size
+// channels per lane of q, k and v (16 bytes) and per wave
+template <typename XT> constexpr int kLaneCh = 16 / static_cast<int>(sizeof(XT));
+template <typename XT> constexpr int kSeg = 64 * kLaneCh<XT>;
+constexpr int kGateSeg = 256;  // channels per wave of the gate, 4 a lane
 
 template <typename XT> __device__ __forceinline__ float to_f(XT x);
 template <> __device__ __forceinline__ float to_f<float>(float x) { return x; }
@@ -42,245 +48,293 @@ template <> __device__ __forceinline__ float from_f<float>(float x) { return x; 
 template <> __device__ __forceinline__ _Float16 from_f<_Float16>(float x) { return static_cast<_Float16>(x); }
 template <> __device__ __forceinline__ bf16_t from_f<bf16_t>(float x) { return bf16_t{f32_to_bf16_bits(x)}; }
 
-// CPL consecutive elements, accessed as one aligned vector.
-template <typename XT, int CPL>
-struct alignas(sizeof(XT) * CPL) Pack {
-    XT e[CPL];
-};
-
-template <typename XT, int CPL>
-__device__ __forceinline__ void ld(const XT* p, float (&x)[CPL]) {
-    const Pack<XT, CPL> v = *reinterpret_cast<const Pack<XT, CPL>*>(p);
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) x[c] = to_f(v.e[c]);
-}
-
-template <typename XT, int CPL>
-__device__ __forceinline__ void st(XT* p, const float (&x)[CPL]) {
-    Pack<XT, CPL> v;
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) v.e[c] = from_f<XT>(x[c]);
-    *reinterpret_cast<Pack<XT, CPL>*>(p) = v;
-}
-
 // Round to XT and back: the value an XT tensor would hold.
 template <typename XT>
 __device__ __forceinline__ float round_to(float x) {
     return to_f(from_f<XT>(x));
 }
 
-
-
-// A small parameter element of a runtime dtype: the load is unconditional
-// (a NULL or out-of-range element reads `fallback`'s first word instead and is
-// masked), so that every load of a unit is issued before any result is used.
-__device__ __forceinline__ RawElem param_load(const void* p, int64_t i, bool valid, const void* fallback,
-                                              int dtype) {
-    return valid ? load_raw_elem(p, i, dtype) : load_raw_elem(fallback, 0, dtype);
+// N consecutive elements held as loaded.  Rows are aligned to their
+// element only (the layer's rows of H (2 K + V) + H + 256 elements are not a
+// multiple of 16 bytes for every H); the compiler emits what that allows.
+template <typename XT, int N>
+struct Raw {
+    static constexpr int W = sizeof(XT) * N / 4;     // words
+    uint32_t w[W];
+};
+template <int N, typename XT>
+__device__ __forceinline__ Raw<XT, N> ldn(const XT* p) {
+    Raw<XT, N> r;
+    __builtin_memcpy(r.w, p, sizeof(r.w));
+    return r;
+}
+template <typename XT, int N>
+__device__ __forceinline__ void unpack(const Raw<XT, N>& r, float (&x)[N]) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+        if constexpr (sizeof(XT) == 4) {
+            x[c] = __uint_as_float(r.w[c]);
+        } else {
+            const uint16_t u = static_cast<uint16_t>(r.w[c / 2] >> (16 * (c % 2)));
+            x[c] = Elem<XT>::code == KDA_DTYPE_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, u))
+                                                   : bf16_bits_to_f32(u);
+        }
+    }
+}
+template <typename XT, int N>
+__device__ __forceinline__ void stn(XT* p, const float (&x)[N]) {
+    XT v[N];
+#pragma unroll
+    for (int c = 0; c < N; ++c) v[c] = from_f<XT>(x[c]);
+    __builtin_memcpy(p, v, sizeof(v));
 }
 
-// ---- prep: one q, k or v head over a token tile ---------------------------
-template <typename XT, int CPL, int TILE>
-__device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t b, int64_t t0, int64_t h, int lane) {
-    constexpr int kRows = TILE + kMaxConv - 1;
-    const int64_t Dh = 64 * CPL;
-    const int64_t D = a.H * Dh;
-    const int64_t ch0 = h * Dh + lane * CPL;
-    const int cs = static_cast<int>(a.conv_size), cm = cs - 1;
+// N consecutive parameters of a runtime dtype from element i on, as fp32.
+template <int N>
+__device__ __forceinline__ void params(const void* p, int64_t i, int dtype, float (&x)[N]) {
+    uint32_t w[N];
+    if (dtype == KDA_DTYPE_F32) {
+        __builtin_memcpy(w, static_cast<const float*>(p) + i, sizeof(w));
+#pragma unroll
+        for (int c = 0; c < N; ++c) x[c] = __uint_as_float(w[c]);
+        return;
+    }
+    __builtin_memcpy(w, static_cast<const uint16_t*>(p) + i, N * 2);
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+        const uint16_t u = static_cast<uint16_t>(w[c / 2] >> (16 * (c % 2)));
+        x[c] = dtype == KDA_DTYPE_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, u)) : bf16_bits_to_f32(u);
+    }
+}
+
+// ---- prep: kSeg channels of q, k or v over a token tile ---------------------
+// DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
+// conv_size when it is 4 (the usual case, no test of the tap count in the
+// loops), else 0.
+template <typename XT, int DH, int TILE, int CS>
+__device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t b, int64_t t0, int64_t seg, int lane) {
+    constexpr int kRows = TILE + kMaxConv - 1, N = kLaneCh<XT>;
+    const int64_t D = a.H * (DH ? DH : a.V);
+    const bool valid = seg * kSeg<XT> + N * lane < D;
+    const int64_t ch0 = valid ? seg * kSeg<XT> + N * lane : 0;
+    const int cs = CS ? CS : static_cast<int>(a.conv_size), cm = cs - 1;
     const int64_t T = a.T;
     const int n = static_cast<int>((T - t0) < TILE ? (T - t0) : TILE);
-    const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0] + ch0;
+    const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0];
     const XT* hist = static_cast<const XT*>(a.hist_in[i]);
-    const XT* hrow = hist != nullptr ? hist + b * cm * D + ch0 : x;
+    const XT* hrow = hist != nullptr ? hist + b * cm * D : x;
 
     // window row r holds token t0 - cm + r: a token of this call, a cached
     // input (t < 0) or zero.  Every row is loaded unconditionally (rows with
     // no data read token 0 and are masked) so that all loads are in flight
     // together.
-    float win[kRows][CPL];
+    Raw<XT, N> win[kRows];
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
         const int64_t tok = t0 - cm + r;
         const bool in_x = tok >= 0 && tok < T;
         const bool in_h = tok < 0 && hist != nullptr;
         const XT* src = in_x ? x + tok * a.x_stride[i][1] : (in_h ? hrow + (cm + tok) * D : x);
-        ld<XT, CPL>(src, win[r]);
+        win[r] = ldn<N>(src + ch0);
         if (!(in_x || in_h)) {
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) win[r][c] = 0.f;
+            for (int c = 0; c < Raw<XT, N>::W; ++c) win[r].w[c] = 0u;
         }
     }
-    RawElem rw[kMaxConv][CPL], rb[CPL];
+    float w[kMaxConv][N], bias[N];
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        rb[c] = param_load(a.conv_b[i], ch0 + c, a.conv_b[i] != nullptr, a.conv_w[i], a.w_dtype);
+    for (int c = 0; c < N; ++c) bias[c] = 0.f;
+    if (a.conv_b[i] != nullptr) params<N>(a.conv_b[i], ch0, a.w_dtype, bias);
+    if constexpr (CS == kMaxConv) {
+        float wc[N * kMaxConv];
+        params<N * kMaxConv>(a.conv_w[i], ch0 * kMaxConv, a.w_dtype, wc);
 #pragma unroll
-        for (int j = 0; j < kMaxConv; ++j)
-            rw[j][c] = param_load(a.conv_w[i], (ch0 + c) * cs + j, j < cs, a.conv_w[i], a.w_dtype);
-    }
-    float w[kMaxConv][CPL], bias[CPL];
+        for (int c = 0; c < N; ++c)
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        bias[c] = a.conv_b[i] != nullptr ? decode_elem(rb[c], a.w_dtype) : 0.f;
+            for (int j = 0; j < kMaxConv; ++j) w[j][c] = wc[kMaxConv * c + j];
+    } else {
 #pragma unroll
-        for (int j = 0; j < kMaxConv; ++j) w[j][c] = j < cs ? decode_elem(rw[j][c], a.w_dtype) : 0.f;
+        for (int c = 0; c < N; ++c)
+#pragma unroll
+            for (int j = 0; j < kMaxConv; ++j)
+                w[j][c] = j < cs ? load_elem(a.conv_w[i], (ch0 + c) * cs + j, a.w_dtype) : 0.f;
     }
 
     XT* out = static_cast<XT*>(i == 0 ? a.q : (i == 1 ? a.k : a.v)) + (b * T + t0) * D + ch0;
     const float inv_eps = 1.f / a.l2_eps;
     // tap j of tile token t reads window row t + j (token t0 + t - cm + j)
+    float xs[kMaxConv][N];
+#pragma unroll
+    for (int j = 0; j < kMaxConv - 1; ++j) unpack(win[j], xs[j]);
 #pragma unroll
     for (int t = 0; t < TILE; ++t) {
-        float s[CPL];
+        unpack(win[t + kMaxConv - 1], xs[(t + kMaxConv - 1) % kMaxConv]);
+        float s[N];
         float ss = 0.f;
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) {
+        for (int c = 0; c < N; ++c) {
             float u = bias[c];
 #pragma unroll
             for (int j = 0; j < kMaxConv; ++j)
-                if (j < cs) u = fmaf(w[j][c], win[t + j][c], u);
+                if (j < cs) u = fmaf(w[j][c], xs[(t + j) % kMaxConv][c], u);
             s[c] = u * sigmoid_f(u);
             ss = fmaf(s[c], s[c], ss);
         }
-        if (i < 2) {
+        if constexpr (DH != 0) {
             // l2 norm over the head: x * min(rsqrt(sum x^2), 1/eps)
-            const float rn = fminf(rsqrtf(wave_sum(ss)), inv_eps);
+            const float rn = fminf(rsqrtf(lanes_sum<DH / N>(ss)), inv_eps);
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) s[c] *= rn;
+            for (int c = 0; c < N; ++c) s[c] *= rn;
         }
-        if (t < n) st<XT, CPL>(out + t * D, s);
+        if (t < n && valid) stn(out + t * D, s);
     }
 
     // the next call's conv cache: inputs T - cm .. T - 1 = window rows n + r
-    if (a.hist_out[i] != nullptr && t0 + n == T) {
+    if (a.hist_out[i] != nullptr && t0 + n == T && valid) {
         XT* ho = static_cast<XT*>(a.hist_out[i]) + b * cm * D + ch0;
 #pragma unroll
         for (int r = 0; r < kMaxConv - 1; ++r) {
-            float hv[CPL];
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) hv[c] = 0.f;
+            Raw<XT, N> hv = win[r];
 #pragma unroll
             for (int rr = 0; rr < kRows; ++rr)
-                if (rr == n + r) {
-#pragma unroll
-                    for (int c = 0; c < CPL; ++c) hv[c] = win[rr][c];
-                }
-            if (r < cm) st<XT, CPL>(ho + r * D, hv);
+                if (rr == n + r) hv = win[rr];
+            if (r < cm) __builtin_memcpy(ho + r * D, hv.w, sizeof(hv.w));
         }
     }
 }
 
-// ---- prep: the forget gate of one head over a token tile, and its beta ----
-template <typename XT, int CPL, int TILE>
-__device__ __forceinline__ void gate_unit(const kda_prep_args& a, int64_t b, int64_t t0, int64_t h, int lane) {
-    const int64_t Dh = 64 * CPL;
-    const int64_t D = a.H * Dh;
-    const int64_t ch0 = h * Dh + lane * CPL;
+// ---- prep: the forget gate of 256 channels over a token tile, and the betas
+// of their heads.  Four channels a lane: g is stored in 32 bits, 16 bytes a
+// lane (eight channels in two stores of 32-byte lanes took 107 us where this
+// takes 78 at B=4 T=2048 H=16 K=128 bf16, the projections included).
+template <typename XT, int DH, int TILE>
+__device__ __forceinline__ void gate_unit(const kda_prep_args& a, int64_t b, int64_t t0, int64_t seg, int lane) {
+    constexpr int kHeads = kGateSeg / DH;        // heads per unit
+    const int64_t D = a.H * DH;
+    const bool valid = seg * kGateSeg + 4 * lane < D;
+    const int64_t ch0 = valid ? seg * kGateSeg + 4 * lane : 0;
     const int64_t T = a.T;
     const int n = static_cast<int>((T - t0) < TILE ? (T - t0) : TILE);
     const XT* gk = static_cast<const XT*>(a.gk) + b * a.gk_stride[0] + ch0;
 
     // every load first (rows past the end re-read the last token)
-    float z[TILE][CPL];
+    Raw<XT, 4> z[TILE];
 #pragma unroll
-    for (int t = 0; t < TILE; ++t) ld<XT, CPL>(gk + (t0 + (t < n ? t : n - 1)) * a.gk_stride[1], z[t]);
-    const int tl = lane < n ? lane : n - 1;
-    const RawElem rlogit =
-        load_raw_elem(a.beta_logit, b * a.beta_stride[0] + (t0 + tl) * a.beta_stride[1] + h, a.x_dtype);
-    RawElem ra[CPL], rd[CPL];
+    for (int t = 0; t < TILE; ++t) z[t] = ldn<4>(gk + (t0 + (t < n ? t : n - 1)) * a.gk_stride[1]);
+    // entry e of the unit's TILE x kHeads betas: token e / kHeads, head e % kHeads
+    constexpr int kB = (TILE * kHeads + 63) / 64;
+    RawElem rl[kB];
+    int64_t bt[kB], bh[kB];
+    bool bv[kB];
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        ra[c] = load_raw_elem(a.a_log, ch0 + c, a.p_dtype);
-        rd[c] = load_raw_elem(a.dt_bias, ch0 + c, a.p_dtype);
+    for (int e = 0; e < kB; ++e) {
+        const int k = lane + 64 * e;
+        bt[e] = t0 + k / kHeads;
+        bh[e] = seg * kHeads + k % kHeads;
+        bv[e] = k < n * kHeads && bh[e] < a.H;
+        rl[e] = load_raw_elem(a.beta_logit,
+                              b * a.beta_stride[0] + (bv[e] ? bt[e] * a.beta_stride[1] + bh[e] : t0 * a.beta_stride[1]),
+                              a.x_dtype);
     }
-    float neg_a[CPL], dtb[CPL];
+    float neg_a[4], dtb[4];
+    params<4>(a.a_log, ch0, a.p_dtype, neg_a);
+    params<4>(a.dt_bias, ch0, a.p_dtype, dtb);
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        neg_a[c] = -__expf(decode_elem(ra[c], a.p_dtype));
-        dtb[c] = decode_elem(rd[c], a.p_dtype);
-    }
+    for (int c = 0; c < 4; ++c) neg_a[c] = -__expf(neg_a[c]);
     float* g = static_cast<float*>(a.g) + (b * T + t0) * D + ch0;
 #pragma unroll
     for (int t = 0; t < TILE; ++t) {
-        float o[CPL];
+        float x[4], o[4];
+        unpack(z[t], x);
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) o[c] = neg_a[c] * softplus(z[t][c] + dtb[c]);
-        if (t < n) st<float, CPL>(g + t * D, o);
+        for (int c = 0; c < 4; ++c) o[c] = neg_a[c] * softplus(x[c] + dtb[c]);
+        if (t < n && valid) stn(g + t * D, o);
     }
-    if (lane < n)
-        static_cast<float*>(a.beta)[(b * T + t0 + lane) * a.H + h] = sigmoid_f(decode_elem(rlogit, a.x_dtype));
+#pragma unroll
+    for (int e = 0; e < kB; ++e)
+        if (bv[e]) static_cast<float*>(a.beta)[(b * T + bt[e]) * a.H + bh[e]] = sigmoid_f(decode_elem(rl[e], a.x_dtype));
 }
 
-// One wave per (batch, tile, part, head), part 0..2 = q, k, v, 3 = gate
-// (nparts = 4, or 3 when the call leaves the gates to the core).  The host
-// keeps the number of units below 2^31, so the unit index is split with
-// 32-bit arithmetic.
-template <typename XT, int CPLK, int CPLV, int TILE>
-__global__ __launch_bounds__(256) void prep_kernel(const kda_prep_args a, uint32_t ntiles, uint32_t units,
-                                                   uint32_t nparts) {
+// Bound by memory from a few thousand tokens on (4.4-4.6 of the 5.2 TB/s of a
+// copy, reading three rows in sixteen twice).  us, two channels a lane and a
+// wave a head -> this, fp16 unless said: B=16 T=2048 H=16 d=128 bf16 210 -> 184;
+// B=4 T=2048 53.5 -> 44; B=1 T=1000 12.0 -> 8.8; a decode step at B=1 4.1 ->
+// 3.5, at B=64 5.6 -> 4.0.
+//
+// One wave per (batch, tile, kSeg channels of q, k, v and, unless the call
+// leaves the gates to the core, of the gate).  The host keeps the number of
+// units below 2^31, so the unit index is split with 32-bit arithmetic.
+template <typename XT, int K, int TILE>
+__global__ __launch_bounds__(256) void prep_kernel(const kda_prep_args a, uint32_t ntiles, uint32_t units) {
     const int lane = threadIdx.x & 63;
     const uint32_t unit = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= units) return;
     const uint32_t H = static_cast<uint32_t>(a.H);
-    uint32_t u = unit;
-    const int64_t h = u % H;
-    u /= H;
-    const int part = static_cast<int>(u % nparts);
-    u /= nparts;
-    const int64_t t0 = static_cast<int64_t>(u % ntiles) * TILE;
-    const int64_t b = u / ntiles;
-    if (part < 2)
-        conv_unit<XT, CPLK, TILE>(a, part, b, t0, h, lane);
-    else if (part == 2)
-        conv_unit<XT, CPLV, TILE>(a, 2, b, t0, h, lane);
-    else
-        gate_unit<XT, CPLK, TILE>(a, b, t0, h, lane);
+    const uint32_t segk = (H * K + kSeg<XT> - 1) / kSeg<XT>;
+    const uint32_t segv = (H * static_cast<uint32_t>(a.V) + kSeg<XT> - 1) / kSeg<XT>;
+    const uint32_t per = 2 * segk + segv + (a.g != nullptr ? (H * K + kGateSeg - 1) / kGateSeg : 0);
+    uint32_t s = unit % per;
+    const uint32_t bt = unit / per;
+    const int64_t t0 = static_cast<int64_t>(bt % ntiles) * TILE, b = bt / ntiles;
+    if (s < 2 * segk) {
+        const int i = s >= segk;
+        if (a.conv_size == 4) conv_unit<XT, K, TILE, 4>(a, i, b, t0, s - i * segk, lane);
+        else conv_unit<XT, K, TILE, 0>(a, i, b, t0, s - i * segk, lane);
+    } else if (s < 2 * segk + segv) {
+        if (a.conv_size == 4) conv_unit<XT, 0, TILE, 4>(a, 2, b, t0, s - 2 * segk, lane);
+        else conv_unit<XT, 0, TILE, 0>(a, 2, b, t0, s - 2 * segk, lane);
+    } else {
+        gate_unit<XT, K, TILE>(a, b, t0, s - 2 * segk - segv, lane);
+    }
 }
 
-// ---- output: one wave per (batch, head, tile of kOutRows tokens) -----------
-constexpr int kOutRows = 8;
+// ---- output: one wave per (batch, tile of tokens, kSeg channels) ------------
+// At copy rate from a few thousand tokens on; us at H=16 V=128 fp16, a wave a
+// head -> this: B=4 T=2048 19.9 -> 19.6 (bf16 21.0 -> 19.2), B=1 T=1000 4.8 ->
+// 3.9, a decode step at B=64 2.9 -> 2.5.  Units of 2 tokens where units of 8
+// leave SIMDs without two waves.
+constexpr int kOutRows = 8;      // tokens per unit (1 for a decode step)
 
-template <typename XT, int CPL>
+template <typename XT, int V, int TILE>
 __global__ __launch_bounds__(256) void output_kernel(const kda_output_args a, uint32_t ntiles, uint32_t units) {
+    constexpr int N = kLaneCh<XT>;
     const int lane = threadIdx.x & 63;
     const uint32_t unit = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= units) return;
-    const uint32_t H = static_cast<uint32_t>(a.H);
-    const int64_t h = unit % H;
-    const uint32_t bt = unit / H;
-    const int64_t t0 = static_cast<int64_t>(bt % ntiles) * kOutRows, b = bt / ntiles;
-    const int n = static_cast<int>((a.T - t0) < kOutRows ? (a.T - t0) : kOutRows);
-    const int64_t V = 64 * CPL;
-    const int64_t c0 = lane * CPL;
+    const uint32_t D = static_cast<uint32_t>(a.H) * V;
+    const uint32_t segs = (D + kSeg<XT> - 1) / kSeg<XT>;
+    const uint32_t ch = (unit % segs) * kSeg<XT> + N * lane, bt = unit / segs;
+    const bool valid = ch < D;
+    const int64_t c0 = valid ? ch : 0, h = c0 / V;
+    const int64_t t0 = static_cast<int64_t>(bt % ntiles) * TILE, b = bt / ntiles;
+    const int n = static_cast<int>((a.T - t0) < TILE ? (a.T - t0) : TILE);
 
     // every load first (rows past the end re-read the last token)
-    const XT* op = static_cast<const XT*>(a.o) + b * a.o_stride[0] + h * a.o_stride[2] + c0;
-    const XT* gp = static_cast<const XT*>(a.gate) + b * a.gate_stride[0] + h * V + c0;
-    float o[kOutRows][CPL], gt[kOutRows][CPL];
+    const XT* op = static_cast<const XT*>(a.o) + b * a.o_stride[0] + h * a.o_stride[2] + c0 % V;
+    const XT* gp = static_cast<const XT*>(a.gate) + b * a.gate_stride[0] + c0;
+    Raw<XT, N> o[TILE], gt[TILE];
 #pragma unroll
-    for (int r = 0; r < kOutRows; ++r) {
+    for (int r = 0; r < TILE; ++r) {
         const int64_t t = t0 + (r < n ? r : n - 1);
-        ld<XT, CPL>(op + t * a.o_stride[1], o[r]);
-        ld<XT, CPL>(gp + t * a.gate_stride[1], gt[r]);
+        o[r] = ldn<N>(op + t * a.o_stride[1]);
+        gt[r] = ldn<N>(gp + t * a.gate_stride[1]);
     }
-    RawElem rw[CPL];
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) rw[c] = load_raw_elem(a.weight, h * V + c0 + c, a.w_dtype);
-    float w[CPL];
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) w[c] = decode_elem(rw[c], a.w_dtype);
+    float w[N];
+    params<N>(a.weight, c0, a.w_dtype, w);
 
-    XT* yp = static_cast<XT*>(a.y) + (b * a.T + t0) * a.H * V + h * V + c0;
+    XT* yp = static_cast<XT*>(a.y) + (b * a.T + t0) * D + c0;
 #pragma unroll
-    for (int r = 0; r < kOutRows; ++r) {
-        float ss = 0.f;
+    for (int r = 0; r < TILE; ++r) {
+        float x[N], g[N], ss = 0.f;
+        unpack(o[r], x);
+        unpack(gt[r], g);
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) ss = fmaf(o[r][c], o[r][c], ss);
-        const float rstd = rsqrtf(wave_sum(ss) / static_cast<float>(V) + a.eps);
-        float y[CPL];
+        for (int c = 0; c < N; ++c) ss = fmaf(x[c], x[c], ss);
+        const float rstd = rsqrtf(lanes_sum<V / N>(ss) / static_cast<float>(V) + a.eps);
+        float y[N];
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) y[c] = round_to<XT>((o[r][c] * rstd) * w[c]) * sigmoid_f(gt[r][c]);
-        if (r < n) st<XT, CPL>(yp + r * a.H * V, y);
+        for (int c = 0; c < N; ++c) y[c] = round_to<XT>((x[c] * rstd) * w[c]) * sigmoid_f(g[c]);
+        if (r < n && valid) stn(yp + r * static_cast<int64_t>(D), y);
     }
 }
 
@@ -302,50 +356,64 @@ bool overlap(const void* a, int64_t na, const void* b, int64_t nb) {
     return a0 < b0 + static_cast<uintptr_t>(nb) && b0 < a0 + static_cast<uintptr_t>(na);
 }
 
-template <typename XT, int CPLK, int CPLV>
+// Tokens per unit: 16; 4 where units of 16 would leave SIMDs without a wave
+// (each also reads the conv_size - 1 rows before it; B=1 T=1000 H=16 K=128
+// without the gates 8.8 us, 9.9 in units of 8; B=2 T=2048 25 us in units of
+// 16, 30 in units of 4; with the gates, whose waves are shorter, B=4 T=2048 H=4
+// 24 us in units of 4 and 28.5 in units of 16); 1 for a decode step.  A conv
+// cache updated in place needs all its tokens in one unit, which then reads
+// the old rows before it writes the new ones: 8 or 16.
+template <typename XT, int K>
 void launch_prep(const kda_prep_args& a, hipStream_t stream) {
-    // a single token (the decode step) gets units of one token
-    const uint32_t nparts = a.g != nullptr ? 4u : 3u;
-    if (a.T == 1) {
-        const int64_t units = a.B * nparts * a.H;
-        hipLaunchKernelGGL((prep_kernel<XT, CPLK, CPLV, 1>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256),
-                           0, stream, a, 1u, static_cast<uint32_t>(units), nparts);
-        return;
-    }
-    const int64_t ntiles = (a.T + kTile - 1) / kTile;
-    const int64_t units = a.B * ntiles * nparts * a.H;
-    hipLaunchKernelGGL((prep_kernel<XT, CPLK, CPLV, kTile>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256),
-                       0, stream, a, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units), nparts);
+    const int64_t segk = (a.H * K + kSeg<XT> - 1) / kSeg<XT>, segv = (a.H * a.V + kSeg<XT> - 1) / kSeg<XT>;
+    const int64_t per = 2 * segk + segv + (a.g != nullptr ? (a.H * K + kGateSeg - 1) / kGateSeg : 0);
+    auto go = [&](auto tile) {
+        constexpr int TILE = decltype(tile)::value;
+        const int64_t ntiles = (a.T + TILE - 1) / TILE, units = a.B * ntiles * per;
+        hipLaunchKernelGGL((prep_kernel<XT, K, TILE>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
+                           stream, a, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units));
+    };
+    const int64_t kWaves = a.g != nullptr ? 4096 : 1280;
+    bool in_place = false;
+    for (int i = 0; i < 3; ++i) in_place = in_place || (a.hist_in[i] != nullptr && a.hist_in[i] == a.hist_out[i]);
+    const bool few = a.B * ((a.T + kTile - 1) / kTile) * per < kWaves;
+    if (a.T == 1) go(std::integral_constant<int, 1>{});
+    else if (few && (!in_place || a.T <= 4)) go(std::integral_constant<int, 4>{});
+    else if (few && a.T <= 8) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, kTile>{});
 }
 
 template <typename XT>
 int launch_prep_dims(const kda_prep_args& a, hipStream_t stream) {
-    const int ck = static_cast<int>(a.K / 64), cv = static_cast<int>(a.V / 64);
-    switch (ck * 10 + cv) {
-        case 11: launch_prep<XT, 1, 1>(a, stream); break;
-        case 12: launch_prep<XT, 1, 2>(a, stream); break;
-        case 14: launch_prep<XT, 1, 4>(a, stream); break;
-        case 21: launch_prep<XT, 2, 1>(a, stream); break;
-        case 22: launch_prep<XT, 2, 2>(a, stream); break;
-        case 24: launch_prep<XT, 2, 4>(a, stream); break;
-        case 41: launch_prep<XT, 4, 1>(a, stream); break;
-        case 42: launch_prep<XT, 4, 2>(a, stream); break;
-        case 44: launch_prep<XT, 4, 4>(a, stream); break;
+    switch (a.K) {
+        case 64: launch_prep<XT, 64>(a, stream); break;
+        case 128: launch_prep<XT, 128>(a, stream); break;
+        case 256: launch_prep<XT, 256>(a, stream); break;
         default: return KDA_ERR_UNSUPPORTED;
     }
     return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
 }
 
+template <typename XT, int V>
+void launch_output(const kda_output_args& a, hipStream_t stream) {
+    const int64_t segs = (a.H * V + kSeg<XT> - 1) / kSeg<XT>;
+    auto go = [&](auto tile) {
+        constexpr int TILE = decltype(tile)::value;
+        const int64_t ntiles = (a.T + TILE - 1) / TILE, units = a.B * ntiles * segs;
+        hipLaunchKernelGGL((output_kernel<XT, V, TILE>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
+                           stream, a, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units));
+    };
+    if (a.T == 1) go(std::integral_constant<int, 1>{});
+    else if (a.B * ((a.T + kOutRows - 1) / kOutRows) * segs < 2048) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, kOutRows>{});
+}
+
 template <typename XT>
 int launch_output_dims(const kda_output_args& a, hipStream_t stream) {
-    const int64_t ntiles = (a.T + kOutRows - 1) / kOutRows;
-    const int64_t units = a.B * ntiles * a.H;
-    const dim3 grid(static_cast<unsigned>((units + 3) / 4)), block(256);
-    const uint32_t nt = static_cast<uint32_t>(ntiles), nu = static_cast<uint32_t>(units);
     switch (a.V) {
-        case 64: hipLaunchKernelGGL((output_kernel<XT, 1>), grid, block, 0, stream, a, nt, nu); break;
-        case 128: hipLaunchKernelGGL((output_kernel<XT, 2>), grid, block, 0, stream, a, nt, nu); break;
-        case 256: hipLaunchKernelGGL((output_kernel<XT, 4>), grid, block, 0, stream, a, nt, nu); break;
+        case 64: launch_output<XT, 64>(a, stream); break;
+        case 128: launch_output<XT, 128>(a, stream); break;
+        case 256: launch_output<XT, 256>(a, stream); break;
         default: return KDA_ERR_UNSUPPORTED;
     }
     return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;

@@ -195,3 +195,67 @@ def test_prep_without_gates_matches_prep_with_gates(ops, T):
     assert g2 is None and b2 is None and g1 is not None
     for a, b in ((q1, q2), (k1, k2), (v1, v2)) + tuple((h1[n], h2[n]) for n in "qkv"):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [
+    (8, 1027, 8, 128, 64, 4),    # 16-token units, a ragged last one; V's 512 channels in one wave
+    (1, 1027, 5, 64, 64, 4),     # 4-token units; 320 channels: a wave with idle lanes
+    (2, 5, 3, 64, 256, 3),       # a second unit of one token; three taps
+])
+def test_prep_units_and_unaligned_rows(ops, dtype, shape):
+    """Every unit length, channel counts that leave lanes of the last wave
+    idle, and rows that start at an odd element (K = 64 only asks for element
+    alignment): the same bounds, and the same bits as contiguous inputs."""
+    B, T, H, K, V, cs = shape
+    xs, ws, bs, gk, a_log, dt_bias, beta_logit = make_prep_inputs(B, T, H, K, V, cs, dtype, seed=T + V)
+    kw = dict(num_heads=H, head_dim=K, value_head_dim=V, l2_eps=1e-6)
+    with torch.no_grad():
+        got = ops.kda_prep(*xs, ws, bs, gk, a_log, dt_bias, beta_logit, **kw)
+    ref = prep_ref(xs, ws, bs, gk, a_log, dt_bias, beta_logit, H, K, V, 1e-6)
+    for name, gt, rf in zip(("q", "k", "v", "g", "beta"), got[:5], ref):
+        ok, err = close(gt, rf, TOL[dtype] if name in "qkv" else 1e-5)
+        assert ok, (name, err)
+    if K == 64 and V == 64:
+        def cut(x):
+            wide = torch.full((*x.shape[:-1], x.shape[-1] + 3), float("nan"), device=DEV, dtype=x.dtype)
+            wide[..., 1:1 + x.shape[-1]] = x
+            return wide[..., 1:1 + x.shape[-1]]
+        with torch.no_grad():
+            odd = ops.kda_prep(*(cut(x) for x in xs), ws, bs, cut(gk), a_log, dt_bias, cut(beta_logit), **kw)
+        for a, b in zip(got[:5], odd[:5]):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T", [2, 5, 8, 9])
+def test_prep_in_place_cache_is_read_before_it_is_written(ops, T):
+    """The in-place cache at the lengths around its units' (4, 8, 16 tokens)."""
+    B, H, K, V, cs = 3, 2, 64, 64, 4
+    xs, ws, bs, gk, a_log, dt_bias, beta_logit = make_prep_inputs(B, T, H, K, V, cs, torch.bfloat16, seed=T)
+    hist = {n: torch.randn(B, cs - 1, H * K, generator=torch.Generator().manual_seed(i)).bfloat16().to(DEV)
+            for i, n in enumerate("qkv")}
+    kw = dict(num_heads=H, head_dim=K, value_head_dim=V, l2_eps=1e-6)
+    with torch.no_grad():
+        want = ops.kda_prep(*xs, ws, bs, gk, a_log, dt_bias, beta_logit, hist=hist, want_hist=True, **kw)
+        buf = {n: t.clone() for n, t in hist.items()}
+        got = ops.kda_prep(*xs, ws, bs, gk, a_log, dt_bias, beta_logit, hist=buf, hist_out=buf, **kw)
+    for a, b in zip(want[:5], got[:5]):
+        assert torch.equal(a, b)
+    for n in "qkv":
+        assert torch.equal(want[5][n], buf[n])
+
+
+@pytest.mark.parametrize("shape", [(4, 1100, 16, 128), (1, 1, 3, 64), (2, 3, 5, 128)])
+def test_output_units(ops, shape):
+    """Units of 8, 1 and 2 tokens; heads that leave lanes of the last wave idle."""
+    B, T, H, V = shape
+    gen = torch.Generator().manual_seed(T)
+    o = torch.randn(B, T, H, V, generator=gen).half()
+    gate = torch.randn(B, T, H * V, generator=gen).half()
+    w = (1 + 0.1 * torch.randn(H, V, generator=gen)).half()
+    with torch.no_grad():
+        y = ops.kda_output(o.to(DEV), gate.to(DEV), w.to(DEV), 1e-6)
+    n = head_rmsnorm_ref(o.float(), w.float(), 1e-6).half().float()
+    ref = (n * torch.sigmoid(gate.float().view(B, T, H, V))).reshape(B, T, H * V)
+    ok, err = close(y, ref, TOL[torch.float16])
+    assert ok, err
