@@ -7,10 +7,13 @@ if it is missing or was built for another ABI version, every call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libkda_hip.so"
+HOST_PATH = Path(__file__).resolve().parent / "_kda_host.so"     # csrc/host_binding.cpp
 ABI_VERSION = 14
 
 DTYPE_F32 = 0
@@ -151,7 +154,8 @@ EXPORTED_SYMBOLS = ("kda_chunkwise_fwd", "kda_recurrent_fwd", "kda_chunkwise_fwd
                     "kda_output_bwd", "kda_output_bwd_workspace_size", "kda_status_str", "kda_abi_version")
 
 _lib = None
-_lock = threading.Lock()
+_host = None
+_lock = threading.RLock()
 
 
 class NativeLibraryError(RuntimeError):
@@ -222,6 +226,36 @@ def load() -> ctypes.CDLL:
                 f"{LIB_PATH} has ABI version {version}, this wrapper expects {ABI_VERSION}; rebuild it")
         _lib = lib
         return lib
+
+
+def host():
+    """The native side of the wrapper (``csrc/host_binding.cpp``), bound to the
+    loaded library: each of its functions answers the common form of a call and
+    returns None for any other."""
+    global _host
+    if _host is not None:
+        return _host
+    with _lock:
+        if _host is not None:
+            return _host
+        lib = load()
+        if not HOST_PATH.exists():
+            raise NativeLibraryError(f"{HOST_PATH} not found: build it with __graft_entry__.build()")
+        import torch
+        loader = importlib.machinery.ExtensionFileLoader("_kda_host", str(HOST_PATH))
+        spec = importlib.util.spec_from_file_location("_kda_host", str(HOST_PATH), loader=loader)
+        try:
+            mod = importlib.util.module_from_spec(spec)
+            loader.exec_module(mod)
+        except ImportError as exc:
+            raise NativeLibraryError(f"cannot load {HOST_PATH}: {exc}") from exc
+        if mod.abi_version() != ABI_VERSION:
+            raise NativeLibraryError(f"{HOST_PATH} has ABI version {mod.abi_version()}, this wrapper expects "
+                                     f"{ABI_VERSION}; rebuild it")
+        mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in EXPORTED_SYMBOLS},
+                 torch._C._cuda_getCurrentRawStream)
+        _host = mod
+        return mod
 
 
 def status_str(code: int) -> str:

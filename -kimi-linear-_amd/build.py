@@ -18,6 +18,7 @@ REPO_DIR = PKG_DIR.parent
 CSRC = PKG_DIR / "csrc"
 INCLUDE = REPO_DIR / "include"
 LIB_PATH = PKG_DIR / "libkda_hip.so"
+HOST_PATH = PKG_DIR / "_kda_host.so"
 BUILD_DIR = PKG_DIR / "_build"
 
 SOURCES = ["kda_api.hip", "kda_recurrent.hip", "kda_chunkwise.hip", "kda_chunkwise_bwd.hip", "kda_layer_ops.hip",
@@ -51,8 +52,27 @@ def _run(cmd: list[str]) -> None:
         print(err, file=sys.stderr)
 
 
+def build_host(verbose: bool = False) -> Path:
+    """Compile the wrapper's native side (host code only) against torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(x for p in include_paths() for x in ("-isystem", p)), f"-I{sysconfig.get_paths()['include']}",
+           f"-I{INCLUDE}", str(CSRC / "host_binding.cpp"), "-o", str(tmp),
+           *(f"-L{p}" for p in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd))
+    _run(cmd)
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build_native(verbose: bool = False) -> Path:
-    """Compile every source for gfx950 and link the shared library."""
+    """Compile every source for gfx950, link the shared library and build the wrapper's native side."""
     hipcc = _hipcc()
     BUILD_DIR.mkdir(exist_ok=True)
     incs = [f"-I{INCLUDE}", f"-I{CSRC}"]
@@ -67,7 +87,9 @@ def build_native(verbose: bool = False) -> Path:
 
     workers = max(1, min(len(SOURCES), int(os.environ.get("MAX_JOBS", "4"))))
     with ThreadPoolExecutor(max_workers=workers) as pool:
+        host = pool.submit(build_host, verbose)
         objs = list(pool.map(compile_one, SOURCES))
+        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     if verbose:

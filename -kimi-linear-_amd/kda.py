@@ -91,6 +91,21 @@ def _strides3(x: torch.Tensor):
     return (ctypes.c_int64 * 3)(*x.stride()[:3])
 
 
+def _common(kind, q, k, v, g, beta, state, chunk_size, state_dtype, state_out=None, gate=(None, None),
+            epilogue=(None, None, 0.0), split=False):
+    """The call in native code if it has the common form (``_native.host``),
+    else None: anything to convert, copy, differentiate or refuse is
+    :func:`_forward`'s.  ``split``: let a long sequence run as segments."""
+    segments = 1
+    if split and isinstance(q, torch.Tensor) and isinstance(v, torch.Tensor) and q.dim() == 4 and v.dim() == 4:
+        segments = long_segments(*q.shape, v.shape[-1], v.dtype)
+    try:
+        return _native.host().core(kind == "recurrent", q, k, v, g, beta, state, chunk_size, state_dtype, state_out,
+                                   *gate, *epilogue, segments)
+    except TypeError:       # an argument of no type a common call has
+        return None
+
+
 def _forward(kind, q, k, v, g, beta, state, chunk_size, state_dtype, state_out=None, ckpt=False, gate=None,
              epilogue=None):
     """Shared forward.  ``ckpt=True`` (chunkwise, inside the autograd
@@ -403,6 +418,9 @@ def kda_chunkwise(q, k, v, g, beta, initial_state=None, chunk_size=64, tile_size
     Returns ``(o [B, T, H, V] in v.dtype, state [B, H, K, V] in state_dtype or v.dtype)``.
     """
     del tile_size
+    done = _common("chunkwise", q, k, v, g, beta, initial_state, int(chunk_size), state_dtype, split=True)
+    if done is not None:
+        return done
     inputs = [x for x in (q, k, v, g, beta, initial_state) if isinstance(x, torch.Tensor)]
     if torch.is_grad_enabled() and any(x.requires_grad for x in inputs):
         K, V = q.shape[-1], v.shape[-1]
@@ -470,6 +488,9 @@ def kda_recurrent(q, k, v, g, beta, state=None, state_dtype=None, *, state_out=N
     buffer.  It is returned as the second output.  Under autograd the state is
     always a new tensor: ``state_out`` is for loops that run without grad.
     """
+    done = _common("recurrent", q, k, v, g, beta, state, 0, state_dtype, state_out)
+    if done is not None:
+        return done
     inputs = [x for x in (q, k, v, g, beta, state) if isinstance(x, torch.Tensor)]
     if torch.is_grad_enabled() and any(x.requires_grad for x in inputs):
         K, V = q.shape[-1], v.shape[-1]
@@ -495,6 +516,10 @@ def kda_chunkwise_gated(q, k, v, gk, beta_logit, a_log, dt_bias, initial_state=N
     in that dtype (converted if they come in another); g and beta never exist
     in memory.  Forward only.  Returns ``(o, state)`` as ``kda_chunkwise``.
     """
+    done = _common("chunkwise", q, k, v, gk, beta_logit, initial_state, int(chunk_size), state_dtype,
+                   gate=(a_log, dt_bias)) if a_log is not None else None
+    if done is not None:
+        return done
     return _forward("chunkwise", q, k, v, gk, beta_logit, initial_state, int(chunk_size), state_dtype,
                     gate=(a_log, dt_bias))
 
@@ -503,6 +528,10 @@ def kda_recurrent_gated(q, k, v, gk, beta_logit, a_log, dt_bias, state=None, sta
                         state_out=None):
     """``kda_recurrent`` with the fused gate of :func:`kda_chunkwise_gated`
     (gate inputs in any float dtype).  ``state_out`` as in ``kda_recurrent``."""
+    done = _common("recurrent", q, k, v, gk, beta_logit, state, 0, state_dtype, state_out,
+                   gate=(a_log, dt_bias)) if a_log is not None else None
+    if done is not None:
+        return done
     return _forward("recurrent", q, k, v, gk, beta_logit, state, 0, state_dtype, state_out, gate=(a_log, dt_bias))
 
 
@@ -519,7 +548,12 @@ def kda_chunkwise_fused(q, k, v, gk, beta_logit, a_log, dt_bias, og, norm_weight
     [H, V]``.  fp16 / bf16 q, k, v; K and V in (64, 128).  Forward only.
     Returns ``(y [B, T, H*V] in v.dtype, state)``.
     """
-    o, s = _forward("chunkwise", q, k, v, gk, beta_logit, initial_state, int(chunk_size), state_dtype,
-                    gate=(a_log, dt_bias), epilogue=(og, norm_weight, eps))
+    done = None
+    if a_log is not None and og is not None:
+        done = _common("chunkwise", q, k, v, gk, beta_logit, initial_state, int(chunk_size), state_dtype,
+                       gate=(a_log, dt_bias), epilogue=(og, norm_weight, eps))
+    o, s = done if done is not None else _forward(
+        "chunkwise", q, k, v, gk, beta_logit, initial_state, int(chunk_size), state_dtype,
+        gate=(a_log, dt_bias), epilogue=(og, norm_weight, eps))
     B, T, H, V = o.shape
     return o.view(B, T, H * V), s

@@ -53,6 +53,7 @@ from types import SimpleNamespace
 import torch
 import torch.nn as nn
 
+from . import _native
 from .kda import (KdaError, kda_chunkwise, kda_chunkwise_fused, kda_chunkwise_gated, kda_recurrent,
                   kda_recurrent_gated, long_segments)
 from .layer_ops import kda_output, kda_output_train, kda_prep, kda_prep_train
@@ -188,7 +189,7 @@ class KimiDeltaAttention(nn.Module):
         call :meth:`refresh_fused_weight` after them."""
         mods = self._input_mods()
         params = [m.weight for m in mods] + [m.bias for m in mods if m.bias is not None]
-        key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in params)
+        key = _native.host().params_key(params)
         if self._wcat is not None and self._wcat[0] == key:
             return self._wcat[1], self._wcat[2]
         with torch.no_grad():
@@ -226,7 +227,7 @@ class KimiDeltaAttention(nn.Module):
         gated core (the reference casts them to fp32 too, ``kda.py:458-459``);
         cached like :meth:`_input_weight` and refilled in place."""
         params = (self.A_log, self.dt_bias)
-        key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in params)
+        key = _native.host().params_key(params)
         if self._gcat is not None and self._gcat[0] == key:
             return self._gcat[1], self._gcat[2]
         with torch.no_grad():

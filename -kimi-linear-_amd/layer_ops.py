@@ -79,6 +79,18 @@ def kda_prep(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta_logit, *
     points (:func:`kimi_linear_amd.kda.kda_chunkwise_gated`).
     """
     H, K, V = int(num_heads), int(head_dim), int(value_head_dim)
+    three = lambda d: (None, None, None) if d is None else (d["q"], d["k"], d["v"])  # noqa: E731
+    try:
+        done = _native.host().prep((q_in, k_in, v_in), conv_w, conv_b, gk, a_log, dt_bias, beta_logit, H, K, V,
+                                   float(l2_eps), three(hist), three(hist_out), bool(want_hist))
+    except TypeError:       # an argument of no type a common call has
+        done = None
+    if done is not None:
+        q, k, v, g, beta, new = done
+        if want_hist:
+            return q, k, v, g, beta, dict(zip("qkv", new))
+        return q, k, v, g, beta, hist_out
+    # the general path: copies what has another layout, says what is wrong
     if q_in.dim() != 3:
         raise KdaError(f"q_in must be [B, T, H*K], got {list(q_in.shape)}")
     B, T = q_in.shape[0], q_in.shape[1]
@@ -186,6 +198,12 @@ def kda_output(o, gate, weight, eps):
     ``o: [B, T, H, V]``, ``gate: [B, T, H*V]`` (same dtype), ``weight: [H, V]``.
     Returns ``[B, T, H*V]``.
     """
+    try:
+        y = _native.host().output(o, gate, weight, float(eps))
+    except TypeError:       # an argument of no type a common call has
+        y = None
+    if y is not None:
+        return y
     if o.dim() != 4:
         raise KdaError(f"o must be [B, T, H, V], got {list(o.shape)}")
     B, T, H, V = o.shape

@@ -1,0 +1,165 @@
+"""The wrapper's native side (``csrc/host_binding.cpp``) against its general
+path: the same bits for every call it answers, and None -- the general path's
+case -- for every call with something to convert, copy, differentiate, trace
+or refuse."""
+
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def kda(kda_pkg):
+    return importlib.import_module("kimi_linear_amd.kda")
+
+
+@pytest.fixture(scope="module")
+def host(kda_pkg):
+    return importlib.import_module("kimi_linear_amd._native").host()
+
+
+def inputs(dtype, B=2, T=64, H=2, K=64, V=64, gate=torch.float32, device=DEV):
+    wl = importlib.import_module("kimi_linear_amd.workloads")
+    i = wl.make_inputs(B, T, H, K, V, device=device, seed=5, qkv_dtype=dtype, gate_dtype=gate, state_std=0.05)
+    return [i[n] for n in ("q", "k", "v", "g", "beta")], i["state"]
+
+
+def call(host, args, state=None, recurrent=False, chunk=32, state_dtype=torch.float32, state_out=None,
+         gate=(None, None), epilogue=(None, None, 0.0), segments=1):
+    return host.core(recurrent, *args, state, chunk, state_dtype, state_out, *gate, *epilogue, segments)
+
+
+def test_declines_what_is_not_a_plain_device_tensor(host):
+    args, state = inputs(torch.float16, device="cpu")
+    assert call(host, args) is None                                       # no HIP device
+    assert call(host, [x.to("meta") for x in args]) is None
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode():
+        fake = [torch.empty(x.shape, dtype=x.dtype, device="cuda") for x in args]
+        assert call(host, fake) is None                                   # a dispatch mode is active
+    assert call(host, fake) is None                                       # a tensor subclass outside it
+    with pytest.raises(TypeError):
+        call(host, [None, *args[1:]])
+    seen = []
+
+    def f(x):
+        seen.append(call(host, [x, *args[1:]]))
+        return x.sum()
+    torch.vmap(f)(torch.stack([args[0]] * 2))
+    assert seen == [None]
+
+
+def test_params_key_follows_every_change(host):
+    a, b = torch.zeros(4), torch.zeros(4)
+    k0 = host.params_key([a, b])
+    assert host.params_key([a, b]) == k0
+    a.add_(1)
+    assert host.params_key([a, b]) != k0
+    k1 = host.params_key([a, b])
+    assert host.params_key([a, b.clone()]) != k1 and host.params_key([b, a]) != k1
+    assert host.params_key([a, a.view(torch.int32)]) != host.params_key([a, a])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,gate", [(torch.float16, torch.float32), (torch.bfloat16, torch.float32),
+                                        (torch.float32, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("kind", ["chunkwise", "recurrent"])
+def test_same_bits_as_the_general_path(kda, host, dtype, gate, kind):
+    args, state = inputs(dtype, gate=gate)
+    rec = kind == "recurrent"
+    forms = {
+        "plain": args,
+        "body": [x[:, :32] for x in args],                                # token rows of a longer buffer
+        "heads": [x.transpose(1, 2).contiguous().transpose(1, 2) for x in args],   # head-major memory
+        "batch": [x[1:] for x in args],
+    }
+    with torch.no_grad():
+        for name, a in forms.items():
+            B = a[0].shape[0]
+            for st in (None, state[:B].contiguous(), state[:B].half()):
+                for sd in (torch.float32, torch.bfloat16, None):
+                    got = call(host, a, st, rec, state_dtype=sd)
+                    if not rec and gate is not torch.float32:
+                        assert got is None                                # the chunk pipeline reads fp32 gates
+                        continue
+                    want = kda._forward(kind, *a, st, 32, sd)
+                    assert got is not None, name
+                    assert got[0].dtype == want[0].dtype and got[1].dtype == want[1].dtype
+                    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), name
+
+
+@pytest.mark.gpu
+def test_declines_what_needs_the_general_path(kda, host):
+    args, state = inputs(torch.float16)
+    q, k, v, g, beta = args
+    none = lambda *a, **kw: call(host, *a, **kw) is None                  # noqa: E731
+    with torch.no_grad():
+        assert none([q.float(), k, v, g, beta])                           # q in another type
+        assert none([q.double(), k.double(), v.double(), g, beta])
+        assert none([q, k, v, g.half(), beta])                            # the chunk pipeline reads fp32 gates
+        assert none([q[..., ::2], k[..., ::2], v, g[..., ::2], beta])     # strided channels
+        assert none([q[:, :1].expand(-1, 64, -1, -1), k, v, g, beta])     # broadcast token rows
+        assert none([q, k, v, g, beta[:, :1].expand(-1, 64, -1)])
+        assert none(args, state.transpose(2, 3))                          # a state of other strides
+        assert none(args, state.double())
+        assert none(args, chunk=48) and none(args, chunk=0)               # T % chunk != 0
+        assert none(args, state_dtype=torch.float64)
+        assert none([q, k[:, :32], v, g, beta]) and none([q, k, v, g, beta[..., :1]])
+        assert none([q, k, v.cpu(), g, beta])
+        assert none(args, state, state_out=state)                         # in place is the recurrence's
+        assert not none(args, state, recurrent=True, state_out=state.clone())
+        assert none(args, state, recurrent=True, state_out=state.half())
+        both = torch.empty(state.numel() + 8, device=DEV)
+        a, b = both[:-8].view(state.shape), both[8:].view(state.shape)
+        assert none(args, a, recurrent=True, state_out=b)                 # partial overlap
+        assert none([x[:0] for x in args]) and none([x[..., :48] for x in (q, k)] + [v, g[..., :48], beta])
+        assert not none(args)
+    qg = q.clone().requires_grad_()
+    assert none([qg, k, v, g, beta])
+    with torch.no_grad():
+        assert not none([qg, k, v, g, beta])
+    import torch.autograd.forward_ad as fwad
+    with fwad.dual_level():
+        assert none([fwad.make_dual(q, torch.ones_like(q)), k, v, g, beta])
+
+
+@pytest.mark.gpu
+def test_layer_kernels_match_their_general_path(kda_pkg, monkeypatch):
+    """kda_prep and kda_output through the native side and with it turned off."""
+    ops = importlib.import_module("kimi_linear_amd.layer_ops")
+    B, T, H, K, V = 2, 21, 2, 64, 128
+    gen = torch.Generator().manual_seed(1)
+    rn = lambda *s: torch.randn(*s, generator=gen).half().to(DEV)          # noqa: E731
+    big = rn(B, T, 3 * H * K + H * V + H)
+    x = big.split((H * K, H * K, H * V, H * K, H), -1)
+    w = [rn(D, 1, 4) for D in (H * K, H * K, H * V)]
+    bias = [rn(H * K), None, rn(H * V)]
+    al, dt = rn(H, K).float(), rn(H, K).float()
+    hist = dict(zip("qkv", (rn(B, 3, D) for D in (H * K, H * K, H * V))))
+    o, wn = rn(B, T, H, V), rn(H, V)
+
+    def run():
+        with torch.no_grad():
+            out = [ops.kda_prep(*x[:3], w, bias, gk, al, dt, x[4], num_heads=H, head_dim=K, value_head_dim=V,
+                                l2_eps=1e-6, hist=h, want_hist=wh)
+                   for gk in (None, x[3]) for h in (None, hist) for wh in (False, True)]
+            return out, ops.kda_output(o, big[..., :H * V], wn, 1e-6)
+
+    got, y = run()
+
+    class Off:
+        prep = output = staticmethod(lambda *a: None)
+    monkeypatch.setattr(ops._native, "host", lambda: Off)
+    want, y2 = run()
+    assert torch.equal(y, y2)
+    for a, b in zip(got, want):
+        for p, r in zip(a, b):
+            if isinstance(r, dict):
+                assert all(torch.equal(p[n], r[n]) for n in "qkv")
+            else:
+                assert (p is None and r is None) or torch.equal(p, r)
