@@ -150,6 +150,7 @@ EXPORTED_SYMBOLS = ("kda_chunkwise_fwd", "kda_recurrent_fwd", "kda_chunkwise_fwd
                     "kda_chunkwise_long_fwd", "kda_chunkwise_long_workspace_size",
                     "kda_chunkwise_bwd",
                     "kda_chunkwise_bwd_workspace_size", "kda_chunkwise_bwd_noalloc",
+                    "kda_chunkwise_split_fwd", "kda_chunkwise_split_workspace_size",
                     "kda_prep_fwd", "kda_output_fwd", "kda_prep_bwd", "kda_prep_bwd_workspace_size",
                     "kda_output_bwd", "kda_output_bwd_workspace_size", "kda_status_str", "kda_abi_version")
 
@@ -188,11 +189,13 @@ def load() -> ctypes.CDLL:
         for name in ("kda_chunkwise_gated_fwd", "kda_recurrent_gated_fwd"):
             getattr(lib, name).argtypes = [ctypes.POINTER(KdaFwdArgs), ctypes.POINTER(KdaGateArgs), ctypes.c_void_p]
             getattr(lib, name).restype = ctypes.c_int
-        lib.kda_chunkwise_long_fwd.argtypes = [ctypes.POINTER(KdaFwdArgs), ctypes.c_int64, ctypes.c_void_p,
-                                               ctypes.c_void_p]
-        lib.kda_chunkwise_long_fwd.restype = ctypes.c_int
-        lib.kda_chunkwise_long_workspace_size.argtypes = [ctypes.c_int64] * 6
-        lib.kda_chunkwise_long_workspace_size.restype = ctypes.c_size_t
+        for name in ("kda_chunkwise_long_fwd", "kda_chunkwise_split_fwd"):
+            getattr(lib, name).argtypes = [ctypes.POINTER(KdaFwdArgs), ctypes.c_int64, ctypes.c_void_p,
+                                           ctypes.c_void_p]
+            getattr(lib, name).restype = ctypes.c_int
+        for name in ("kda_chunkwise_long_workspace_size", "kda_chunkwise_split_workspace_size"):
+            getattr(lib, name).argtypes = [ctypes.c_int64] * 6
+            getattr(lib, name).restype = ctypes.c_size_t
         lib.kda_chunkwise_fused_fwd.argtypes = [ctypes.POINTER(KdaFwdArgs), ctypes.POINTER(KdaGateArgs),
                                                 ctypes.POINTER(KdaOutEpilogue), ctypes.c_void_p]
         lib.kda_chunkwise_fused_fwd.restype = ctypes.c_int

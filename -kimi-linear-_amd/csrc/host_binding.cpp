@@ -41,6 +41,8 @@ struct Fns {
     decltype(&kda_chunkwise_fused_fwd) fused = nullptr;
     decltype(&kda_chunkwise_long_fwd) long_fwd = nullptr;
     decltype(&kda_chunkwise_long_workspace_size) long_ws = nullptr;
+    decltype(&kda_chunkwise_split_fwd) split_fwd = nullptr;
+    decltype(&kda_chunkwise_split_workspace_size) split_ws = nullptr;
     decltype(&kda_prep_fwd) prep = nullptr;
     decltype(&kda_output_fwd) output = nullptr;
 };
@@ -62,6 +64,8 @@ void bind(const py::dict& addr, const py::object& stream_fn) {
     take(fn.fused, addr, "kda_chunkwise_fused_fwd");
     take(fn.long_fwd, addr, "kda_chunkwise_long_fwd");
     take(fn.long_ws, addr, "kda_chunkwise_long_workspace_size");
+    take(fn.split_fwd, addr, "kda_chunkwise_split_fwd");
+    take(fn.split_ws, addr, "kda_chunkwise_split_workspace_size");
     take(fn.prep, addr, "kda_prep_fwd");
     take(fn.output, addr, "kda_output_fwd");
     Py_INCREF(stream_fn.ptr());
@@ -210,8 +214,11 @@ py::object core(bool recurrent, const Tensor& q, const Tensor& k, const Tensor& 
     int status;
     Tensor keep;                                     // alive until the launches that read it are enqueued
     if (segments > 1) {
-        keep = at::empty({static_cast<int64_t>(fn.long_ws(B, T, H, K, V, segments))}, v.options().dtype(at::kByte));
-        status = fn.long_fwd(&a, segments, keep.data_ptr(), stream);
+        // the form whose transition columns end when they are zero, where there is one
+        const size_t split = fn.split_ws(B, T, H, K, V, segments);
+        const size_t bytes = split != 0 ? split : fn.long_ws(B, T, H, K, V, segments);
+        keep = at::empty({static_cast<int64_t>(bytes)}, v.options().dtype(at::kByte).requires_grad(false));
+        status = (split != 0 ? fn.split_fwd : fn.long_fwd)(&a, segments, keep.data_ptr(), stream);
     } else if (og) {
         keep = weight->detach().to(at::kFloat).contiguous();
         kda_out_epilogue e{};

@@ -413,10 +413,16 @@ __device__ __forceinline__ f4 mm_f32(const f4& xt, const f4& y, f4 c) {
 // the identity and see v = 0 -- beside the V columns of its own state from
 // zero; no o is written, unless TOUT: then the outputs of every state column
 // are written in fp32, those of the V columns (the outputs from a zero
-// initial state) to o, those of the transition columns (per token, the
-// coefficients of the initial state in the outputs) to a second buffer.
+// initial state) to long_out.oz, those of the transition columns (per token,
+// the coefficients of the initial state in the outputs) to long_out.c.
+// kToutBoth: both kinds of column in one launch.  Or two launches: the
+// transition columns (kToutTrans), whose workgroup ends once its columns are
+// all zero (they stay zero, and the coefficients with them) and leaves the
+// number of chunks it wrote in long_out.n; then the V columns (kToutV), whose
+// outputs past those chunks are final and go to o in its own type.
+enum { kToutBoth = 1, kToutTrans = 2, kToutV = 3 };
 template <int K, int NC, typename TQ, bool GATED, int CG = 1, bool EPI = false, bool TRANS = false,
-          bool TOUT = false, bool CKPT = false>
+          int TOUT = 0, bool CKPT = false>
 struct Kern {
     static constexpr int KT = K / 16;                   // 16-row state tiles
     static constexpr int KU = K / 32;                   // 32-wide k blocks
@@ -474,7 +480,8 @@ struct Kern {
     // consumers' loop keeps an exact count of its outstanding vector memory
     // operations; the other kernels have no record stores at all.
     static constexpr bool kFlatRec = CKPT && Elem<TQ>::code == KDA_DTYPE_F16;
-    float* cout = nullptr;                   // TOUT: the transition columns' outputs [B, T, H, K]
+    long_out lo{};                           // TOUT
+    int nz = 0;                              // TOUT: blocks whose V outputs go to oz; later ones go to o
     int nblk = 0;                            // blocks of the real chunks (records exist for these)
 
     // A, L, N of the chunk holding block blk (row-major 32 x 32, consecutive)
@@ -982,7 +989,7 @@ struct Kern {
     static constexpr bool RANGE = Elem<TQ>::code == KDA_DTYPE_BF16;
     mutable float sig = 1.f, isig = 1.f;
     __device__ void v_load(uint32_t (&vr)[VW], int chunk, int grp) const {
-        if (TRANS && vzero) {
+        if (TOUT == kToutTrans || (TRANS && TOUT != kToutV && vzero)) {
 #pragma unroll
             for (int i = 0; i < VW; ++i) vr[i] = 0u;
             return;
@@ -1084,7 +1091,8 @@ struct Kern {
         const auto s1 = __builtin_amdgcn_permlane16_swap(px[1], py[1], false, false);
         __builtin_amdgcn_raw_buffer_store_b128(u4{s0[0], s1[0], s0[1], s1[1]}, r, vo, 0, 0);
     }
-    __device__ void store_chunk(const f4 (&O)[CG][CB], int blk, int64_t colw) const {
+    // on = false: stores of an empty range
+    __device__ void store_chunk(const f4 (&O)[CG][CB], int blk, int64_t colw, bool on = true) const {
         static_assert(CG == 1 || CG == 2, "output tiles of one or two column groups");
         if constexpr (sizeof(TQ) == 4) {
 #pragma unroll
@@ -1099,7 +1107,7 @@ struct Kern {
             if constexpr (CG == 1) {
                 // lane group lg: row ln of block lg % 2, columns 8 (lg / 2) ..
                 const auto r = make_rsrc(static_cast<TQ*>(a.o) + e,
-                                         static_cast<uint32_t>((rows_in(blk) + rows_in(blk + 1)) * rs * es));
+                                         on ? static_cast<uint32_t>((rows_in(blk) + rows_in(blk + 1)) * rs * es) : 0u);
                 const int vo = static_cast<int>(((ln + BT * (lg & 1)) * rs + colw + 8 * (lg >> 1)) * es);
                 store_pair(O[0][0], O[0][1], r, vo);
             } else {
@@ -1108,25 +1116,25 @@ struct Kern {
 #pragma unroll
                 for (int bk = 0; bk < CB; ++bk) {
                     const auto r = make_rsrc(static_cast<TQ*>(a.o) + e + BT * bk * rs,
-                                             static_cast<uint32_t>(rows_in(blk + bk) * rs * es));
+                                             on ? static_cast<uint32_t>(rows_in(blk + bk) * rs * es) : 0u);
                     store_pair(O[0][bk], O[1][bk], r, vo);
                 }
             }
         }
     }
 
-    // TOUT: a chunk's outputs in fp32, the V columns' to o ([B, T, H, V]
-    // fp32), the transition columns' to cout ([B, T, H, K]); the choice is
-    // wave-uniform and taken by selecting the base, not by a branch.
+    // TOUT: a chunk's outputs in fp32, the V columns' to oz ([B, T, H, V]),
+    // the transition columns' to c ([B, T, H, K]); the choice is uniform over
+    // the workgroup and taken by selecting the base, not by a branch.
     __device__ void store_fp32_chunk(const f4 (&O)[CG][CB], int blk, int64_t colw) const {
-        const bool tr = vzero;
-        float* base = tr ? cout : static_cast<float*>(a.o);
+        const bool tr = vzero, on = TOUT != kToutV || blk < nz;
+        float* base = tr ? lo.c : lo.oz;
         const int64_t W = tr ? K : a.V, col = tr ? colw - a.V : colw;
         const int64_t rs = a.H * W;
         const int64_t e = (b * T + static_cast<int64_t>(blk) * BT) * rs + h * W;
 #pragma unroll
         for (int bk = 0; bk < CB; ++bk) {
-            const auto r = make_rsrc(base + e + BT * bk * rs, static_cast<uint32_t>(rows_in(blk + bk) * rs * 4));
+            const auto r = make_rsrc(base + e + BT * bk * rs, on ? static_cast<uint32_t>(rows_in(blk + bk) * rs * 4) : 0u);
 #pragma unroll
             for (int g = 0; g < CG; ++g)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, O[g][bk]), r,
@@ -1395,6 +1403,7 @@ struct Kern {
             pd.blk = blk;
         } else if constexpr (TOUT) {
             store_fp32_chunk(O, blk, colw);
+            if constexpr (TOUT == kToutV) store_chunk(O, blk, colw, blk >= nz);
         } else if constexpr (!TRANS) {
             store_chunk(O, blk, colw);
         }
@@ -1423,17 +1432,18 @@ struct Kern {
 // barriers; every prefetch is issued unconditionally (a block past T loads
 // zeros).  The chunks cover T rounded up to whole chunks: a padded block
 // (all rows past T) is neutral and is built like any other.
-// ckpt: CKPT, the chunk records; TOUT, the transition columns' outputs.
+// ckpt: CKPT, the chunk records; lout: TOUT, where the first pass writes.
 template <int K, int NC, typename TQ, bool GATED, int CG = 1, bool EPI = false, bool TRANS = false, bool CKPT = false,
-          bool TOUT = false>
+          int TOUT = 0>
 __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd_args a, float* ckpt,
                                                                    const kda_gate_args gate,
-                                                                   const kda_out_epilogue epi) {
-    static_assert(!TOUT || TRANS, "fp32 outputs belong to the transition pass");
+                                                                   const kda_out_epilogue epi, const long_out lout) {
+    static_assert(TOUT == 0 || TRANS, "fp32 outputs belong to the transition pass");
     using KN = Kern<K, NC, TQ, GATED, CG, EPI, TRANS, TOUT, CKPT>;
     constexpr int KT = KN::KT, VT = KN::VT, CH = KN::CH;
     static_assert(K % 32 == 0 && K <= 128, "chunkwise supports K in {32, 64, 128}");
     __shared__ Smem<K, CG, EPI> sm;
+    __shared__ int alive[2];         // kToutTrans: a column was not zero after superstep s (slot s % 2)
     KN kn(a, sm);
     if constexpr (EPI) {
         kn.og = epi.gate;
@@ -1444,13 +1454,15 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
 
     const int64_t H = a.H, V = a.V;
     const int64_t VS = V + (TRANS ? K : 0);             // state columns
-    const int nvt = static_cast<int>(VS / VT);
     // XCD-aware order: workgroups are dealt round-robin over the 8 XCDs, so
     // renumber them to put consecutive logical workgroups -- the V-tiles of
     // one head, which all read the head's q, k and g -- on one XCD and its L2.
     int bid = blockIdx.x;
     if (gridDim.x % kXcds == 0) bid = (bid % kXcds) * (gridDim.x / kXcds) + bid / kXcds;
-    const int vt = bid % nvt;
+    // the tiles of a head in this launch, and the first of them
+    const int nvt = static_cast<int>((TOUT == kToutTrans ? K : (TOUT == kToutV ? V : VS)) / VT);
+    const int first = TOUT == kToutTrans ? static_cast<int>(V / VT) : 0;
+    const int tile = bid % nvt, vt = first + tile;
     bid /= nvt;
     kn.h = bid % H;
     kn.b = bid / H;
@@ -1471,8 +1483,17 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
     if constexpr (CKPT) {
         if (ckpt != nullptr && vt == 0) kn.ckm = ckpt + (kn.b * H + kn.h) * ncc * ckpt_record(K, V);
     }
-    if constexpr (TOUT) kn.cout = ckpt;
+    if constexpr (TOUT != 0) kn.lo = lout;
     const int nss = (ncc + NCH - 1) / NCH;               // supersteps
+    if constexpr (TOUT == kToutV) {
+        int n = 0;
+        const int nt = K / static_cast<int>(trans_tile(K, V));
+        for (int i = 0; i < nt; ++i) {
+            const int x = lout.n[(kn.b * H + kn.h) * nt + i];
+            n = x > n ? x : n;
+        }
+        kn.nz = __builtin_amdgcn_readfirstlane(CB * n);
+    }
 
     const bool consumer = wave < NC;
     // consumer state: S[g][t][j] = S[16t + 4lg + j][colw + 16g + ln]
@@ -1531,7 +1552,8 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
             if constexpr (!EPI && (!CKPT || KN::kFlatRec) && (!TRANS || TOUT)) {
                 // (distinct offsets: identical stores would be merged away;
                 // flat records: the chunk's state and R stores as well)
-                constexpr int ns = TOUT ? CB * CG : KN::kOutStores + (CKPT ? CG * (KN::KT + CB) * 4 : 0);
+                constexpr int ns = (TOUT ? CB * CG : 0) + (TOUT == 0 || TOUT == kToutV ? KN::kOutStores : 0) +
+                                   (CKPT ? CG * (KN::KT + CB) * 4 : 0);
                 const auto none = make_rsrc(a.o, 0u);
 #pragma unroll
                 for (int i = 0; i < ns; ++i)
@@ -1585,9 +1607,11 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
                 }
             }
         };
+        if (TOUT == kToutTrans && threadIdx.x == 0) alive[0] = 0;
         __syncthreads();
         solve_next(-1);
         __syncthreads();
+        int done = nss;                                  // supersteps run
         for (int s = 0; s < nss; ++s) {
 #pragma unroll
             for (int cj = 0; cj < NCH; ++cj) {
@@ -1597,7 +1621,24 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
                                                      : nullptr;
                 kn.consume(sm.set[s & 1][cj], NB * s + CB * cj, vr[cj], vt, S, colw, ck, pd[cj], wave);
             }
+            if constexpr (TOUT == kToutTrans) {
+                bool on = false;
+#pragma unroll
+                for (int g = 0; g < CG; ++g)
+#pragma unroll
+                    for (int t = 0; t < KT; ++t)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) on = on || !(S[g][t][j] == 0.f);
+                if (__any(on) && kn.lane == 0) alive[s & 1] = 1;
+            }
             __syncthreads();
+            if constexpr (TOUT == kToutTrans) {
+                if (threadIdx.x == 0) alive[(s + 1) & 1] = 0;
+                if (__builtin_amdgcn_readfirstlane(alive[s & 1]) == 0) {   // every wave reads the same
+                    done = s + 1;
+                    break;
+                }
+            }
             if constexpr (EPI) {
 #pragma unroll
                 for (int cj = 0; cj < NCH; ++cj)
@@ -1605,6 +1646,10 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
             }
             solve_next(s);
             __syncthreads();
+        }
+        if constexpr (TOUT == kToutTrans) {
+            if (threadIdx.x == 0)
+                lout.n[(kn.b * H + kn.h) * (K / VT) + tile] = NCH * done < ncc ? NCH * done : ncc;
         }
         // a null state_out (the output pass of a split long sequence) keeps no final state
         if (a.state_out != nullptr) {
@@ -1639,6 +1684,9 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
             ChunkOps<K>& co = sm.set[(s + 1) & 1][p / CB];
             if (s + 1 < nss) kn.phase1(raw, w, p, co, blk + NB);
             __syncthreads();
+            if constexpr (TOUT == kToutTrans) {
+                if (s >= 0 && __builtin_amdgcn_readfirstlane(alive[s & 1]) == 0) break;
+            }
             if (s + 1 < nss) kn.phase2(p, blk, co);
             __syncthreads();
         }
@@ -1646,28 +1694,47 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
 }
 
 template <int K, int NC, typename TQ, bool GATED, int CG = 1, bool EPI = false, bool TRANS = false, bool CKPT = false,
-          bool TOUT = false>
+          int TOUT = 0>
 int launch_knq(const kda_fwd_args& a, hipStream_t stream, float* ckpt, const kda_gate_args& gate,
-               const kda_out_epilogue& epi = kda_out_epilogue{}) {
-    const int64_t blocks = a.B * a.H * ((a.V + (TRANS ? K : 0)) / (16 * NC * CG));
+               const kda_out_epilogue& epi = kda_out_epilogue{}, const long_out& lout = long_out{}) {
+    const int64_t cols = TOUT == kToutTrans ? K : (TRANS && TOUT != kToutV ? a.V + K : a.V);
+    const int64_t blocks = a.B * a.H * (cols / (16 * NC * CG));
     hipLaunchKernelGGL((chunkwise_kernel<K, NC, TQ, GATED, CG, EPI, TRANS, CKPT, TOUT>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(64 * (NC + NB)), 0, stream, a, ckpt, gate, epi);
+                       dim3(64 * (NC + NB)), 0, stream, a, ckpt, gate, epi, lout);
     return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
 }
 
 // The first pass of a split long sequence: 64-column tiles over the V state
 // columns and the K transition columns (128-column tiles when they would
-// outnumber the CUs).
+// outnumber the CUs).  With outputs in two launches (lout->part), tiles of
+// trans_tile() columns over one kind.
 template <int K, typename TQ>
-int launch_trans(const kda_fwd_args& a, hipStream_t stream, float* cout) {
+int launch_trans(const kda_fwd_args& a, hipStream_t stream, const long_out* lout) {
     const kda_gate_args none{nullptr, nullptr};
-    const bool wide = a.B * a.H * ((a.V + K) / 64) > 256 && (a.V + K) % 128 == 0;
-    if (cout != nullptr) {
-        if (wide) return launch_knq<K, 4, TQ, false, 2, false, true, false, true>(a, stream, cout, none);
-        return launch_knq<K, 4, TQ, false, 1, false, true, false, true>(a, stream, cout, none);
+    auto go = [&](auto cg, auto tout) {
+        constexpr int CG = decltype(cg)::value, TOUT = decltype(tout)::value;
+        return launch_knq<K, 4, TQ, false, CG, false, true, false, TOUT>(a, stream, nullptr, none, {},
+                                                                         lout ? *lout : long_out{});
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    if (lout != nullptr && lout->part != long_out::kBoth) {
+        const bool trans = lout->part == long_out::kTrans;
+        if constexpr (K == 128) {
+            if (trans_tile(K, a.V) == 128)
+                return trans ? go(I2{}, std::integral_constant<int, kToutTrans>{})
+                             : go(I2{}, std::integral_constant<int, kToutV>{});
+        }
+        return trans ? go(I1{}, std::integral_constant<int, kToutTrans>{})
+                     : go(I1{}, std::integral_constant<int, kToutV>{});
     }
-    if (wide) return launch_knq<K, 4, TQ, false, 2, false, true>(a, stream, nullptr, none);
-    return launch_knq<K, 4, TQ, false, 1, false, true>(a, stream, nullptr, none);
+    const bool wide = a.B * a.H * ((a.V + K) / 64) > 256 && (a.V + K) % 128 == 0;
+    if (lout != nullptr) {
+        using Both = std::integral_constant<int, kToutBoth>;
+        return wide ? go(I2{}, Both{}) : go(I1{}, Both{});
+    }
+    return wide ? go(I2{}, I0{}) : go(I1{}, I0{});
 }
 
 // The fused output epilogue: one workgroup per (b, h), 4 consumer waves of
@@ -1808,13 +1875,13 @@ bool chunkwise_trans_supported(const kda_fwd_args& a) {
            (a.qkv_dtype == KDA_DTYPE_F16 || a.qkv_dtype == KDA_DTYPE_BF16);
 }
 
-int chunkwise_trans_launch(const kda_fwd_args& a, hipStream_t stream, float* cout) {
+int chunkwise_trans_launch(const kda_fwd_args& a, hipStream_t stream, const long_out* lout) {
     const int st = chunkwise_check(a, false);
     if (st != KDA_OK) return st;
     if (!chunkwise_trans_supported(a)) return KDA_ERR_UNSUPPORTED;
     if (a.qkv_dtype == KDA_DTYPE_F16)
-        return a.K == 64 ? launch_trans<64, _Float16>(a, stream, cout) : launch_trans<128, _Float16>(a, stream, cout);
-    return a.K == 64 ? launch_trans<64, bf16_t>(a, stream, cout) : launch_trans<128, bf16_t>(a, stream, cout);
+        return a.K == 64 ? launch_trans<64, _Float16>(a, stream, lout) : launch_trans<128, _Float16>(a, stream, lout);
+    return a.K == 64 ? launch_trans<64, bf16_t>(a, stream, lout) : launch_trans<128, bf16_t>(a, stream, lout);
 }
 
 int chunkwise_launch(const kda_fwd_args& a, hipStream_t stream, float* ckpt, const kda_gate_args* gate) {

@@ -32,10 +32,23 @@ int chunkwise_launch(const kda_fwd_args& a, hipStream_t stream, float* ckpt = nu
                      const kda_gate_args* gate = nullptr);
 // The first pass of a split long sequence (kda_chunkwise_long_fwd): per chain
 // the state from zero and the transition, state_out [B, H, K, V + K] fp32;
-// with cout, also the outputs in fp32: o [B, T, H, V] from the zero state and
-// cout [B, T, H, K] those of the transition columns.
+// with lout, also the outputs in fp32: oz [B, T, H, V] from the zero state and
+// c [B, T, H, K] those of the transition columns (the coefficients of the
+// initial state).  In two launches (kTrans, kV) the transition columns' 64- or
+// 128-column tiles write only the n[(b, h), tile] 32-token chunks in which
+// they may not be zero, and the V columns' outputs after those chunks go to o
+// [B, T, H, V] instead of oz.
+struct long_out {
+    float* oz;
+    float* c;
+    int* n;
+    int part;
+    static constexpr int kBoth = 0, kTrans = 1, kV = 2;
+};
+// columns of a transition tile with lout
+__host__ __device__ constexpr int64_t trans_tile(int64_t K, int64_t V) { return K == 128 && V % 128 == 0 ? 128 : 64; }
 bool chunkwise_trans_supported(const kda_fwd_args& a);
-int chunkwise_trans_launch(const kda_fwd_args& a, hipStream_t stream, float* cout = nullptr);
+int chunkwise_trans_launch(const kda_fwd_args& a, hipStream_t stream, const long_out* lout = nullptr);
 // The chunkwise forward with the layer's output epilogue (kda_chunkwise_fused_fwd).
 bool chunkwise_fused_supported(const kda_fwd_args& a);
 int chunkwise_fused_launch(const kda_fwd_args& a, hipStream_t stream, const kda_gate_args* gate,
@@ -45,6 +58,11 @@ int chunkwise_fused_launch(const kda_fwd_args& a, hipStream_t stream, const kda_
 // segments, and the three passes (T % P == 0, checked by the caller).
 int64_t long_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P);
 int long_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t stream);
+// The few-chain form with transition columns that end when they are zero, in
+// P segments or a power of two times as many: workspace bytes (0: no such
+// form for this shape) and the launch.
+int64_t split_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P);
+int split_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t stream);
 
 // Chunkwise backward (kda_chunkwise_bwd.hip).
 bool chunkwise_bwd_supported(int64_t K, int64_t V);

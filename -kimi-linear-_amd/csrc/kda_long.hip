@@ -22,6 +22,20 @@
 // coefficients of the initial state in the outputs) -- and
 //   3'. o[t] = oz[t] + c[t] S_start[p] (long_correct_kernel), rounded once;
 // the outputs are linear in the initial state, so this is the same function.
+//
+// A chain forgets its initial state: with decays that average e^-0.8 a token
+// in the slowest channel the transition columns are exactly zero after about
+// 110 tokens of a segment.  The split form (kda_chunkwise_split_fwd) runs the
+// transition columns before the V columns: a workgroup whose columns are all
+// zero ends (they stay zero) and says how many chunks it wrote; the V
+// columns' outputs after those chunks are final, oz + 0, and 3' leaves them
+// (unless S_start holds an infinity or a NaN, whose product with zero is NaN:
+// then it takes those tokens too, with c = 0).  Each of the two launches has
+// the chip to itself, so a segment is half as long.  B=1 T=32768 H=16 K=V=128
+// fp16: 8 segments in one launch 537 us, 16 in two 316 (trans 34, V columns
+// 215, combine 48, correction 37: the kernels alone).  With decays 1000 times
+// weaker, where nothing is forgotten, it costs about a tenth more than the one
+// launch (632 -> 700 us on a GPU not yet at its settled clock).
 #include "kda_common.h"
 #include "kda_launch.h"
 
@@ -36,24 +50,28 @@ typedef uint32_t w4 __attribute__((ext_vector_type(4)));
 typedef uint32_t w2 __attribute__((ext_vector_type(2)));
 
 constexpr int kCombineCols = 16;   // state columns per combine workgroup
-constexpr int kCombineThreads = 256;
+// one wave per 16 rows of Phi (two tiles a wave measured 55 us at 16 segments of
+// 16 heads, K = V = 128, one 49)
+constexpr int combine_threads(int K) { return 4 * K; }
 constexpr int kCombinePad = 20;    // LDS row of the state strip: conflict-free B-operand reads
 
-// One workgroup of four waves per (b, h, 16 state columns):
+// One workgroup of K / 16 waves per (b, h, 16 state columns):
 // S_start[p] = S; S = Phi_p S + S_loc_p for p = 0 .. P - 1; S_out = S.
-// The strip S (K x 16) sits in LDS; wave w computes rows 16 (TPW w + t) ..
-// + 15 of Phi_p S on the fp32 matrix cores (v_mfma_f32_16x16x4f32, exact
+// The strip S (K x 16) sits in LDS; wave w computes rows 16 w .. + 15 of
+// Phi_p S on the fp32 matrix cores (v_mfma_f32_16x16x4f32, exact
 // products): lane (ln, lg) feeds Phi[r0 + ln][16 U + 4 lg + u] (one 16-byte
 // load of the row covers u = 0 .. 3) against S[16 U + 4 lg + u][ln].
 // seg: [B P, H, K, V + K] fp32 (columns [0, V) S_loc, [V, V + K) Phi);
 // sstart: [B P, H, K, V] fp32; s0 (nullable, any dtype) and sout: [B, H, K, V].
+// nonfinite (nullable): [B P, H, V / 16, waves], whether S_start[p]'s part is
+// not finite (a byte a wave).
 template <int K>
-__global__ __launch_bounds__(kCombineThreads) void long_combine_kernel(const float* seg, float* sstart,
+__global__ __launch_bounds__(combine_threads(K)) void long_combine_kernel(const float* seg, float* sstart,
                                                                        const void* s0, int s0_dtype, void* sout,
                                                                        int sout_dtype, int64_t B, int64_t H,
-                                                                       int64_t V, int64_t P) {
+                                                                       int64_t V, int64_t P, uint8_t* nonfinite) {
     static_assert(K == 64 || K == 128, "the split path takes K in {64, 128}");
-    constexpr int TPW = K / 64;                     // 16-row tiles per wave
+    constexpr int kCombineThreads = combine_threads(K), kCombineWaves = kCombineThreads / 64;
     constexpr int EPT = K * kCombineCols / kCombineThreads;   // strip elements per thread
     __shared__ float S[K][kCombinePad];
     const int t = threadIdx.x, w = t >> 6, lane = t & 63, ln = lane & 15, lg = lane >> 4;
@@ -72,46 +90,41 @@ __global__ __launch_bounds__(kCombineThreads) void long_combine_kernel(const flo
     }
     __syncthreads();
     // segment p + 1's Phi rows and S_loc are fetched while segment p is composed
-    f4 ph[TPW][K / 16], sl[TPW];
+    const int r0 = 16 * w;
+    f4 ph[K / 16], sl;
     auto fetch = [&](int64_t p) {
         const float* base = seg + ((b * P + p) * H + h) * K * VS;
 #pragma unroll
-        for (int tt = 0; tt < TPW; ++tt) {
-            const int r0 = 16 * (TPW * w + tt);
+        for (int j = 0; j < 4; ++j) sl[j] = base[(r0 + 4 * lg + j) * VS + c0 + ln];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) sl[tt][j] = base[(r0 + 4 * lg + j) * VS + c0 + ln];
-#pragma unroll
-            for (int U = 0; U < K / 16; ++U)
-                ph[tt][U] = *reinterpret_cast<const f4*>(base + (r0 + ln) * VS + V + 16 * U + 4 * lg);
-        }
+        for (int U = 0; U < K / 16; ++U)
+            ph[U] = *reinterpret_cast<const f4*>(base + (r0 + ln) * VS + V + 16 * U + 4 * lg);
     };
     if (P > 0) fetch(0);
     for (int64_t p = 0; p < P; ++p) {
         const int64_t bp = b * P + p;
+        bool odd = false;
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
             const int e = t + kCombineThreads * m, r = e / kCombineCols, j = e % kCombineCols;
-            sstart[((bp * H + h) * K + r) * V + c0 + j] = S[r][j];
+            const float x = S[r][j];
+            sstart[((bp * H + h) * K + r) * V + c0 + j] = x;
+            odd = odd || !(fabsf(x) <= 3.4028235e38f);
         }
-        f4 acc[TPW];
+        // one byte a wave: its part of the strip holds an infinity or a NaN
+        const bool any_odd = __any(odd);
+        if (nonfinite != nullptr && lane == 0)
+            nonfinite[((bp * H + h) * nct + c0 / kCombineCols) * kCombineWaves + w] = any_odd;
+        f4 acc = sl;
 #pragma unroll
-        for (int tt = 0; tt < TPW; ++tt) {
-            acc[tt] = sl[tt];
+        for (int U = 0; U < K / 16; ++U)
 #pragma unroll
-            for (int U = 0; U < K / 16; ++U)
-#pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    acc[tt] = __builtin_amdgcn_mfma_f32_16x16x4f32(ph[tt][U][u], S[16 * U + 4 * lg + u][ln], acc[tt],
-                                                                   0, 0, 0);
-        }
+            for (int u = 0; u < 4; ++u)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ph[U][u], S[16 * U + 4 * lg + u][ln], acc, 0, 0, 0);
         if (p + 1 < P) fetch(p + 1);
         __syncthreads();                    // every wave's reads of S are done
 #pragma unroll
-        for (int tt = 0; tt < TPW; ++tt) {
-            const int r0 = 16 * (TPW * w + tt);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) S[r0 + 4 * lg + j][ln] = acc[tt][j];
-        }
+        for (int j = 0; j < 4; ++j) S[r0 + 4 * lg + j][ln] = acc[j];
         __syncthreads();
     }
 #pragma unroll
@@ -152,7 +165,10 @@ constexpr int kCorrectTokens = 256;   // tokens per correction workgroup
 // segment that starts from zero (no initial state) takes oz as it is.  Rows
 // past the segment's end are outside the descriptors' ranges (read as zero,
 // stores dropped).  oz, cf: [B T, H, V] and [B T, H, K] fp32; sstart:
-// [B P, H, K, V] fp32; o: [B T, H, V] in the output dtype.
+// [B P, H, K, V] fp32; o: [B T, H, V] in the output dtype.  nch: [B P, H, K /
+// tile], the 32-token chunks of the segment whose coefficients of a tile of
+// channels were written (zero after them, and the outputs in o instead of
+// oz), or null: all; nonfinite: of the combine.
 template <int K>
 struct CorrectSmem {
     uint16_t hi[2][16][K + 8];
@@ -161,7 +177,8 @@ struct CorrectSmem {
 template <int K, typename TO>
 __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, const float* cf, const float* sstart,
                                                             TO* o, int64_t T, int64_t H, int64_t V, int64_t P,
-                                                            int zero_first) {
+                                                            int zero_first, const int* nch, int tile,
+                                                            const uint32_t* nonfinite) {
     __shared__ CorrectSmem<K> sm;
     const int t = threadIdx.x, lane = t & 63, ln = lane & 15, lg = lane >> 4;
     const int nthr = static_cast<int>(blockDim.x);
@@ -176,13 +193,31 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
     const bool none = zero_first && bp % P == 0;    // S_start = 0
     const int64_t c0 = 16 * w;
     const int64_t t0 = tb * kCorrectTokens;
-    const int rows = static_cast<int>(Ts - t0 < kCorrectTokens ? Ts - t0 : kCorrectTokens);
     const int64_t row0 = bp * Ts + t0;              // flat token index b T + p Ts + t0
+    // rows of this workgroup's tokens with coefficients, per channel tile
+    // (one or two); and whether S_start is not finite (a word a strip)
+    const int64_t left = Ts - t0 < kCorrectTokens ? Ts - t0 : kCorrectTokens;
+    int n0 = static_cast<int>(left), n1 = n0;
+    uint32_t odd = 0;
+    if (nch != nullptr) {
+        const int* nc = nch + (bp * H + h) * (K / tile);
+        auto with_c = [&](int i) {
+            const int64_t r = 32 * static_cast<int64_t>(nc[i]) - t0;
+            return static_cast<int>(r < 0 ? 0 : (r < left ? r : left));
+        };
+        n0 = with_c(0);
+        n1 = K / tile > 1 ? with_c(1) : n0;
+        constexpr int kWords = combine_threads(K) / 64 / 4;     // a strip's bytes
+        for (int i = 0; i < static_cast<int>(V / kCombineCols) * kWords; ++i)
+            odd |= nonfinite[(bp * H + h) * (V / kCombineCols) * kWords + i];
+    }
+    const int rows = n0 > n1 ? n0 : n1;             // whose V outputs are in oz
+    if (rows == 0 && !odd) return;                  // the others are final
     const int64_t hk = H * K, hv = H * V;
-    const auto rc = make_rsrc(cf + row0 * hk + h * K, static_cast<uint32_t>(((rows - 1) * hk + K) * 4));
-    const auto rz = make_rsrc(oz + row0 * hv + h * V, static_cast<uint32_t>(((rows - 1) * hv + V) * 4));
+    const auto rc = make_rsrc(cf + row0 * hk + h * K, rows ? static_cast<uint32_t>(((rows - 1) * hk + K) * 4) : 0u);
+    const auto rz = make_rsrc(oz + row0 * hv + h * V, rows ? static_cast<uint32_t>(((rows - 1) * hv + V) * 4) : 0u);
     const auto ro = make_rsrc(o + row0 * hv + h * V,
-                              static_cast<uint32_t>(((rows - 1) * hv + V) * static_cast<int64_t>(sizeof(TO))));
+                              static_cast<uint32_t>(((left - 1) * hv + V) * static_cast<int64_t>(sizeof(TO))));
     auto store_out = [&](const f4& y, int orow) {
         if constexpr (sizeof(TO) == 4) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(w4, y), ro, orow * 4, 0, 0);
@@ -232,8 +267,10 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
         for (int m = 0; m < 2; ++m) {
             const int i = t + nthr * m;
             const int r = i / (K / 4), c4 = i % (K / 4);
-            // a slot past the step's pieces reads past the range: no memory access
-            const int off = i < NP ? static_cast<int>(((tt + r) * hk + 4 * c4) * 4) : 0x7ffffff0;
+            // a slot past the step's pieces, or past the coefficients of its
+            // channels, reads past the range: no memory access, zeros
+            const int nr = 4 * c4 < tile ? n0 : n1;
+            const int off = i < NP && tt + r < nr ? static_cast<int>(((tt + r) * hk + 4 * c4) * 4) : 0x7ffffff0;
             fc[m] = __builtin_bit_cast(w4, __builtin_amdgcn_raw_buffer_load_b128(rc, off, 0, 0));
         }
     };
@@ -295,6 +332,25 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
         z = zn;
         buf ^= 1;
     }
+    if (odd) {
+        // the tokens after them: o + 0 S_start, a NaN in the columns of S_start
+        // that hold an infinity or a NaN
+        f4 nan = {0.f, 0.f, 0.f, 0.f};
+        const bf8 zero = __builtin_bit_cast(bf8, w4{0u, 0u, 0u, 0u});
+#pragma unroll
+        for (int u = 0; u < K / 32; ++u) {
+            nan = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sh[u], zero, nan, 0, 0, 0);
+            nan = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sl[u], zero, nan, 0, 0, 0);
+        }
+        for (int tt = rows; tt < left; tt += 16) {
+            const int orow = oz_row(tt);
+            f4 y;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                y[j] = tt + ln < left ? load_elem(o, row0 * hv + h * V + orow + j, Elem<TO>::code) + nan[j] : 0.f;
+            store_out(y, orow);
+        }
+    }
 }
 
 // The [B, T, ...] view of a chain input as a [B P, T / P, ...] view: one
@@ -308,24 +364,52 @@ bool split_strides(int64_t (&st)[3], int64_t B, int64_t T, int64_t P) {
 
 }  // namespace
 
-// The few-chain form: the first pass in one round of 128-column workgroups
-// on the current device (and V <= 256: one correction wave per 16 columns).
-static bool long_correct_form(int64_t B, int64_t H, int64_t K, int64_t V, int64_t P) {
-    if (V > 256) return false;
+static int64_t cu_count() {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    return (V + K) % 128 == 0 && B * P * H * ((V + K) / 128) <= cus;
+    return cus;
+}
+
+// The few-chain form: the first pass in one round of 128-column workgroups
+// on the current device (and V <= 256: one correction wave per 16 columns).
+static bool long_correct_form(int64_t B, int64_t H, int64_t K, int64_t V, int64_t P) {
+    return V <= 256 && V % 64 == 0 && (V + K) % 128 == 0 && B * P * H * ((V + K) / 128) <= cu_count();
+}
+
+// Bytes of P segments' states, transitions and initial states, and in the
+// few-chain form of the fp32 outputs oz and coefficients c after them.
+static int64_t segment_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P, bool outputs) {
+    return 4 * (B * P * H * K * (2 * V + K) + (outputs ? B * T * H * (V + K) : 0));
 }
 
 int64_t long_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P) {
-    // segment states and transitions, initial states; in the few-chain form
-    // the fp32 outputs oz and c after them
-    return 4 * (B * P * H * K * (2 * V + K) + (long_correct_form(B, H, K, V, P) ? B * T * H * (V + K) : 0));
+    return segment_bytes(B, T, H, K, V, P, long_correct_form(B, H, K, V, P));
 }
 
-int long_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t stream) {
+// Segments of the split form: twice P (or the power of two times P) while the
+// V columns fit one round of workgroups and a segment keeps kSplitSegment
+// tokens; none (0) where P cannot be doubled: its one launch holds both kinds
+// of columns side by side.
+static int64_t split_segments(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P) {
+    constexpr int64_t kSplitSegment = 1024;
+    if ((K != 64 && K != 128) || T % P != 0 || !long_correct_form(B, H, K, V, P)) return 0;
+    const int64_t cus = cu_count(), tiles = B * H * (V / trans_tile(K, V)), P0 = P;
+    while (2 * P * tiles <= cus && T % (2 * P) == 0 && T / (2 * P) >= kSplitSegment) P *= 2;
+    return P > P0 ? P : 0;
+}
+
+int64_t split_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P) {
+    P = split_segments(B, T, H, K, V, P);
+    if (P == 0) return 0;
+    // and the chunk counts and the combine's bytes
+    return segment_bytes(B, T, H, K, V, P, true) + 4 * B * P * H * (K / trans_tile(K, V) + V / kCombineCols * (K / 64));
+}
+
+// The three kernels (ends: transition columns may end early).
+static int run_segments(const kda_fwd_args& a, int64_t P, bool correct, bool ends, void* workspace,
+                        hipStream_t stream) {
     const int64_t B = a.B, T = a.T, H = a.H, K = a.K, V = a.V;
     kda_fwd_args s = a;
     s.B = B * P;
@@ -334,30 +418,39 @@ int long_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t s
         !split_strides(s.v_stride, B, T, P) || !split_strides(s.g_stride, B, T, P) ||
         !split_strides(s.beta_stride, B, T, P))
         return KDA_ERR_UNSUPPORTED;
+    const int tile = static_cast<int>(trans_tile(K, V));
     float* seg = static_cast<float*>(workspace);
     float* sstart = seg + B * P * H * K * (V + K);
     float* oz = sstart + B * P * H * K * V;
     float* cf = oz + B * T * H * V;
-    const bool correct = long_correct_form(B, H, K, V, P);
+    int* nch = ends ? reinterpret_cast<int*>(cf + B * T * H * K) : nullptr;
+    uint32_t* nonfinite = ends ? reinterpret_cast<uint32_t*>(nch + B * P * H * (K / tile)) : nullptr;
 
     // 1. per chain: the state from zero and the transition (and in the
-    // few-chain form the fp32 outputs oz and c)
+    // few-chain form the outputs from zero and the coefficients c)
     kda_fwd_args a1 = s;
     a1.state_in = nullptr;
     a1.state_out = seg;
     a1.state_out_dtype = KDA_DTYPE_F32;
-    a1.o = correct ? oz : nullptr;
-    int st = chunkwise_trans_launch(a1, stream, correct ? cf : nullptr);
+    a1.o = ends ? a.o : nullptr;
+    long_out lout{oz, cf, nch, ends ? long_out::kTrans : long_out::kBoth};
+    int st = chunkwise_trans_launch(a1, stream, correct ? &lout : nullptr);
+    if (st == KDA_OK && ends) {
+        lout.part = long_out::kV;
+        st = chunkwise_trans_launch(a1, stream, &lout);
+    }
     if (st != KDA_OK) return st;
 
     // 2. the segments in order
-    const int64_t blocks = B * H * (V / kCombineCols);
+    const dim3 cgrid(static_cast<unsigned>(B * H * (V / kCombineCols)));
+    const dim3 cblock(static_cast<unsigned>(combine_threads(static_cast<int>(K))));
+    auto* bad = reinterpret_cast<uint8_t*>(nonfinite);
     if (K == 64)
-        hipLaunchKernelGGL((long_combine_kernel<64>), dim3(static_cast<unsigned>(blocks)), dim3(kCombineThreads), 0,
-                           stream, seg, sstart, a.state_in, a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P);
+        hipLaunchKernelGGL((long_combine_kernel<64>), cgrid, cblock, 0, stream, seg, sstart, a.state_in,
+                           a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P, bad);
     else
-        hipLaunchKernelGGL((long_combine_kernel<128>), dim3(static_cast<unsigned>(blocks)), dim3(kCombineThreads), 0,
-                           stream, seg, sstart, a.state_in, a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P);
+        hipLaunchKernelGGL((long_combine_kernel<128>), cgrid, cblock, 0, stream, seg, sstart, a.state_in,
+                           a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P, bad);
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
 
     if (correct) {
@@ -367,7 +460,7 @@ int long_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t s
         const int zero_first = a.state_in == nullptr ? 1 : 0;
 #define KDA_CORRECT(KK, TO)                                                                                    \
     hipLaunchKernelGGL((long_correct_kernel<KK, TO>), grid, block, 0, stream, oz, cf, sstart,                   \
-                       static_cast<TO*>(a.o), T, H, V, P, zero_first)
+                       static_cast<TO*>(a.o), T, H, V, P, zero_first, nch, tile, nonfinite)
         if (a.qkv_dtype == KDA_DTYPE_F16) {
             if (K == 64) KDA_CORRECT(64, _Float16); else KDA_CORRECT(128, _Float16);
         } else {
@@ -385,6 +478,16 @@ int long_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t s
     a3.state_out = nullptr;
     a3.state_out_dtype = KDA_DTYPE_F32;
     return chunkwise_launch(a3, stream);
+}
+
+int long_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t stream) {
+    return run_segments(a, P, long_correct_form(a.B, a.H, a.K, a.V, P), false, workspace, stream);
+}
+
+int split_launch(const kda_fwd_args& a, int64_t P, void* workspace, hipStream_t stream) {
+    P = split_segments(a.B, a.T, a.H, a.K, a.V, P);
+    if (P == 0) return KDA_ERR_UNSUPPORTED;
+    return run_segments(a, P, true, true, workspace, stream);
 }
 
 }  // namespace kda

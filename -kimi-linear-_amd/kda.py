@@ -254,10 +254,13 @@ def _forward(kind, q, k, v, g, beta, state, chunk_size, state_dtype, state_out=N
             if B == 1 or all(x.stride(0) == T * x.stride(1) for x in (q, k, v, g, beta)):
                 segments = long_segments(B, T, H, K, V, qk_dtype)
         if segments > 1:
-            ws = torch.empty(int(lib.kda_chunkwise_long_workspace_size(B, T, H, K, V, segments)), device=dev,
-                             dtype=torch.uint8)
-            status = lib.kda_chunkwise_long_fwd(ctypes.byref(args), ctypes.c_int64(segments),
-                                                ctypes.c_void_p(ws.data_ptr()), stream)
+            # the form whose transition columns end when they are zero, where there is one
+            size, fwd = int(lib.kda_chunkwise_split_workspace_size(B, T, H, K, V, segments)), lib.kda_chunkwise_split_fwd
+            if size == 0:
+                size, fwd = int(lib.kda_chunkwise_long_workspace_size(B, T, H, K, V, segments)), \
+                    lib.kda_chunkwise_long_fwd
+            ws = torch.empty(size, device=dev, dtype=torch.uint8)
+            status = fwd(ctypes.byref(args), ctypes.c_int64(segments), ctypes.c_void_p(ws.data_ptr()), stream)
         elif epilogue is not None:
             gargs = None
             if gate is not None:
@@ -301,8 +304,9 @@ CU_COUNT = 256
 
 
 def long_segments(B, T, H, K, V, dtype) -> int:
-    """Segments for kda_chunkwise_long_fwd; 1 (one pass) when the chains alone
-    fill half the CUs or the shape has no split kernel.
+    """Segments for kda_chunkwise_split_fwd (which may double them) or, where
+    that has no form, kda_chunkwise_long_fwd; 1 (one pass) when the chains
+    alone fill half the CUs or the shape has no split kernel.
 
     With V + K a multiple of 128 and V <= 256 the split takes its few-chain
     form whenever its first pass (every segment's state columns and transition

@@ -187,6 +187,17 @@ int kda_chunkwise_fused_fwd(const kda_fwd_args* args, const kda_gate_args* gate,
 size_t kda_chunkwise_long_workspace_size(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t segments);
 int kda_chunkwise_long_fwd(const kda_fwd_args* args, int64_t segments, void* workspace, void* stream);
 
+/*
+ * The few-chain form of the split (K in {64, 128}, V <= 256, V + K a multiple
+ * of 128, B segments H (V + K) / 128 at most the device's compute units) in
+ * `segments` segments or a power of two times as many, with the work on a
+ * segment's dependence on its initial state ending once that dependence is
+ * exactly zero.  The same function and errors as kda_chunkwise_long_fwd;
+ * KDA_ERR_UNSUPPORTED where the size function returns 0 (no such form).
+ */
+size_t kda_chunkwise_split_workspace_size(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t segments);
+int kda_chunkwise_split_fwd(const kda_fwd_args* args, int64_t segments, void* workspace, void* stream);
+
 /* ---------------------------------------------------------------------------
  * Backward of the chunkwise forward.  The reference differentiates
  * kda_chunkwise (kimi_linear/kda.py:58-185) with autograd and trains through
