@@ -13,6 +13,7 @@
 // In Python a call's checks, its argument structure and its device and stream
 // lookups took about 20 us (a decode step at B=1 takes 4 us on the GPU).
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/utils/pybind.h>
@@ -45,6 +46,7 @@ struct Fns {
     decltype(&kda_chunkwise_split_workspace_size) split_ws = nullptr;
     decltype(&kda_prep_fwd) prep = nullptr;
     decltype(&kda_output_fwd) output = nullptr;
+    decltype(&kda_linear_fwd) linear = nullptr;
 };
 Fns fn;
 // torch._C._cuda_getCurrentRawStream; kept for the process's life
@@ -68,6 +70,7 @@ void bind(const py::dict& addr, const py::object& stream_fn) {
     take(fn.split_ws, addr, "kda_chunkwise_split_workspace_size");
     take(fn.prep, addr, "kda_prep_fwd");
     take(fn.output, addr, "kda_output_fwd");
+    take(fn.linear, addr, "kda_linear_fwd");
     Py_INCREF(stream_fn.ptr());
     raw_stream = stream_fn.ptr();
 }
@@ -359,6 +362,78 @@ py::object output(const Tensor& o, const Tensor& gate, const Tensor& weight, dou
     return py::cast(y);
 }
 
+// Rows of x [B, T, K] one stride apart, as few as kda_linear_fwd takes, and w [N, K].
+bool linear_ok(const Plain& plain, const Tensor& x, const Tensor& w) {
+    const auto dt = x.scalar_type();
+    return plain.ok && (dt == at::kHalf || dt == at::kBFloat16) && x.dim() == 3 && x.numel() > 0 && w.numel() > 0 &&
+           w.dim() == 2 && x.size(0) <= 64 && x.size(1) <= 64 && x.size(0) * x.size(1) <= 64 && x.stride(2) == 1 &&
+           (x.size(0) == 1 || x.size(1) == 1 || x.stride(0) == x.size(1) * x.stride(1)) && w.size(1) == x.size(2) &&
+           w.scalar_type() == dt && w.is_contiguous();
+}
+
+int64_t row_stride(const Tensor& x) { return x.size(1) == 1 ? x.stride(0) : x.stride(1); }
+
+void linear_operands(kda_linear_args& a, int i, const Tensor& x, const Tensor& w, const Tensor& y) {
+    a.x[i] = x.data_ptr();
+    a.x_stride[i] = row_stride(x);
+    a.w[i] = w.data_ptr();
+    a.N[i] = w.size(0);
+    a.y[i] = y.data_ptr();
+}
+
+// Autocast would choose the projection's type: its calls are the general path's.
+bool autocast_on() { return at::autocast::is_autocast_enabled(at::kCUDA); }
+
+// x w^T of few rows, [B, T, N]; residual [B, T, N]: their sum; out: written
+// there.  The result, or None for the calls of the library product.
+py::object linear(const Tensor& x, const Tensor& w, const OptTensor& residual, const OptTensor& out) {
+    Plain plain(x);
+    plain.add(w).add(residual).add(out);
+    if (!linear_ok(plain, x, w) || autocast_on()) return py::none();
+    const int64_t B = x.size(0), T = x.size(1), N = w.size(0);
+    if (residual && (!sized(*residual, {B, T, N}) || residual->scalar_type() != x.scalar_type() ||
+                     residual->stride(2) != 1 ||
+                     (B > 1 && T > 1 && residual->stride(0) != T * residual->stride(1))))
+        return py::none();
+    if (out && (!sized(*out, {B, T, N}) || out->scalar_type() != x.scalar_type() || !out->is_contiguous() ||
+                overlaps(*out, x) || overlaps(*out, w) || (residual && overlaps(*out, *residual))))
+        return py::none();
+    const c10::DeviceGuard guard(plain.dev);
+    Tensor y = out ? *out : at::empty({B, T, N}, x.options().requires_grad(false));
+    kda_linear_args a{};
+    a.M = B * T;
+    a.K = x.size(2);
+    linear_operands(a, 0, x, w, y);
+    if (residual) {
+        a.residual = residual->data_ptr();
+        a.residual_stride = row_stride(*residual);
+    }
+    a.dtype = code(x);
+    if (fn.linear(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    return py::cast(y);
+}
+
+// Two such products of one depth in one launch: (y0, y1) or None.
+py::object linear2(const Tensor& x0, const Tensor& w0, const Tensor& x1, const Tensor& w1) {
+    Plain plain(x0);
+    plain.add(w0).add(x1).add(w1);
+    if (!linear_ok(plain, x0, w0) || !linear_ok(plain, x1, w1) || !x0.sizes().equals(x1.sizes()) ||
+        x0.scalar_type() != x1.scalar_type() || autocast_on())
+        return py::none();
+    const c10::DeviceGuard guard(plain.dev);
+    const auto opt = x0.options().requires_grad(false);
+    Tensor y0 = at::empty({x0.size(0), x0.size(1), w0.size(0)}, opt);
+    Tensor y1 = at::empty({x0.size(0), x0.size(1), w1.size(0)}, opt);
+    kda_linear_args a{};
+    a.M = x0.size(0) * x0.size(1);
+    a.K = x0.size(2);
+    linear_operands(a, 0, x0, w0, y0);
+    linear_operands(a, 1, x1, w1, y1);
+    a.dtype = code(x0);
+    if (fn.linear(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    return py::make_tuple(y0, y1);
+}
+
 // What decides whether a copy made of these parameters is still theirs:
 // storage address, version, type and device of each.
 py::bytes params_key(const std::vector<Tensor>& params) {
@@ -382,5 +457,7 @@ PYBIND11_MODULE(_kda_host, m) {
     m.def("core", &core);
     m.def("prep", &prep);
     m.def("output", &output);
+    m.def("linear", &linear);
+    m.def("linear2", &linear2);
     m.def("params_key", &params_key);
 }

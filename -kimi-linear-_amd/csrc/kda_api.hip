@@ -250,6 +250,27 @@ int kda_chunkwise_bwd_noalloc(const kda_bwd_args* a, void* stream) {
     return kda::chunkwise_bwd_launch(b, static_cast<hipStream_t>(stream));
 }
 
+int kda_linear_fwd(const kda_linear_args* a, void* stream) {
+    if (a == nullptr) return KDA_ERR_NULL_POINTER;
+    const int mats = a->x[1] ? 2 : 1;
+    if (a->M < 0 || a->K <= 0) return KDA_ERR_BAD_SHAPE;
+    if (a->dtype != KDA_DTYPE_F16 && a->dtype != KDA_DTYPE_BF16) return KDA_ERR_BAD_DTYPE;
+    if (!kda::linear_supported(*a) || (mats == 2 && a->residual)) return KDA_ERR_UNSUPPORTED;
+    if (a->M == 0) return KDA_OK;
+    const auto misaligned = [](const void* p, int64_t stride, uintptr_t n) {
+        return reinterpret_cast<uintptr_t>(p) % n != 0 || stride * 2 % static_cast<int64_t>(n) != 0;
+    };
+    for (int i = 0; i < mats; ++i) {
+        if (!a->x[i] || !a->w[i] || !a->y[i]) return KDA_ERR_NULL_POINTER;
+        if (a->N[i] <= 0 || a->N[i] / 16 > INT32_MAX) return KDA_ERR_BAD_SHAPE;
+        if (a->N[i] % 16 != 0 || misaligned(a->x[i], a->x_stride[i], 16) || misaligned(a->w[i], 0, 16) ||
+            misaligned(a->y[i], 0, 8))
+            return KDA_ERR_UNSUPPORTED;
+    }
+    if (a->residual && misaligned(a->residual, a->residual_stride, 8)) return KDA_ERR_UNSUPPORTED;
+    return kda::linear_launch(*a, static_cast<hipStream_t>(stream));
+}
+
 const char* kda_status_str(int status) {
     switch (status) {
         case KDA_OK: return "ok";

@@ -72,4 +72,8 @@ int chunkwise_bwd_launch(const kda_bwd_args& a, hipStream_t stream);
 // on the current device; resolved once per device.  KDA_OK or KDA_ERR_LAUNCH.
 int chunkwise_bwd_scratch(void** ptr);
 
+// y = x W^T of few rows (kda_linear.hip); shapes and alignment checked by the caller.
+bool linear_supported(const kda_linear_args& a);
+int linear_launch(const kda_linear_args& a, hipStream_t stream);
+
 }  // namespace kda

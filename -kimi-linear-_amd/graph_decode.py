@@ -103,10 +103,16 @@ class KdaGraphedDecoder:
     def _step(self):
         """The captured region: one token through every layer on the static buffers."""
         h = self.input_static
-        for layer, st in zip(self.layers, self.static_states):
+        result = self.output_static.unsqueeze(1)
+        for i, (layer, st) in enumerate(zip(self.layers, self.static_states)):
+            if self.residual and getattr(layer.decode_step_, "__func__", None) is KimiDeltaAttention.decode_step_:
+                # the residual add belongs to the output projection, which writes the result in place
+                h = layer._decode(h, st, h, result if i + 1 == len(self.layers) else None)
+                continue
             out = layer.decode_step_(h, st)
             h = h + out if self.residual else out
-        self.output_static.copy_(h[:, -1, :])
+        if h is not result:
+            self.output_static.copy_(h[:, -1, :])
 
     # ------------------------------------------------------------ state plumbing
     def _snapshot(self):

@@ -133,6 +133,28 @@ def linear_attn_config(**kw) -> SimpleNamespace:
     return SimpleNamespace(linear_attn_config=la, **top)
 
 
+def _plain_weight(mod):
+    """The weight of a module that is just x W^T: an ``nn.Linear`` as torch has it,
+    without a bias, hooks or a forward of its own; else None."""
+    if (type(mod) is not nn.Linear or mod.bias is not None or mod._forward_hooks or mod._forward_pre_hooks
+            or "forward" in mod.__dict__ or nn.modules.module._has_any_global_hook()):
+        return None
+    return mod.weight
+
+
+def _project(mod, x, residual=None, out=None):
+    """``mod(x)``, plus ``residual``, into ``out``: in the few-row kernel
+    (``kda_linear_fwd``, up to 64 rows) where it applies, else as written."""
+    w = _plain_weight(mod) if x.shape[0] * x.shape[1] <= 64 else None
+    y = _native.host().linear(x, w, residual, out) if w is not None else None
+    if y is not None:
+        return y
+    y = mod(x)
+    if residual is not None:
+        y = residual + y
+    return y if out is None else out.copy_(y)
+
+
 class KimiDeltaAttention(nn.Module):
     """The KDA layer (``kda.py:331-536``) with the native core."""
 
@@ -285,10 +307,19 @@ class KimiDeltaAttention(nn.Module):
         convs = (self.conv_q.conv, self.conv_k.conv, self.conv_v.conv)
         H, K, V = self.num_heads, self.head_dim, self.value_head_dim
         w, b = self._input_weight()
-        y = torch.nn.functional.linear(x, w, b)
+        few = x.shape[0] * x.shape[1] <= 64
+        y = _native.host().linear(x, w, None, None) if few and b is None else None
+        if y is None:
+            y = torch.nn.functional.linear(x, w, b)
         q_in, k_in, v_in, beta_logit, gk_low, og_low = torch.split(
             y, (H * K, H * K, H * V, H, self.gk_proj[0].out_features, self.og_proj[0].out_features), dim=-1)
-        gk = self.gk_proj[1](gk_low)
+        gk = gate = None
+        if few:                       # both up-projections in one launch
+            w_gk, w_og = _plain_weight(self.gk_proj[1]), _plain_weight(self.og_proj[1])
+            if w_gk is not None and w_og is not None:
+                gk, gate = _native.host().linear2(gk_low, w_gk, og_low, w_og) or (None, None)
+        if gk is None:
+            gk = self.gk_proj[1](gk_low)
         gate_in = (gk, *self._gate_params(), beta_logit) if gates else (None, None, None, None)
         q, k, v, g, beta, new_conv = kda_prep(
             q_in, k_in, v_in,
@@ -298,17 +329,23 @@ class KimiDeltaAttention(nn.Module):
             l2_eps=self.l2norm_eps, hist=hist, hist_out=conv_out if use_cache else None,
             want_hist=use_cache and conv_out is None)
         if gates:
-            return q, k, v, g, beta, new_conv, og_low
-        return q, k, v, gk.view(x.shape[0], x.shape[1], H, K), beta_logit, new_conv, og_low
+            return q, k, v, g, beta, new_conv, (og_low, gate)
+        return q, k, v, gk.view(x.shape[0], x.shape[1], H, K), beta_logit, new_conv, (og_low, gate)
 
-    def _output(self, o_core, og_low):
+    def _output_gate(self, og):
+        """The output gate's up-projection from what :meth:`_projections` returned for it."""
+        og_low, gate = og
+        return self.og_proj[1](og_low) if gate is None else gate
+
+    def _output(self, o_core, og, residual=None, out=None):
         """Head-wise RMSNorm, sigmoid output gate (one fused kernel,
         :func:`kda_output`) and the output projection (``kda.py:464-470``);
-        ``og_low`` is the output gate's down-projection of x."""
-        gate = self.og_proj[1](og_low)
+        ``og`` is the output gate from :meth:`_projections`.  With ``residual``
+        their sum, with ``out`` written there."""
+        gate = self._output_gate(og)
         if gate.dtype != o_core.dtype:
             gate = gate.to(o_core.dtype)
-        return self.o_proj(kda_output(o_core, gate, self.g_norm.weight, self.g_norm.eps))
+        return _project(self.o_proj, kda_output(o_core, gate, self.g_norm.weight, self.g_norm.eps), residual, out)
 
     def decode_step_(self, x, state):
         """One cached decode token (x: [B, 1, d]) that updates ``state`` in
@@ -318,17 +355,21 @@ class KimiDeltaAttention(nn.Module):
         the reference instead copies each new state back into its static
         buffers (``graph_decode.py:257-262``), a full extra read and write of
         the state per layer and token."""
+        return self._decode(x, state)
+
+    def _decode(self, x, state, residual=None, out=None):
+        """:meth:`decode_step_`, plus ``residual`` [B, 1, d], into ``out`` [B, 1, d]."""
         if x.shape[1] != 1:
             raise ValueError(f"decode_step_ takes one token, got x of shape {tuple(x.shape)}")
-        q, k, v, gk, bl, _, og_low = self._projections(x, conv_cache=state["conv"], use_cache=True,
-                                                       conv_out=state["conv"])
+        q, k, v, gk, bl, _, og = self._projections(x, conv_cache=state["conv"], use_cache=True,
+                                                   conv_out=state["conv"])
         rec = state["recurrent"]
         if rec is None:
             raise ValueError("decode_step_ needs an allocated recurrent state (run a prefill first)")
         a_log, dt_bias = self._gate_params()
         o_core, _ = kda_recurrent_gated(q, k, v, gk, bl, a_log, dt_bias, state=rec, state_dtype=rec.dtype,
                                         state_out=rec)
-        return self._output(o_core, og_low)
+        return self._output(o_core, og, residual, out)
 
     def _train_forward(self, x):
         """The layer's forward for training (``kda.py:473-536`` differentiated by
@@ -394,16 +435,15 @@ class KimiDeltaAttention(nn.Module):
         # H=16 d=128: 179 against 347 us for the core).
         split = (not fused and not (use_cache and T == 1) and body > 0 and (B == 1 or body == T)
                  and long_segments(B, body, self.num_heads, self.head_dim, self.value_head_dim, x.dtype) > 1)
-        q, k, v, g, beta, new_conv, og_low = self._projections(x, conv_cache=conv_cache, use_cache=use_cache,
-                                                               gates=split)
+        q, k, v, g, beta, new_conv, og = self._projections(x, conv_cache=conv_cache, use_cache=use_cache,
+                                                           gates=split)
         gate = self._gate_params()      # unless split, g and beta above are gk and the beta logits
         if fused:
             # one chunkwise body and no tail: the output epilogue runs on the
             # chunk kernel's tiles and its result is the o_proj input
-            og = self.og_proj[1](og_low)
-            y, new_rec = kda_chunkwise_fused(q, k, v, g, beta, *gate, og, self.g_norm.weight, self.g_norm.eps,
+            y, new_rec = kda_chunkwise_fused(q, k, v, g, beta, *gate, self._output_gate(og), self.g_norm.weight, self.g_norm.eps,
                                              initial_state=rec, chunk_size=C, state_dtype=sdtype)
-            out = self.o_proj(y)
+            out = _project(self.o_proj, y)
             if use_cache:
                 return out, {"conv": new_conv, "recurrent": new_rec}
             return out
@@ -442,7 +482,7 @@ class KimiDeltaAttention(nn.Module):
             if o_core is None:
                 o_core = x.new_zeros(B, T, self.num_heads, self.value_head_dim)
             new_rec = rec
-        out = self._output(o_core, og_low)
+        out = self._output(o_core, og)
         if use_cache:
             return out, {"conv": new_conv, "recurrent": new_rec}
         return out

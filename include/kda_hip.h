@@ -360,6 +360,28 @@ typedef struct kda_output_args {
 
 int kda_output_fwd(const kda_output_args* args, void* stream);
 
+/* y[i] = x[i] W[i]^T for few rows: a decode step's projections, which are reads
+ * of their weights (nn.Linear without a bias, kimi_linear/kda.py:345-384).  One
+ * matrix, or two of one K in one launch (x[1] not NULL).  Sums in fp32, the
+ * result rounded to the activation type.  residual (one matrix only):
+ * y = residual + that rounded result, the add of a residual stream.  K a
+ * multiple of 32, N of 16, at most 16 rows (32 for K <= 1024, 64 for K <= 512);
+ * x rows and weights 16-byte aligned, residual rows and y 8-byte; other calls return KDA_ERR_UNSUPPORTED.  y overlaps no input. */
+typedef struct kda_linear_args {
+    int64_t M;                     /* rows */
+    int64_t K;
+    int64_t N[2];
+    const void* x[2];              /* [M, K] */
+    int64_t x_stride[2];           /* row strides in elements */
+    const void* w[2];              /* [N, K] contiguous */
+    void* y[2];                    /* [M, N] contiguous */
+    const void* residual;          /* [M, N[0]] or NULL */
+    int64_t residual_stride;
+    int32_t dtype;                 /* KDA_DTYPE_F16 or KDA_DTYPE_BF16, of all tensors */
+} kda_linear_args;
+
+int kda_linear_fwd(const kda_linear_args* args, void* stream);
+
 /* Gradients of kda_prep_fwd, for training through the layer (the reference
  * differentiates _projections, kimi_linear/kda.py:399-461, by autograd;
  * scripts/train_musicgpt_fp16.py:519-523 trains the whole layer).  Given dy,
