@@ -151,7 +151,8 @@ EXPORTED_SYMBOLS = ("kda_chunkwise_fwd", "kda_recurrent_fwd", "kda_chunkwise_fwd
                     "kda_chunkwise_bwd",
                     "kda_chunkwise_bwd_workspace_size", "kda_chunkwise_bwd_noalloc",
                     "kda_chunkwise_split_fwd", "kda_chunkwise_split_workspace_size",
-                    "kda_prep_fwd", "kda_output_fwd", "kda_linear_fwd", "kda_prep_bwd", "kda_prep_bwd_workspace_size",
+                    "kda_prep_fwd", "kda_output_fwd", "kda_linear_fwd", "kda_linear_wgrad",
+                    "kda_linear_wgrad_workspace_size", "kda_prep_bwd", "kda_prep_bwd_workspace_size",
                     "kda_output_bwd", "kda_output_bwd_workspace_size", "kda_status_str", "kda_abi_version")
 
 _lib = None
@@ -213,6 +214,10 @@ def load() -> ctypes.CDLL:
         lib.kda_output_fwd.restype = ctypes.c_int
         lib.kda_linear_fwd.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
         lib.kda_linear_fwd.restype = ctypes.c_int
+        lib.kda_linear_wgrad.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+        lib.kda_linear_wgrad.restype = ctypes.c_int
+        lib.kda_linear_wgrad_workspace_size.argtypes = [ctypes.c_int64] * 3
+        lib.kda_linear_wgrad_workspace_size.restype = ctypes.c_size_t
         lib.kda_prep_bwd.argtypes = [ctypes.POINTER(KdaPrepBwdArgs), ctypes.c_void_p]
         lib.kda_prep_bwd.restype = ctypes.c_int
         lib.kda_prep_bwd_workspace_size.argtypes = [ctypes.c_int64] * 6

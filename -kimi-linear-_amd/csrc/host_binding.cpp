@@ -47,6 +47,8 @@ struct Fns {
     decltype(&kda_prep_fwd) prep = nullptr;
     decltype(&kda_output_fwd) output = nullptr;
     decltype(&kda_linear_fwd) linear = nullptr;
+    decltype(&kda_linear_wgrad) wgrad = nullptr;
+    decltype(&kda_linear_wgrad_workspace_size) wgrad_ws = nullptr;
 };
 Fns fn;
 // torch._C._cuda_getCurrentRawStream; kept for the process's life
@@ -71,6 +73,8 @@ void bind(const py::dict& addr, const py::object& stream_fn) {
     take(fn.prep, addr, "kda_prep_fwd");
     take(fn.output, addr, "kda_output_fwd");
     take(fn.linear, addr, "kda_linear_fwd");
+    take(fn.wgrad, addr, "kda_linear_wgrad");
+    take(fn.wgrad_ws, addr, "kda_linear_wgrad_workspace_size");
     Py_INCREF(stream_fn.ptr());
     raw_stream = stream_fn.ptr();
 }
@@ -434,6 +438,40 @@ py::object linear2(const Tensor& x0, const Tensor& w0, const Tensor& x1, const T
     return py::make_tuple(y0, y1);
 }
 
+// Rows of [B, T, D] one stride apart.
+bool one_stride(const Tensor& t) {
+    return t.stride(2) == 1 && (t.size(0) == 1 || t.size(1) == 1 || t.stride(0) == t.size(1) * t.stride(1));
+}
+
+// dy^T x over the tokens, [N, K], or None for the calls of the library product.
+py::object linear_wgrad(const Tensor& dy, const Tensor& x) {
+    Plain plain(dy);
+    plain.add(x);
+    const auto dt = dy.scalar_type();
+    if (!plain.ok || (dt != at::kHalf && dt != at::kBFloat16) || x.scalar_type() != dt || dy.dim() != 3 ||
+        x.dim() != 3 || dy.size(0) != x.size(0) || dy.size(1) != x.size(1) || dy.numel() == 0 || x.numel() == 0 ||
+        !one_stride(dy) || !one_stride(x))
+        return py::none();
+    kda_linear_wgrad_args a{};
+    a.M = dy.size(0) * dy.size(1);
+    a.N = dy.size(2);
+    a.K = x.size(2);
+    const size_t bytes = fn.wgrad_ws(a.M, a.N, a.K);
+    if (bytes == 0) return py::none();
+    const c10::DeviceGuard guard(plain.dev);
+    const auto opt = x.options().requires_grad(false);
+    Tensor dw = at::empty({a.N, a.K}, opt), ws = at::empty({static_cast<int64_t>(bytes)}, opt.dtype(at::kByte));
+    a.dy = dy.data_ptr();
+    a.dy_stride = row_stride(dy);
+    a.x = x.data_ptr();
+    a.x_stride = row_stride(x);
+    a.dw = dw.data_ptr();
+    a.workspace = ws.data_ptr();
+    a.dtype = code(x);
+    if (fn.wgrad(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    return py::cast(dw);
+}
+
 // What decides whether a copy made of these parameters is still theirs:
 // storage address, version, type and device of each.
 py::bytes params_key(const std::vector<Tensor>& params) {
@@ -459,5 +497,6 @@ PYBIND11_MODULE(_kda_host, m) {
     m.def("output", &output);
     m.def("linear", &linear);
     m.def("linear2", &linear2);
+    m.def("linear_wgrad", &linear_wgrad);
     m.def("params_key", &params_key);
 }

@@ -271,6 +271,24 @@ int kda_linear_fwd(const kda_linear_args* a, void* stream) {
     return kda::linear_launch(*a, static_cast<hipStream_t>(stream));
 }
 
+size_t kda_linear_wgrad_workspace_size(int64_t M, int64_t N, int64_t K) {
+    if (!kda::linear_wgrad_supported(M, N, K)) return 0;
+    return static_cast<size_t>(kda::linear_wgrad_workspace_bytes(M, N, K));
+}
+
+int kda_linear_wgrad(const kda_linear_wgrad_args* a, void* stream) {
+    if (a == nullptr) return KDA_ERR_NULL_POINTER;
+    if (a->M < 0 || a->N < 0 || a->K < 0) return KDA_ERR_BAD_SHAPE;
+    if (a->dtype != KDA_DTYPE_F16 && a->dtype != KDA_DTYPE_BF16) return KDA_ERR_BAD_DTYPE;
+    if (!kda::linear_wgrad_supported(a->M, a->N, a->K)) return KDA_ERR_UNSUPPORTED;
+    if (!a->dy || !a->x || !a->dw || !a->workspace) return KDA_ERR_NULL_POINTER;
+    const auto at = [](const void* p, uintptr_t n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
+    if (!at(a->dy, 8) || !at(a->x, 8) || !at(a->dw, 8) || !at(a->workspace, 16) || a->dy_stride % 4 != 0 ||
+        a->x_stride % 4 != 0)
+        return KDA_ERR_UNSUPPORTED;
+    return kda::linear_wgrad_launch(*a, static_cast<hipStream_t>(stream));
+}
+
 const char* kda_status_str(int status) {
     switch (status) {
         case KDA_OK: return "ok";

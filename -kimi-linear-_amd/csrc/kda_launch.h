@@ -75,5 +75,8 @@ int chunkwise_bwd_scratch(void** ptr);
 // y = x W^T of few rows (kda_linear.hip); shapes and alignment checked by the caller.
 bool linear_supported(const kda_linear_args& a);
 int linear_launch(const kda_linear_args& a, hipStream_t stream);
+bool linear_wgrad_supported(int64_t M, int64_t N, int64_t K);
+int64_t linear_wgrad_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int linear_wgrad_launch(const kda_linear_wgrad_args& a, hipStream_t stream);
 
 }  // namespace kda

@@ -37,6 +37,15 @@ template <> struct Mat<bf16_t> {
     }
 };
 
+// Four neighbouring elements in one store.
+template <typename T>
+__device__ __forceinline__ void store4(T* p, f4 v) {
+    struct alignas(4 * sizeof(T)) { T e[4]; } out;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) Elem<T>::st(&out.e[j], v[j]);
+    __builtin_memcpy(__builtin_assume_aligned(p, 4 * sizeof(T)), &out, sizeof(out));
+}
+
 constexpr int kDepth = 8;        // steps whose loads are in flight together
 
 // N steps of 32 from the lane's addresses on.
@@ -113,7 +122,6 @@ __global__ __launch_bounds__(64 * SPLIT) void linear_kernel(kda_linear_args a) {
         }
         const int64_t row = 16 * (i % MT) + ln, n = n0 + 16 * (i / MT) + 4 * lg;
         if (row >= a.M || n >= N) continue;
-        T out[4];
         if (a.residual) {
             const uint2 raw = *reinterpret_cast<const uint2*>(static_cast<const T*>(a.residual) +
                                                               row * a.residual_stride + n);
@@ -122,11 +130,7 @@ __global__ __launch_bounds__(64 * SPLIT) void linear_kernel(kda_linear_args a) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) r[j] = Elem<T>::ld(&res[j]) + round_elem<T>(r[j]);
         }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) Elem<T>::st(&out[j], r[j]);
-        uint2 raw;
-        __builtin_memcpy(&raw, out, 8);
-        *reinterpret_cast<uint2*>(static_cast<T*>(a.y[mat]) + row * N + n) = raw;
+        store4(static_cast<T*>(a.y[mat]) + row * N + n, r);
     }
 }
 
@@ -160,6 +164,153 @@ int launch_type(const kda_linear_args& a, hipStream_t stream) {
     return a.N[0] >= 6144 ? launch_rows<T, 2>(a, stream) : launch_rows<T, 1>(a, stream);
 }
 
+// ---- dW = dy^T x over many rows --------------------------------------------
+// The weight gradient of the gates' up-projections: few outputs (N K =
+// 2048 x 128) that each sum over every token, which the library's product
+// leaves to 64 workgroups.  A wave takes 64 rows and 128 columns of dW and a
+// share of the tokens, 32 a step; four waves meet in LDS and the workgroups'
+// sums, enough of them to fill the chip, in a second kernel, both in a fixed
+// order.  Both operands have the contraction along their rows: a lane loads 4
+// neighbouring channels of 8 tokens and turns them into four fragments of 8
+// tokens in registers, so the tile's rows are n0 + 4 i + j for fragment j, and
+// four column fragments end in 16 contiguous bytes of dW.
+// The loads bound it: one step of each wave is in flight behind the current
+// one, with 128 accumulators a wave leaving room for one wave a SIMD.  us in
+// a graph of 40, bf16, library / here: 8192 tokens, N = 2048 63.5 / 20.2
+// (1.7 TB/s of dy), 32768 tokens 150 / 59.6, N = 512 at 8192 tokens 63.8 /
+// 15.8; 1024 tokens, N = 2048 11.3 / 10.5, 256 tokens 6.5 / 6.6.
+constexpr int kWgN = 64, kWgK = 128;
+
+struct Rows8 {
+    uint2 r[8];
+};
+// 8 tokens' 4 channels -> fragment J: channel J of the 8 tokens
+template <int J>
+__device__ __forceinline__ uint4 frag(const Rows8& v) {
+    constexpr uint32_t sel = J % 2 == 0 ? 0x05040100u : 0x07060302u;
+    const auto word = [&](int i) { return J / 2 == 0 ? v.r[i].x : v.r[i].y; };
+    return uint4{__builtin_amdgcn_perm(word(1), word(0), sel), __builtin_amdgcn_perm(word(3), word(2), sel),
+                 __builtin_amdgcn_perm(word(5), word(4), sel), __builtin_amdgcn_perm(word(7), word(6), sel)};
+}
+
+template <typename T>
+__device__ __forceinline__ void load_rows(Rows8& v, const T* p, int64_t stride, int64_t row, int64_t M) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v.r[i] = *reinterpret_cast<const uint2*>(p + min(row + i, M - 1) * stride);
+    if (row + 8 > M) {                                  // tokens past the last count as zero
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (row + i >= M) v.r[i] = uint2{0, 0};
+    }
+}
+
+// Grid (N / 64 * K / 128, splits); out: fp32 [splits, N, K], or one split's dw itself.
+template <typename T, typename OT>
+__global__ __launch_bounds__(256) void wgrad_kernel(kda_linear_wgrad_args a, OT* out, int64_t per) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ln = lane & 15, lg = lane >> 4;
+    const int64_t nt = a.N / kWgN;
+    const int64_t n0 = blockIdx.x % nt * kWgN, k0 = blockIdx.x / nt * kWgK;
+    const T* dy = static_cast<const T*>(a.dy) + n0 + 4 * ln;
+    const T* x = static_cast<const T*>(a.x) + k0 + 4 * ln;
+    const int64_t end = min((static_cast<int64_t>(blockIdx.y) + 1) * per, (a.M + 31) / 32);
+    int64_t s = static_cast<int64_t>(blockIdx.y) * per + wave;
+
+    f4 acc[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    Rows8 na, nb[2];
+    const auto fetch = [&](int64_t step) {
+        const int64_t row = 32 * step + 8 * lg;
+        load_rows(na, dy, a.dy_stride, row, a.M);
+        load_rows(nb[0], x, a.x_stride, row, a.M);
+        load_rows(nb[1], x + 64, a.x_stride, row, a.M);
+    };
+    if (s < end) fetch(s);
+    for (; s < end; s += 4) {
+        const uint4 fa[4] = {frag<0>(na), frag<1>(na), frag<2>(na), frag<3>(na)};
+        const uint4 fb[8] = {frag<0>(nb[0]), frag<1>(nb[0]), frag<2>(nb[0]), frag<3>(nb[0]),
+                             frag<0>(nb[1]), frag<1>(nb[1]), frag<2>(nb[1]), frag<3>(nb[1])};
+        if (s + 4 < end) fetch(s + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[i][j] = Mat<T>::mma(fa[i], fb[j], acc[i][j]);
+    }
+
+    // waves 2 and 3 hand their sums to 0 and 1; those exchange halves
+    __shared__ f4 red[2][32][64];
+    if (wave >= 2) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) red[wave - 2][i][lane] = acc[i / 8][i % 8];
+    }
+    __syncthreads();
+    if (wave < 2) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) acc[i / 8][i % 8] += red[wave][i][lane];
+    }
+    __syncthreads();
+    if (wave < 2) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i)
+            if (i / 16 != wave) red[wave][i][lane] = acc[i / 8][i % 8];
+    }
+    __syncthreads();
+    if (wave >= 2) return;
+    out += static_cast<int64_t>(blockIdx.y) * a.N * a.K;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (i / 2 != wave) continue;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] += red[1 - wave][8 * i + j][lane];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t n = n0 + 4 * (4 * lg + q) + i;
+                store4(out + n * a.K + k0 + 64 * h + 4 * ln,
+                       f4{acc[i][4 * h][q], acc[i][4 * h + 1][q], acc[i][4 * h + 2][q], acc[i][4 * h + 3][q]});
+            }
+    }
+}
+
+// dw[e] = the sum of the splits' shares, in order; four elements a thread.
+template <typename T>
+__global__ __launch_bounds__(256) void wgrad_sum_kernel(const float* part, T* dw, int64_t n, int splits) {
+    const int64_t e = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (e >= n) return;
+    f4 s = *reinterpret_cast<const f4*>(part + e);
+#pragma unroll 8
+    for (int i = 1; i < splits; ++i) s += *reinterpret_cast<const f4*>(part + i * n + e);
+    store4(dw + e, s);
+}
+
+// One workgroup a CU, each with at least two steps a wave.
+int64_t wgrad_splits(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = (N / kWgN) * (K / kWgK), steps = (M + 31) / 32;
+    return max(int64_t{1}, min(256 / tiles, steps / 8));
+}
+
+template <typename T>
+int launch_wgrad(const kda_linear_wgrad_args& a, hipStream_t stream) {
+    const int64_t splits = wgrad_splits(a.M, a.N, a.K), steps = (a.M + 31) / 32;
+    const int64_t per = (steps + splits - 1) / splits;
+    const dim3 grid(static_cast<unsigned>((a.N / kWgN) * (a.K / kWgK)), static_cast<unsigned>(splits));
+    if (splits == 1) {
+        wgrad_kernel<T, T><<<grid, 256, 0, stream>>>(a, static_cast<T*>(a.dw), per);
+        return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
+    }
+    float* part = static_cast<float*>(a.workspace);
+    wgrad_kernel<T, float><<<grid, 256, 0, stream>>>(a, part, per);
+    if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
+    const int64_t n = a.N * a.K;
+    wgrad_sum_kernel<T><<<static_cast<unsigned>((n / 4 + 255) / 256), 256, 0, stream>>>(part, static_cast<T*>(a.dw), n,
+                                                                                        static_cast<int>(splits));
+    return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
+}
+
 }  // namespace
 
 // The shapes this kernel is the better one for.  Each workgroup reads all rows
@@ -180,6 +331,18 @@ bool linear_supported(const kda_linear_args& a) {
 
 int linear_launch(const kda_linear_args& a, hipStream_t stream) {
     return a.dtype == KDA_DTYPE_F16 ? launch_type<_Float16>(a, stream) : launch_type<bf16_t>(a, stream);
+}
+
+// From 512 tokens on (measured above); up to 64 tiles, beyond which the
+// library's product has workgroups enough by itself.
+bool linear_wgrad_supported(int64_t M, int64_t N, int64_t K) {
+    return M >= 512 && N > 0 && K > 0 && N % kWgN == 0 && K % kWgK == 0 && N <= 4096 && K <= 4096 &&
+           (N / kWgN) * (K / kWgK) <= 64 && M <= int64_t{1} << 40;
+}
+int64_t linear_wgrad_workspace_bytes(int64_t M, int64_t N, int64_t K) { return wgrad_splits(M, N, K) * N * K * 4; }
+
+int linear_wgrad_launch(const kda_linear_wgrad_args& a, hipStream_t stream) {
+    return a.dtype == KDA_DTYPE_F16 ? launch_wgrad<_Float16>(a, stream) : launch_wgrad<bf16_t>(a, stream);
 }
 
 }  // namespace kda

@@ -133,6 +133,36 @@ def linear_attn_config(**kw) -> SimpleNamespace:
     return SimpleNamespace(linear_attn_config=la, **top)
 
 
+class _LinearFn(torch.autograd.Function):
+    """x W^T whose weight gradient, a few outputs that sum over every token, has
+    a kernel (``kda_linear_wgrad``); the rest are library products."""
+
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return torch.nn.functional.linear(x, w)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        dx = torch.matmul(dy, w) if ctx.needs_input_grad[0] else None
+        dw = None
+        if ctx.needs_input_grad[1]:
+            dw = _native.host().linear_wgrad(dy, x)
+            if dw is None:
+                dw = torch.matmul(dy.reshape(-1, dy.shape[-1]).t(), x.reshape(-1, x.shape[-1]))
+        return dx, dw
+
+
+def _project_train(mod, x):
+    """``mod(x)``, differentiable; :class:`_LinearFn` where that is all the module does."""
+    w = _plain_weight(mod)
+    if (w is None or mod._backward_hooks or mod._backward_pre_hooks or w.dtype != x.dtype
+            or x.dtype not in (torch.float16, torch.bfloat16) or torch.is_autocast_enabled(x.device.type)):
+        return mod(x)
+    return _LinearFn.apply(x, w)
+
+
 def _plain_weight(mod):
     """The weight of a module that is just x W^T: an ``nn.Linear`` as torch has it,
     without a bias, hooks or a forward of its own; else None."""
@@ -397,13 +427,13 @@ class KimiDeltaAttention(nn.Module):
         if T == 0:
             return self.o_proj(x.new_zeros(B, 0, H * V))
         convs = (self.conv_q.conv, self.conv_k.conv, self.conv_v.conv)
-        gk = self.gk_proj[1](gk_low)
+        gk = _project_train(self.gk_proj[1], gk_low)
         q, k, v, g, beta = kda_prep_train(q_in, k_in, v_in, tuple(c.weight for c in convs),
                                           tuple(c.bias for c in convs), gk, self.A_log, self.dt_bias, beta_logit,
                                           num_heads=H, head_dim=K, value_head_dim=V, l2_eps=self.l2norm_eps)
         C = self.chunk_size if T % self.chunk_size == 0 else T
         o_core, _ = kda_chunkwise(q, k, v, g, beta, chunk_size=C, state_dtype=self._state_dtype(x))
-        gate = self.og_proj[1](og_low)
+        gate = _project_train(self.og_proj[1], og_low)
         if gate.dtype != o_core.dtype:
             gate = gate.to(o_core.dtype)
         return self.o_proj(kda_output_train(o_core, gate, self.g_norm.weight, self.g_norm.eps))

@@ -382,6 +382,26 @@ typedef struct kda_linear_args {
 
 int kda_linear_fwd(const kda_linear_args* args, void* stream);
 
+/* dw = dy^T x, the gradient of a small weight (the gates' up-projections) from
+ * many rows.  Sums in fp32, rounded to the activation type once, in a fixed
+ * order.  M at least 512, N a multiple of 64, K of 128, N K at most 64 * 64 * 128; dy and x rows
+ * 8-byte aligned, dw 8-byte, workspace 16-byte and
+ * kda_linear_wgrad_workspace_size() bytes (0: no kernel for the shape); other
+ * calls return KDA_ERR_UNSUPPORTED. */
+typedef struct kda_linear_wgrad_args {
+    int64_t M, N, K;
+    const void* dy;                /* [M, N] */
+    int64_t dy_stride;             /* row strides in elements */
+    const void* x;                 /* [M, K] */
+    int64_t x_stride;
+    void* dw;                      /* [N, K] contiguous */
+    void* workspace;
+    int32_t dtype;                 /* KDA_DTYPE_F16 or KDA_DTYPE_BF16, of all tensors */
+} kda_linear_wgrad_args;
+
+size_t kda_linear_wgrad_workspace_size(int64_t M, int64_t N, int64_t K);
+int kda_linear_wgrad(const kda_linear_wgrad_args* args, void* stream);
+
 /* Gradients of kda_prep_fwd, for training through the layer (the reference
  * differentiates _projections, kimi_linear/kda.py:399-461, by autograd;
  * scripts/train_musicgpt_fp16.py:519-523 trains the whole layer).  Given dy,

@@ -93,3 +93,55 @@ def test_modules_with_a_behaviour_of_their_own_are_called(kda_pkg):
         mod.forward = lambda a: a.new_ones(1, 1, 32)
         assert torch.equal(layer._project(mod, x), torch.ones_like(x[..., :32]))
     assert layer._plain_weight(torch.nn.Linear(64, 32)) is None           # a bias
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(512, 64, 128), (513, 2048, 128), (545, 64, 256), (1000, 1024, 128),
+                                   (8192, 2048, 128), (8225, 64, 128)])
+def test_weight_gradient(host, M, N, K, dtype):
+    """dy^T x: rows left over by a step, by the waves and by the splits, strided
+    rows.  Bound: the result's rounding and M fp32 additions."""
+    gen = torch.Generator().manual_seed(M)
+    dy = torch.randn(M, N, generator=gen).to(dtype).to(DEV)
+    big = torch.full((1, M, K + 24), float("nan"), dtype=dtype, device=DEV)
+    big[0, :, 8:K + 8] = torch.randn(M, K, generator=gen).to(dtype)
+    x = big[..., 8:K + 8]
+    dw = host.linear_wgrad(dy.view(1, M, N), x)
+    assert torch.equal(dw, host.linear_wgrad(dy.view(1, M, N), x))
+    check_bound = dy.double().t() @ x[0].double()
+    mag = dy.double().abs().t() @ x[0].double().abs()
+    ulp = 2.0 ** (-11 if dtype == torch.float16 else -8)
+    assert bool(((dw.double() - check_bound).abs() <= ulp * check_bound.abs() + M * 2.0 ** -24 * mag + 2.0 ** -24).all())
+
+
+@pytest.mark.gpu
+def test_weight_gradient_left_to_the_library(host):
+    dy = torch.zeros(2, 300, 64, device=DEV, dtype=torch.float16)
+    x = torch.zeros(2, 300, 128, device=DEV, dtype=torch.float16)
+    assert host.linear_wgrad(dy, x) is not None
+    assert host.linear_wgrad(dy[..., :32], x[..., :32]) is None
+    assert host.linear_wgrad(dy.float(), x.float()) is None
+    assert host.linear_wgrad(dy, x.bfloat16()) is None
+    assert host.linear_wgrad(dy[:, :280], x[:, :280]) is None             # rows of two strides
+    assert host.linear_wgrad(dy[:1], x[:1]) is None                       # 300 tokens
+    assert host.linear_wgrad(dy[:, :0], x[:, :0]) is None
+    odd = torch.zeros(2, 300, 130, device=DEV, dtype=torch.float16)
+    assert host.linear_wgrad(dy, odd[..., 1:129]) is None                 # rows not 8-byte aligned
+
+
+@pytest.mark.gpu
+def test_linear_function_gradients(kda_pkg):
+    """The training path's up-projection against autograd's own linear layer."""
+    layer = importlib.import_module("kimi_linear_amd.layer")
+    mod = torch.nn.Linear(128, 256, bias=False, device=DEV, dtype=torch.float16)
+    x = torch.randn(2, 400, 128, device=DEV, dtype=torch.float16, requires_grad=True)
+    dy = torch.randn(2, 400, 256, device=DEV, dtype=torch.float16)
+    y, ref = layer._project_train(mod, x), mod(x)
+    assert torch.equal(y, ref) and type(y.grad_fn).__name__ == "_LinearFnBackward"
+    dx, dw = torch.autograd.grad(y, (x, mod.weight), dy)
+    rx, rw = torch.autograd.grad(ref, (x, mod.weight), dy)
+    for a, b in ((dx, rx), (dw, rw)):       # two roundings of sums of 800 products, a few tens in size
+        assert bool(((a.double() - b.double()).abs() <= 2.0 ** -10 * b.double().abs() + 800 * 2.0 ** -23 * 60).all())
+    mod.register_full_backward_hook(lambda *a: None)
+    assert type(layer._project_train(mod, x).grad_fn).__name__ != "_LinearFnBackward"
