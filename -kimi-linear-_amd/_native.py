@@ -14,7 +14,7 @@ from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libkda_hip.so"
 HOST_PATH = Path(__file__).resolve().parent / "_kda_host.so"     # csrc/host_binding.cpp
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 DTYPE_F32 = 0
 DTYPE_F16 = 1
@@ -128,6 +128,7 @@ class KdaPrepBwdArgs(ctypes.Structure):
         ("da_log", ctypes.c_void_p), ("ddt_bias", ctypes.c_void_p),
         ("l2_eps", ctypes.c_float), ("x_dtype", ctypes.c_int32),
         ("workspace", ctypes.c_void_p),
+        ("dx_stride", ctypes.c_int64), ("typed_param_grads", ctypes.c_int32),
     ]
 
 
@@ -141,7 +142,7 @@ class KdaOutputBwdArgs(ctypes.Structure):
         ("weight", ctypes.c_void_p), ("w_dtype", ctypes.c_int32),
         ("dy", ctypes.c_void_p), ("d_o", ctypes.c_void_p), ("dgate", ctypes.c_void_p),
         ("dweight", ctypes.c_void_p), ("eps", ctypes.c_float), ("x_dtype", ctypes.c_int32),
-        ("workspace", ctypes.c_void_p),
+        ("workspace", ctypes.c_void_p), ("typed_param_grads", ctypes.c_int32),
     ]
 
 

@@ -6,15 +6,14 @@
 // scripts/train_musicgpt_fp16.py:519-523).  The core has its own backward
 // (kda_chunkwise_bwd); these kernels carry the gradients the rest of the way:
 //
-//   prep_bwd_kernel, one wave per (batch, 64-token tile, tensor, head), lanes
-//     across the head's channels as in the forward.  q, k, v: the forward is
-//     re-evaluated from the saved projections (conv, SiLU, L2 norm), then
+//   prep_bwd_kernel, one workgroup per (batch, 64-token tile, run of channels),
+//     eight channels a lane as in the forward.  q, k, v: the forward is re-evaluated
+//     from the saved projections (conv, SiLU, L2 norm), then
 //       ds = rn dy - s rn^3 <s, dy>      (L2 norm; ds = dy / eps when clamped)
 //       du = ds sigmoid(u) (1 + u (1 - sigmoid(u)))          (SiLU)
 //       dx[t] = sum_j w[j] du[t + cm - j]                     (causal conv)
 //     and the tile's shares of dw[j] = sum_t du[t] x[t - cm + j], db = sum du.
-//     An 8-token step needs du for cm rows past itself: those are evaluated
-//     again by the next step (short steps keep the wave's registers few).  Gates: dgk = dg (-exp(A_log)) sigmoid(z),
+//     Gates: dgk = dg (-exp(A_log)) sigmoid(z),
 //     dbeta_logit = dbeta beta (1 - beta), and the tile's shares of
 //     dA_log = sum dg g and ddt_bias = sum dgk.
 //   output_bwd_kernel, one wave per (batch, 32-token tile, head):
@@ -27,26 +26,19 @@
 // Both are HBM-streaming: every input element is read once per use (plus the
 // conv halo), every gradient written once.
 #include "kda_common.h"
+#include "kda_rows.h"
 
 namespace kda {
 
 namespace {
 
 constexpr int kMaxConvB = 4;      // largest conv_size (as the forward)
-constexpr int kStep = 8;          // tokens per step of a prep unit
-constexpr int kPrepTile = 64;     // tokens per prep unit
+constexpr int kGroup = 4;         // tokens per step of a conv unit: the convolution's window, so a row's slot is its index
+constexpr int kStep = 8;          // tokens per step of a gate unit
+constexpr int kPrepTile = 64;     // tokens per prep unit, a workgroup's
+constexpr int kSub = 4;           // its waves, a quarter of the tile each
 constexpr int kOutStep = 8;       // tokens per step of an output unit
 constexpr int kOutTile = 32;      // tokens per output unit
-
-template <typename XT> __device__ __forceinline__ float to_f(XT x);
-template <> __device__ __forceinline__ float to_f<float>(float x) { return x; }
-template <> __device__ __forceinline__ float to_f<_Float16>(_Float16 x) { return static_cast<float>(x); }
-template <> __device__ __forceinline__ float to_f<bf16_t>(bf16_t x) { return bf16_bits_to_f32(x.bits); }
-
-template <typename XT> __device__ __forceinline__ XT from_f(float x);
-template <> __device__ __forceinline__ float from_f<float>(float x) { return x; }
-template <> __device__ __forceinline__ _Float16 from_f<_Float16>(float x) { return static_cast<_Float16>(x); }
-template <> __device__ __forceinline__ bf16_t from_f<bf16_t>(float x) { return bf16_t{f32_to_bf16_bits(x)}; }
 
 template <typename XT, int CPL>
 struct alignas(sizeof(XT) * CPL) Vec {
@@ -100,234 +92,267 @@ int64_t prep_ws_floats(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, in
     return prep_rows(B, T) * ((2 * H * K + H * V) * (cs + 1) + 2 * H * K);
 }
 
-// ---- q, k or v: one head over a 64-token tile ------------------------------
-template <typename XT, int CPL>
-__device__ void conv_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int i, int64_t b, int64_t tile,
-                              int64_t h, int lane) {
-    constexpr int R = kStep + kMaxConvB - 1;   // du rows of a step: its own and cm more
-    constexpr int W = R + kMaxConvB - 1;       // x rows those need
-    const int64_t Dh = 64 * CPL;
-    const int64_t D = a.H * Dh;
-    const int64_t ch0 = h * Dh + lane * CPL;
-    const int cs = static_cast<int>(a.conv_size), cm = cs - 1;
-    const int64_t T = a.T;
-    const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0] + ch0;
-    const XT* dy = static_cast<const XT*>(a.dy[i]) + b * T * D + ch0;
-    XT* dx = static_cast<XT*>(a.dx[i]) + b * T * D + ch0;
-
-    RawElem rw[kMaxConvB][CPL], rb[CPL];
+// Sums over the waves of a tile, in their order; wave 0 has them.
+template <int N>
+__device__ __forceinline__ void sum_waves(float (&v)[N], float* red, int wave, int lane) {
+    if (wave > 0) {
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        rb[c] = load_raw_elem(a.conv_b[i] != nullptr ? a.conv_b[i] : a.conv_w[i],
-                              a.conv_b[i] != nullptr ? ch0 + c : 0, a.w_dtype);
-#pragma unroll
-        for (int j = 0; j < kMaxConvB; ++j)
-            rw[j][c] = load_raw_elem(a.conv_w[i], j < cs ? (ch0 + c) * cs + j : 0, a.w_dtype);
+        for (int i = 0; i < N; ++i) red[((wave - 1) * N + i) * 64 + lane] = v[i];
     }
-    float w[kMaxConvB][CPL], bias[CPL];
+    __syncthreads();
+    if (wave == 0) {
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        bias[c] = a.conv_b[i] != nullptr ? decode_elem(rb[c], a.w_dtype) : 0.f;
+        for (int w = 0; w < kSub - 1; ++w)
 #pragma unroll
-        for (int j = 0; j < kMaxConvB; ++j) w[j][c] = j < cs ? decode_elem(rw[j][c], a.w_dtype) : 0.f;
-    }
-    // the taps in reverse, wr[j] = w[cm - j]: dx[t] = sum_j wr[j] du[t + j]
-    float wr[kMaxConvB][CPL];
-#pragma unroll
-    for (int jp = 0; jp < kMaxConvB; ++jp)
-#pragma unroll
-        for (int c = 0; c < CPL; ++c) {
-            float v = 0.f;
-#pragma unroll
-            for (int j = 0; j < kMaxConvB; ++j) v = j + jp == cm ? w[j][c] : v;
-            wr[jp][c] = v;
-        }
-    const float inv_eps = 1.f / a.l2_eps;
-
-    float dws[kMaxConvB][CPL], dbs[CPL];
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        dbs[c] = 0.f;
-#pragma unroll
-        for (int j = 0; j < kMaxConvB; ++j) dws[j][c] = 0.f;
-    }
-    const int64_t t0 = tile * kPrepTile;
-    for (int step = 0; step < kPrepTile / kStep; ++step) {
-        const int64_t s0 = t0 + step * kStep;
-        if (s0 >= T) break;
-        // x row r is token s0 - cm + r, dy and du row r token s0 + r; rows
-        // outside [0, T) read a valid row and count as zero
-        float xw[W][CPL], dyr[R][CPL];
-#pragma unroll
-        for (int r = 0; r < W; ++r) {
-            const int64_t tok = s0 - cm + r;
-            const bool in = tok >= 0 && tok < T;
-            vld<XT, CPL>(x + (in ? tok : 0) * a.x_stride[i][1], xw[r]);
-            if (!in) {
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) xw[r][c] = 0.f;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int64_t tok = s0 + r;
-            const bool in = tok < T;
-            vld<XT, CPL>(dy + (in ? tok : 0) * D, dyr[r]);
-            if (!in) {
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) dyr[r][c] = 0.f;
-            }
-        }
-        float du[R][CPL];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            float u[CPL], sg[CPL], s[CPL];
-            float ss = 0.f, sd = 0.f;
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                u[c] = bias[c];
-#pragma unroll
-                for (int j = 0; j < kMaxConvB; ++j)
-                    if (j < cs) u[c] = fmaf(w[j][c], xw[r + j][c], u[c]);
-                sg[c] = sigmoid_f(u[c]);
-                s[c] = u[c] * sg[c];
-                ss = fmaf(s[c], s[c], ss);
-                sd = fmaf(s[c], dyr[r][c], sd);
-            }
-            float ds[CPL];
-            if (i < 2) {
-                // y = s min(rsqrt(sum s^2), 1/eps): a clamped row is s / eps
-                const float tot = wave_sum(ss), dot = wave_sum(sd);
-                const float rn = rsqrtf(tot);
-                const bool clamped = !(rn < inv_eps);
-                const float k3 = rn * rn * rn * dot;
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) ds[c] = clamped ? dyr[r][c] * inv_eps : fmaf(rn, dyr[r][c], -s[c] * k3);
-            } else {
-#pragma unroll
-                for (int c = 0; c < CPL; ++c) ds[c] = dyr[r][c];
-            }
-            const bool in = s0 + r < T;
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                const float d = ds[c] * sg[c] * fmaf(u[c], 1.f - sg[c], 1.f);
-                du[r][c] = in ? d : 0.f;
-            }
-        }
-        // the step's tokens: dx, and their shares of dw and db
-#pragma unroll
-        for (int t = 0; t < kStep; ++t) {
-            float g[CPL];
-#pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                float acc = 0.f;
-#pragma unroll
-                for (int j = 0; j < kMaxConvB; ++j) acc = fmaf(wr[j][c], du[t + j][c], acc);
-                g[c] = acc;
-                dbs[c] += du[t][c];
-#pragma unroll
-                for (int j = 0; j < kMaxConvB; ++j)
-                    if (j < cs) dws[j][c] = fmaf(du[t][c], xw[t + j][c], dws[j][c]);
-            }
-            if (s0 + t < T) vst<XT, CPL>(dx + (s0 + t) * D, g);
-        }
-    }
-    const int64_t row = b * ((T + kPrepTile - 1) / kPrepTile) + tile;
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-#pragma unroll
-        for (int j = 0; j < kMaxConvB; ++j)
-            if (j < cs) pp.dw[i][(row * D + ch0 + c) * cs + j] = dws[j][c];
-        if (a.db[i] != nullptr) pp.db[i][row * D + ch0 + c] = dbs[c];
+            for (int i = 0; i < N; ++i) v[i] += red[(w * N + i) * 64 + lane];
     }
 }
 
-// ---- the gates of one head over a 64-token tile ----------------------------
-template <typename XT, int CPL>
-__device__ void gate_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int64_t b, int64_t tile, int64_t h,
-                              int lane) {
-    const int64_t Dh = 64 * CPL;
-    const int64_t D = a.H * Dh;
-    const int64_t ch0 = h * Dh + lane * CPL;
-    const int64_t T = a.T;
-    float neg_a[CPL], dtb[CPL];
+// ---- q, k or v: kSeg channels over a token tile ------------------------------
+// DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
+// conv_size when it is 4, else 0.  The tokens go by once: du[t] needs the x
+// rows t - 3 .. t and completes dx[t - 3], so four x rows and four partial dx
+// rows are held, in slots by the token's index modulo 4, and a wave's last
+// three dx take du of three tokens past its own.  wl[L] is the tap of lag L:
+// u[t] = sum_L wl[L] x[t - L], dx[t] = sum_L wl[L] du[t + L].
+template <typename XT, int DH, int CS>
+__device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int i, int64_t b,
+                                              int64_t tile, int64_t seg, int wave, int lane, float* red) {
+    constexpr int N = kLaneCh<XT>, G = kGroup;
+    static_assert(G == kMaxConvB, "a row's slot is its index in the group");
+    const int64_t D = a.H * (DH ? DH : a.V), T = a.T;
+    const bool valid = seg * kSeg<XT> + N * lane < D;
+    const int64_t ch0 = valid ? seg * kSeg<XT> + N * lane : 0;
+    const int cs = CS ? CS : static_cast<int>(a.conv_size), cm = cs - 1;
+    const int64_t dxs = a.dx_stride ? a.dx_stride : D;
+    const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0] + ch0;
+    const XT* dy = static_cast<const XT*>(a.dy[i]) + b * T * D + ch0;
+    XT* dx = static_cast<XT*>(a.dx[i]) + b * T * dxs + ch0;
+    const int64_t t0 = tile * kPrepTile + wave * (kPrepTile / kSub);
+    const int n = static_cast<int>(T - t0 < kPrepTile / kSub ? T - t0 : kPrepTile / kSub);     // <= 0: no token
+
+    Raw<XT, N> nx[G], ny[G];
+    const auto fetch = [&](int idx) {                   // rows past the end re-read the last token
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        neg_a[c] = -__expf(load_elem(a.a_log, ch0 + c, a.p_dtype));
-        dtb[c] = load_elem(a.dt_bias, ch0 + c, a.p_dtype);
+        for (int r = 0; r < G; ++r) {
+            const int64_t tok = t0 + idx + r < T ? t0 + idx + r : T - 1;
+            nx[r] = ldn<N>(x + tok * a.x_stride[i][1]);
+            ny[r] = ldn<N>(dy + tok * D);
+        }
+    };
+    fetch(0);
+    float xs[G][N], dxa[G][N], wl[G][N], bias[N], dws[G][N], dbs[N];
+#pragma unroll
+    for (int r = 1; r < G; ++r) {                       // tokens t0 - 3 .. t0 - 1
+        const int64_t tok = t0 - G + r;
+        const Raw<XT, N> h = ldn<N>(x + (tok < 0 ? 0 : (tok < T ? tok : T - 1)) * a.x_stride[i][1]);
+        unpack(h, xs[r]);
+        if (tok < 0) {
+#pragma unroll
+            for (int c = 0; c < N; ++c) xs[r][c] = 0.f;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < N; ++c) bias[c] = dbs[c] = 0.f;
+    if (a.conv_b[i] != nullptr) params<N>(a.conv_b[i], ch0, a.w_dtype, bias);
+    if constexpr (CS == kMaxConvB) {
+        float wc[N * kMaxConvB];
+        params<N * kMaxConvB>(a.conv_w[i], ch0 * kMaxConvB, a.w_dtype, wc);
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+#pragma unroll
+            for (int L = 0; L < G; ++L) wl[L][c] = wc[kMaxConvB * c + kMaxConvB - 1 - L];
+    } else {
+#pragma unroll
+        for (int c = 0; c < N; ++c)
+#pragma unroll
+            for (int L = 0; L < G; ++L)
+                wl[L][c] = L <= cm ? load_elem(a.conv_w[i], (ch0 + c) * cs + cm - L, a.w_dtype) : 0.f;
+    }
+#pragma unroll
+    for (int L = 0; L < G; ++L)
+#pragma unroll
+        for (int c = 0; c < N; ++c) dws[L][c] = dxa[L][c] = 0.f;
+    const float inv_eps = 1.f / a.l2_eps;
+
+    for (int idx0 = 0; n > 0 && idx0 < n + G - 1; idx0 += G) {
+        Raw<XT, N> cx[G], cy[G];
+#pragma unroll
+        for (int r = 0; r < G; ++r) cx[r] = nx[r], cy[r] = ny[r];
+        fetch(idx0 + G);
+#pragma unroll
+        for (int r = 0; r < G; ++r) {
+            const int idx = idx0 + r;
+            float d[N], u[N], sg[N], s[N];
+            unpack(cx[r], xs[r]);
+            unpack(cy[r], d);
+            float ss = 0.f, sd = 0.f;
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                u[c] = bias[c];
+#pragma unroll
+                for (int L = G - 1; L >= 0; --L)
+                    if (L <= cm) u[c] = fmaf(wl[L][c], xs[(r - L + G) % G][c], u[c]);
+                sg[c] = sigmoid_f(u[c]);
+                s[c] = u[c] * sg[c];
+                ss = fmaf(s[c], s[c], ss);
+                sd = fmaf(s[c], d[c], sd);
+            }
+            if constexpr (DH != 0) {
+                // y = s min(rsqrt(sum s^2), 1/eps): a clamped row is s / eps
+                const float rn = rsqrtf(lanes_sum<DH / N>(ss)), dot = lanes_sum<DH / N>(sd);
+                const bool clamped = !(rn < inv_eps);
+                const float k3 = rn * rn * rn * dot;
+#pragma unroll
+                for (int c = 0; c < N; ++c) d[c] = clamped ? d[c] * inv_eps : fmaf(rn, d[c], -s[c] * k3);
+            }
+            const bool in = t0 + idx < T;
+#pragma unroll
+            for (int c = 0; c < N; ++c) {
+                d[c] *= sg[c] * fmaf(u[c], 1.f - sg[c], 1.f);
+                d[c] = in ? d[c] : 0.f;
+                dxa[r][c] = wl[0][c] * d[c];
+#pragma unroll
+                for (int L = 1; L < G; ++L)
+                    if (L <= cm) dxa[(r - L + G) % G][c] = fmaf(wl[L][c], d[c], dxa[(r - L + G) % G][c]);
+            }
+            if (idx < n) {                              // the tile's own tokens
+#pragma unroll
+                for (int c = 0; c < N; ++c) {
+                    dbs[c] += d[c];
+#pragma unroll
+                    for (int L = 0; L < G; ++L)
+                        if (L <= cm) dws[L][c] = fmaf(d[c], xs[(r - L + G) % G][c], dws[L][c]);
+                }
+            }
+            const int e = idx - (G - 1);
+            if (e >= 0 && e < n && valid) stn(dx + (t0 + e) * dxs, dxa[(r + 1) % G]);
+        }
+    }
+    float sums[(G + 1) * N];
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+#pragma unroll
+        for (int L = 0; L < G; ++L) sums[L * N + c] = dws[L][c];
+        sums[G * N + c] = dbs[c];
+    }
+    sum_waves(sums, red, wave, lane);
+    if (!valid || wave > 0) return;
+    const int64_t row = b * ((T + kPrepTile - 1) / kPrepTile) + tile;
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+#pragma unroll
+        for (int L = 0; L < G; ++L)
+            if (L <= cm) pp.dw[i][(row * D + ch0 + c) * cs + cm - L] = sums[L * N + c];
+        if (a.db[i] != nullptr) pp.db[i][row * D + ch0 + c] = sums[G * N + c];
+    }
+}
+
+// ---- the gates of 256 channels over a token tile, and the betas of their heads
+template <typename XT, int DH>
+__device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int64_t b, int64_t tile,
+                                              int64_t seg, int wave, int lane, float* red) {
+    constexpr int N = 4, kHeads = kGateSeg / DH;
+    const int64_t D = a.H * DH, T = a.T;
+    const bool valid = seg * kGateSeg + N * lane < D;
+    const int64_t ch0 = valid ? seg * kGateSeg + N * lane : 0;
+    float neg_a[N], dtb[N], sa[N], sd[N];
+    params<N>(a.a_log, ch0, a.p_dtype, neg_a);
+    params<N>(a.dt_bias, ch0, a.p_dtype, dtb);
+#pragma unroll
+    for (int c = 0; c < N; ++c) {
+        neg_a[c] = -__expf(neg_a[c]);
+        sa[c] = sd[c] = 0.f;
     }
     const XT* gk = static_cast<const XT*>(a.gk) + b * a.gk_stride[0] + ch0;
     const float* dg = a.dg + b * T * D + ch0;
     XT* dgk = static_cast<XT*>(a.dgk) + b * T * D + ch0;
-    float sa[CPL], sd[CPL];
-#pragma unroll
-    for (int c = 0; c < CPL; ++c) sa[c] = sd[c] = 0.f;
-    const int64_t t0 = tile * kPrepTile;
-    for (int step = 0; step < kPrepTile / kStep; ++step) {
-        const int64_t s0 = t0 + step * kStep;
-        if (s0 >= T) break;
-        float z[kStep][CPL], d[kStep][CPL];
+    const int64_t dls = a.dx_stride ? a.dx_stride : a.H;
+    const int64_t t0 = tile * kPrepTile + wave * (kPrepTile / kSub);
+    const int64_t t1 = t0 + kPrepTile / kSub < T ? t0 + kPrepTile / kSub : T;
+    // lane e < kStep kHeads of a step takes the beta of its token e / kHeads, head e % kHeads
+    const int64_t bh = seg * kHeads + lane % kHeads;
+    const bool beta_lane = lane < kStep * kHeads && bh < a.H;
+    for (int64_t s0 = t0; s0 < t1; s0 += kStep) {
+        Raw<XT, N> z[kStep];
+        Raw<float, N> d[kStep];
 #pragma unroll
         for (int t = 0; t < kStep; ++t) {
-            const int64_t tok = s0 + t < T ? s0 + t : s0;
-            vld<XT, CPL>(gk + tok * a.gk_stride[1], z[t]);
-            vld<float, CPL>(dg + tok * D, d[t]);
+            const int64_t tok = s0 + t < t1 ? s0 + t : s0;
+            z[t] = ldn<N>(gk + tok * a.gk_stride[1]);
+            d[t] = ldn<N>(dg + tok * D);
         }
 #pragma unroll
         for (int t = 0; t < kStep; ++t) {
-            if (s0 + t >= T) break;
-            float o[CPL];
+            if (s0 + t >= t1) break;
+            float zz[N], dd[N], o[N];
+            unpack(z[t], zz);
+            unpack(d[t], dd);
 #pragma unroll
-            for (int c = 0; c < CPL; ++c) {
-                const float zz = z[t][c] + dtb[c];
+            for (int c = 0; c < N; ++c) {
+                zz[c] += dtb[c];
                 // softplus(z) = z above torch's threshold (20), and its
                 // derivative 1 there; sigmoid(z) below
-                const float sp = softplus(zz);
-                const float sl = zz > 20.f ? 1.f : sigmoid_f(zz);
-                o[c] = d[t][c] * neg_a[c] * sl;
+                const float sp = softplus(zz[c]);
+                const float sl = zz[c] > 20.f ? 1.f : sigmoid_f(zz[c]);
+                o[c] = dd[c] * neg_a[c] * sl;
                 sd[c] += o[c];
-                sa[c] = fmaf(d[t][c], neg_a[c] * sp, sa[c]);
+                sa[c] = fmaf(dd[c], neg_a[c] * sp, sa[c]);
             }
-            vst<XT, CPL>(dgk + (s0 + t) * D, o);
+            if (valid) stn(dgk + (s0 + t) * D, o);
         }
-        // beta: lane t of the step takes token s0 + t
-        if (lane < kStep && s0 + lane < T) {
-            const int64_t tok = s0 + lane;
-            const float x = load_elem(a.beta_logit, b * a.beta_stride[0] + tok * a.beta_stride[1] + h, a.x_dtype);
+        const int64_t tok = s0 + lane / kHeads;
+        if (beta_lane && tok < t1) {
+            const float x = load_elem(a.beta_logit, b * a.beta_stride[0] + tok * a.beta_stride[1] + bh, a.x_dtype);
             const float bt = sigmoid_f(x);
-            const float g = a.dbeta[(b * T + tok) * a.H + h] * bt * (1.f - bt);
-            store_elem(a.dbeta_logit, (b * T + tok) * a.H + h, a.x_dtype, g);
+            const float g = a.dbeta[(b * T + tok) * a.H + bh] * bt * (1.f - bt);
+            store_elem(a.dbeta_logit, (b * T + tok) * dls + bh, a.x_dtype, g);
         }
     }
+    float sums[2 * N];
+#pragma unroll
+    for (int c = 0; c < N; ++c) sums[c] = sa[c], sums[N + c] = sd[c];
+    sum_waves(sums, red, wave, lane);
+    if (!valid || wave > 0) return;
     const int64_t row = b * ((T + kPrepTile - 1) / kPrepTile) + tile;
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) {
-        pp.da[row * D + ch0 + c] = sa[c];
-        pp.ddt[row * D + ch0 + c] = sd[c];
+    for (int c = 0; c < N; ++c) {
+        pp.da[row * D + ch0 + c] = sums[c];
+        pp.ddt[row * D + ch0 + c] = sums[N + c];
     }
 }
 
-// One wave per (batch, tile, part, head); part 0..2 = q, k, v, 3 = the gates.
-template <typename XT, int CPLK, int CPLV>
-__global__ __launch_bounds__(256) void prep_bwd_kernel(const kda_prep_bwd_args a, const PrepParts pp,
-                                                       uint32_t ntiles, uint32_t units, uint32_t nparts) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t unit = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (unit >= units) return;
-    const uint32_t H = static_cast<uint32_t>(a.H);
-    uint32_t u = unit;
-    const int64_t h = u % H;
-    u /= H;
-    const int part = static_cast<int>(u % nparts);
-    u /= nparts;
-    const int64_t tile = u % ntiles;
-    const int64_t b = u / ntiles;
-    if (part < 2)
-        conv_bwd_unit<XT, CPLK>(a, pp, part, b, tile, h, lane);
-    else if (part == 2)
-        conv_bwd_unit<XT, CPLV>(a, pp, 2, b, tile, h, lane);
-    else
-        gate_bwd_unit<XT, CPLK>(a, pp, b, tile, h, lane);
+// One workgroup per (batch, tile, kSeg channels of q, k, v or kGateSeg of the
+// gates), the gates' shorter units last, into what the others leave free.
+// Bound by the arithmetic on the channels (about 40 operations each, two of
+// them transcendental) at two waves a SIMD.  A wave a head, two channels a
+// lane, took 11 rows of du for 8 tokens and a 64-lane sum a row.  us of
+// kda_prep_backward, then -> this, H=16 d=128 unless said, a wave a whole tile
+// in brackets: B=4 T=2048 bf16 213 -> 135 (139), fp16 177 -> 138 (141), fp32
+// 202 -> 184 (197); B=1 T=2048 bf16 65 -> 42 (55); B=1 T=500 52 -> 22 (49);
+// B=1 T=1024 H=8 d=64 fp16 42 -> 20 (48).
+template <typename XT, int K, bool FULL>
+__global__ __launch_bounds__(64 * kSub, 2) void prep_bwd_kernel(const kda_prep_bwd_args a, const PrepParts pp,
+                                                         uint32_t ntiles, uint32_t convs) {
+    constexpr int CS = FULL ? kMaxConvB : 0;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __shared__ float red[(kSub - 1) * (kGroup + 1) * kLaneCh<XT> * 64];
+    if (blockIdx.x >= convs) {
+        const uint32_t u = blockIdx.x - convs, segs = (static_cast<uint32_t>(a.H) * K + kGateSeg - 1) / kGateSeg;
+        const uint32_t bt = u / segs;
+        gate_bwd_unit<XT, K>(a, pp, bt / ntiles, bt % ntiles, u % segs, wave, lane, red);
+        return;
+    }
+    const uint32_t segk = (static_cast<uint32_t>(a.H) * K + kSeg<XT> - 1) / kSeg<XT>;
+    const uint32_t segv = static_cast<uint32_t>((a.H * a.V + kSeg<XT> - 1) / kSeg<XT>);
+    const uint32_t per = 2 * segk + segv, s = blockIdx.x % per, bt = blockIdx.x / per;
+    const int64_t tile = bt % ntiles, b = bt / ntiles;
+    if (s < 2 * segk) {
+        const int i = s >= segk;
+        conv_bwd_unit<XT, K, CS>(a, pp, i, b, tile, s - i * segk, wave, lane, red);
+    } else {
+        conv_bwd_unit<XT, 0, CS>(a, pp, 2, b, tile, s - 2 * segk, wave, lane, red);
+    }
 }
 
 // ---- output: one wave per (batch, 32-token tile, head) ---------------------
@@ -399,8 +424,9 @@ __global__ __launch_bounds__(256) void output_bwd_kernel(const kda_output_bwd_ar
 // ---- sums of the tiles' shares ---------------------------------------------
 struct ColSum {
     const float* src;              // [rows][n]
-    float* dst;                    // [n]
+    void* dst;                     // [n]
     int64_t n;
+    int32_t dtype;                 // of dst
 };
 struct ColSums {
     ColSum s[8];
@@ -422,7 +448,8 @@ __global__ __launch_bounds__(256) void colsum_kernel(const ColSums c) {
 #pragma unroll
     for (int u = 0; u < 8; ++u)
         if (r + u < c.rows) acc[u] += d.src[(r + u) * d.n + k];
-    d.dst[k] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+    store_elem(d.dst, k, d.dtype,
+               ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7])));
 }
 
 int launch_colsum(const ColSums& c, int count, hipStream_t stream) {
@@ -466,6 +493,9 @@ int validate_prep_bwd(const kda_prep_bwd_args* a) {
     if (!a->workspace) return KDA_ERR_NULL_POINTER;
     if (!aligned(a->workspace, 16)) return KDA_ERR_BAD_SHAPE;
     if (prep_rows(a->B, a->T) * 4 * a->H > INT32_MAX) return KDA_ERR_BAD_SHAPE;
+    const int64_t hk = a->H * a->K, hv = a->H * a->V;
+    if (a->dx_stride != 0 && (a->dx_stride < (hk > hv ? hk : hv) || a->dx_stride % (a->K > a->V ? a->K / 64 : a->V / 64)))
+        return KDA_ERR_BAD_SHAPE;
     return KDA_OK;
 }
 
@@ -487,39 +517,41 @@ int validate_output_bwd(const kda_output_bwd_args* a) {
     return KDA_OK;
 }
 
-template <typename XT, int CPLK, int CPLV>
+template <typename XT, int K, bool FULL>
 int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
     const PrepParts pp = prep_parts(a.workspace, a.B, a.T, a.H, a.K, a.V, a.conv_size);
-    const uint32_t nparts = a.gk != nullptr ? 4u : 3u;
-    const int64_t ntiles = (a.T + kPrepTile - 1) / kPrepTile;
-    const int64_t units = a.B * ntiles * nparts * a.H;
-    hipLaunchKernelGGL((prep_bwd_kernel<XT, CPLK, CPLV>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
-                       stream, a, pp, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units), nparts);
+    const int64_t ntiles = (a.T + kPrepTile - 1) / kPrepTile, hk = a.H * a.K, hv = a.H * a.V;
+    const auto segs = [](int64_t d, int64_t n) { return (d + n - 1) / n; };
+    const int64_t convs = pp.rows * (2 * segs(hk, kSeg<XT>) + segs(hv, kSeg<XT>));
+    const int64_t gates = a.gk != nullptr ? pp.rows * segs(hk, kGateSeg) : 0;
+    const dim3 grid(static_cast<unsigned>(convs + gates));
+    const uint32_t nt = static_cast<uint32_t>(ntiles), nc = static_cast<uint32_t>(convs);
+    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, FULL>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc);
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
     ColSums c{};
     c.rows = pp.rows;
     int n = 0;
     const int64_t D[3] = {a.H * a.K, a.H * a.K, a.H * a.V};
+    const int32_t wt = a.typed_param_grads ? a.w_dtype : KDA_DTYPE_F32;
+    const int32_t pt = a.typed_param_grads ? a.p_dtype : KDA_DTYPE_F32;
     for (int i = 0; i < 3; ++i) {
-        c.s[n++] = ColSum{pp.dw[i], a.dw[i], D[i] * a.conv_size};
-        if (a.db[i] != nullptr) c.s[n++] = ColSum{pp.db[i], a.db[i], D[i]};
+        c.s[n++] = ColSum{pp.dw[i], a.dw[i], D[i] * a.conv_size, wt};
+        if (a.db[i] != nullptr) c.s[n++] = ColSum{pp.db[i], a.db[i], D[i], wt};
     }
     if (a.gk != nullptr) {
-        c.s[n++] = ColSum{pp.da, a.da_log, a.H * a.K};
-        c.s[n++] = ColSum{pp.ddt, a.ddt_bias, a.H * a.K};
+        c.s[n++] = ColSum{pp.da, a.da_log, a.H * a.K, pt};
+        c.s[n++] = ColSum{pp.ddt, a.ddt_bias, a.H * a.K, pt};
     }
     return launch_colsum(c, n, stream);
 }
 
 template <typename XT>
 int launch_prep_bwd_dims(const kda_prep_bwd_args& a, hipStream_t stream) {
-    switch ((a.K / 64) * 10 + a.V / 64) {
-        case 11: return launch_prep_bwd<XT, 1, 1>(a, stream);
-        case 12: return launch_prep_bwd<XT, 1, 2>(a, stream);
-        case 21: return launch_prep_bwd<XT, 2, 1>(a, stream);
-        case 22: return launch_prep_bwd<XT, 2, 2>(a, stream);
-        default: return KDA_ERR_UNSUPPORTED;
-    }
+    if (a.K == 64)
+        return a.conv_size == kMaxConvB ? launch_prep_bwd<XT, 64, true>(a, stream)
+                                        : launch_prep_bwd<XT, 64, false>(a, stream);
+    return a.conv_size == kMaxConvB ? launch_prep_bwd<XT, 128, true>(a, stream)
+                                    : launch_prep_bwd<XT, 128, false>(a, stream);
 }
 
 template <typename XT>
@@ -536,7 +568,7 @@ int launch_output_bwd(const kda_output_bwd_args& a, hipStream_t stream) {
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
     ColSums c{};
     c.rows = a.B * ntiles;
-    c.s[0] = ColSum{part, a.dweight, a.H * a.V};
+    c.s[0] = ColSum{part, a.dweight, a.H * a.V, a.typed_param_grads ? a.w_dtype : KDA_DTYPE_F32};
     return launch_colsum(c, 1, stream);
 }
 

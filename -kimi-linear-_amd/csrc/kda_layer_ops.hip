@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "kda_common.h"
+#include "kda_rows.h"
 
 namespace kda {
 
@@ -33,80 +34,6 @@ namespace {
 
 constexpr int kTile = 16;      // tokens per prep unit at most; an in-place conv cache needs T <= this
 constexpr int kMaxConv = 4;    // largest conv_size
-// channels per lane of q, k and v (16 bytes) and per wave
-template <typename XT> constexpr int kLaneCh = 16 / static_cast<int>(sizeof(XT));
-template <typename XT> constexpr int kSeg = 64 * kLaneCh<XT>;
-constexpr int kGateSeg = 256;  // channels per wave of the gate, 4 a lane
-
-template <typename XT> __device__ __forceinline__ float to_f(XT x);
-template <> __device__ __forceinline__ float to_f<float>(float x) { return x; }
-template <> __device__ __forceinline__ float to_f<_Float16>(_Float16 x) { return static_cast<float>(x); }
-template <> __device__ __forceinline__ float to_f<bf16_t>(bf16_t x) { return bf16_bits_to_f32(x.bits); }
-
-template <typename XT> __device__ __forceinline__ XT from_f(float x);
-template <> __device__ __forceinline__ float from_f<float>(float x) { return x; }
-template <> __device__ __forceinline__ _Float16 from_f<_Float16>(float x) { return static_cast<_Float16>(x); }
-template <> __device__ __forceinline__ bf16_t from_f<bf16_t>(float x) { return bf16_t{f32_to_bf16_bits(x)}; }
-
-// Round to XT and back: the value an XT tensor would hold.
-template <typename XT>
-__device__ __forceinline__ float round_to(float x) {
-    return to_f(from_f<XT>(x));
-}
-
-// N consecutive elements held as loaded.  Rows are aligned to their
-// element only (the layer's rows of H (2 K + V) + H + 256 elements are not a
-// multiple of 16 bytes for every H); the compiler emits what that allows.
-template <typename XT, int N>
-struct Raw {
-    static constexpr int W = sizeof(XT) * N / 4;     // words
-    uint32_t w[W];
-};
-template <int N, typename XT>
-__device__ __forceinline__ Raw<XT, N> ldn(const XT* p) {
-    Raw<XT, N> r;
-    __builtin_memcpy(r.w, p, sizeof(r.w));
-    return r;
-}
-template <typename XT, int N>
-__device__ __forceinline__ void unpack(const Raw<XT, N>& r, float (&x)[N]) {
-#pragma unroll
-    for (int c = 0; c < N; ++c) {
-        if constexpr (sizeof(XT) == 4) {
-            x[c] = __uint_as_float(r.w[c]);
-        } else {
-            const uint16_t u = static_cast<uint16_t>(r.w[c / 2] >> (16 * (c % 2)));
-            x[c] = Elem<XT>::code == KDA_DTYPE_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, u))
-                                                   : bf16_bits_to_f32(u);
-        }
-    }
-}
-template <typename XT, int N>
-__device__ __forceinline__ void stn(XT* p, const float (&x)[N]) {
-    XT v[N];
-#pragma unroll
-    for (int c = 0; c < N; ++c) v[c] = from_f<XT>(x[c]);
-    __builtin_memcpy(p, v, sizeof(v));
-}
-
-// N consecutive parameters of a runtime dtype from element i on, as fp32.
-template <int N>
-__device__ __forceinline__ void params(const void* p, int64_t i, int dtype, float (&x)[N]) {
-    uint32_t w[N];
-    if (dtype == KDA_DTYPE_F32) {
-        __builtin_memcpy(w, static_cast<const float*>(p) + i, sizeof(w));
-#pragma unroll
-        for (int c = 0; c < N; ++c) x[c] = __uint_as_float(w[c]);
-        return;
-    }
-    __builtin_memcpy(w, static_cast<const uint16_t*>(p) + i, N * 2);
-#pragma unroll
-    for (int c = 0; c < N; ++c) {
-        const uint16_t u = static_cast<uint16_t>(w[c / 2] >> (16 * (c % 2)));
-        x[c] = dtype == KDA_DTYPE_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, u)) : bf16_bits_to_f32(u);
-    }
-}
-
 // ---- prep: kSeg channels of q, k or v over a token tile ---------------------
 // DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
 // conv_size when it is 4 (the usual case, no test of the tap count in the

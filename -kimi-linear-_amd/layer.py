@@ -56,7 +56,7 @@ import torch.nn as nn
 from . import _native
 from .kda import (KdaError, kda_chunkwise, kda_chunkwise_fused, kda_chunkwise_gated, kda_recurrent,
                   kda_recurrent_gated, long_segments)
-from .layer_ops import kda_output, kda_output_train, kda_prep, kda_prep_train
+from .layer_ops import kda_output, kda_output_train, kda_prep, kda_prep_train, split_joined
 
 
 def l2norm(x, eps: float):
@@ -422,15 +422,16 @@ class KimiDeltaAttention(nn.Module):
         w = torch.cat([m.weight for m in mods], 0)
         b = torch.cat([m.bias for m in mods]) if mods[0].bias is not None else None
         y = torch.nn.functional.linear(x, w, b)
-        q_in, k_in, v_in, beta_logit, gk_low, og_low = torch.split(
-            y, (H * K, H * K, H * V, H, self.gk_proj[0].out_features, self.og_proj[0].out_features), dim=-1)
+        q_in, k_in, v_in, beta_logit, gk_low, og_low = split_joined(
+            y, (H * K, H * K, H * V, H, self.gk_proj[0].out_features, self.og_proj[0].out_features))
         if T == 0:
             return self.o_proj(x.new_zeros(B, 0, H * V))
         convs = (self.conv_q.conv, self.conv_k.conv, self.conv_v.conv)
         gk = _project_train(self.gk_proj[1], gk_low)
         q, k, v, g, beta = kda_prep_train(q_in, k_in, v_in, tuple(c.weight for c in convs),
                                           tuple(c.bias for c in convs), gk, self.A_log, self.dt_bias, beta_logit,
-                                          num_heads=H, head_dim=K, value_head_dim=V, l2_eps=self.l2norm_eps)
+                                          num_heads=H, head_dim=K, value_head_dim=V, l2_eps=self.l2norm_eps,
+                                          row=y.shape[-1])
         C = self.chunk_size if T % self.chunk_size == 0 else T
         o_core, _ = kda_chunkwise(q, k, v, g, beta, chunk_size=C, state_dtype=self._state_dtype(x))
         gate = _project_train(self.og_proj[1], og_low)

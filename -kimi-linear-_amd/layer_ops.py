@@ -236,7 +236,7 @@ def _c(t):
 
 
 def kda_prep_backward(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta_logit, dq, dk, dv, dg, dbeta, *,
-                      num_heads, head_dim, value_head_dim, l2_eps):
+                      num_heads, head_dim, value_head_dim, l2_eps, row=None):
     """Gradients of :func:`kda_prep` (a call without a conv cache) from those
     of its outputs: ``dq, dk [B, T, H, K]``, ``dv [B, T, H, V]`` and, with the
     gates, ``dg [B, T, H, K]``, ``dbeta [B, T, H]`` (fp32).
@@ -247,6 +247,8 @@ def kda_prep_backward(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta
     dtype, and for the gates ``dgk [B, T, H*K]``, ``dbeta_logit [B, T, H]``,
     ``da_log``, ``ddt_bias`` (shaped and typed as ``a_log``, ``dt_bias``), or
     None without gates.  Sums over tokens are fp32 and run in a fixed order.
+    ``row`` (with the gates): dq_in, dk_in, dv_in and dbeta_logit are the first
+    channels, in this order, of one ``[B, T, row]`` tensor.
     """
     H, K, V = int(num_heads), int(head_dim), int(value_head_dim)
     B, T = q_in.shape[0], q_in.shape[1]
@@ -260,9 +262,12 @@ def kda_prep_backward(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta
     bs = [_c(b) if b is not None else None for b in conv_b]
     gates = gk is not None
     dev = xs[0].device
-    dxs = [torch.empty_like(x, memory_format=torch.contiguous_format) for x in xs]
-    dws = [torch.empty(D, cs, device=dev, dtype=torch.float32) for D in (Dk, Dk, Dv)]
-    dbs = [torch.empty(D, device=dev, dtype=torch.float32) if b is not None else None
+    if row is not None:
+        *dxs, dlogit = torch.empty(B, T, row, device=dev, dtype=dt)[..., :2 * Dk + Dv + H].split((Dk, Dk, Dv, H), -1)
+    else:
+        dxs = [torch.empty_like(x, memory_format=torch.contiguous_format) for x in xs]
+    dws = [torch.empty(D, 1, cs, device=dev, dtype=wdt) for D in (Dk, Dk, Dv)]
+    dbs = [torch.empty(D, device=dev, dtype=wdt) if b is not None else None
            for b, D in zip(bs, (Dk, Dk, Dv))]
     out_g = (None, None, None, None)
     if gates:
@@ -272,9 +277,10 @@ def kda_prep_backward(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta
         dg = _c(dg.float()).view(B, T, Dk)
         dbeta = _c(dbeta.float()).view(B, T, H)
         dgk = torch.empty(B, T, Dk, device=dev, dtype=dt)
-        dlogit = torch.empty(B, T, H, device=dev, dtype=dt)
-        dal = torch.empty(Dk, device=dev, dtype=torch.float32)
-        ddt = torch.empty(Dk, device=dev, dtype=torch.float32)
+        if row is None:
+            dlogit = torch.empty(B, T, H, device=dev, dtype=dt)
+        dal = torch.empty(a_log.shape, device=dev, dtype=a_log.dtype)
+        ddt = torch.empty(dt_bias.shape, device=dev, dtype=dt_bias.dtype)
     if B * T * H > 0:
         lib = _native.load()
         ws_bytes = lib.kda_prep_bwd_workspace_size(B, T, H, K, V, cs)
@@ -305,15 +311,14 @@ def kda_prep_backward(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta
         a.l2_eps = float(l2_eps)
         a.x_dtype = _code("activations", xs[0])
         a.workspace = work.data_ptr()
+        a.dx_stride, a.typed_param_grads = row or 0, 1
         _call(lib.kda_prep_bwd, a, dev, f"kda_prep_bwd (B={B}, T={T}, H={H}, K={K}, V={V}, conv {cs})")
     else:
         for t in dxs + dws + [d for d in dbs if d is not None] + ([dgk, dlogit, dal, ddt] if gates else []):
             t.zero_()
     if gates:
-        out_g = (dgk, dlogit, dal.view_as(a_log).to(a_log.dtype), ddt.view_as(dt_bias).to(dt_bias.dtype))
-    dw = tuple(d.view(-1, 1, cs).to(wdt) for d in dws)
-    db = tuple(d.to(wdt) if d is not None else None for d in dbs)
-    return (dxs[0], dxs[1], dxs[2], dw, db) + out_g
+        out_g = (dgk, dlogit, dal, ddt)
+    return (dxs[0], dxs[1], dxs[2], tuple(dws), tuple(dbs)) + out_g
 
 
 def kda_output_backward(o, gate, weight, eps, dy):
@@ -330,10 +335,9 @@ def kda_output_backward(o, gate, weight, eps, dy):
     dev = o.device
     do = torch.empty(B, T, H, V, device=dev, dtype=o.dtype)
     dgate = torch.empty(B, T, H * V, device=dev, dtype=o.dtype)
-    dw = torch.empty(H * V, device=dev, dtype=torch.float32)
+    dw = torch.empty(H, V, device=dev, dtype=weight.dtype)
     if do.numel() == 0:
-        dw.zero_()
-        return do, dgate, dw.view(H, V).to(weight.dtype)
+        return do, dgate, dw.zero_()
     lib = _native.load()
     work = torch.empty(max(1, (lib.kda_output_bwd_workspace_size(B, T, H, V) + 3) // 4), device=dev,
                        dtype=torch.float32)
@@ -346,8 +350,9 @@ def kda_output_backward(o, gate, weight, eps, dy):
     a.weight, a.w_dtype = weight.data_ptr(), _code("weight", weight)
     a.dy, a.d_o, a.dgate, a.dweight = dy.data_ptr(), do.data_ptr(), dgate.data_ptr(), dw.data_ptr()
     a.eps, a.x_dtype, a.workspace = float(eps), _code("o", o), work.data_ptr()
+    a.typed_param_grads = 1
     _call(lib.kda_output_bwd, a, dev, f"kda_output_bwd (B={B}, T={T}, H={H}, V={V})")
-    return do, dgate, dw.view(H, V).to(weight.dtype)
+    return do, dgate, dw
 
 
 class _PrepFn(torch.autograd.Function):
@@ -355,7 +360,7 @@ class _PrepFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q_in, k_in, v_in, wq, wk, wv, bq, bk, bv, gk, beta_logit, a_log, dt_bias, meta):
-        H, K, V, eps = meta
+        H, K, V, eps, _ = meta
         q, k, v, g, beta, _ = kda_prep(q_in, k_in, v_in, (wq, wk, wv), (bq, bk, bv), gk, a_log, dt_bias, beta_logit,
                                        num_heads=H, head_dim=K, value_head_dim=V, l2_eps=eps)
         ctx.save_for_backward(q_in, k_in, v_in, wq, wk, wv, bq, bk, bv, gk, beta_logit, a_log, dt_bias)
@@ -365,7 +370,7 @@ class _PrepFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dq, dk, dv, dg, dbeta):
         q_in, k_in, v_in, wq, wk, wv, bq, bk, bv, gk, beta_logit, a_log, dt_bias = ctx.saved_tensors
-        H, K, V, eps = ctx.meta
+        H, K, V, eps, row = ctx.meta
         B, T = q_in.shape[0], q_in.shape[1]
         z = lambda *s: torch.zeros(*s, device=q_in.device, dtype=torch.float32)  # noqa: E731
         dq = dq if dq is not None else z(B, T, H, K)
@@ -375,7 +380,7 @@ class _PrepFn(torch.autograd.Function):
         dbeta = dbeta if dbeta is not None else z(B, T, H)
         dqi, dki, dvi, dw, db, dgk, dlogit, dal, ddt = kda_prep_backward(
             q_in, k_in, v_in, (wq, wk, wv), (bq, bk, bv), gk, a_log, dt_bias, beta_logit, dq, dk, dv, dg, dbeta,
-            num_heads=H, head_dim=K, value_head_dim=V, l2_eps=eps)
+            num_heads=H, head_dim=K, value_head_dim=V, l2_eps=eps, row=row)
         return (dqi, dki, dvi, dw[0], dw[1], dw[2], db[0], db[1], db[2], dgk, dlogit, dal, ddt, None)
 
 
@@ -396,11 +401,62 @@ class _OutputFn(torch.autograd.Function):
 
 
 def kda_prep_train(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta_logit, *, num_heads, head_dim,
-                   value_head_dim, l2_eps):
+                   value_head_dim, l2_eps, row=None):
     """:func:`kda_prep` with the gates and without a conv cache, differentiable
-    (native forward and backward kernels): ``(q, k, v, g, beta)``."""
+    (native forward and backward kernels): ``(q, k, v, g, beta)``.  ``row``: as
+    in :func:`kda_prep_backward`, for projections split by :func:`split_joined`."""
     return _PrepFn.apply(q_in, k_in, v_in, *conv_w, *conv_b, gk, beta_logit, a_log, dt_bias,
-                         (int(num_heads), int(head_dim), int(value_head_dim), float(l2_eps)))
+                         (int(num_heads), int(head_dim), int(value_head_dim), float(l2_eps), row))
+
+
+class _SplitFn(torch.autograd.Function):
+    """torch.split over the last dimension.  Backward: gradients that are already
+    slices of one tensor in the split's layout, the leading ones of
+    :func:`kda_prep_backward` with ``row``, stay where they are and the others
+    are written beside them; any others are concatenated."""
+
+    @staticmethod
+    def forward(ctx, y, sizes):
+        ctx.sizes, ctx.rows = sizes, tuple(y.shape[:-1])
+        ctx.set_materialize_grads(False)
+        return tuple(y.split(sizes, -1))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        some = next((g for g in grads if g is not None), None)
+        if some is None:
+            return None, None
+        joined = None if torch.is_grad_enabled() else _joined(grads, ctx.rows, ctx.sizes)
+        if joined is not None:
+            return joined, None
+        return torch.cat([g if g is not None else some.new_zeros(*ctx.rows, n)
+                          for g, n in zip(grads, ctx.sizes)], -1), None
+
+
+def _joined(grads, rows, sizes):
+    """The tensor [*rows, sum(sizes)] that the leading gradient is a slice of,
+    completed with the others; None if there is none."""
+    base = grads[0]._base if grads[0] is not None else None
+    shape = (*rows, sum(sizes))
+    if (base is None or tuple(base.shape) != shape or not base.is_contiguous() or base.dtype != grads[0].dtype
+            or base.requires_grad):
+        return None
+    parts, missing = base.split(sizes, -1), []
+    for g, p in zip(grads, parts):
+        if g is not None and g._base is base:
+            if g.shape != p.shape or g.stride() != p.stride() or g.storage_offset() != p.storage_offset():
+                return None
+        else:
+            missing.append((g, p))
+    for g, p in missing:
+        p.zero_() if g is None else p.copy_(g)
+    return base
+
+
+def split_joined(y, sizes):
+    """``torch.split(y, sizes, -1)``, differentiable, for projections whose
+    gradients :func:`kda_prep_train` writes in place with ``row``."""
+    return _SplitFn.apply(y, tuple(sizes))
 
 
 def kda_output_train(o, gate, weight, eps):

@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define KDA_ABI_VERSION 14
+#define KDA_ABI_VERSION 15
 
 /* Element types accepted at the boundary. */
 typedef enum kda_dtype {
@@ -429,8 +429,8 @@ typedef struct kda_prep_bwd_args {
     int32_t w_dtype;               /* kda_dtype of conv_w and conv_b */
     const void* dy[3];             /* gradients of q, k [B, T, H, K] and v [B, T, H, V], contiguous, x dtype */
     void* dx[3];                   /* [B, T, D] contiguous, x dtype */
-    float* dw[3];                  /* [D, conv_size] */
-    float* db[3];                  /* [D] or NULL */
+    void* dw[3];                   /* [D, conv_size] */
+    void* db[3];                   /* [D] or NULL */
     const void* gk;                /* [B, T, H*K] gate up-projection, x dtype, or NULL (no gates) */
     int64_t gk_stride[2];
     const void* a_log;             /* [H*K] */
@@ -442,11 +442,14 @@ typedef struct kda_prep_bwd_args {
     const float* dbeta;            /* [B, T, H] contiguous */
     void* dgk;                     /* [B, T, H*K] contiguous, x dtype */
     void* dbeta_logit;             /* [B, T, H] contiguous, x dtype */
-    float* da_log;                 /* [H*K] */
-    float* ddt_bias;               /* [H*K] */
+    void* da_log;                  /* [H*K] */
+    void* ddt_bias;                /* [H*K] */
     float l2_eps;
     int32_t x_dtype;
     void* workspace;
+    int64_t dx_stride;             /* 0, or the row stride of the dx and of dbeta_logit (batches T rows apart):
+                                    * slices of one gradient of the joined projections */
+    int32_t typed_param_grads;     /* 0: dw, db, da_log, ddt_bias in fp32; 1: in w_dtype and p_dtype, rounded once */
 } kda_prep_bwd_args;
 
 size_t kda_prep_bwd_workspace_size(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t conv_size);
@@ -469,10 +472,11 @@ typedef struct kda_output_bwd_args {
     const void* dy;                /* [B, T, H*V] contiguous, x dtype */
     void* d_o;                     /* [B, T, H, V] contiguous, x dtype */
     void* dgate;                   /* [B, T, H*V] contiguous, x dtype */
-    float* dweight;                /* [H*V] */
+    void* dweight;                 /* [H*V] */
     float eps;
     int32_t x_dtype;
     void* workspace;               /* kda_output_bwd_workspace_size() bytes */
+    int32_t typed_param_grads;     /* 0: dweight in fp32; 1: in w_dtype, rounded once */
 } kda_output_bwd_args;
 
 size_t kda_output_bwd_workspace_size(int64_t B, int64_t T, int64_t H, int64_t V);

@@ -1,0 +1,95 @@
+"""The pre-processing's backward at the edges of its units (tokens per tile,
+channels per wave, conv sizes), and its gradients as slices of one tensor."""
+
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+from test_gpu_layer_train import DEV, TOL_K, _prep_inputs, _prep_ref, rel
+
+
+@pytest.fixture(scope="module")
+def ops(kda_pkg):
+    return importlib.import_module("kimi_linear_amd.layer_ops")
+
+
+def run(ops, inp, up, dtype, H, K, V, row=None):
+    dev = lambda t: t.to(DEV) if t is not None else None  # noqa: E731
+    return ops.kda_prep_backward(
+        *(dev(x) for x in inp["x"]), [dev(w.to(dtype)) for w in inp["w"]],
+        [dev(b.to(dtype)) if b is not None else None for b in inp["b"]], dev(inp["gk"]), dev(inp["a_log"]),
+        dev(inp["dt_bias"]), dev(inp["logit"]), *(dev(up[n]) for n in ("dq", "dk", "dv", "dg", "dbeta")),
+        num_heads=H, head_dim=K, value_head_dim=V, l2_eps=1e-6, row=row)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,T,H,K,V,cs", [(1, 1, 1, 64, 64, 4), (2, 3, 3, 64, 128, 4), (1, 61, 5, 128, 64, 1),
+                                          (2, 65, 9, 64, 64, 3), (1, 33, 5, 128, 128, 4), (3, 132, 2, 128, 64, 4),
+                                          (2, 67, 1, 64, 64, 2), (1, 128, 1, 64, 64, 4)])
+def test_unit_edges(ops, dtype, B, T, H, K, V, cs):
+    """Tiles with 1 to 4 rows left and one row into the next, channel runs that end
+    inside a wave.  Bounds as for the same kernels elsewhere."""
+    inp, up = _prep_inputs(B, T, H, K, V, cs, dtype, seed=T + cs)
+    got = run(ops, inp, up, dtype, H, K, V)
+    ref_in = dict(inp, w=[w.to(dtype) for w in inp["w"]], b=[b.to(dtype) for b in inp["b"]])
+    outs, leaves = _prep_ref(ref_in, H, K, V, 1e-6)
+    ups = [up[n].to(dtype if i < 3 else torch.float32).double() for i, n in enumerate(("dq", "dk", "dv", "dg", "dbeta"))]
+    torch.autograd.backward(outs, ups)
+    ref = ([x.grad for x in leaves["x"]], [w.grad for w in leaves["w"]], [b.grad for b in leaves["b"]],
+           leaves["gk"].grad, leaves["logit"].grad, leaves["a_log"].grad, leaves["dt_bias"].grad)
+    pairs = [*zip(got[:3], ref[0]), *zip(got[3], ref[1]), *zip(got[4], ref[2]), *zip(got[5:], ref[3:])]
+    for i, (a, b) in enumerate(pairs):
+        assert a.shape == b.shape and rel(a, b) <= TOL_K[dtype], i
+    # the same as slices of one tensor's rows
+    width = H * (2 * K + V) + H
+    row = run(ops, inp, up, dtype, H, K, V, row=width + 19 * (K // 64) * (V // 64) + width % 2)
+    for a, b in zip([*got[:3], *got[3], *got[4], *got[5:]], [*row[:3], *row[3], *row[4], *row[5:]]):
+        assert torch.equal(a, b)
+    assert row[0]._base is row[6]._base and row[0]._base.shape[-1] >= width
+
+
+class Halves(torch.autograd.Function):
+    """a and b as they are; their gradients as slices of one [.., row] tensor."""
+
+    @staticmethod
+    def forward(ctx, a, b, row):
+        ctx.row = row
+        return a.clone(), b.clone()
+
+    @staticmethod
+    def backward(ctx, da, db):
+        n, m = da.shape[-1], db.shape[-1]
+        with torch.no_grad():
+            a, b = da.new_full((*da.shape[:-1], ctx.row), float("nan"))[..., :n + m].split((n, m), -1)
+            a.copy_(da)
+            b.copy_(db)
+        return a, b, None
+
+
+@pytest.mark.parametrize("case", ["joined", "missing", "narrower", "foreign", "create_graph", "twice"])
+def test_split_gradient(ops, case):
+    """split_joined's gradient is torch.split's, whatever the parts' gradients are made of."""
+    gen = torch.Generator().manual_seed(0)
+    y = torch.randn(2, 3, 10, generator=gen, requires_grad=True)
+    w = torch.randn(2, 3, 10, generator=gen)
+    sizes = (3, 4, 2, 1)
+
+    def loss(parts):
+        a, b, c, d = parts
+        if case != "foreign":
+            a, b = Halves.apply(a, b, 9 if case == "narrower" else 10)
+        terms = [a * w[..., :3], b * w[..., 3:7], c * w[..., 7:9]] + ([] if case == "missing" else [d * w[..., 9:]])
+        return sum((t ** 2).sum() for t in terms)
+
+    graph = case in ("create_graph", "twice")
+    out = loss(ops.split_joined(y, sizes))
+    ref = torch.autograd.grad(loss(y.split(sizes, -1)), y)[0]
+    got = torch.autograd.grad(out, y, create_graph=case == "create_graph", retain_graph=graph)[0]
+    assert torch.equal(got, ref)
+    if case == "twice":
+        again = torch.autograd.grad(out, y)[0]
+        assert torch.equal(again, ref) and torch.equal(got, ref)
