@@ -449,7 +449,7 @@ class KimiDeltaAttention(nn.Module):
                 raise KdaError("the training path (grad mode with parameters that require grad) takes no cache "
                                "or state; run cached prefill and decode under torch.no_grad()")
             return self._train_forward(x)
-        if use_cache and state is None:
+        if use_cache and state is None and x.shape[1] == 0:     # with tokens, no conv cache counts as zeros
             state = self.init_state(x.shape[0], device=x.device, dtype=x.dtype)
         conv_cache = state["conv"] if state is not None else None
         rec = state["recurrent"] if state is not None else None
