@@ -3,7 +3,8 @@
 Mirrors ``kimi_linear/kda.py:258-536`` -- same parameters (names and shapes, so a
 reference ``state_dict`` loads unchanged), same forward semantics and dispatch
 rules -- with the core recurrence running on the gfx950 kernels of
-:mod:`kimi_linear_amd.kda`.  The projections are library GEMMs; the
+:mod:`kimi_linear_amd.kda`.  The projections are library GEMMs (a few
+rows' ones the kernel of ``kda_linear_fwd``); the
 elementwise work between them and the core (short convolutions with their
 cache, SiLU, L2 norms, gates; RMSNorm and output gate) runs in the two fused
 kernels of :mod:`kimi_linear_amd.layer_ops`.  ``ShortConv``,
