@@ -253,6 +253,7 @@ def host():
         if not HOST_PATH.exists():
             raise NativeLibraryError(f"{HOST_PATH} not found: build it with __graft_entry__.build()")
         import torch
+        from .kda import KdaError
         loader = importlib.machinery.ExtensionFileLoader("_kda_host", str(HOST_PATH))
         spec = importlib.util.spec_from_file_location("_kda_host", str(HOST_PATH), loader=loader)
         try:
@@ -264,7 +265,7 @@ def host():
             raise NativeLibraryError(f"{HOST_PATH} has ABI version {mod.abi_version()}, this wrapper expects "
                                      f"{ABI_VERSION}; rebuild it")
         mod.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in EXPORTED_SYMBOLS},
-                 torch._C._cuda_getCurrentRawStream)
+                 torch._C._cuda_getCurrentRawStream, KdaError, "cuda")
         _host = mod
         return mod
 

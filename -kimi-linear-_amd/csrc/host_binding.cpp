@@ -8,7 +8,8 @@
 // dispatch mode or tensor subclass at work -- and returns None for any other
 // call, before doing anything: the Python wrapper then takes its general path,
 // which converts, copies or raises.  So a call has one meaning, and this file
-// only answers for the part of it that needs no decision.
+// only answers for the part of it that needs no decision.  A launch that fails
+// raises: it may have run.
 //
 // In Python a call's checks, its argument structure and its device and stream
 // lookups took about 20 us (a decode step at B=1 takes 4 us on the GPU).
@@ -49,18 +50,22 @@ struct Fns {
     decltype(&kda_linear_fwd) linear = nullptr;
     decltype(&kda_linear_wgrad) wgrad = nullptr;
     decltype(&kda_linear_wgrad_workspace_size) wgrad_ws = nullptr;
+    decltype(&kda_status_str) status_str = nullptr;
 };
 Fns fn;
-// torch._C._cuda_getCurrentRawStream; kept for the process's life
+// torch._C._cuda_getCurrentRawStream and the wrapper's KdaError; kept for the process's life
 PyObject* raw_stream = nullptr;
+PyObject* error = nullptr;
+at::DeviceType device_type = at::kCUDA;      // whose tensors the calls take
 
 template <typename F>
 void take(F& f, const py::dict& addr, const char* name) {
     f = reinterpret_cast<F>(addr[name].cast<uintptr_t>());
 }
 
-// The loaded library's entry points (name -> address) and torch's stream lookup.
-void bind(const py::dict& addr, const py::object& stream_fn) {
+// The loaded library's entry points (name -> address), torch's stream lookup,
+// the wrapper's exception and the type of the library's device.
+void bind(const py::dict& addr, const py::object& stream_fn, const py::object& error_class, const std::string& device) {
     take(fn.chunkwise, addr, "kda_chunkwise_fwd");
     take(fn.recurrent, addr, "kda_recurrent_fwd");
     take(fn.chunkwise_gated, addr, "kda_chunkwise_gated_fwd");
@@ -75,8 +80,23 @@ void bind(const py::dict& addr, const py::object& stream_fn) {
     take(fn.linear, addr, "kda_linear_fwd");
     take(fn.wgrad, addr, "kda_linear_wgrad");
     take(fn.wgrad_ws, addr, "kda_linear_wgrad_workspace_size");
-    Py_INCREF(stream_fn.ptr());
-    raw_stream = stream_fn.ptr();
+    take(fn.status_str, addr, "kda_status_str");
+    device_type = at::Device(device).type();
+    raw_stream = stream_fn.inc_ref().ptr();
+    error = error_class.inc_ref().ptr();
+}
+
+// Whether the library refused the call, before any launch: the general path
+// reports or answers it.  A failed launch is no refusal (the status is read
+// after the launch and may be an older error of the thread: the kernels, or the
+// first ones of several, may have run).  The general path would run them a
+// second time, on a state updated in place, so it raises here.
+bool refused(int status, const char* name) {
+    if (status == KDA_ERR_LAUNCH) {
+        PyErr_Format(error, "%s failed: %s", name, fn.status_str(status));
+        throw py::error_already_set();
+    }
+    return status != KDA_OK;
 }
 
 int code(const Tensor& t) {
@@ -96,7 +116,7 @@ struct Plain {
     bool ok = true;
     explicit Plain(const Tensor& first)
         : dev(first.defined() ? first.device() : at::Device(at::kCPU)) {
-        ok = dev.is_cuda() && c10::impl::TorchDispatchModeTLS::stack_len() == 0;
+        ok = dev.type() == device_type && c10::impl::TorchDispatchModeTLS::stack_len() == 0;
         add(first);
     }
     Plain& add(const Tensor& t) {
@@ -240,7 +260,7 @@ py::object core(bool recurrent, const Tensor& q, const Tensor& k, const Tensor& 
     } else {
         status = (recurrent ? fn.recurrent : fn.chunkwise)(&a, stream);
     }
-    if (status != KDA_OK) return py::none();         // refused before any launch: the wrapper reports it
+    if (refused(status, recurrent ? "kda_recurrent" : "kda_chunkwise")) return py::none();
     return py::make_tuple(o, s);
 }
 
@@ -331,7 +351,7 @@ py::object prep(const std::array<Tensor, 3>& x, const std::array<Tensor, 3>& w, 
     a.v = out[2].data_ptr();
     a.l2_eps = static_cast<float>(l2_eps);
     a.x_dtype = dt;
-    if (fn.prep(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    if (refused(fn.prep(&a, stream_of(plain.dev)), "kda_prep_fwd")) return py::none();
     py::object pg = py::none(), pb = py::none(), ph = py::none();
     if (gates) pg = py::cast(g), pb = py::cast(beta);
     if (hn[0].defined()) ph = py::make_tuple(hn[0], hn[1], hn[2]);
@@ -362,7 +382,7 @@ py::object output(const Tensor& o, const Tensor& gate, const Tensor& weight, dou
     a.y = y.data_ptr();
     a.eps = static_cast<float>(eps);
     a.x_dtype = code(o);
-    if (fn.output(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    if (refused(fn.output(&a, stream_of(plain.dev)), "kda_output_fwd")) return py::none();
     return py::cast(y);
 }
 
@@ -413,7 +433,7 @@ py::object linear(const Tensor& x, const Tensor& w, const OptTensor& residual, c
         a.residual_stride = row_stride(*residual);
     }
     a.dtype = code(x);
-    if (fn.linear(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    if (refused(fn.linear(&a, stream_of(plain.dev)), "kda_linear_fwd")) return py::none();
     return py::cast(y);
 }
 
@@ -434,7 +454,7 @@ py::object linear2(const Tensor& x0, const Tensor& w0, const Tensor& x1, const T
     linear_operands(a, 0, x0, w0, y0);
     linear_operands(a, 1, x1, w1, y1);
     a.dtype = code(x0);
-    if (fn.linear(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    if (refused(fn.linear(&a, stream_of(plain.dev)), "kda_linear_fwd")) return py::none();
     return py::make_tuple(y0, y1);
 }
 
@@ -468,7 +488,7 @@ py::object linear_wgrad(const Tensor& dy, const Tensor& x) {
     a.dw = dw.data_ptr();
     a.workspace = ws.data_ptr();
     a.dtype = code(x);
-    if (fn.wgrad(&a, stream_of(plain.dev)) != KDA_OK) return py::none();
+    if (refused(fn.wgrad(&a, stream_of(plain.dev)), "kda_linear_wgrad")) return py::none();
     return py::cast(dw);
 }
 

@@ -163,3 +163,81 @@ def test_layer_kernels_match_their_general_path(kda_pkg, monkeypatch):
                 assert all(torch.equal(p[n], r[n]) for n in "qkv")
             else:
                 assert (p is None and r is None) or torch.equal(p, r)
+
+
+# ---- the native side on CPU tensors, bound to stand-ins for the library's entry points
+@pytest.fixture
+def stand_in(kda_pkg, tmp_path):
+    """``bind(**entries)``: a copy of the native module of its own whose library
+    consists of the given callables (args, stream, ..) -> status."""
+    import ctypes
+    import importlib.util
+    import shutil
+    native = importlib.import_module("kimi_linear_amd._native")
+    error = importlib.import_module("kimi_linear_amd.kda").KdaError
+    path = shutil.copy(native.HOST_PATH, tmp_path / "_kda_host.so")
+    spec = importlib.util.spec_from_file_location("_kda_host", str(path))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    keep, lib = [], native.load()
+
+    def bind(**entries):
+        addr = {n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in native.EXPORTED_SYMBOLS}
+        for n, f in entries.items():
+            if not isinstance(f, int):
+                keep.append(ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_void_p] * 4)(f))
+                f = ctypes.cast(keep[-1], ctypes.c_void_p).value
+            addr[n] = f
+        mod.bind(addr, lambda index: 0, error, "cpu")
+        return mod
+    yield bind
+    keep.clear()
+
+
+def host_calls(mod):
+    """entry point -> a call of the native side that ends in it"""
+    args, state = inputs(torch.float16, device="cpu")
+    B, T, H, K = args[0].shape
+    V = args[2].shape[-1]
+    ga = (torch.rand(H, K), torch.rand(H, K))
+    gated = [*args[:3], args[3].half(), args[4].half()]
+    og, wn = torch.rand(B, T, H * V).half(), torch.rand(H, V)
+    long = [x[:1, :1].expand(1, 4096, *x.shape[2:]).contiguous() for x in args]
+    x = torch.rand(B, T, H * K).half()
+    w = [torch.rand(H * D, 1, 4).half() for D in (K, K, V)]
+    hist = [torch.rand(B, 3, H * D).half() for D in (K, K, V)]
+    few, wl = torch.rand(2, 1, 64).half(), torch.rand(32, 64).half()
+    none = (None, None, None)
+    return {
+        "kda_recurrent_fwd": lambda: call(mod, args, state, True, state_out=state),
+        "kda_recurrent_gated_fwd": lambda: call(mod, gated, state, True, state_out=state, gate=ga),
+        "kda_chunkwise_fwd": lambda: call(mod, args),
+        "kda_chunkwise_gated_fwd": lambda: call(mod, gated, gate=ga),
+        "kda_chunkwise_fused_fwd": lambda: call(mod, gated, gate=ga, epilogue=(og, wn, 1e-6)),
+        "kda_chunkwise_long_fwd": lambda: call(mod, long, segments=2),
+        "kda_prep_fwd": lambda: mod.prep((x, x, x), w, none, None, None, None, None, H, K, V, 1e-6, hist, hist, False),
+        "kda_output_fwd": lambda: mod.output(args[2], og, wn.half(), 1e-6),
+        "kda_linear_fwd": lambda: mod.linear(few, wl, None, None),
+        "kda_linear_wgrad": lambda: mod.linear_wgrad(torch.rand(1, 512, 64).half(), torch.rand(1, 512, 128).half()),
+    }
+
+
+@pytest.mark.parametrize("status", ["launch", "refused", "ok"])
+def test_a_failed_launch_is_not_run_again(stand_in, kda, status):
+    """A launch error raises after one call (its kernels may have run, on a state
+    in place); only a refusal, which launches nothing, is the general path's."""
+    code = {"launch": 6, "refused": 4, "ok": 0}[status]
+    seen = []
+    names = list(host_calls(None))
+    entry = {n: (lambda *a, n=n: seen.append(n) or code) for n in names}
+    # (the segmented call in its one-launch form: no split workspace)
+    mod = stand_in(**entry, kda_chunkwise_split_workspace_size=lambda *a: 0)
+    for n, f in host_calls(mod).items():
+        with torch.no_grad():
+            if status == "launch":
+                with pytest.raises(kda.KdaError, match="launch failed"):
+                    f()
+            else:
+                assert (f() is None) == (status == "refused")
+        assert seen == [n]
+        seen.clear()
