@@ -141,6 +141,17 @@ void* stream_of(const at::Device& dev) {
     return reinterpret_cast<void*>(s.cast<uintptr_t>());
 }
 
+// f(stream), f the allocations and the C ABI call of one entry, on dev and its
+// current stream.  Without the interpreter lock: an allocation or a launch into
+// a full queue waits for the device, and other threads run meanwhile.
+template <typename F>
+int run(const at::Device& dev, F&& f) {
+    void* stream = stream_of(dev);
+    const py::gil_scoped_release unlocked;
+    const c10::DeviceGuard guard(dev);
+    return f(stream);
+}
+
 bool sized(const Tensor& t, std::initializer_list<int64_t> s) { return t.sizes() == at::IntArrayRef(s); }
 
 // [B, T, H, D]: contiguous channels, token rows that do not overlap.
@@ -212,54 +223,52 @@ py::object core(bool recurrent, const Tensor& q, const Tensor& k, const Tensor& 
             if (B != 1 && x->stride(0) != T * x->stride(1)) segments = 1;
     }
 
-    const c10::DeviceGuard guard(plain.dev);
-    Tensor o = at::empty({B, T, H, V}, v.options().requires_grad(false));
-    Tensor s = state_out ? *state_out : at::empty({B, H, K, V}, v.options().dtype(st).requires_grad(false));
-    kda_fwd_args a{};
-    a.B = B; a.T = T; a.H = H; a.K = K; a.V = V;
-    a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.g = g.data_ptr(); a.beta = beta.data_ptr();
-    strides3(a.q_stride, q);
-    strides3(a.k_stride, k);
-    strides3(a.v_stride, v);
-    strides3(a.g_stride, g);
-    strides3(a.beta_stride, beta);
-    a.qkv_dtype = dt; a.g_dtype = gt; a.beta_dtype = bt;
-    a.state_in = state ? state->data_ptr() : nullptr;
-    a.state_in_dtype = state ? code(*state) : KDA_DTYPE_F32;
-    a.state_out = s.data_ptr();
-    a.state_out_dtype = code(s);
-    a.o = o.data_ptr();
-    a.scale = static_cast<float>(std::pow(static_cast<double>(K), -0.5));
-    a.clamp_fp16_out = recurrent ? 1 : 0;
-    a.chunk_size = recurrent ? 1 : chunk_size;
-    kda_gate_args ga{};
-    if (gated) {
-        ga.a_log = static_cast<const float*>(a_log->data_ptr());
-        ga.dt_bias = static_cast<const float*>(dt_bias->data_ptr());
-    }
-    void* stream = stream_of(plain.dev);
-    int status;
-    Tensor keep;                                     // alive until the launches that read it are enqueued
-    if (segments > 1) {
-        // the form whose transition columns end when they are zero, where there is one
-        const size_t split = fn.split_ws(B, T, H, K, V, segments);
-        const size_t bytes = split != 0 ? split : fn.long_ws(B, T, H, K, V, segments);
-        keep = at::empty({static_cast<int64_t>(bytes)}, v.options().dtype(at::kByte).requires_grad(false));
-        status = (split != 0 ? fn.split_fwd : fn.long_fwd)(&a, segments, keep.data_ptr(), stream);
-    } else if (og) {
-        keep = weight->detach().to(at::kFloat).contiguous();
-        kda_out_epilogue e{};
-        e.gate = og->data_ptr();
-        e.gate_stride[0] = og->stride(0);
-        e.gate_stride[1] = og->stride(1);
-        e.weight = static_cast<const float*>(keep.data_ptr());
-        e.eps = static_cast<float>(eps);
-        status = fn.fused(&a, gated ? &ga : nullptr, &e, stream);
-    } else if (gated) {
-        status = (recurrent ? fn.recurrent_gated : fn.chunkwise_gated)(&a, &ga, stream);
-    } else {
-        status = (recurrent ? fn.recurrent : fn.chunkwise)(&a, stream);
-    }
+    Tensor o, s, keep;                               // keep: alive until the launches that read it are enqueued
+    const int status = run(plain.dev, [&](void* stream) -> int {
+        o = at::empty({B, T, H, V}, v.options().requires_grad(false));
+        s = state_out ? *state_out : at::empty({B, H, K, V}, v.options().dtype(st).requires_grad(false));
+        kda_fwd_args a{};
+        a.B = B; a.T = T; a.H = H; a.K = K; a.V = V;
+        a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.g = g.data_ptr(); a.beta = beta.data_ptr();
+        strides3(a.q_stride, q);
+        strides3(a.k_stride, k);
+        strides3(a.v_stride, v);
+        strides3(a.g_stride, g);
+        strides3(a.beta_stride, beta);
+        a.qkv_dtype = dt; a.g_dtype = gt; a.beta_dtype = bt;
+        a.state_in = state ? state->data_ptr() : nullptr;
+        a.state_in_dtype = state ? code(*state) : KDA_DTYPE_F32;
+        a.state_out = s.data_ptr();
+        a.state_out_dtype = code(s);
+        a.o = o.data_ptr();
+        a.scale = static_cast<float>(std::pow(static_cast<double>(K), -0.5));
+        a.clamp_fp16_out = recurrent ? 1 : 0;
+        a.chunk_size = recurrent ? 1 : chunk_size;
+        kda_gate_args ga{};
+        if (gated) {
+            ga.a_log = static_cast<const float*>(a_log->data_ptr());
+            ga.dt_bias = static_cast<const float*>(dt_bias->data_ptr());
+        }
+        if (segments > 1) {
+            // the form whose transition columns end when they are zero, where there is one
+            const size_t split = fn.split_ws(B, T, H, K, V, segments);
+            const size_t bytes = split != 0 ? split : fn.long_ws(B, T, H, K, V, segments);
+            keep = at::empty({static_cast<int64_t>(bytes)}, v.options().dtype(at::kByte).requires_grad(false));
+            return (split != 0 ? fn.split_fwd : fn.long_fwd)(&a, segments, keep.data_ptr(), stream);
+        }
+        if (og) {
+            keep = weight->detach().to(at::kFloat).contiguous();
+            kda_out_epilogue e{};
+            e.gate = og->data_ptr();
+            e.gate_stride[0] = og->stride(0);
+            e.gate_stride[1] = og->stride(1);
+            e.weight = static_cast<const float*>(keep.data_ptr());
+            e.eps = static_cast<float>(eps);
+            return fn.fused(&a, gated ? &ga : nullptr, &e, stream);
+        }
+        if (gated) return (recurrent ? fn.recurrent_gated : fn.chunkwise_gated)(&a, &ga, stream);
+        return (recurrent ? fn.recurrent : fn.chunkwise)(&a, stream);
+    });
     if (refused(status, recurrent ? "kda_recurrent" : "kda_chunkwise")) return py::none();
     return py::make_tuple(o, s);
 }
@@ -312,46 +321,48 @@ py::object prep(const std::array<Tensor, 3>& x, const std::array<Tensor, 3>& w, 
             return py::none();
     }
 
-    const c10::DeviceGuard guard(plain.dev);
-    const auto opt = x[0].options().requires_grad(false);
-    Tensor out[3] = {at::empty({B, T, H, K}, opt), at::empty({B, T, H, K}, opt), at::empty({B, T, H, V}, opt)};
-    Tensor g, beta, hn[3];
-    kda_prep_args a{};
-    a.B = B; a.T = T; a.H = H; a.K = K; a.V = V; a.conv_size = cs;
-    for (int i = 0; i < 3; ++i) {
-        a.x[i] = x[i].data_ptr();
-        a.x_stride[i][0] = x[i].stride(0);
-        a.x_stride[i][1] = x[i].stride(1);
-        a.conv_w[i] = w[i].data_ptr();
-        a.conv_b[i] = bias[i] ? bias[i]->data_ptr() : nullptr;
-        a.hist_in[i] = hist[i] ? hist[i]->data_ptr() : nullptr;
-        if (want_hist) hn[i] = at::empty({B, keep, H * (i == 2 ? V : K)}, opt);
-        else if (have_out) hn[i] = *hist_out[i];
-        a.hist_out[i] = hn[i].defined() ? hn[i].data_ptr() : nullptr;
-    }
-    a.w_dtype = wt;
-    a.p_dtype = KDA_DTYPE_F32;
-    if (gates) {
-        g = at::empty({B, T, H, K}, opt.dtype(at::kFloat));
-        beta = at::empty({B, T, H}, opt.dtype(at::kFloat));
-        a.gk = gk->data_ptr();
-        a.gk_stride[0] = gk->stride(0);
-        a.gk_stride[1] = gk->stride(1);
-        a.a_log = a_log->data_ptr();
-        a.dt_bias = dt_bias->data_ptr();
-        a.p_dtype = code(*a_log);
-        a.beta_logit = beta_logit->data_ptr();
-        a.beta_stride[0] = beta_logit->stride(0);
-        a.beta_stride[1] = beta_logit->stride(1);
-        a.g = static_cast<float*>(g.data_ptr());
-        a.beta = static_cast<float*>(beta.data_ptr());
-    }
-    a.q = out[0].data_ptr();
-    a.k = out[1].data_ptr();
-    a.v = out[2].data_ptr();
-    a.l2_eps = static_cast<float>(l2_eps);
-    a.x_dtype = dt;
-    if (refused(fn.prep(&a, stream_of(plain.dev)), "kda_prep_fwd")) return py::none();
+    Tensor out[3], g, beta, hn[3];
+    const int status = run(plain.dev, [&](void* stream) -> int {
+        const auto opt = x[0].options().requires_grad(false);
+        for (int i = 0; i < 3; ++i) out[i] = at::empty({B, T, H, i == 2 ? V : K}, opt);
+        kda_prep_args a{};
+        a.B = B; a.T = T; a.H = H; a.K = K; a.V = V; a.conv_size = cs;
+        for (int i = 0; i < 3; ++i) {
+            a.x[i] = x[i].data_ptr();
+            a.x_stride[i][0] = x[i].stride(0);
+            a.x_stride[i][1] = x[i].stride(1);
+            a.conv_w[i] = w[i].data_ptr();
+            a.conv_b[i] = bias[i] ? bias[i]->data_ptr() : nullptr;
+            a.hist_in[i] = hist[i] ? hist[i]->data_ptr() : nullptr;
+            if (want_hist) hn[i] = at::empty({B, keep, H * (i == 2 ? V : K)}, opt);
+            else if (have_out) hn[i] = *hist_out[i];
+            a.hist_out[i] = hn[i].defined() ? hn[i].data_ptr() : nullptr;
+        }
+        a.w_dtype = wt;
+        a.p_dtype = KDA_DTYPE_F32;
+        if (gates) {
+            g = at::empty({B, T, H, K}, opt.dtype(at::kFloat));
+            beta = at::empty({B, T, H}, opt.dtype(at::kFloat));
+            a.gk = gk->data_ptr();
+            a.gk_stride[0] = gk->stride(0);
+            a.gk_stride[1] = gk->stride(1);
+            a.a_log = a_log->data_ptr();
+            a.dt_bias = dt_bias->data_ptr();
+            a.p_dtype = code(*a_log);
+            a.beta_logit = beta_logit->data_ptr();
+            a.beta_stride[0] = beta_logit->stride(0);
+            a.beta_stride[1] = beta_logit->stride(1);
+            a.g = static_cast<float*>(g.data_ptr());
+            a.beta = static_cast<float*>(beta.data_ptr());
+        }
+        a.q = out[0].data_ptr();
+        a.k = out[1].data_ptr();
+        a.v = out[2].data_ptr();
+        a.l2_eps = static_cast<float>(l2_eps);
+        a.x_dtype = dt;
+        return fn.prep(&a, stream);
+    });
+    if (refused(status, "kda_prep_fwd")) return py::none();
     py::object pg = py::none(), pb = py::none(), ph = py::none();
     if (gates) pg = py::cast(g), pb = py::cast(beta);
     if (hn[0].defined()) ph = py::make_tuple(hn[0], hn[1], hn[2]);
@@ -368,21 +379,24 @@ py::object output(const Tensor& o, const Tensor& gate, const Tensor& weight, dou
         !sized(gate, {B, T, H * V}) || gate.scalar_type() != o.scalar_type() || gate.stride(2) != 1 ||
         !sized(weight, {H, V}) || !weight.is_contiguous() || !vec_ok(o, V / 64) || !vec_ok(gate, V / 64))
         return py::none();
-    const c10::DeviceGuard guard(plain.dev);
-    Tensor y = at::empty({B, T, H * V}, o.options().requires_grad(false));
-    kda_output_args a{};
-    a.B = B; a.T = T; a.H = H; a.V = V;
-    a.o = o.data_ptr();
-    strides3(a.o_stride, o);
-    a.gate = gate.data_ptr();
-    a.gate_stride[0] = gate.stride(0);
-    a.gate_stride[1] = gate.stride(1);
-    a.weight = weight.data_ptr();
-    a.w_dtype = code(weight);
-    a.y = y.data_ptr();
-    a.eps = static_cast<float>(eps);
-    a.x_dtype = code(o);
-    if (refused(fn.output(&a, stream_of(plain.dev)), "kda_output_fwd")) return py::none();
+    Tensor y;
+    const int status = run(plain.dev, [&](void* stream) -> int {
+        y = at::empty({B, T, H * V}, o.options().requires_grad(false));
+        kda_output_args a{};
+        a.B = B; a.T = T; a.H = H; a.V = V;
+        a.o = o.data_ptr();
+        strides3(a.o_stride, o);
+        a.gate = gate.data_ptr();
+        a.gate_stride[0] = gate.stride(0);
+        a.gate_stride[1] = gate.stride(1);
+        a.weight = weight.data_ptr();
+        a.w_dtype = code(weight);
+        a.y = y.data_ptr();
+        a.eps = static_cast<float>(eps);
+        a.x_dtype = code(o);
+        return fn.output(&a, stream);
+    });
+    if (refused(status, "kda_output_fwd")) return py::none();
     return py::cast(y);
 }
 
@@ -422,18 +436,21 @@ py::object linear(const Tensor& x, const Tensor& w, const OptTensor& residual, c
     if (out && (!sized(*out, {B, T, N}) || out->scalar_type() != x.scalar_type() || !out->is_contiguous() ||
                 overlaps(*out, x) || overlaps(*out, w) || (residual && overlaps(*out, *residual))))
         return py::none();
-    const c10::DeviceGuard guard(plain.dev);
-    Tensor y = out ? *out : at::empty({B, T, N}, x.options().requires_grad(false));
-    kda_linear_args a{};
-    a.M = B * T;
-    a.K = x.size(2);
-    linear_operands(a, 0, x, w, y);
-    if (residual) {
-        a.residual = residual->data_ptr();
-        a.residual_stride = row_stride(*residual);
-    }
-    a.dtype = code(x);
-    if (refused(fn.linear(&a, stream_of(plain.dev)), "kda_linear_fwd")) return py::none();
+    Tensor y;
+    const int status = run(plain.dev, [&](void* stream) -> int {
+        y = out ? *out : at::empty({B, T, N}, x.options().requires_grad(false));
+        kda_linear_args a{};
+        a.M = B * T;
+        a.K = x.size(2);
+        linear_operands(a, 0, x, w, y);
+        if (residual) {
+            a.residual = residual->data_ptr();
+            a.residual_stride = row_stride(*residual);
+        }
+        a.dtype = code(x);
+        return fn.linear(&a, stream);
+    });
+    if (refused(status, "kda_linear_fwd")) return py::none();
     return py::cast(y);
 }
 
@@ -444,17 +461,20 @@ py::object linear2(const Tensor& x0, const Tensor& w0, const Tensor& x1, const T
     if (!linear_ok(plain, x0, w0) || !linear_ok(plain, x1, w1) || !x0.sizes().equals(x1.sizes()) ||
         x0.scalar_type() != x1.scalar_type() || autocast_on())
         return py::none();
-    const c10::DeviceGuard guard(plain.dev);
-    const auto opt = x0.options().requires_grad(false);
-    Tensor y0 = at::empty({x0.size(0), x0.size(1), w0.size(0)}, opt);
-    Tensor y1 = at::empty({x0.size(0), x0.size(1), w1.size(0)}, opt);
-    kda_linear_args a{};
-    a.M = x0.size(0) * x0.size(1);
-    a.K = x0.size(2);
-    linear_operands(a, 0, x0, w0, y0);
-    linear_operands(a, 1, x1, w1, y1);
-    a.dtype = code(x0);
-    if (refused(fn.linear(&a, stream_of(plain.dev)), "kda_linear_fwd")) return py::none();
+    Tensor y0, y1;
+    const int status = run(plain.dev, [&](void* stream) -> int {
+        const auto opt = x0.options().requires_grad(false);
+        y0 = at::empty({x0.size(0), x0.size(1), w0.size(0)}, opt);
+        y1 = at::empty({x0.size(0), x0.size(1), w1.size(0)}, opt);
+        kda_linear_args a{};
+        a.M = x0.size(0) * x0.size(1);
+        a.K = x0.size(2);
+        linear_operands(a, 0, x0, w0, y0);
+        linear_operands(a, 1, x1, w1, y1);
+        a.dtype = code(x0);
+        return fn.linear(&a, stream);
+    });
+    if (refused(status, "kda_linear_fwd")) return py::none();
     return py::make_tuple(y0, y1);
 }
 
@@ -478,17 +498,21 @@ py::object linear_wgrad(const Tensor& dy, const Tensor& x) {
     a.K = x.size(2);
     const size_t bytes = fn.wgrad_ws(a.M, a.N, a.K);
     if (bytes == 0) return py::none();
-    const c10::DeviceGuard guard(plain.dev);
-    const auto opt = x.options().requires_grad(false);
-    Tensor dw = at::empty({a.N, a.K}, opt), ws = at::empty({static_cast<int64_t>(bytes)}, opt.dtype(at::kByte));
-    a.dy = dy.data_ptr();
-    a.dy_stride = row_stride(dy);
-    a.x = x.data_ptr();
-    a.x_stride = row_stride(x);
-    a.dw = dw.data_ptr();
-    a.workspace = ws.data_ptr();
-    a.dtype = code(x);
-    if (refused(fn.wgrad(&a, stream_of(plain.dev)), "kda_linear_wgrad")) return py::none();
+    Tensor dw;
+    const int status = run(plain.dev, [&](void* stream) -> int {
+        const auto opt = x.options().requires_grad(false);
+        dw = at::empty({a.N, a.K}, opt);
+        const Tensor ws = at::empty({static_cast<int64_t>(bytes)}, opt.dtype(at::kByte));
+        a.dy = dy.data_ptr();
+        a.dy_stride = row_stride(dy);
+        a.x = x.data_ptr();
+        a.x_stride = row_stride(x);
+        a.dw = dw.data_ptr();
+        a.workspace = ws.data_ptr();
+        a.dtype = code(x);
+        return fn.wgrad(&a, stream);
+    });
+    if (refused(status, "kda_linear_wgrad")) return py::none();
     return py::cast(dw);
 }
 

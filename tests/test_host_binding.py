@@ -241,3 +241,14 @@ def test_a_failed_launch_is_not_run_again(stand_in, kda, status):
                 assert (f() is None) == (status == "refused")
         assert seen == [n]
         seen.clear()
+
+
+def test_launches_run_without_the_interpreter_lock(stand_in):
+    """Other Python threads run while a launch waits for a full queue: the entry
+    points are called without the lock (PyGILState_Check is 0, their KDA_OK)."""
+    import ctypes
+    check = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    mod = stand_in(**{n: check for n in host_calls(None)}, kda_chunkwise_split_workspace_size=lambda *a: 0)
+    for n, f in host_calls(mod).items():
+        with torch.no_grad():
+            assert f() is not None, n
