@@ -261,6 +261,9 @@ def host():
             loader.exec_module(mod)
         except ImportError as exc:
             raise NativeLibraryError(f"cannot load {HOST_PATH}: {exc}") from exc
+        if mod.torch_version != torch.__version__:
+            raise NativeLibraryError(f"{HOST_PATH} was compiled against torch {mod.torch_version}, this is torch "
+                                     f"{torch.__version__}; rebuild it")
         if mod.abi_version() != ABI_VERSION:
             raise NativeLibraryError(f"{HOST_PATH} has ABI version {mod.abi_version()}, this wrapper expects "
                                      f"{ABI_VERSION}; rebuild it")

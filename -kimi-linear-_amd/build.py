@@ -61,6 +61,7 @@ def build_host(verbose: bool = False) -> Path:
     tmp = HOST_PATH.with_suffix(".so.tmp")
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DKDA_TORCH_VERSION="{torch.__version__}"',
            *(x for p in include_paths() for x in ("-isystem", p)), f"-I{sysconfig.get_paths()['include']}",
            f"-I{INCLUDE}", str(CSRC / "host_binding.cpp"), "-o", str(tmp),
            *(f"-L{p}" for p in library_paths()), "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]

@@ -535,6 +535,7 @@ py::bytes params_key(const std::vector<Tensor>& params) {
 
 PYBIND11_MODULE(_kda_host, m) {
     m.def("abi_version", [] { return KDA_ABI_VERSION; });
+    m.attr("torch_version") = KDA_TORCH_VERSION;    // it was compiled against; its C++ interface is not stable
     m.def("bind", &bind);
     m.def("core", &core);
     m.def("prep", &prep);

@@ -252,3 +252,14 @@ def test_launches_run_without_the_interpreter_lock(stand_in):
     for n, f in host_calls(mod).items():
         with torch.no_grad():
             assert f() is not None, n
+
+
+def test_another_torch_than_it_was_compiled_against(kda_pkg, monkeypatch):
+    """torch's C++ interface changes between releases: the native side refuses to run under another one."""
+    native = importlib.import_module("kimi_linear_amd._native")
+    monkeypatch.setattr(native, "_host", None)
+    assert native.host().torch_version == torch.__version__
+    monkeypatch.setattr(native, "_host", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    with pytest.raises(native.NativeLibraryError, match="torch 0.0.1; rebuild"):
+        native.host()
