@@ -263,7 +263,7 @@ def kda_prep_backward(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta
     gates = gk is not None
     dev = xs[0].device
     if row is not None:
-        *dxs, dlogit = torch.empty(B, T, row, device=dev, dtype=dt)[..., :2 * Dk + Dv + H].split((Dk, Dk, Dv, H), -1)
+        *dxs, dlogit = joined_gradient((B, T, row), (Dk, Dk, Dv, H), dt, dev)
     else:
         dxs = [torch.empty_like(x, memory_format=torch.contiguous_format) for x in xs]
     dws = [torch.empty(D, 1, cs, device=dev, dtype=wdt) for D in (Dk, Dk, Dv)]
@@ -409,9 +409,17 @@ def kda_prep_train(q_in, k_in, v_in, conv_w, conv_b, gk, a_log, dt_bias, beta_lo
                          (int(num_heads), int(head_dim), int(value_head_dim), float(l2_eps), row))
 
 
+def joined_gradient(shape, sizes, dtype, device):
+    """The first parts, ``sizes`` channels each, of one empty ``[.., row]``
+    gradient that :class:`_SplitFn` may complete: nobody else holds it."""
+    joined = torch.empty(shape, device=device, dtype=dtype)
+    joined.kda_parts = len(sizes)           # kept as long as a part refers to the tensor
+    return joined[..., :sum(sizes)].split(sizes, -1)
+
+
 class _SplitFn(torch.autograd.Function):
-    """torch.split over the last dimension.  Backward: gradients that are already
-    slices of one tensor in the split's layout, the leading ones of
+    """torch.split over the last dimension.  Backward: gradients that are the
+    parts of a :func:`joined_gradient` in the split's layout, the leading ones of
     :func:`kda_prep_backward` with ``row``, stay where they are and the others
     are written beside them; any others are concatenated."""
 
@@ -434,21 +442,21 @@ class _SplitFn(torch.autograd.Function):
 
 
 def _joined(grads, rows, sizes):
-    """The tensor [*rows, sum(sizes)] that the leading gradient is a slice of,
-    completed with the others; None if there is none."""
+    """The :func:`joined_gradient` of shape [*rows, sum(sizes)] whose parts the
+    leading gradients are, all of them, completed with the others; None if
+    there is none."""
     base = grads[0]._base if grads[0] is not None else None
-    shape = (*rows, sum(sizes))
-    if (base is None or tuple(base.shape) != shape or not base.is_contiguous() or base.dtype != grads[0].dtype
-            or base.requires_grad):
+    n = getattr(base, "kda_parts", 0)
+    if (not 0 < n <= len(grads) or tuple(base.shape) != (*rows, sum(sizes)) or base.dtype != grads[0].dtype
+            or base.requires_grad or any(g is None or g._base is not base for g in grads[:n])
+            or any(g is not None and g._base is base for g in grads[n:])):
         return None
-    parts, missing = base.split(sizes, -1), []
-    for g, p in zip(grads, parts):
-        if g is not None and g._base is base:
-            if g.shape != p.shape or g.stride() != p.stride() or g.storage_offset() != p.storage_offset():
-                return None
-        else:
-            missing.append((g, p))
-    for g, p in missing:
+    parts = base.split(sizes, -1)
+    for g, p in zip(grads[:n], parts):
+        if g.shape != p.shape or g.stride() != p.stride() or g.storage_offset() != p.storage_offset():
+            return None
+    del base.kda_parts
+    for g, p in zip(grads[n:], parts[n:]):
         p.zero_() if g is None else p.copy_(g)
     return base
 

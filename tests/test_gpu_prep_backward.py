@@ -93,3 +93,62 @@ def test_split_gradient(ops, case):
     if case == "twice":
         again = torch.autograd.grad(out, y)[0]
         assert torch.equal(again, ref) and torch.equal(got, ref)
+
+
+class Parts(torch.autograd.Function):
+    """a and b as they are; their gradients as the caller's own tensors."""
+
+    @staticmethod
+    def forward(ctx, a, b, grads):
+        ctx.grads = grads
+        return a.clone(), b.clone()
+
+    @staticmethod
+    def backward(ctx, da, db):
+        return (*ctx.grads, None)
+
+
+def test_split_gradient_leaves_the_callers_tensors(ops):
+    """Gradients that are slices of a tensor of the caller's, in the split's very
+    layout: it is neither written to nor returned."""
+    y = torch.randn(2, 3, 10, requires_grad=True)
+    own = torch.randn(2, 3, 10)
+    before = own.clone()
+    a, b, c, d = ops.split_joined(y, (3, 4, 2, 1))
+    a, b = Parts.apply(a, b, own.split((3, 4, 2, 1), -1)[:2])
+    got = torch.autograd.grad((a.sum(), b.sum(), (2 * c).sum()), y, [torch.tensor(1.)] * 3)[0]
+    assert torch.equal(own, before)
+    assert got.data_ptr() != own.data_ptr()
+    assert torch.equal(got, torch.cat([before[..., :7], torch.full((2, 3, 2), 2.), torch.zeros(2, 3, 1)], -1))
+
+
+def test_split_gradient_of_two_splits(ops):
+    """The parts of one joined gradient that belong to two splits: each gets its own."""
+    y, z = torch.randn(2, 3, 10, requires_grad=True), torch.randn(2, 3, 10, requires_grad=True)
+    sizes = (3, 4, 2, 1)
+    joined = ops.joined_gradient((2, 3, 10), sizes[:2], torch.float32, y.device)
+    want = [torch.randn_like(p) for p in joined]
+    for p, w in zip(joined, want):
+        p.copy_(w)
+    a, b = Parts.apply(ops.split_joined(y, sizes)[0], ops.split_joined(z, sizes)[1], joined)
+    gy, gz = torch.autograd.grad((a.sum(), b.sum()), (y, z))
+    assert torch.equal(gy, torch.cat([want[0], torch.zeros(2, 3, 7)], -1))
+    assert torch.equal(gz, torch.cat([torch.zeros(2, 3, 3), want[1], torch.zeros(2, 3, 3)], -1))
+
+
+@pytest.mark.parametrize("case", ["joined", "missing", "narrower", "create_graph"])
+def test_split_gradient_in_place(ops, case):
+    """Parts of a joined gradient stay where they are, beside the others."""
+    sizes, row = (3, 4, 2, 1), 9 if case == "narrower" else 10
+    y = torch.randn(2, 3, 10, requires_grad=True)
+    joined = ops.joined_gradient((2, 3, row), sizes[:2], torch.float32, y.device)
+    for p in joined:
+        p.normal_()
+    want = [p.clone() for p in joined]
+    a, b, c, d = ops.split_joined(y, sizes)
+    a, b = Parts.apply(a, b, joined)
+    out = a.sum() + b.sum() + (2 * c).sum() + (0 if case == "missing" else (3 * d).sum())
+    got = torch.autograd.grad(out, y, create_graph=case == "create_graph")[0]
+    want += [torch.full((2, 3, 2), 2.), torch.full((2, 3, 1), 0. if case == "missing" else 3.)]
+    assert torch.equal(got, torch.cat(want, -1))
+    assert (got.data_ptr() == joined[0].data_ptr()) == (case in ("joined", "missing"))
