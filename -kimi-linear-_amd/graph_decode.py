@@ -105,7 +105,7 @@ class KdaGraphedDecoder:
         h = self.input_static
         result = self.output_static.unsqueeze(1)
         for i, (layer, st) in enumerate(zip(self.layers, self.static_states)):
-            if self.residual and getattr(layer.decode_step_, "__func__", None) is KimiDeltaAttention.decode_step_:
+            if self.residual and isinstance(layer, KimiDeltaAttention) and layer._unmodified("decode_step_"):
                 # the residual add belongs to the output projection, which writes the result in place
                 h = layer._decode(h, st, h, result if i + 1 == len(self.layers) else None)
                 continue

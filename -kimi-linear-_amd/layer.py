@@ -319,6 +319,11 @@ class KimiDeltaAttention(nn.Module):
         z = lambda dim: torch.zeros(batch, keep, dim, device=device, dtype=dtype)  # noqa: E731
         return {"conv": {"q": z(H * K), "k": z(H * K), "v": z(H * V)}, "recurrent": None}
 
+    def _unmodified(self, *methods):
+        """Whether these methods are the ones written here, not a subclass's, the
+        instance's or a later replacement: only then may a call go by them."""
+        return all(getattr(type(self), n) is _METHODS[n] and n not in self.__dict__ for n in methods)
+
     def _projections(self, x, conv_cache=None, use_cache=False, conv_out=None, gates=False):
         """q, k, v, the gate's up-projection gk ``[B, T, H, K]``, the beta logits
         ``[B, T, H]``, the new conv cache and the output gate's down-projection
@@ -333,6 +338,11 @@ class KimiDeltaAttention(nn.Module):
         places of gk and the logits, for the ungated core.  ``conv_out``: write
         the new conv cache into these tensors (may be ``conv_cache`` itself for
         T <= 16) instead of returning new ones."""
+        return self._inputs(x, conv_cache, use_cache, conv_out, gates, output_gate=False)[:7]
+
+    def _inputs(self, x, conv_cache=None, use_cache=False, conv_out=None, gates=False, output_gate=True):
+        """What :meth:`_projections` returns and the output gate's up-projection
+        where (few rows) both up-projections are one launch, else None."""
         keep = max(self.conv_size - 1, 0)
         hist = conv_cache if (use_cache and conv_cache is not None and keep > 0) else None
         convs = (self.conv_q.conv, self.conv_k.conv, self.conv_v.conv)
@@ -345,7 +355,7 @@ class KimiDeltaAttention(nn.Module):
         q_in, k_in, v_in, beta_logit, gk_low, og_low = torch.split(
             y, (H * K, H * K, H * V, H, self.gk_proj[0].out_features, self.og_proj[0].out_features), dim=-1)
         gk = gate = None
-        if few:                       # both up-projections in one launch
+        if few and output_gate:       # both up-projections in one launch
             w_gk, w_og = _plain_weight(self.gk_proj[1]), _plain_weight(self.og_proj[1])
             if w_gk is not None and w_og is not None:
                 gk, gate = _native.host().linear2(gk_low, w_gk, og_low, w_og) or (None, None)
@@ -360,20 +370,34 @@ class KimiDeltaAttention(nn.Module):
             l2_eps=self.l2norm_eps, hist=hist, hist_out=conv_out if use_cache else None,
             want_hist=use_cache and conv_out is None)
         if gates:
-            return q, k, v, g, beta, new_conv, (og_low, gate)
-        return q, k, v, gk.view(x.shape[0], x.shape[1], H, K), beta_logit, new_conv, (og_low, gate)
+            return q, k, v, g, beta, new_conv, og_low, gate
+        return q, k, v, gk.view(x.shape[0], x.shape[1], H, K), beta_logit, new_conv, og_low, gate
 
-    def _output_gate(self, og):
-        """The output gate's up-projection from what :meth:`_projections` returned for it."""
-        og_low, gate = og
-        return self.og_proj[1](og_low) if gate is None else gate
+    def _core_inputs(self, x, **kw):
+        """:meth:`_inputs`, through :meth:`_projections` if that or :meth:`_output` has been replaced."""
+        if self._unmodified("_projections", "_output"):
+            return self._inputs(x, **kw)
+        return (*self._projections(x, **kw), None)
 
-    def _output(self, o_core, og, residual=None, out=None):
+    def _output(self, o_core, og_low):
         """Head-wise RMSNorm, sigmoid output gate (one fused kernel,
         :func:`kda_output`) and the output projection (``kda.py:464-470``);
-        ``og`` is the output gate from :meth:`_projections`.  With ``residual``
+        ``og_low`` is the output gate's down-projection of x."""
+        return self._result(o_core, og_low, None)
+
+    def _layer_output(self, o_core, og_low, gate, residual=None, out=None):
+        """:meth:`_output` from what :meth:`_core_inputs` returned; with ``residual``
         their sum, with ``out`` written there."""
-        gate = self._output_gate(og)
+        if self._unmodified("_output"):
+            return self._result(o_core, og_low, gate, residual, out)
+        y = self._output(o_core, og_low)
+        if residual is not None:
+            y = residual + y
+        return y if out is None else out.copy_(y)
+
+    def _result(self, o_core, og_low, gate, residual=None, out=None):
+        if gate is None:
+            gate = self.og_proj[1](og_low)
         if gate.dtype != o_core.dtype:
             gate = gate.to(o_core.dtype)
         return _project(self.o_proj, kda_output(o_core, gate, self.g_norm.weight, self.g_norm.eps), residual, out)
@@ -392,15 +416,14 @@ class KimiDeltaAttention(nn.Module):
         """:meth:`decode_step_`, plus ``residual`` [B, 1, d], into ``out`` [B, 1, d]."""
         if x.shape[1] != 1:
             raise ValueError(f"decode_step_ takes one token, got x of shape {tuple(x.shape)}")
-        q, k, v, gk, bl, _, og = self._projections(x, conv_cache=state["conv"], use_cache=True,
-                                                   conv_out=state["conv"])
+        q, k, v, gk, bl, _, *og = self._core_inputs(x, conv_cache=state["conv"], use_cache=True, conv_out=state["conv"])
         rec = state["recurrent"]
         if rec is None:
             raise ValueError("decode_step_ needs an allocated recurrent state (run a prefill first)")
         a_log, dt_bias = self._gate_params()
         o_core, _ = kda_recurrent_gated(q, k, v, gk, bl, a_log, dt_bias, state=rec, state_dtype=rec.dtype,
                                         state_out=rec)
-        return self._output(o_core, og, residual, out)
+        return self._layer_output(o_core, *og, residual, out)
 
     def _train_forward(self, x):
         """The layer's forward for training (``kda.py:473-536`` differentiated by
@@ -450,7 +473,8 @@ class KimiDeltaAttention(nn.Module):
                 raise KdaError("the training path (grad mode with parameters that require grad) takes no cache "
                                "or state; run cached prefill and decode under torch.no_grad()")
             return self._train_forward(x)
-        if use_cache and state is None and x.shape[1] == 0:     # with tokens, no conv cache counts as zeros
+        # (with tokens, no conv cache counts as zeros)
+        if use_cache and state is None and (x.shape[1] == 0 or not self._unmodified("init_state")):
             state = self.init_state(x.shape[0], device=x.device, dtype=x.dtype)
         conv_cache = state["conv"] if state is not None else None
         rec = state["recurrent"] if state is not None else None
@@ -467,14 +491,16 @@ class KimiDeltaAttention(nn.Module):
         # H=16 d=128: 179 against 347 us for the core).
         split = (not fused and not (use_cache and T == 1) and body > 0 and (B == 1 or body == T)
                  and long_segments(B, body, self.num_heads, self.head_dim, self.value_head_dim, x.dtype) > 1)
-        q, k, v, g, beta, new_conv, og = self._projections(x, conv_cache=conv_cache, use_cache=use_cache,
-                                                           gates=split)
+        q, k, v, g, beta, new_conv, *og = self._core_inputs(x, conv_cache=conv_cache, use_cache=use_cache, gates=split)
         gate = self._gate_params()      # unless split, g and beta above are gk and the beta logits
         if fused:
             # one chunkwise body and no tail: the output epilogue runs on the
             # chunk kernel's tiles and its result is the o_proj input
-            y, new_rec = kda_chunkwise_fused(q, k, v, g, beta, *gate, self._output_gate(og), self.g_norm.weight, self.g_norm.eps,
-                                             initial_state=rec, chunk_size=C, state_dtype=sdtype)
+            og_low, og_gate = og
+            y, new_rec = kda_chunkwise_fused(q, k, v, g, beta, *gate,
+                                             self.og_proj[1](og_low) if og_gate is None else og_gate,
+                                             self.g_norm.weight, self.g_norm.eps, initial_state=rec, chunk_size=C,
+                                             state_dtype=sdtype)
             out = _project(self.o_proj, y)
             if use_cache:
                 return out, {"conv": new_conv, "recurrent": new_rec}
@@ -514,7 +540,10 @@ class KimiDeltaAttention(nn.Module):
             if o_core is None:
                 o_core = x.new_zeros(B, T, self.num_heads, self.value_head_dim)
             new_rec = rec
-        out = self._output(o_core, og)
+        out = self._layer_output(o_core, *og)
         if use_cache:
             return out, {"conv": new_conv, "recurrent": new_rec}
         return out
+
+
+_METHODS = {n: getattr(KimiDeltaAttention, n) for n in ("_projections", "_output", "init_state", "decode_step_")}

@@ -207,3 +207,67 @@ def test_layer_long_prefill_takes_the_split_core(kda_pkg, monkeypatch):
     print(f"  vs oracle: out {e:.3e} state {es:.3e}; vs one pass: out {e1:.3e} state {es1:.3e}", flush=True)
     assert e <= TOL[dtype] and es <= TOL[dtype]
     assert e1 <= TOL[dtype] and es1 <= TOL[dtype]
+
+
+# ----------------------------------------------------------------- methods of a subclass
+@pytest.mark.parametrize("where", ["subclass", "instance", "class"])
+def test_replaced_methods_are_called(kda_pkg, monkeypatch, where):
+    """_projections, _output, init_state and decode_step_ replaced by a subclass,
+    on the instance or on the class keep their arguments and results and take
+    part in prefill, decode and the graph decoder."""
+    import importlib
+    import types
+    decoder = importlib.import_module("kimi_linear_amd.graph_decode").KdaGraphedDecoder
+    base = kda_pkg.KimiDeltaAttention
+    old = {n: getattr(base, n) for n in ("_projections", "_output", "init_state", "decode_step_")}
+    seen = []
+
+    def _projections(self, x, conv_cache=None, use_cache=False, conv_out=None, gates=False):
+        seen.append("_projections")
+        *rest, og_low = old["_projections"](self, x, conv_cache=conv_cache, use_cache=use_cache, conv_out=conv_out,
+                                            gates=gates)
+        assert len(rest) == 6 and og_low.shape[:2] == x.shape[:2]
+        return (*rest, og_low * 0)                  # an output gate of 1/2
+
+    def _output(self, o_core, og_low):
+        seen.append("_output")
+        return old["_output"](self, o_core, og_low) + 1
+
+    def init_state(self, batch, device=None, dtype=None):
+        seen.append("init_state")
+        state = old["init_state"](self, batch, device=device, dtype=dtype)
+        state["conv"]["q"].fill_(0.5)
+        return state
+
+    def decode_step_(self, x, state):
+        seen.append("decode_step_")
+        return old["decode_step_"](self, x, state) * 2
+
+    new = dict(_projections=_projections, _output=_output, init_state=init_state, decode_step_=decode_step_)
+    mod, x = make_layer(kda_pkg, torch.float16)[0], make_x(2, 5, 256, torch.float16, 3).to(DEV)
+    with torch.no_grad():
+        start = old["init_state"](mod, 2, device=x.device, dtype=x.dtype)
+        start["conv"]["q"].fill_(0.5)
+        keep = mod.og_proj[1].weight.clone()        # the same layer by hand: a gate of 1/2 everywhere
+        mod.og_proj[1].weight.zero_()
+        y, st = mod(x[:, :4], state=start, use_cache=True)
+        want = [y + 1, 2 * (mod.decode_step_(x[:, 4:], st) + 1)]
+        mod.og_proj[1].weight.copy_(keep)
+    if where == "subclass":
+        mod.__class__ = type("Sub", (base,), new)
+    for n, f in new.items():
+        if where == "instance":
+            setattr(mod, n, types.MethodType(f, mod))
+        elif where == "class":
+            monkeypatch.setattr(base, n, f)
+    with torch.no_grad():
+        y, st = mod(x[:, :4], use_cache=True)
+        assert seen == ["init_state", "_projections", "_output"]
+        step = mod.decode_step_(x[:, 4:], st)
+        tol = TOL[torch.float16]        # the up-projections one by one: other sums, rounded the same
+        assert rel(y, want[0]) <= tol and rel(step, want[1]) <= tol
+        seen.clear()
+        dec = decoder([mod])
+        dec.prefill(x[:, :4])
+        assert seen.count("decode_step_") == 4 and seen.count("_output") == 5      # 3 warm-up steps and the capture
+        assert rel(dec.step(x[:, 4:]), (x[:, 4:] + want[1])[:, 0]) <= tol
