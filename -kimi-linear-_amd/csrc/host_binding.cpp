@@ -163,9 +163,16 @@ void strides3(int64_t (&out)[3], const Tensor& t) {
     for (int i = 0; i < 3; ++i) out[i] = t.stride(i);
 }
 
+// From a tensor's first byte to past its last, the gaps of its strides included.
+size_t extent(const Tensor& t) {
+    int64_t last = 0;
+    for (int64_t i = 0; i < t.dim(); ++i) last += (t.size(i) - 1) * t.stride(i);
+    return t.numel() == 0 ? 0 : static_cast<size_t>((last + 1) * t.element_size());
+}
+
 bool overlaps(const Tensor& a, const Tensor& b) {
     const auto a0 = reinterpret_cast<uintptr_t>(a.data_ptr()), b0 = reinterpret_cast<uintptr_t>(b.data_ptr());
-    return a0 < b0 + b.nbytes() && b0 < a0 + a.nbytes();
+    return a0 < b0 + extent(b) && b0 < a0 + extent(a);
 }
 
 // kda_chunkwise / kda_recurrent (recurrent), with the gates' parameters their

@@ -263,3 +263,19 @@ def test_another_torch_than_it_was_compiled_against(kda_pkg, monkeypatch):
     monkeypatch.setattr(torch, "__version__", "0.0.1")
     with pytest.raises(native.NativeLibraryError, match="torch 0.0.1; rebuild"):
         native.host()
+
+
+def test_an_output_among_the_rows_of_an_input_is_the_general_paths(stand_in):
+    """x or the residual as every other row of a buffer whose last row is the output:
+    it lies past as many bytes as they hold, before their end."""
+    mod = stand_in(kda_linear_fwd=lambda *a: 0)
+    w = torch.rand(64, 64).half()
+    buf = torch.rand(8, 1, 64).half()
+    rows, out = buf[:7:2], buf[5:6]                       # rows 0, 2, 4, 6
+    with torch.no_grad():
+        assert mod.linear(rows[:3], w, None, buf[5:8]) is not None
+        assert mod.linear(rows, w, None, buf[4:8]) is None
+        assert mod.linear(buf[:1].expand(1, 1, 64), w, rows[:1], out) is not None
+        x = torch.rand(4, 1, 64).half()
+        assert mod.linear(x, w, rows, buf[4:8]) is None and mod.linear(x, w, rows, None) is not None
+        assert mod.linear(x, w[:16], None, x.view(-1)[64:128].view(4, 1, 16)) is None
