@@ -53,6 +53,7 @@ from types import SimpleNamespace
 
 import torch
 import torch.nn as nn
+from torch.overrides import has_torch_function
 
 from . import _native
 from .kda import (KdaError, kda_chunkwise, kda_chunkwise_fused, kda_chunkwise_gated, kda_recurrent,
@@ -157,18 +158,20 @@ class _LinearFn(torch.autograd.Function):
 
 def _project_train(mod, x):
     """``mod(x)``, differentiable; :class:`_LinearFn` where that is all the module does."""
-    w = _plain_weight(mod)
+    w = _plain_weight(mod, x)
     if (w is None or mod._backward_hooks or mod._backward_pre_hooks or w.dtype != x.dtype
             or x.dtype not in (torch.float16, torch.bfloat16) or torch.is_autocast_enabled(x.device.type)):
         return mod(x)
     return _LinearFn.apply(x, w)
 
 
-def _plain_weight(mod):
+def _plain_weight(mod, *inputs):
     """The weight of a module that is just x W^T: an ``nn.Linear`` as torch has it,
-    without a bias, hooks or a forward of its own; else None."""
+    without a bias, hooks or a forward of its own, with no torch function mode
+    or tensor subclass that takes part in ``F.linear``; else None."""
     if (type(mod) is not nn.Linear or mod.bias is not None or mod._forward_hooks or mod._forward_pre_hooks
-            or "forward" in mod.__dict__ or nn.modules.module._has_any_global_hook()):
+            or "forward" in mod.__dict__ or nn.modules.module._has_any_global_hook()
+            or has_torch_function((mod.weight, *inputs))):
         return None
     return mod.weight
 
@@ -176,7 +179,7 @@ def _plain_weight(mod):
 def _project(mod, x, residual=None, out=None):
     """``mod(x)``, plus ``residual``, into ``out``: in the few-row kernel
     (``kda_linear_fwd``, up to 64 rows) where it applies, else as written."""
-    w = _plain_weight(mod) if x.shape[0] * x.shape[1] <= 64 else None
+    w = _plain_weight(mod, x) if x.shape[0] * x.shape[1] <= 64 else None
     y = _native.host().linear(x, w, residual, out) if w is not None else None
     if y is not None:
         return y
@@ -348,7 +351,7 @@ class KimiDeltaAttention(nn.Module):
         convs = (self.conv_q.conv, self.conv_k.conv, self.conv_v.conv)
         H, K, V = self.num_heads, self.head_dim, self.value_head_dim
         w, b = self._input_weight()
-        few = x.shape[0] * x.shape[1] <= 64
+        few = x.shape[0] * x.shape[1] <= 64 and not has_torch_function((x,))
         y = _native.host().linear(x, w, None, None) if few and b is None else None
         if y is None:
             y = torch.nn.functional.linear(x, w, b)

@@ -57,3 +57,26 @@ def test_l2norm(kda_pkg):
     tiny = torch.full((1, 64), 1e-9)                      # rsqrt clamped to 1 / eps
     assert torch.allclose(kda_pkg.l2norm(tiny, 1e-6), tiny * 1e6)
     assert kda_pkg.l2norm(x.half(), 1e-6).dtype == torch.float16
+
+
+def test_a_function_mode_or_subclass_sees_the_projections(kda_pkg):
+    """A torch function mode or a tensor subclass may change ``F.linear``: the
+    projections are then the module's own call."""
+    import importlib
+    from torch.overrides import TorchFunctionMode
+    layer = importlib.import_module("kimi_linear_amd.layer")
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    mod, x = torch.nn.Linear(8, 4, bias=False), torch.randn(1, 1, 8)
+    assert layer._plain_weight(mod, x) is mod.weight
+    assert layer._plain_weight(mod, x.as_subclass(Sub)) is None
+    with Mode():
+        assert layer._plain_weight(mod, x) is None
+    mod.weight = torch.nn.Parameter(mod.weight.detach().as_subclass(Sub))
+    assert layer._plain_weight(mod, x) is None
