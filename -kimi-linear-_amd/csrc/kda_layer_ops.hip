@@ -36,15 +36,16 @@ constexpr int kTile = 16;      // tokens per prep unit at most; an in-place conv
 constexpr int kMaxConv = 4;    // largest conv_size
 // ---- prep: kSeg channels of q, k or v over a token tile ---------------------
 // DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
-// conv_size when it is 4 (the usual case, no test of the tap count in the
-// loops), else 0.
+// conv_size, so that the taps of a lane's channels are a few wide loads: with a
+// runtime size each was a load and a wait of its own (us, bf16 unless said: a
+// decode step at B=33 H=16 K=V=128 conv_size 2 6.0 -> 3.0, two channels a lane
+// took 3.7; B=4 T=125 H=16 fp16 conv_size 3 with the gates 12.1 -> 7.6, 9.6).
 template <typename XT, int DH, int TILE, int CS>
 __device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t b, int64_t t0, int64_t seg, int lane) {
-    constexpr int kRows = TILE + kMaxConv - 1, N = kLaneCh<XT>;
+    constexpr int cs = CS, cm = cs - 1, kRows = TILE + cm, N = kLaneCh<XT>;
     const int64_t D = a.H * (DH ? DH : a.V);
     const bool valid = seg * kSeg<XT> + N * lane < D;
     const int64_t ch0 = valid ? seg * kSeg<XT> + N * lane : 0;
-    const int cs = CS ? CS : static_cast<int>(a.conv_size), cm = cs - 1;
     const int64_t T = a.T;
     const int n = static_cast<int>((T - t0) < TILE ? (T - t0) : TILE);
     const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0];
@@ -68,42 +69,32 @@ __device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t
             for (int c = 0; c < Raw<XT, N>::W; ++c) win[r].w[c] = 0u;
         }
     }
-    float w[kMaxConv][N], bias[N];
+    float w[cs][N], wc[N * cs], bias[N];
 #pragma unroll
     for (int c = 0; c < N; ++c) bias[c] = 0.f;
     if (a.conv_b[i] != nullptr) params<N>(a.conv_b[i], ch0, a.w_dtype, bias);
-    if constexpr (CS == kMaxConv) {
-        float wc[N * kMaxConv];
-        params<N * kMaxConv>(a.conv_w[i], ch0 * kMaxConv, a.w_dtype, wc);
+    params<N * cs>(a.conv_w[i], ch0 * cs, a.w_dtype, wc);
 #pragma unroll
-        for (int c = 0; c < N; ++c)
+    for (int c = 0; c < N; ++c)
 #pragma unroll
-            for (int j = 0; j < kMaxConv; ++j) w[j][c] = wc[kMaxConv * c + j];
-    } else {
-#pragma unroll
-        for (int c = 0; c < N; ++c)
-#pragma unroll
-            for (int j = 0; j < kMaxConv; ++j)
-                w[j][c] = j < cs ? load_elem(a.conv_w[i], (ch0 + c) * cs + j, a.w_dtype) : 0.f;
-    }
+        for (int j = 0; j < cs; ++j) w[j][c] = wc[cs * c + j];
 
     XT* out = static_cast<XT*>(i == 0 ? a.q : (i == 1 ? a.k : a.v)) + (b * T + t0) * D + ch0;
     const float inv_eps = 1.f / a.l2_eps;
     // tap j of tile token t reads window row t + j (token t0 + t - cm + j)
-    float xs[kMaxConv][N];
+    float xs[cs][N];
 #pragma unroll
-    for (int j = 0; j < kMaxConv - 1; ++j) unpack(win[j], xs[j]);
+    for (int j = 0; j < cm; ++j) unpack(win[j], xs[j]);
 #pragma unroll
     for (int t = 0; t < TILE; ++t) {
-        unpack(win[t + kMaxConv - 1], xs[(t + kMaxConv - 1) % kMaxConv]);
+        unpack(win[t + cm], xs[(t + cm) % cs]);
         float s[N];
         float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < N; ++c) {
             float u = bias[c];
 #pragma unroll
-            for (int j = 0; j < kMaxConv; ++j)
-                if (j < cs) u = fmaf(w[j][c], xs[(t + j) % kMaxConv][c], u);
+            for (int j = 0; j < cs; ++j) u = fmaf(w[j][c], xs[(t + j) % cs][c], u);
             s[c] = u * sigmoid_f(u);
             ss = fmaf(s[c], s[c], ss);
         }
@@ -120,12 +111,12 @@ __device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t
     if (a.hist_out[i] != nullptr && t0 + n == T && valid) {
         XT* ho = static_cast<XT*>(a.hist_out[i]) + b * cm * D + ch0;
 #pragma unroll
-        for (int r = 0; r < kMaxConv - 1; ++r) {
+        for (int r = 0; r < cm; ++r) {
             Raw<XT, N> hv = win[r];
 #pragma unroll
             for (int rr = 0; rr < kRows; ++rr)
                 if (rr == n + r) hv = win[rr];
-            if (r < cm) __builtin_memcpy(ho + r * D, hv.w, sizeof(hv.w));
+            __builtin_memcpy(ho + r * D, hv.w, sizeof(hv.w));
         }
     }
 }
@@ -203,13 +194,19 @@ __global__ __launch_bounds__(256) void prep_kernel(const kda_prep_args a, uint32
     uint32_t s = unit % per;
     const uint32_t bt = unit / per;
     const int64_t t0 = static_cast<int64_t>(bt % ntiles) * TILE, b = bt / ntiles;
+    const auto conv = [&](auto dh, int i, int64_t seg) {
+        constexpr int DH = decltype(dh)::value;
+        switch (a.conv_size) {
+            case 4: conv_unit<XT, DH, TILE, 4>(a, i, b, t0, seg, lane); break;
+            case 3: conv_unit<XT, DH, TILE, 3>(a, i, b, t0, seg, lane); break;
+            case 2: conv_unit<XT, DH, TILE, 2>(a, i, b, t0, seg, lane); break;
+            default: conv_unit<XT, DH, TILE, 1>(a, i, b, t0, seg, lane);
+        }
+    };
     if (s < 2 * segk) {
-        const int i = s >= segk;
-        if (a.conv_size == 4) conv_unit<XT, K, TILE, 4>(a, i, b, t0, s - i * segk, lane);
-        else conv_unit<XT, K, TILE, 0>(a, i, b, t0, s - i * segk, lane);
+        conv(std::integral_constant<int, K>{}, s >= segk, s - (s >= segk) * segk);
     } else if (s < 2 * segk + segv) {
-        if (a.conv_size == 4) conv_unit<XT, 0, TILE, 4>(a, 2, b, t0, s - 2 * segk, lane);
-        else conv_unit<XT, 0, TILE, 0>(a, 2, b, t0, s - 2 * segk, lane);
+        conv(std::integral_constant<int, 0>{}, 2, s - 2 * segk);
     } else {
         gate_unit<XT, K, TILE>(a, b, t0, s - 2 * segk - segv, lane);
     }
