@@ -110,7 +110,8 @@ __device__ __forceinline__ void sum_waves(float (&v)[N], float* red, int wave, i
 
 // ---- q, k or v: kSeg channels over a token tile ------------------------------
 // DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
-// conv_size when it is 4, else 0.  The tokens go by once: du[t] needs the x
+// conv_size, so that the taps are a few wide loads (one load and wait for each
+// took 60.6 us at B=20 T=704 H=1 d=64 conv_size 2, before this split 37.0).  The tokens go by once: du[t] needs the x
 // rows t - 3 .. t and completes dx[t - 3], so four x rows and four partial dx
 // rows are held, in slots by the token's index modulo 4, and a wave's last
 // three dx take du of three tokens past its own.  wl[L] is the tap of lag L:
@@ -123,7 +124,7 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
     const int64_t D = a.H * (DH ? DH : a.V), T = a.T;
     const bool valid = seg * kSeg<XT> + N * lane < D;
     const int64_t ch0 = valid ? seg * kSeg<XT> + N * lane : 0;
-    const int cs = CS ? CS : static_cast<int>(a.conv_size), cm = cs - 1;
+    constexpr int cs = CS, cm = cs - 1;
     const int64_t dxs = a.dx_stride ? a.dx_stride : D;
     const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0] + ch0;
     const XT* dy = static_cast<const XT*>(a.dy[i]) + b * T * D + ch0;
@@ -141,7 +142,7 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
         }
     };
     fetch(0);
-    float xs[G][N], dxa[G][N], wl[G][N], bias[N], dws[G][N], dbs[N];
+    float xs[G][N], dxa[G][N], wl[cs][N], wc[N * cs], bias[N], dws[cs][N], dbs[N];
 #pragma unroll
     for (int r = 1; r < G; ++r) {                       // tokens t0 - 3 .. t0 - 1
         const int64_t tok = t0 - G + r;
@@ -155,24 +156,18 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
 #pragma unroll
     for (int c = 0; c < N; ++c) bias[c] = dbs[c] = 0.f;
     if (a.conv_b[i] != nullptr) params<N>(a.conv_b[i], ch0, a.w_dtype, bias);
-    if constexpr (CS == kMaxConvB) {
-        float wc[N * kMaxConvB];
-        params<N * kMaxConvB>(a.conv_w[i], ch0 * kMaxConvB, a.w_dtype, wc);
+    params<N * cs>(a.conv_w[i], ch0 * cs, a.w_dtype, wc);
 #pragma unroll
-        for (int c = 0; c < N; ++c)
+    for (int c = 0; c < N; ++c)
 #pragma unroll
-            for (int L = 0; L < G; ++L) wl[L][c] = wc[kMaxConvB * c + kMaxConvB - 1 - L];
-    } else {
-#pragma unroll
-        for (int c = 0; c < N; ++c)
-#pragma unroll
-            for (int L = 0; L < G; ++L)
-                wl[L][c] = L <= cm ? load_elem(a.conv_w[i], (ch0 + c) * cs + cm - L, a.w_dtype) : 0.f;
-    }
+        for (int L = 0; L < cs; ++L) {
+            wl[L][c] = wc[cs * c + cm - L];
+            dws[L][c] = 0.f;
+        }
 #pragma unroll
     for (int L = 0; L < G; ++L)
 #pragma unroll
-        for (int c = 0; c < N; ++c) dws[L][c] = dxa[L][c] = 0.f;
+        for (int c = 0; c < N; ++c) dxa[L][c] = 0.f;
     const float inv_eps = 1.f / a.l2_eps;
 
     for (int idx0 = 0; n > 0 && idx0 < n + G - 1; idx0 += G) {
@@ -191,8 +186,7 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
             for (int c = 0; c < N; ++c) {
                 u[c] = bias[c];
 #pragma unroll
-                for (int L = G - 1; L >= 0; --L)
-                    if (L <= cm) u[c] = fmaf(wl[L][c], xs[(r - L + G) % G][c], u[c]);
+                for (int L = cm; L >= 0; --L) u[c] = fmaf(wl[L][c], xs[(r - L + G) % G][c], u[c]);
                 sg[c] = sigmoid_f(u[c]);
                 s[c] = u[c] * sg[c];
                 ss = fmaf(s[c], s[c], ss);
@@ -213,28 +207,28 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
                 d[c] = in ? d[c] : 0.f;
                 dxa[r][c] = wl[0][c] * d[c];
 #pragma unroll
-                for (int L = 1; L < G; ++L)
-                    if (L <= cm) dxa[(r - L + G) % G][c] = fmaf(wl[L][c], d[c], dxa[(r - L + G) % G][c]);
+                for (int L = 1; L < cs; ++L)
+                    dxa[(r - L + G) % G][c] = fmaf(wl[L][c], d[c], dxa[(r - L + G) % G][c]);
             }
             if (idx < n) {                              // the tile's own tokens
 #pragma unroll
                 for (int c = 0; c < N; ++c) {
                     dbs[c] += d[c];
 #pragma unroll
-                    for (int L = 0; L < G; ++L)
-                        if (L <= cm) dws[L][c] = fmaf(d[c], xs[(r - L + G) % G][c], dws[L][c]);
+                    for (int L = 0; L < cs; ++L)
+                        dws[L][c] = fmaf(d[c], xs[(r - L + G) % G][c], dws[L][c]);
                 }
             }
             const int e = idx - (G - 1);
             if (e >= 0 && e < n && valid) stn(dx + (t0 + e) * dxs, dxa[(r + 1) % G]);
         }
     }
-    float sums[(G + 1) * N];
+    float sums[(cs + 1) * N];
 #pragma unroll
     for (int c = 0; c < N; ++c) {
 #pragma unroll
-        for (int L = 0; L < G; ++L) sums[L * N + c] = dws[L][c];
-        sums[G * N + c] = dbs[c];
+        for (int L = 0; L < cs; ++L) sums[L * N + c] = dws[L][c];
+        sums[cs * N + c] = dbs[c];
     }
     sum_waves(sums, red, wave, lane);
     if (!valid || wave > 0) return;
@@ -242,9 +236,8 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
 #pragma unroll
     for (int c = 0; c < N; ++c) {
 #pragma unroll
-        for (int L = 0; L < G; ++L)
-            if (L <= cm) pp.dw[i][(row * D + ch0 + c) * cs + cm - L] = sums[L * N + c];
-        if (a.db[i] != nullptr) pp.db[i][row * D + ch0 + c] = sums[G * N + c];
+        for (int L = 0; L < cs; ++L) pp.dw[i][(row * D + ch0 + c) * cs + cm - L] = sums[L * N + c];
+        if (a.db[i] != nullptr) pp.db[i][row * D + ch0 + c] = sums[cs * N + c];
     }
 }
 
@@ -331,10 +324,9 @@ __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const 
 // in brackets: B=4 T=2048 bf16 213 -> 135 (139), fp16 177 -> 138 (141), fp32
 // 202 -> 184 (197); B=1 T=2048 bf16 65 -> 42 (55); B=1 T=500 52 -> 22 (49);
 // B=1 T=1024 H=8 d=64 fp16 42 -> 20 (48).
-template <typename XT, int K, bool FULL>
+template <typename XT, int K, int CS>
 __global__ __launch_bounds__(64 * kSub, 2) void prep_bwd_kernel(const kda_prep_bwd_args a, const PrepParts pp,
                                                          uint32_t ntiles, uint32_t convs) {
-    constexpr int CS = FULL ? kMaxConvB : 0;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __shared__ float red[(kSub - 1) * (kGroup + 1) * kLaneCh<XT> * 64];
     if (blockIdx.x >= convs) {
@@ -517,7 +509,7 @@ int validate_output_bwd(const kda_output_bwd_args* a) {
     return KDA_OK;
 }
 
-template <typename XT, int K, bool FULL>
+template <typename XT, int K, int CS>
 int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
     const PrepParts pp = prep_parts(a.workspace, a.B, a.T, a.H, a.K, a.V, a.conv_size);
     const int64_t ntiles = (a.T + kPrepTile - 1) / kPrepTile, hk = a.H * a.K, hv = a.H * a.V;
@@ -526,7 +518,7 @@ int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
     const int64_t gates = a.gk != nullptr ? pp.rows * segs(hk, kGateSeg) : 0;
     const dim3 grid(static_cast<unsigned>(convs + gates));
     const uint32_t nt = static_cast<uint32_t>(ntiles), nc = static_cast<uint32_t>(convs);
-    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, FULL>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc);
+    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, CS>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc);
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
     ColSums c{};
     c.rows = pp.rows;
@@ -545,13 +537,19 @@ int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
     return launch_colsum(c, n, stream);
 }
 
+template <typename XT, int K>
+int launch_prep_bwd_conv(const kda_prep_bwd_args& a, hipStream_t stream) {
+    switch (a.conv_size) {
+        case 4: return launch_prep_bwd<XT, K, 4>(a, stream);
+        case 3: return launch_prep_bwd<XT, K, 3>(a, stream);
+        case 2: return launch_prep_bwd<XT, K, 2>(a, stream);
+        default: return launch_prep_bwd<XT, K, 1>(a, stream);
+    }
+}
+
 template <typename XT>
 int launch_prep_bwd_dims(const kda_prep_bwd_args& a, hipStream_t stream) {
-    if (a.K == 64)
-        return a.conv_size == kMaxConvB ? launch_prep_bwd<XT, 64, true>(a, stream)
-                                        : launch_prep_bwd<XT, 64, false>(a, stream);
-    return a.conv_size == kMaxConvB ? launch_prep_bwd<XT, 128, true>(a, stream)
-                                    : launch_prep_bwd<XT, 128, false>(a, stream);
+    return a.K == 64 ? launch_prep_bwd_conv<XT, 64>(a, stream) : launch_prep_bwd_conv<XT, 128>(a, stream);
 }
 
 template <typename XT>
