@@ -114,11 +114,12 @@ __device__ __forceinline__ void sum_waves(float (&v)[N], float* red, int wave, i
 // took 60.6 us at B=20 T=704 H=1 d=64 conv_size 2, before this split 37.0).  The tokens go by once: du[t] needs the x
 // rows t - 3 .. t and completes dx[t - 3], so four x rows and four partial dx
 // rows are held, in slots by the token's index modulo 4, and a wave's last
-// three dx take du of three tokens past its own.  wl[L] is the tap of lag L:
+// three dx take du of three tokens past its own.  tw: tokens a wave, a quarter
+// of the tile, or of a shorter sequence, in whole groups.  wl[L] is the tap of lag L:
 // u[t] = sum_L wl[L] x[t - L], dx[t] = sum_L wl[L] du[t + L].
 template <typename XT, int DH, int CS>
 __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int i, int64_t b,
-                                              int64_t tile, int64_t seg, int wave, int lane, float* red) {
+                                              int64_t tile, int64_t seg, int wave, int lane, int tw, float* red) {
     constexpr int N = kLaneCh<XT>, G = kGroup;
     static_assert(G == kMaxConvB, "a row's slot is its index in the group");
     const int64_t D = a.H * (DH ? DH : a.V), T = a.T;
@@ -129,8 +130,8 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
     const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0] + ch0;
     const XT* dy = static_cast<const XT*>(a.dy[i]) + b * T * D + ch0;
     XT* dx = static_cast<XT*>(a.dx[i]) + b * T * dxs + ch0;
-    const int64_t t0 = tile * kPrepTile + wave * (kPrepTile / kSub);
-    const int n = static_cast<int>(T - t0 < kPrepTile / kSub ? T - t0 : kPrepTile / kSub);     // <= 0: no token
+    const int64_t t0 = tile * kPrepTile + wave * tw;
+    const int n = static_cast<int>(T - t0 < tw ? T - t0 : tw);      // <= 0: no token
 
     Raw<XT, N> nx[G], ny[G];
     const auto fetch = [&](int idx) {                   // rows past the end re-read the last token
@@ -244,7 +245,7 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
 // ---- the gates of 256 channels over a token tile, and the betas of their heads
 template <typename XT, int DH>
 __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int64_t b, int64_t tile,
-                                              int64_t seg, int wave, int lane, float* red) {
+                                              int64_t seg, int wave, int lane, int tw, float* red) {
     constexpr int N = 4, kHeads = kGateSeg / DH;
     const int64_t D = a.H * DH, T = a.T;
     const bool valid = seg * kGateSeg + N * lane < D;
@@ -261,8 +262,8 @@ __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const 
     const float* dg = a.dg + b * T * D + ch0;
     XT* dgk = static_cast<XT*>(a.dgk) + b * T * D + ch0;
     const int64_t dls = a.dx_stride ? a.dx_stride : a.H;
-    const int64_t t0 = tile * kPrepTile + wave * (kPrepTile / kSub);
-    const int64_t t1 = t0 + kPrepTile / kSub < T ? t0 + kPrepTile / kSub : T;
+    const int64_t t0 = tile * kPrepTile + wave * tw;
+    const int64_t t1 = t0 + tw < T ? t0 + tw : T;
     // lane e < kStep kHeads of a step takes the beta of its token e / kHeads, head e % kHeads
     const int64_t bh = seg * kHeads + lane % kHeads;
     const bool beta_lane = lane < kStep * kHeads && bh < a.H;
@@ -326,13 +327,13 @@ __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const 
 // B=1 T=1024 H=8 d=64 fp16 42 -> 20 (48).
 template <typename XT, int K, int CS>
 __global__ __launch_bounds__(64 * kSub, 2) void prep_bwd_kernel(const kda_prep_bwd_args a, const PrepParts pp,
-                                                         uint32_t ntiles, uint32_t convs) {
+                                                         uint32_t ntiles, uint32_t convs, int tw) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __shared__ float red[(kSub - 1) * (kGroup + 1) * kLaneCh<XT> * 64];
     if (blockIdx.x >= convs) {
         const uint32_t u = blockIdx.x - convs, segs = (static_cast<uint32_t>(a.H) * K + kGateSeg - 1) / kGateSeg;
         const uint32_t bt = u / segs;
-        gate_bwd_unit<XT, K>(a, pp, bt / ntiles, bt % ntiles, u % segs, wave, lane, red);
+        gate_bwd_unit<XT, K>(a, pp, bt / ntiles, bt % ntiles, u % segs, wave, lane, tw, red);
         return;
     }
     const uint32_t segk = (static_cast<uint32_t>(a.H) * K + kSeg<XT> - 1) / kSeg<XT>;
@@ -341,9 +342,9 @@ __global__ __launch_bounds__(64 * kSub, 2) void prep_bwd_kernel(const kda_prep_b
     const int64_t tile = bt % ntiles, b = bt / ntiles;
     if (s < 2 * segk) {
         const int i = s >= segk;
-        conv_bwd_unit<XT, K, CS>(a, pp, i, b, tile, s - i * segk, wave, lane, red);
+        conv_bwd_unit<XT, K, CS>(a, pp, i, b, tile, s - i * segk, wave, lane, tw, red);
     } else {
-        conv_bwd_unit<XT, 0, CS>(a, pp, 2, b, tile, s - 2 * segk, wave, lane, red);
+        conv_bwd_unit<XT, 0, CS>(a, pp, 2, b, tile, s - 2 * segk, wave, lane, tw, red);
     }
 }
 
@@ -518,7 +519,11 @@ int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
     const int64_t gates = a.gk != nullptr ? pp.rows * segs(hk, kGateSeg) : 0;
     const dim3 grid(static_cast<unsigned>(convs + gates));
     const uint32_t nt = static_cast<uint32_t>(ntiles), nc = static_cast<uint32_t>(convs);
-    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, CS>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc);
+    // a sequence of one tile is shared out among its waves (us with 16 tokens a
+    // wave -> this: B=52 T=18 H=8 d=128 bf16 32.8 -> 24.1, B=16 T=24 H=16 d=64 fp16
+    // conv 2 16.6 -> 12.6; a wave a head took 27.0 and 14.2)
+    const int tw = ntiles > 1 ? kPrepTile / kSub : static_cast<int>((a.T + kGroup * kSub - 1) / (kGroup * kSub)) * kGroup;
+    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, CS>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc, tw);
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
     ColSums c{};
     c.rows = pp.rows;
