@@ -108,7 +108,7 @@ __device__ __forceinline__ void sum_waves(float (&v)[N], float* red, int wave, i
     }
 }
 
-// ---- q, k or v: kSeg channels over a token tile ------------------------------
+// ---- q, k or v: 64 N channels over a token tile ------------------------------
 // DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
 // conv_size, so that the taps are a few wide loads (one load and wait for each
 // took 60.6 us at B=20 T=704 H=1 d=64 conv_size 2, before this split 37.0).  The tokens go by once: du[t] needs the x
@@ -117,14 +117,14 @@ __device__ __forceinline__ void sum_waves(float (&v)[N], float* red, int wave, i
 // three dx take du of three tokens past its own.  tw: tokens a wave, a quarter
 // of the tile, or of a shorter sequence, in whole groups.  wl[L] is the tap of lag L:
 // u[t] = sum_L wl[L] x[t - L], dx[t] = sum_L wl[L] du[t + L].
-template <typename XT, int DH, int CS>
+template <typename XT, int DH, int CS, int N>
 __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const PrepParts& pp, int i, int64_t b,
                                               int64_t tile, int64_t seg, int wave, int lane, int tw, float* red) {
-    constexpr int N = kLaneCh<XT>, G = kGroup;
+    constexpr int G = kGroup;
     static_assert(G == kMaxConvB, "a row's slot is its index in the group");
     const int64_t D = a.H * (DH ? DH : a.V), T = a.T;
-    const bool valid = seg * kSeg<XT> + N * lane < D;
-    const int64_t ch0 = valid ? seg * kSeg<XT> + N * lane : 0;
+    const bool valid = seg * (64 * N) + N * lane < D;
+    const int64_t ch0 = valid ? seg * (64 * N) + N * lane : 0;
     constexpr int cs = CS, cm = cs - 1;
     const int64_t dxs = a.dx_stride ? a.dx_stride : D;
     const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0] + ch0;
@@ -156,8 +156,8 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
     }
 #pragma unroll
     for (int c = 0; c < N; ++c) bias[c] = dbs[c] = 0.f;
-    if (a.conv_b[i] != nullptr) params<N>(a.conv_b[i], ch0, a.w_dtype, bias);
-    params<N * cs>(a.conv_w[i], ch0 * cs, a.w_dtype, wc);
+    if (a.conv_b[i] != nullptr) decode(ld_params<N>(a.conv_b[i], ch0, a.w_dtype), a.w_dtype, bias);
+    decode(ld_params<N * cs>(a.conv_w[i], ch0 * cs, a.w_dtype), a.w_dtype, wc);
 #pragma unroll
     for (int c = 0; c < N; ++c)
 #pragma unroll
@@ -182,7 +182,6 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
             float d[N], u[N], sg[N], s[N];
             unpack(cx[r], xs[r]);
             unpack(cy[r], d);
-            float ss = 0.f, sd = 0.f;
 #pragma unroll
             for (int c = 0; c < N; ++c) {
                 u[c] = bias[c];
@@ -190,12 +189,10 @@ __device__ __forceinline__ void conv_bwd_unit(const kda_prep_bwd_args& a, const 
                 for (int L = cm; L >= 0; --L) u[c] = fmaf(wl[L][c], xs[(r - L + G) % G][c], u[c]);
                 sg[c] = sigmoid_f(u[c]);
                 s[c] = u[c] * sg[c];
-                ss = fmaf(s[c], s[c], ss);
-                sd = fmaf(s[c], d[c], sd);
             }
             if constexpr (DH != 0) {
                 // y = s min(rsqrt(sum s^2), 1/eps): a clamped row is s / eps
-                const float rn = rsqrtf(lanes_sum<DH / N>(ss)), dot = lanes_sum<DH / N>(sd);
+                const float rn = rsqrtf(head_dot<XT, DH>(s, s)), dot = head_dot<XT, DH>(s, d);
                 const bool clamped = !(rn < inv_eps);
                 const float k3 = rn * rn * rn * dot;
 #pragma unroll
@@ -251,8 +248,8 @@ __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const 
     const bool valid = seg * kGateSeg + N * lane < D;
     const int64_t ch0 = valid ? seg * kGateSeg + N * lane : 0;
     float neg_a[N], dtb[N], sa[N], sd[N];
-    params<N>(a.a_log, ch0, a.p_dtype, neg_a);
-    params<N>(a.dt_bias, ch0, a.p_dtype, dtb);
+    decode(ld_params<N>(a.a_log, ch0, a.p_dtype), a.p_dtype, neg_a);
+    decode(ld_params<N>(a.dt_bias, ch0, a.p_dtype), a.p_dtype, dtb);
 #pragma unroll
     for (int c = 0; c < N; ++c) {
         neg_a[c] = -__expf(neg_a[c]);
@@ -316,7 +313,7 @@ __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const 
     }
 }
 
-// One workgroup per (batch, tile, kSeg channels of q, k, v or kGateSeg of the
+// One workgroup per (batch, tile, 64 N channels of q, k, v or kGateSeg of the
 // gates), the gates' shorter units last, into what the others leave free.
 // Bound by the arithmetic on the channels (about 40 operations each, two of
 // them transcendental) at two waves a SIMD.  A wave a head, two channels a
@@ -325,26 +322,25 @@ __device__ __forceinline__ void gate_bwd_unit(const kda_prep_bwd_args& a, const 
 // in brackets: B=4 T=2048 bf16 213 -> 135 (139), fp16 177 -> 138 (141), fp32
 // 202 -> 184 (197); B=1 T=2048 bf16 65 -> 42 (55); B=1 T=500 52 -> 22 (49);
 // B=1 T=1024 H=8 d=64 fp16 42 -> 20 (48).
-template <typename XT, int K, int CS>
+template <typename XT, int K, int CS, int N>
 __global__ __launch_bounds__(64 * kSub, 2) void prep_bwd_kernel(const kda_prep_bwd_args a, const PrepParts pp,
                                                          uint32_t ntiles, uint32_t convs, int tw) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    __shared__ float red[(kSub - 1) * (kGroup + 1) * kLaneCh<XT> * 64];
+    __shared__ float red[(kSub - 1) * ((CS + 1) * N > 8 ? (CS + 1) * N : 8) * 64];    // (the gates: 8 sums a lane)
     if (blockIdx.x >= convs) {
         const uint32_t u = blockIdx.x - convs, segs = (static_cast<uint32_t>(a.H) * K + kGateSeg - 1) / kGateSeg;
         const uint32_t bt = u / segs;
         gate_bwd_unit<XT, K>(a, pp, bt / ntiles, bt % ntiles, u % segs, wave, lane, tw, red);
         return;
     }
-    const uint32_t segk = (static_cast<uint32_t>(a.H) * K + kSeg<XT> - 1) / kSeg<XT>;
-    const uint32_t segv = static_cast<uint32_t>((a.H * a.V + kSeg<XT> - 1) / kSeg<XT>);
+    const uint32_t segk = static_cast<uint32_t>(segments(a.H * K, N)), segv = static_cast<uint32_t>(segments(a.H * a.V, N));
     const uint32_t per = 2 * segk + segv, s = blockIdx.x % per, bt = blockIdx.x / per;
     const int64_t tile = bt % ntiles, b = bt / ntiles;
     if (s < 2 * segk) {
         const int i = s >= segk;
-        conv_bwd_unit<XT, K, CS>(a, pp, i, b, tile, s - i * segk, wave, lane, tw, red);
+        conv_bwd_unit<XT, K, CS, N>(a, pp, i, b, tile, s - i * segk, wave, lane, tw, red);
     } else {
-        conv_bwd_unit<XT, 0, CS>(a, pp, 2, b, tile, s - 2 * segk, wave, lane, tw, red);
+        conv_bwd_unit<XT, 0, CS, N>(a, pp, 2, b, tile, s - 2 * segk, wave, lane, tw, red);
     }
 }
 
@@ -510,20 +506,19 @@ int validate_output_bwd(const kda_output_bwd_args* a) {
     return KDA_OK;
 }
 
-template <typename XT, int K, int CS>
-int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
+template <typename XT, int K, int CS, int N>
+int launch_prep_bwd_n(const kda_prep_bwd_args& a, hipStream_t stream) {
     const PrepParts pp = prep_parts(a.workspace, a.B, a.T, a.H, a.K, a.V, a.conv_size);
     const int64_t ntiles = (a.T + kPrepTile - 1) / kPrepTile, hk = a.H * a.K, hv = a.H * a.V;
-    const auto segs = [](int64_t d, int64_t n) { return (d + n - 1) / n; };
-    const int64_t convs = pp.rows * (2 * segs(hk, kSeg<XT>) + segs(hv, kSeg<XT>));
-    const int64_t gates = a.gk != nullptr ? pp.rows * segs(hk, kGateSeg) : 0;
+    const int64_t convs = pp.rows * (2 * segments(hk, N) + segments(hv, N));
+    const int64_t gates = a.gk != nullptr ? pp.rows * ((hk + kGateSeg - 1) / kGateSeg) : 0;
     const dim3 grid(static_cast<unsigned>(convs + gates));
     const uint32_t nt = static_cast<uint32_t>(ntiles), nc = static_cast<uint32_t>(convs);
     // a sequence of one tile is shared out among its waves (us with 16 tokens a
     // wave -> this: B=52 T=18 H=8 d=128 bf16 32.8 -> 24.1, B=16 T=24 H=16 d=64 fp16
     // conv 2 16.6 -> 12.6; a wave a head took 27.0 and 14.2)
     const int tw = ntiles > 1 ? kPrepTile / kSub : static_cast<int>((a.T + kGroup * kSub - 1) / (kGroup * kSub)) * kGroup;
-    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, CS>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc, tw);
+    hipLaunchKernelGGL((prep_bwd_kernel<XT, K, CS, N>), grid, dim3(64 * kSub), 0, stream, a, pp, nt, nc, tw);
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
     ColSums c{};
     c.rows = pp.rows;
@@ -540,6 +535,11 @@ int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
         c.s[n++] = ColSum{pp.ddt, a.ddt_bias, a.H * a.K, pt};
     }
     return launch_colsum(c, n, stream);
+}
+
+template <typename XT, int K, int CS>
+int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
+    return launch_prep_bwd_n<XT, K, CS, kLaneCh<XT>>(a, stream);
 }
 
 template <typename XT, int K>

@@ -23,6 +23,10 @@
 // eight channels.  Every load of a unit is issued unconditionally before its
 // first use (rows past the data re-read a valid row and are masked), so a
 // wave keeps all of its rows in flight at once instead of waiting on each.
+// The parameters' loads come before the rows': used first in a row's store,
+// which is conditional, a later load of theirs was waited for in every row,
+// and with it the store of the row before (B=4 T=3048 H=16 V=128 bf16, output:
+// 26.4 -> 24.0 us; B=48 T=184 20.2 -> 18.9).
 #include <type_traits>
 
 #include "kda_common.h"
@@ -34,23 +38,28 @@ namespace {
 
 constexpr int kTile = 16;      // tokens per prep unit at most; an in-place conv cache needs T <= this
 constexpr int kMaxConv = 4;    // largest conv_size
-// ---- prep: kSeg channels of q, k or v over a token tile ---------------------
+// ---- prep: 64 N channels of q, k or v over a token tile ---------------------
 // DH: the head size whose L2 norm is taken (q and k), 0 for none (v).  CS:
 // conv_size, so that the taps of a lane's channels are a few wide loads: with a
 // runtime size each was a load and a wait of its own (us, bf16 unless said: a
 // decode step at B=33 H=16 K=V=128 conv_size 2 6.0 -> 3.0, two channels a lane
 // took 3.7; B=4 T=125 H=16 fp16 conv_size 3 with the gates 12.1 -> 7.6, 9.6).
-template <typename XT, int DH, int TILE, int CS>
+template <typename XT, int DH, int TILE, int CS, int N>
 __device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t b, int64_t t0, int64_t seg, int lane) {
-    constexpr int cs = CS, cm = cs - 1, kRows = TILE + cm, N = kLaneCh<XT>;
+    constexpr int cs = CS, cm = cs - 1, kRows = TILE + cm;
     const int64_t D = a.H * (DH ? DH : a.V);
-    const bool valid = seg * kSeg<XT> + N * lane < D;
-    const int64_t ch0 = valid ? seg * kSeg<XT> + N * lane : 0;
+    const bool valid = seg * (64 * N) + N * lane < D;
+    const int64_t ch0 = valid ? seg * (64 * N) + N * lane : 0;
     const int64_t T = a.T;
     const int n = static_cast<int>((T - t0) < TILE ? (T - t0) : TILE);
     const XT* x = static_cast<const XT*>(a.x[i]) + b * a.x_stride[i][0];
     const XT* hist = static_cast<const XT*>(a.hist_in[i]);
     const XT* hrow = hist != nullptr ? hist + b * cm * D : x;
+
+    // the parameters first: what waits for a row has them then
+    const RawParams<N * cs> rw = ld_params<N * cs>(a.conv_w[i], ch0 * cs, a.w_dtype);
+    RawParams<N> rb{};
+    if (a.conv_b[i] != nullptr) rb = ld_params<N>(a.conv_b[i], ch0, a.w_dtype);
 
     // window row r holds token t0 - cm + r: a token of this call, a cached
     // input (t < 0) or zero.  Every row is loaded unconditionally (rows with
@@ -70,10 +79,8 @@ __device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t
         }
     }
     float w[cs][N], wc[N * cs], bias[N];
-#pragma unroll
-    for (int c = 0; c < N; ++c) bias[c] = 0.f;
-    if (a.conv_b[i] != nullptr) params<N>(a.conv_b[i], ch0, a.w_dtype, bias);
-    params<N * cs>(a.conv_w[i], ch0 * cs, a.w_dtype, wc);
+    decode(rw, a.w_dtype, wc);
+    decode(rb, a.w_dtype, bias);
 #pragma unroll
     for (int c = 0; c < N; ++c)
 #pragma unroll
@@ -89,18 +96,16 @@ __device__ __forceinline__ void conv_unit(const kda_prep_args& a, int i, int64_t
     for (int t = 0; t < TILE; ++t) {
         unpack(win[t + cm], xs[(t + cm) % cs]);
         float s[N];
-        float ss = 0.f;
 #pragma unroll
         for (int c = 0; c < N; ++c) {
             float u = bias[c];
 #pragma unroll
             for (int j = 0; j < cs; ++j) u = fmaf(w[j][c], xs[(t + j) % cs][c], u);
             s[c] = u * sigmoid_f(u);
-            ss = fmaf(s[c], s[c], ss);
         }
         if constexpr (DH != 0) {
             // l2 norm over the head: x * min(rsqrt(sum x^2), 1/eps)
-            const float rn = fminf(rsqrtf(lanes_sum<DH / N>(ss)), inv_eps);
+            const float rn = fminf(rsqrtf(head_dot<XT, DH>(s, s)), inv_eps);
 #pragma unroll
             for (int c = 0; c < N; ++c) s[c] *= rn;
         }
@@ -135,6 +140,7 @@ __device__ __forceinline__ void gate_unit(const kda_prep_args& a, int64_t b, int
     const int n = static_cast<int>((T - t0) < TILE ? (T - t0) : TILE);
     const XT* gk = static_cast<const XT*>(a.gk) + b * a.gk_stride[0] + ch0;
 
+    const RawParams<4> ra = ld_params<4>(a.a_log, ch0, a.p_dtype), rd = ld_params<4>(a.dt_bias, ch0, a.p_dtype);
     // every load first (rows past the end re-read the last token)
     Raw<XT, 4> z[TILE];
 #pragma unroll
@@ -155,8 +161,8 @@ __device__ __forceinline__ void gate_unit(const kda_prep_args& a, int64_t b, int
                               a.x_dtype);
     }
     float neg_a[4], dtb[4];
-    params<4>(a.a_log, ch0, a.p_dtype, neg_a);
-    params<4>(a.dt_bias, ch0, a.p_dtype, dtb);
+    decode(ra, a.p_dtype, neg_a);
+    decode(rd, a.p_dtype, dtb);
 #pragma unroll
     for (int c = 0; c < 4; ++c) neg_a[c] = -__expf(neg_a[c]);
     float* g = static_cast<float*>(a.g) + (b * T + t0) * D + ch0;
@@ -179,17 +185,16 @@ __device__ __forceinline__ void gate_unit(const kda_prep_args& a, int64_t b, int
 // B=4 T=2048 53.5 -> 44; B=1 T=1000 12.0 -> 8.8; a decode step at B=1 4.1 ->
 // 3.5, at B=64 5.6 -> 4.0.
 //
-// One wave per (batch, tile, kSeg channels of q, k, v and, unless the call
+// One wave per (batch, tile, 64 N channels of q, k, v and, unless the call
 // leaves the gates to the core, of the gate).  The host keeps the number of
 // units below 2^31, so the unit index is split with 32-bit arithmetic.
-template <typename XT, int K, int TILE>
+template <typename XT, int K, int TILE, int N>
 __global__ __launch_bounds__(256) void prep_kernel(const kda_prep_args a, uint32_t ntiles, uint32_t units) {
     const int lane = threadIdx.x & 63;
     const uint32_t unit = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= units) return;
     const uint32_t H = static_cast<uint32_t>(a.H);
-    const uint32_t segk = (H * K + kSeg<XT> - 1) / kSeg<XT>;
-    const uint32_t segv = (H * static_cast<uint32_t>(a.V) + kSeg<XT> - 1) / kSeg<XT>;
+    const uint32_t segk = segments(H * K, N), segv = segments(H * static_cast<uint32_t>(a.V), N);
     const uint32_t per = 2 * segk + segv + (a.g != nullptr ? (H * K + kGateSeg - 1) / kGateSeg : 0);
     uint32_t s = unit % per;
     const uint32_t bt = unit / per;
@@ -197,10 +202,10 @@ __global__ __launch_bounds__(256) void prep_kernel(const kda_prep_args a, uint32
     const auto conv = [&](auto dh, int i, int64_t seg) {
         constexpr int DH = decltype(dh)::value;
         switch (a.conv_size) {
-            case 4: conv_unit<XT, DH, TILE, 4>(a, i, b, t0, seg, lane); break;
-            case 3: conv_unit<XT, DH, TILE, 3>(a, i, b, t0, seg, lane); break;
-            case 2: conv_unit<XT, DH, TILE, 2>(a, i, b, t0, seg, lane); break;
-            default: conv_unit<XT, DH, TILE, 1>(a, i, b, t0, seg, lane);
+            case 4: conv_unit<XT, DH, TILE, 4, N>(a, i, b, t0, seg, lane); break;
+            case 3: conv_unit<XT, DH, TILE, 3, N>(a, i, b, t0, seg, lane); break;
+            case 2: conv_unit<XT, DH, TILE, 2, N>(a, i, b, t0, seg, lane); break;
+            default: conv_unit<XT, DH, TILE, 1, N>(a, i, b, t0, seg, lane);
         }
     };
     if (s < 2 * segk) {
@@ -212,28 +217,28 @@ __global__ __launch_bounds__(256) void prep_kernel(const kda_prep_args a, uint32
     }
 }
 
-// ---- output: one wave per (batch, tile of tokens, kSeg channels) ------------
+// ---- output: one wave per (batch, tile of tokens, 64 N channels) ------------
 // At copy rate from a few thousand tokens on; us at H=16 V=128 fp16, a wave a
 // head -> this: B=4 T=2048 19.9 -> 19.6 (bf16 21.0 -> 19.2), B=1 T=1000 4.8 ->
 // 3.9, a decode step at B=64 2.9 -> 2.5.  Units of 2 tokens where units of 8
 // leave SIMDs without two waves.
 constexpr int kOutRows = 8;      // tokens per unit (1 for a decode step)
 
-template <typename XT, int V, int TILE>
+template <typename XT, int V, int TILE, int N>
 __global__ __launch_bounds__(256) void output_kernel(const kda_output_args a, uint32_t ntiles, uint32_t units) {
-    constexpr int N = kLaneCh<XT>;
     const int lane = threadIdx.x & 63;
     const uint32_t unit = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (unit >= units) return;
     const uint32_t D = static_cast<uint32_t>(a.H) * V;
-    const uint32_t segs = (D + kSeg<XT> - 1) / kSeg<XT>;
-    const uint32_t ch = (unit % segs) * kSeg<XT> + N * lane, bt = unit / segs;
+    const uint32_t segs = segments(D, N);
+    const uint32_t ch = (unit % segs) * (64 * N) + N * lane, bt = unit / segs;
     const bool valid = ch < D;
     const int64_t c0 = valid ? ch : 0, h = c0 / V;
     const int64_t t0 = static_cast<int64_t>(bt % ntiles) * TILE, b = bt / ntiles;
     const int n = static_cast<int>((a.T - t0) < TILE ? (a.T - t0) : TILE);
 
-    // every load first (rows past the end re-read the last token)
+    // every load first, the weights' before the rows' (rows past the end re-read the last token)
+    const RawParams<N> rw = ld_params<N>(a.weight, c0, a.w_dtype);
     const XT* op = static_cast<const XT*>(a.o) + b * a.o_stride[0] + h * a.o_stride[2] + c0 % V;
     const XT* gp = static_cast<const XT*>(a.gate) + b * a.gate_stride[0] + c0;
     Raw<XT, N> o[TILE], gt[TILE];
@@ -244,17 +249,15 @@ __global__ __launch_bounds__(256) void output_kernel(const kda_output_args a, ui
         gt[r] = ldn<N>(gp + t * a.gate_stride[1]);
     }
     float w[N];
-    params<N>(a.weight, c0, a.w_dtype, w);
+    decode(rw, a.w_dtype, w);
 
     XT* yp = static_cast<XT*>(a.y) + (b * a.T + t0) * D + c0;
 #pragma unroll
     for (int r = 0; r < TILE; ++r) {
-        float x[N], g[N], ss = 0.f;
+        float x[N], g[N];
         unpack(o[r], x);
         unpack(gt[r], g);
-#pragma unroll
-        for (int c = 0; c < N; ++c) ss = fmaf(x[c], x[c], ss);
-        const float rstd = rsqrtf(lanes_sum<V / N>(ss) / static_cast<float>(V) + a.eps);
+        const float rstd = rsqrtf(head_dot<XT, V>(x, x) / static_cast<float>(V) + a.eps);
         float y[N];
 #pragma unroll
         for (int c = 0; c < N; ++c) y[c] = round_to<XT>((x[c] * rstd) * w[c]) * sigmoid_f(g[c]);
@@ -287,24 +290,28 @@ bool overlap(const void* a, int64_t na, const void* b, int64_t nb) {
 // 24 us in units of 4 and 28.5 in units of 16); 1 for a decode step.  A conv
 // cache updated in place needs all its tokens in one unit, which then reads
 // the old rows before it writes the new ones: 8 or 16.
-template <typename XT, int K>
-void launch_prep(const kda_prep_args& a, hipStream_t stream) {
-    const int64_t segk = (a.H * K + kSeg<XT> - 1) / kSeg<XT>, segv = (a.H * a.V + kSeg<XT> - 1) / kSeg<XT>;
-    const int64_t per = 2 * segk + segv + (a.g != nullptr ? (a.H * K + kGateSeg - 1) / kGateSeg : 0);
+template <typename XT, int K, int N>
+void launch_prep_n(const kda_prep_args& a, hipStream_t stream) {
+    const int64_t per = 2 * segments(a.H * K, N) + segments(a.H * a.V, N) +
+                        (a.g != nullptr ? (a.H * K + kGateSeg - 1) / kGateSeg : 0);
     auto go = [&](auto tile) {
         constexpr int TILE = decltype(tile)::value;
         const int64_t ntiles = (a.T + TILE - 1) / TILE, units = a.B * ntiles * per;
-        hipLaunchKernelGGL((prep_kernel<XT, K, TILE>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
+        hipLaunchKernelGGL((prep_kernel<XT, K, TILE, N>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
                            stream, a, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units));
     };
+    if (a.T == 1) return go(std::integral_constant<int, 1>{});
     const int64_t kWaves = a.g != nullptr ? 4096 : 1280;
     bool in_place = false;
     for (int i = 0; i < 3; ++i) in_place = in_place || (a.hist_in[i] != nullptr && a.hist_in[i] == a.hist_out[i]);
     const bool few = a.B * ((a.T + kTile - 1) / kTile) * per < kWaves;
-    if (a.T == 1) go(std::integral_constant<int, 1>{});
-    else if (few && (!in_place || a.T <= 4)) go(std::integral_constant<int, 4>{});
+    if (few && (!in_place || a.T <= 4)) go(std::integral_constant<int, 4>{});
     else if (few && a.T <= 8) go(std::integral_constant<int, 8>{});
     else go(std::integral_constant<int, kTile>{});
+}
+template <typename XT, int K>
+void launch_prep(const kda_prep_args& a, hipStream_t stream) {
+    launch_prep_n<XT, K, kLaneCh<XT>>(a, stream);
 }
 
 template <typename XT>
@@ -318,18 +325,22 @@ int launch_prep_dims(const kda_prep_args& a, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
 }
 
-template <typename XT, int V>
-void launch_output(const kda_output_args& a, hipStream_t stream) {
-    const int64_t segs = (a.H * V + kSeg<XT> - 1) / kSeg<XT>;
+template <typename XT, int V, int N>
+void launch_output_n(const kda_output_args& a, hipStream_t stream) {
+    const int64_t segs = segments(a.H * V, N);
     auto go = [&](auto tile) {
         constexpr int TILE = decltype(tile)::value;
         const int64_t ntiles = (a.T + TILE - 1) / TILE, units = a.B * ntiles * segs;
-        hipLaunchKernelGGL((output_kernel<XT, V, TILE>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
+        hipLaunchKernelGGL((output_kernel<XT, V, TILE, N>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
                            stream, a, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units));
     };
     if (a.T == 1) go(std::integral_constant<int, 1>{});
     else if (a.B * ((a.T + kOutRows - 1) / kOutRows) * segs < 2048) go(std::integral_constant<int, 2>{});
     else go(std::integral_constant<int, kOutRows>{});
+}
+template <typename XT, int V>
+void launch_output(const kda_output_args& a, hipStream_t stream) {
+    launch_output_n<XT, V, kLaneCh<XT>>(a, stream);
 }
 
 template <typename XT>

@@ -6,9 +6,10 @@
 
 namespace kda {
 
-// channels per lane of q, k and v (16 bytes) and per wave
+// channels per lane of q, k and v: 16 bytes
 template <typename XT> constexpr int kLaneCh = 16 / static_cast<int>(sizeof(XT));
-template <typename XT> constexpr int kSeg = 64 * kLaneCh<XT>;
+// Runs of 64 n channels, a wave's, in rows of D.
+__host__ __device__ constexpr int64_t segments(int64_t D, int n) { return (D + 64 * n - 1) / (64 * n); }
 constexpr int kGateSeg = 256;  // channels per wave of the gate, 4 a lane
 
 template <typename XT> __device__ __forceinline__ float to_f(XT x);
@@ -18,7 +19,12 @@ template <> __device__ __forceinline__ float to_f<bf16_t>(bf16_t x) { return bf1
 
 template <typename XT> __device__ __forceinline__ XT from_f(float x);
 template <> __device__ __forceinline__ float from_f<float>(float x) { return x; }
-template <> __device__ __forceinline__ _Float16 from_f<_Float16>(float x) { return static_cast<_Float16>(x); }
+template <> __device__ __forceinline__ _Float16 from_f<_Float16>(float x) {
+    // x as the 32-bit value it is: v_fma_mixlo_f16, which the compiler takes in
+    // some kernels and not in others, would round a product before it to 16 bits at once
+    asm("" : "+v"(x));
+    return static_cast<_Float16>(x);
+}
 template <> __device__ __forceinline__ bf16_t from_f<bf16_t>(float x) { return bf16_t{f32_to_bf16_bits(x)}; }
 
 // Round to XT and back: the value an XT tensor would hold.
@@ -62,22 +68,42 @@ __device__ __forceinline__ void stn(XT* p, const float (&x)[N]) {
     __builtin_memcpy(p, v, sizeof(v));
 }
 
-// N consecutive parameters of a runtime dtype from element i on, as fp32.
+// N consecutive parameters of a runtime dtype from element i on: as loaded, and
+// as fp32.  Apart, so that the wait for them comes where they are used: a
+// conversion beside the load would wait for it before the loads after it.
 template <int N>
-__device__ __forceinline__ void params(const void* p, int64_t i, int dtype, float (&x)[N]) {
+struct RawParams {
     uint32_t w[N];
+};
+template <int N>
+__device__ __forceinline__ RawParams<N> ld_params(const void* p, int64_t i, int dtype) {
+    RawParams<N> r;
+    if (dtype == KDA_DTYPE_F32) __builtin_memcpy(r.w, static_cast<const float*>(p) + i, N * 4);
+    else __builtin_memcpy(r.w, static_cast<const uint16_t*>(p) + i, N * 2);
+    return r;
+}
+template <int N>
+__device__ __forceinline__ void decode(const RawParams<N>& r, int dtype, float (&x)[N]) {
+    const auto half = [&](int c) { return static_cast<uint16_t>(r.w[c / 2] >> (16 * (c % 2))); };
     if (dtype == KDA_DTYPE_F32) {
-        __builtin_memcpy(w, static_cast<const float*>(p) + i, sizeof(w));
 #pragma unroll
-        for (int c = 0; c < N; ++c) x[c] = __uint_as_float(w[c]);
-        return;
-    }
-    __builtin_memcpy(w, static_cast<const uint16_t*>(p) + i, N * 2);
+        for (int c = 0; c < N; ++c) x[c] = __uint_as_float(r.w[c]);
+    } else if (dtype == KDA_DTYPE_F16) {
 #pragma unroll
-    for (int c = 0; c < N; ++c) {
-        const uint16_t u = static_cast<uint16_t>(w[c / 2] >> (16 * (c % 2)));
-        x[c] = dtype == KDA_DTYPE_F16 ? static_cast<float>(__builtin_bit_cast(_Float16, u)) : bf16_bits_to_f32(u);
+        for (int c = 0; c < N; ++c) x[c] = static_cast<float>(__builtin_bit_cast(_Float16, half(c)));
+    } else {
+#pragma unroll
+        for (int c = 0; c < N; ++c) x[c] = bf16_bits_to_f32(half(c));
     }
+}
+
+// sum_c x[c] y[c] over a head of DH channels, N a lane (all-reduce).
+template <typename XT, int DH, int N>
+__device__ __forceinline__ float head_dot(const float (&x)[N], const float (&y)[N]) {
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < N; ++c) s = fmaf(x[c], y[c], s);
+    return lanes_sum<DH / N>(s);
 }
 
 }  // namespace kda
