@@ -539,7 +539,12 @@ int launch_prep_bwd_n(const kda_prep_bwd_args& a, hipStream_t stream) {
 
 template <typename XT, int K, int CS>
 int launch_prep_bwd(const kda_prep_bwd_args& a, hipStream_t stream) {
-    return launch_prep_bwd_n<XT, K, CS, kLaneCh<XT>>(a, stream);
+    // us, eight channels a lane -> four: B=39 T=348 H=2 K=64 V=128 fp16 57.0 -> 43.4,
+    // B=42 T=210 H=1 K=128 V=64 fp16 43.4 -> 34.2 (a wave a head 46.6 and 42.2)
+    if constexpr (kLaneCh<XT> == 8) {
+        if (fills(a.H * K, 8) && fills(a.H * a.V, 8)) return launch_prep_bwd_n<XT, K, CS, 8>(a, stream);
+    }
+    return launch_prep_bwd_n<XT, K, CS, 4>(a, stream);
 }
 
 template <typename XT, int K>

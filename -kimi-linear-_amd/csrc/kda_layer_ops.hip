@@ -20,7 +20,10 @@
 // ones a lane (16 bytes of a 16-bit row), so a wave takes 512 channels of a
 // row: the heads' sums of squares are DPP sums over K / 8 lanes, and the
 // per-row work (addresses, the sum's exchange, the row's rsqrt) is shared by
-// eight channels.  Every load of a unit is issued unconditionally before its
+// eight channels.  A row of at most 256 channels takes four a lane (the output
+// kernel two up to 128), which keeps lanes that would be idle at work, and so
+// does a decode step of the pre-processing, whose time is its chain's; the
+// norms' sums keep their order (head_dot), so the bits are the same.  Every load of a unit is issued unconditionally before its
 // first use (rows past the data re-read a valid row and are masked), so a
 // wave keeps all of its rows in flight at once instead of waiting on each.
 // The parameters' loads come before the rows': used first in a row's store,
@@ -300,7 +303,9 @@ void launch_prep_n(const kda_prep_args& a, hipStream_t stream) {
         hipLaunchKernelGGL((prep_kernel<XT, K, TILE, N>), dim3(static_cast<unsigned>((units + 3) / 4)), dim3(256), 0,
                            stream, a, static_cast<uint32_t>(ntiles), static_cast<uint32_t>(units));
     };
-    if (a.T == 1) return go(std::integral_constant<int, 1>{});
+    if constexpr (N == 4) {
+        if (a.T == 1) return go(std::integral_constant<int, 1>{});
+    }
     const int64_t kWaves = a.g != nullptr ? 4096 : 1280;
     bool in_place = false;
     for (int i = 0; i < 3; ++i) in_place = in_place || (a.hist_in[i] != nullptr && a.hist_in[i] == a.hist_out[i]);
@@ -311,7 +316,12 @@ void launch_prep_n(const kda_prep_args& a, hipStream_t stream) {
 }
 template <typename XT, int K>
 void launch_prep(const kda_prep_args& a, hipStream_t stream) {
-    launch_prep_n<XT, K, kLaneCh<XT>>(a, stream);
+    // us, eight channels a lane -> this: decode step, B=9 H=2 d=64 bf16 3.2 -> 2.8,
+    // B=16 H=32 K=64 V=128 3.7 -> 2.7 (two channels a lane 2.8 and 3.9)
+    if constexpr (kLaneCh<XT> == 8) {
+        if (a.T > 1 && fills(a.H * K, 8) && fills(a.H * a.V, 8)) return launch_prep_n<XT, K, 8>(a, stream);
+    }
+    launch_prep_n<XT, K, 4>(a, stream);
 }
 
 template <typename XT>
@@ -340,7 +350,16 @@ void launch_output_n(const kda_output_args& a, hipStream_t stream) {
 }
 template <typename XT, int V>
 void launch_output(const kda_output_args& a, hipStream_t stream) {
-    launch_output_n<XT, V, kLaneCh<XT>>(a, stream);
+    const int64_t D = a.H * V;
+    // us, eight channels a lane with the weights after the rows -> this (a wave a
+    // head): H=1 V=64, B=5 T=2230 bf16 5.3 -> 3.5 (4.0), B=16 T=338 fp16 4.4 -> 2.7 (3.2)
+    if constexpr (kLaneCh<XT> == 8) {
+        if (a.T == 1 || fills(D, 8)) return launch_output_n<XT, V, 8>(a, stream);
+        if constexpr (V <= 128) {
+            if (D <= 128) return launch_output_n<XT, V, 2>(a, stream);
+        }
+    }
+    launch_output_n<XT, V, 4>(a, stream);
 }
 
 template <typename XT>

@@ -259,3 +259,59 @@ def test_output_units(ops, shape):
     ref = (n * torch.sigmoid(gate.float().view(B, T, H, V))).reshape(B, T, H * V)
     ok, err = close(y, ref, TOL[torch.float16])
     assert ok, err
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,K,V,cs", [(8, 64, 64, 4), (4, 128, 128, 3), (4, 128, 256, 2), (2, 256, 256, 1),
+                                      (12, 64, 128, 4)])
+def test_prep_bits_do_not_depend_on_the_call(ops, dtype, H, K, V, cs):
+    """A token's head gives the same bits in a wide call, alone with its cache and
+    without the other heads: two, four or eight channels a lane, one order of the
+    norm's sum.  Every conv_size."""
+    B, T = 2, 9
+    xs, ws, bs, gk, a_log, dt_bias, beta_logit = make_prep_inputs(B, T, H, K, V, cs, dtype, seed=H + V)
+    dims = (K, K, V)
+
+    def call(t, h0, h1, hist):
+        cut = lambda x, D: x[:, t, h0 * D:h1 * D].contiguous()  # noqa: E731
+        with torch.no_grad():
+            return ops.kda_prep(*(cut(x, D) for x, D in zip(xs, dims)), [w[h0 * D:h1 * D] for w, D in zip(ws, dims)],
+                                [b[h0 * D:h1 * D] for b, D in zip(bs, dims)], cut(gk, K), a_log[h0:h1], dt_bias[h0:h1],
+                                cut(beta_logit, 1), num_heads=h1 - h0, head_dim=K, value_head_dim=V, l2_eps=1e-6,
+                                hist=hist, want_hist=True)
+
+    want = call(slice(None), 0, H, None)
+    for h in range(H):
+        for a, b in zip(want[:5], call(slice(None), h, h + 1, None)[:5]):
+            assert torch.equal(a[:, :, h:h + 1], b)
+    hist = None
+    for t in range(T):
+        one = call(slice(t, t + 1), 0, H, hist)
+        hist = one[5]
+        for a, b in zip(want[:5], one[:5]):
+            assert torch.equal(a[:, t:t + 1], b)
+    for n in "qkv":
+        assert torch.equal(want[5][n], hist[n])
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,V", [(8, 64), (4, 128), (2, 256), (6, 128), (12, 64)])
+def test_output_bits_do_not_depend_on_the_call(ops, dtype, H, V):
+    """As for the pre-processing: all heads, one or two of them, one token."""
+    B, T = 2, 5
+    gen = torch.Generator().manual_seed(H + V)
+    o = torch.randn(B, T, H, V, generator=gen).to(dtype).to(DEV)
+    gate = torch.randn(B, T, H * V, generator=gen).to(dtype).to(DEV)
+    w = (1 + 0.1 * torch.randn(H, V, generator=gen)).to(dtype).to(DEV)
+    with torch.no_grad():
+        y = ops.kda_output(o, gate, w, 1e-6)
+        for n in (1, 2):
+            for h in range(0, H, n):
+                cut = slice(h * V, (h + n) * V)
+                assert torch.equal(y[..., cut], ops.kda_output(o[:, :, h:h + n], gate[..., cut], w[h:h + n], 1e-6))
+        for t in range(T):
+            assert torch.equal(y[:, t:t + 1], ops.kda_output(o[:, t:t + 1], gate[:, t:t + 1], w, 1e-6))
+    n = head_rmsnorm_ref(o.float().cpu(), w.float().cpu(), 1e-6).to(dtype).float()
+    ref = (n * torch.sigmoid(gate.float().cpu().view(B, T, H, V))).reshape(B, T, H * V)
+    ok, err = close(y, ref, TOL[dtype])
+    assert ok, err

@@ -152,3 +152,27 @@ def test_split_gradient_in_place(ops, case):
     want += [torch.full((2, 3, 2), 2.), torch.full((2, 3, 1), 0. if case == "missing" else 3.)]
     assert torch.equal(got, torch.cat(want, -1))
     assert (got.data_ptr() == joined[0].data_ptr()) == (case in ("joined", "missing"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,K,V,cs", [(70, 8, 64, 64, 4), (19, 4, 128, 128, 3), (5, 4, 128, 128, 2), (33, 6, 128, 64, 1)])
+def test_bits_do_not_depend_on_the_other_heads(ops, dtype, T, H, K, V, cs):
+    """A head's gradients are the same bits in a wide call and alone (eight or four channels a lane)."""
+    B = 2
+    inp, up = _prep_inputs(B, T, H, K, V, cs, dtype, seed=T)
+    want = run(ops, inp, up, dtype, H, K, V)
+    dims = (K, K, V)
+    for h in range(H):
+        ch = [slice(h * D, (h + 1) * D) for D in dims]
+        one_in = dict(inp, x=[x[..., c].contiguous() for x, c in zip(inp["x"], ch)], w=[w[c] for w, c in zip(inp["w"], ch)],
+                      b=[b[c] for b, c in zip(inp["b"], ch)], gk=inp["gk"][..., ch[0]].contiguous(),
+                      logit=inp["logit"][..., h:h + 1].contiguous(), a_log=inp["a_log"][h:h + 1],
+                      dt_bias=inp["dt_bias"][h:h + 1])
+        one_up = {n: u[:, :, h:h + 1].contiguous() for n, u in up.items()}
+        got = run(ops, one_in, one_up, dtype, 1, K, V)
+        for i in range(3):
+            assert torch.equal(want[i][..., ch[i]], got[i]), i
+            assert torch.equal(want[3][i][ch[i]], got[3][i]) and torch.equal(want[4][i][ch[i]], got[4][i]), i
+        assert torch.equal(want[5][..., ch[0]], got[5]) and torch.equal(want[6][..., h:h + 1], got[6])
+        assert torch.equal(want[7][h:h + 1], got[7]) and torch.equal(want[8][h:h + 1], got[8])
