@@ -134,17 +134,23 @@ __global__ __launch_bounds__(64 * SPLIT) void linear_kernel(kda_linear_args a) {
     }
 }
 
+// As many waves as leave each at least four steps (8 at K >= 1024, 4 at 512,
+// one at 128), where the steps divide evenly.
+int waves(int64_t K) {
+    const int64_t st = K / 32;
+    return st >= 32 && st % 8 == 0 ? 8 : (st >= 16 && st % 4 == 0 ? 4 : 1);
+}
+
 template <typename T, int MT, int NT>
 int launch(const kda_linear_args& a, hipStream_t stream) {
     const int mats = a.x[1] ? 2 : 1;
     const int64_t n = mats == 2 && a.N[1] > a.N[0] ? a.N[1] : a.N[0];
     const dim3 grid(static_cast<unsigned>((n + 16 * NT - 1) / (16 * NT)), static_cast<unsigned>(mats));
-    // as many waves as leave each at least four steps (8 at K >= 1024, 4 at
-    // 512, one at 128), where the steps divide evenly
-    const int64_t st = a.K / 32;
-    if (st >= 32 && st % 8 == 0) linear_kernel<T, MT, NT, 8><<<grid, 512, 0, stream>>>(a);
-    else if (st >= 16 && st % 4 == 0) linear_kernel<T, MT, NT, 4><<<grid, 256, 0, stream>>>(a);
-    else linear_kernel<T, MT, NT, 1><<<grid, 64, 0, stream>>>(a);
+    switch (waves(a.K)) {
+        case 8: linear_kernel<T, MT, NT, 8><<<grid, 512, 0, stream>>>(a); break;
+        case 4: linear_kernel<T, MT, NT, 4><<<grid, 256, 0, stream>>>(a); break;
+        default: linear_kernel<T, MT, NT, 1><<<grid, 64, 0, stream>>>(a);
+    }
     return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
 }
 
@@ -155,13 +161,14 @@ int launch_rows(const kda_linear_args& a, hipStream_t stream) {
     return launch<T, 4, NT>(a, stream);
 }
 
-// 32 rows of W a workgroup halve the reads of x, but only a wide projection
-// still has workgroups for the chip's 256 CUs: at N = 6416, K = 2048, 1 and 16
-// rows 8.0 and 9.9 us -> 6.9 and 8.1; at N = 4096, 256 workgroups of 16 rows
-// against 128 of 32: 5.8 and 6.3 against 6.6 and 8.0.
+// 32 rows of W a workgroup halve the reads of x, where 16 are more workgroups
+// than the chip's 256 CUs.  us, 16 / 32 rows a workgroup, fp16, 1 and 16 rows of
+// x: K = 2048, N = 4096 5.9 / 6.7 and 6.6 / 8.1, N = 4112 7.2 / 6.8 and 9.4 / 8.1,
+// N = 6416 8.1 / 7.0 and 10.1 / 8.3; K = 512, N = 4112 3.0 / 3.1 and 3.7 / 3.6.
+// With one wave a workgroup it is always 16 (K = 2080, N = 6416 9.8 / 14.1).
 template <typename T>
 int launch_type(const kda_linear_args& a, hipStream_t stream) {
-    return a.N[0] >= 6144 ? launch_rows<T, 2>(a, stream) : launch_rows<T, 1>(a, stream);
+    return a.N[0] > 4096 && waves(a.K) > 1 ? launch_rows<T, 2>(a, stream) : launch_rows<T, 1>(a, stream);
 }
 
 // ---- dW = dy^T x over many rows --------------------------------------------
@@ -313,17 +320,19 @@ int launch_wgrad(const kda_linear_wgrad_args& a, hipStream_t stream) {
 
 }  // namespace
 
-// The shapes this kernel is the better one for.  Each workgroup reads all rows
-// of x, which with up to 16 costs less than the 16 or 32 rows of W beside
-// them; with more it still wins where the library's product is bound by its
-// launch.  us a product in a graph of 40, library / here, fp16 (N, K, rows):
-//   6416, 2048:  1: 8.8 / 6.9   16: 8.8 / 8.1   32: 8.8 / 9.8   64: 9.5 / 13.6
-//   2048, 2048:  1: 7.8 / 4.6   16: 8.0 / 6.0   32: 8.2 / 7.8   64: 8.6 / 11.4
-//   3344, 1024:  1: 4.5 / 3.4   16: 4.8 / 4.2   32: 7.8 / 5.1   64: 7.0 / 7.0
-//   1808,  512:  1: 3.6 / 2.4   16: 3.6 / 2.8   32: 4.8 / 3.4   64: 5.5 / 4.4
-//   2048,  128:  1: 3.2 / 1.9   16: 3.5 / 2.1   32: 3.5 / 2.2   64: 3.7 / 2.7
+// Each workgroup reads all rows of x, which with up to 16 costs less than the 16
+// or 32 rows of W beside them; with more it still wins where the library's
+// product is bound by its launch.  us a product in a graph of 24, library / here,
+// fp16 (N, K, rows):
+//   6416, 2048:  1: 8.9 / 7.0   16: 8.9 / 8.3
+//   2048, 2048:  1: 7.8 / 4.7   16: 8.1 / 6.0
+//   4096, 1024:  1: 5.5 / 3.7   16: 5.8 / 4.4   32: 8.1 / 5.4
+//   2048,  512:  1: 3.7 / 2.6   16: 3.8 / 3.0   32: 4.9 / 3.5   64: 5.5 / 4.5
+//   2048,  128:  1: 3.2 / 1.9   16: 3.6 / 2.1   32: 3.5 / 2.3   64: 3.7 / 2.6
 // (two of the last in one launch: 2.0 and 2.8 us at 1 and 64 rows).  At one
-// row the 6416 x 2048 weight goes by at 3.8 TB/s, 5.3 without the launch.
+// row the 6416 x 2048 weight goes by at 3.8 TB/s, 5.3 without the launch.  The
+// layer takes the library's product for the widths and depths where it is the
+// faster one (layer.py, _few_rows).
 bool linear_supported(const kda_linear_args& a) {
     if (a.M > 64 || a.K % 32 != 0) return false;
     return a.M <= 16 || a.K <= (a.M <= 32 ? 1024 : 512);

@@ -176,10 +176,34 @@ def _plain_weight(mod, *inputs):
     return mod.weight
 
 
+def _few_rows(x, n: int) -> bool:
+    """Whether ``kda_linear_fwd`` is the faster product for x [B, T, K] and n
+    outputs, by measurement over K 256 to 4096 and n 512 to 12576 (us, library /
+    kernel, fp16).  More than 8192 outputs are more workgroups than the chip
+    holds: K = 2048, n = 12576 10.7 / 11.8 at one row, 512 4.9 at K = 512 (8.6).
+    Beyond K = 2048 only the reads of W count that fill the chip at once: K =
+    2304, 4 rows, n = 4096 6.7 / 5.8, n = 6416 7.9 / 8.1, n = 512 4.8 / 4.8; 16
+    rows, n = 2048 6.4 / 6.5.  Steps of 32 that do not divide over four waves
+    leave one a workgroup: K = 1568, n = 2048 5.8 / 6.3, n = 4096 8.4 / 6.8."""
+    rows, k = x.shape[0] * x.shape[1], x.shape[2]
+    if rows > 64 or k % 32 != 0:
+        return False
+    one_wave = k % 128 != 0 or k < 512
+    if k > 2048:
+        return rows <= 4 and k <= 4096 and 2048 <= n <= 4096 and not one_wave
+    if n > 8192:
+        return rows <= 32 and k <= 512
+    if k > 1536 and one_wave:
+        return rows <= 16 and n >= 4096
+    return rows <= 16 or k <= (1024 if rows <= 32 else 512)
+
+
 def _project(mod, x, residual=None, out=None):
     """``mod(x)``, plus ``residual``, into ``out``: in the few-row kernel
-    (``kda_linear_fwd``, up to 64 rows) where it applies, else as written."""
+    (``kda_linear_fwd``) where it applies, else as written."""
     w = _plain_weight(mod, x) if x.shape[0] * x.shape[1] <= 64 else None
+    if w is not None and not _few_rows(x, w.shape[0]):
+        w = None
     y = _native.host().linear(x, w, residual, out) if w is not None else None
     if y is not None:
         return y
@@ -352,7 +376,7 @@ class KimiDeltaAttention(nn.Module):
         H, K, V = self.num_heads, self.head_dim, self.value_head_dim
         w, b = self._input_weight()
         few = x.shape[0] * x.shape[1] <= 64 and not has_torch_function((x,))
-        y = _native.host().linear(x, w, None, None) if few and b is None else None
+        y = _native.host().linear(x, w, None, None) if few and b is None and _few_rows(x, w.shape[0]) else None
         if y is None:
             y = torch.nn.functional.linear(x, w, b)
         q_in, k_in, v_in, beta_logit, gk_low, og_low = torch.split(
@@ -360,7 +384,8 @@ class KimiDeltaAttention(nn.Module):
         gk = gate = None
         if few and output_gate:       # both up-projections in one launch
             w_gk, w_og = _plain_weight(self.gk_proj[1]), _plain_weight(self.og_proj[1])
-            if w_gk is not None and w_og is not None:
+            if (w_gk is not None and w_og is not None and _few_rows(gk_low, w_gk.shape[0])
+                    and _few_rows(og_low, w_og.shape[0])):
                 gk, gate = _native.host().linear2(gk_low, w_gk, og_low, w_og) or (None, None)
         if gk is None:
             gk = self.gk_proj[1](gk_low)

@@ -145,3 +145,15 @@ def test_linear_function_gradients(kda_pkg):
         assert bool(((a.double() - b.double()).abs() <= 2.0 ** -10 * b.double().abs() + 800 * 2.0 ** -23 * 60).all())
     mod.register_full_backward_hook(lambda *a: None)
     assert type(layer._project_train(mod, x).grad_fn).__name__ != "_LinearFnBackward"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("K,N", [(512, 4096), (512, 4112), (1024, 4112), (544, 6160), (96, 4128)])
+def test_rows_of_w_per_workgroup(host, M, K, N):
+    """Around 4096 outputs: 16 or 32 rows of W a workgroup, a last one half empty, one wave a workgroup."""
+    x, w = data(M, K, N, torch.float16, seed=N)
+    y = host.linear(x.view(M, 1, K), w, None, None)
+    check(y[:, 0], x, w)
+    part = host.linear(x.view(M, 1, K), w[:2048], None, None)       # 16 rows a workgroup: the same sums
+    assert torch.equal(y[..., :2048], part)

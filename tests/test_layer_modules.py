@@ -80,3 +80,18 @@ def test_a_function_mode_or_subclass_sees_the_projections(kda_pkg):
         assert layer._plain_weight(mod, x) is None
     mod.weight = torch.nn.Parameter(mod.weight.detach().as_subclass(Sub))
     assert layer._plain_weight(mod, x) is None
+
+
+@pytest.mark.parametrize("rows,k,n,own", [
+    (1, 2048, 6416, True), (16, 2048, 2048, True), (17, 2048, 2048, False), (32, 1024, 4096, True), (33, 1024, 4096, False),
+    (64, 512, 2048, True), (65, 128, 2048, False), (64, 128, 2048, True),
+    (1, 2048, 12576, False), (32, 512, 12576, True), (33, 512, 12576, False), (1, 2048, 8192, True),
+    (4, 2304, 4096, True), (5, 2304, 4096, False), (1, 2304, 6416, False), (1, 2304, 512, False), (1, 4096, 2304, True),
+    (1, 4128, 4096, False), (1, 3104, 4096, False), (1, 1568, 2048, False), (16, 1568, 4096, True), (1, 1056, 2048, True), (17, 1056, 4096, False),
+    (1, 544, 2048, True), (1, 48, 2048, False)])
+def test_few_row_projections_where_they_are_faster(kda_pkg, rows, k, n, own):
+    import importlib
+    layer = importlib.import_module("kimi_linear_amd.layer")
+    assert layer._few_rows(torch.empty(rows, 1, k, device="meta"), n) is own
+    if own:       # nothing that the kernel refuses
+        assert k % 32 == 0 and (rows <= 16 or k <= (1024 if rows <= 32 else 512))
