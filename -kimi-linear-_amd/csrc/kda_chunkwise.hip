@@ -324,18 +324,29 @@ __device__ __forceinline__ void load_state(f4 (&S)[KT], const void* p, int dtype
         load_state_t<KT>(S, static_cast<const bf16_t*>(p), off, V);
     }
 }
-template <int KT, typename TS>
+// A bf16 state is rounded in integer operations (INT), but for the gated fp16
+// kernels': the compiler lays out the registers of the whole kernel with this
+// code.  us with the conversion / this, H=16 d=128, B=8 T=4096 and B=4 T=2048:
+// plain fp16 310.6 / 308.9 and 151.1 / 149.6, plain bf16 (outputs in pairs)
+// 323 / 323 and 157 / 158, gated fp16 353.4 / 354.3 and 177 / 180, gated bf16
+// (B=4 T=4096 H=8 d=64) 253 / 249.
+template <typename TS, bool INT>
+__device__ __forceinline__ void store_state_elem(TS* p, float x) {
+    if constexpr (INT && Elem<TS>::code == KDA_DTYPE_BF16) p->bits = f32_to_bf16_bits_int(x);
+    else Elem<TS>::st(p, x);
+}
+template <int KT, bool INT, typename TS>
 __device__ __forceinline__ void store_state_t(const f4 (&S)[KT], TS* p, int64_t off, int64_t V) {
 #pragma unroll
     for (int t = 0; t < KT; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) Elem<TS>::st(p + off + (16 * t + j) * V, S[t][j]);
+        for (int j = 0; j < 4; ++j) store_state_elem<TS, INT>(p + off + (16 * t + j) * V, S[t][j]);
 }
-template <int KT>
+template <int KT, bool INT>
 __device__ __forceinline__ void store_state(const f4 (&S)[KT], void* p, int dtype, int64_t off, int64_t V) {
-    if (dtype == KDA_DTYPE_F32) store_state_t<KT>(S, static_cast<float*>(p), off, V);
-    else if (dtype == KDA_DTYPE_F16) store_state_t<KT>(S, static_cast<_Float16*>(p), off, V);
-    else store_state_t<KT>(S, static_cast<bf16_t*>(p), off, V);
+    if (dtype == KDA_DTYPE_F32) store_state_t<KT, INT>(S, static_cast<float*>(p), off, V);
+    else if (dtype == KDA_DTYPE_F16) store_state_t<KT, INT>(S, static_cast<_Float16*>(p), off, V);
+    else store_state_t<KT, INT>(S, static_cast<bf16_t*>(p), off, V);
 }
 
 // Level whose product supplies entry (row c, column i) of a diagonal block:
@@ -1060,8 +1071,8 @@ struct Kern {
             __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, to_h4(O)), r, vo, 0, 0);
         } else {
             u2 w;
-            w[0] = static_cast<uint32_t>(f32_to_bf16_bits(O[0])) | (static_cast<uint32_t>(f32_to_bf16_bits(O[1])) << 16);
-            w[1] = static_cast<uint32_t>(f32_to_bf16_bits(O[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(O[3])) << 16);
+            w[0] = bf16_pair(O[0], O[1]);
+            w[1] = bf16_pair(O[2], O[3]);
             __builtin_amdgcn_raw_buffer_store_b64(w, r, vo, 0, 0);
         }
     }
@@ -1072,8 +1083,8 @@ struct Kern {
             return __builtin_bit_cast(u2, to_h4(O));
         } else {
             u2 w;
-            w[0] = static_cast<uint32_t>(f32_to_bf16_bits(O[0])) | (static_cast<uint32_t>(f32_to_bf16_bits(O[1])) << 16);
-            w[1] = static_cast<uint32_t>(f32_to_bf16_bits(O[2])) | (static_cast<uint32_t>(f32_to_bf16_bits(O[3])) << 16);
+            w[0] = bf16_pair(O[0], O[1]);
+            w[1] = bf16_pair(O[2], O[3]);
             return w;
         }
     }
@@ -1091,8 +1102,10 @@ struct Kern {
         const auto s1 = __builtin_amdgcn_permlane16_swap(px[1], py[1], false, false);
         __builtin_amdgcn_raw_buffer_store_b128(u4{s0[0], s1[0], s0[1], s1[1]}, r, vo, 0, 0);
     }
-    // on = false: stores of an empty range
-    __device__ void store_chunk(const f4 (&O)[CG][CB], int blk, int64_t colw, bool on = true) const {
+    // on = false: stores of an empty range (a constant where the range is always
+    // the rows': its own code order, as without the argument)
+    template <typename On = std::true_type>
+    __device__ void store_chunk(const f4 (&O)[CG][CB], int blk, int64_t colw, On on = {}) const {
         static_assert(CG == 1 || CG == 2, "output tiles of one or two column groups");
         if constexpr (sizeof(TQ) == 4) {
 #pragma unroll
@@ -1653,6 +1666,7 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
         }
         // a null state_out (the output pass of a split long sequence) keeps no final state
         if (a.state_out != nullptr) {
+            constexpr bool kIntState = !(GATED && Elem<TQ>::code == KDA_DTYPE_F16);
             if constexpr (KN::RANGE) {
 #pragma unroll
                 for (int g = 0; g < CG; ++g)
@@ -1661,7 +1675,7 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
             }
 #pragma unroll
             for (int g = 0; g < CG; ++g)
-                store_state<KT>(S[g], a.state_out, a.state_out_dtype, sbase + (4 * kn.lg) * VS + colw + 16 * g + kn.ln,
+                store_state<KT, kIntState>(S[g], a.state_out, a.state_out_dtype, sbase + (4 * kn.lg) * VS + colw + 16 * g + kn.ln,
                                 VS);
         }
     } else {

@@ -21,13 +21,26 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint16_t b) {
 }
 
 // Round-to-nearest-even fp32 -> bf16 bits (NaN stays a quiet NaN): gfx950's
-// v_cvt_pk_bf16_f32, which converts two values at once where the compiler
-// finds two.  The integer form took five operations a value (kernel trace,
-// bf16, H=16 d=128, integer -> this: fused chunkwise kernel at B=16 T=2048
-// 404 -> 321 us, pre-processing 244 -> 210; its backward at B=4 T=2048 201 ->
-// 160, output 24.4 -> 22.1).
+// v_cvt_pk_bf16_f32.  The integer form took five operations a value (kernel
+// trace, bf16, H=16 d=128, integer -> this: fused chunkwise kernel at B=16
+// T=2048 404 -> 321 us, pre-processing 244 -> 210; its backward at B=4 T=2048
+// 201 -> 160, output 24.4 -> 22.1).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
     return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
+}
+// The same of two values, lo in the low half, in one instruction: the compiler
+// makes two conversions, a shift and an or of two f32_to_bf16_bits.
+__device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{lo, hi}, b2));
+}
+// The same in integer operations.
+__device__ __forceinline__ uint16_t f32_to_bf16_bits_int(float f) {
+    uint32_t u = __float_as_uint(f);
+    if ((u & 0x7f800000u) == 0x7f800000u && (u & 0x007fffffu)) return static_cast<uint16_t>((u >> 16) | 0x40u);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return static_cast<uint16_t>(u >> 16);
 }
 
 __device__ __forceinline__ float load_elem(const void* p, int64_t i, int dtype) {
