@@ -177,11 +177,12 @@ bool overlaps(const Tensor& a, const Tensor& b) {
 
 // kda_chunkwise / kda_recurrent (recurrent), with the gates' parameters their
 // gated forms, with og also kda_chunkwise_fused.  segments > 1: the split of a
-// long sequence the wrapper's rule asks for.  (o, state) or None.
+// long sequence the wrapper's rule asks for; transitions_first: in
+// kda_chunkwise_split_fwd where that has a form.  (o, state) or None.
 py::object core(bool recurrent, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& beta,
                 const OptTensor& state, int64_t chunk_size, const std::optional<at::ScalarType>& state_dtype,
                 const OptTensor& state_out, const OptTensor& a_log, const OptTensor& dt_bias, const OptTensor& og,
-                const OptTensor& weight, double eps, int64_t segments) {
+                const OptTensor& weight, double eps, int64_t segments, bool transitions_first) {
     Plain plain(q);
     plain.add(k).add(v).add(g).add(beta).add(state).add(state_out).add(a_log).add(dt_bias).add(og);
     if (!plain.ok || (weight && !weight->defined())) return py::none();
@@ -258,7 +259,7 @@ py::object core(bool recurrent, const Tensor& q, const Tensor& k, const Tensor& 
         }
         if (segments > 1) {
             // the form whose transition columns end when they are zero, where there is one
-            const size_t split = fn.split_ws(B, T, H, K, V, segments);
+            const size_t split = transitions_first ? fn.split_ws(B, T, H, K, V, segments) : 0;
             const size_t bytes = split != 0 ? split : fn.long_ws(B, T, H, K, V, segments);
             keep = at::empty({static_cast<int64_t>(bytes)}, v.options().dtype(at::kByte).requires_grad(false));
             return (split != 0 ? fn.split_fwd : fn.long_fwd)(&a, segments, keep.data_ptr(), stream);
@@ -544,7 +545,10 @@ PYBIND11_MODULE(_kda_host, m) {
     m.def("abi_version", [] { return KDA_ABI_VERSION; });
     m.attr("torch_version") = KDA_TORCH_VERSION;    // it was compiled against; its C++ interface is not stable
     m.def("bind", &bind);
-    m.def("core", &core);
+    m.def("core", &core, py::arg("recurrent"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("beta"),
+          py::arg("state"), py::arg("chunk_size"), py::arg("state_dtype"), py::arg("state_out"), py::arg("a_log"),
+          py::arg("dt_bias"), py::arg("og"), py::arg("weight"), py::arg("eps"), py::arg("segments"),
+          py::arg("transitions_first") = true);
     m.def("prep", &prep);
     m.def("output", &output);
     m.def("linear", &linear);

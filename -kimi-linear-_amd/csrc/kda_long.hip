@@ -32,10 +32,12 @@
 // (unless S_start holds an infinity or a NaN, whose product with zero is NaN:
 // then it takes those tokens too, with c = 0).  Each of the two launches has
 // the chip to itself, so a segment is half as long.  B=1 T=32768 H=16 K=V=128
-// fp16: 8 segments in one launch 537 us, 16 in two 316 (trans 34, V columns
-// 215, combine 48, correction 37: the kernels alone).  With decays 1000 times
-// weaker, where nothing is forgotten, it costs about a tenth more than the one
-// launch (632 -> 700 us on a GPU not yet at its settled clock).
+// fp16: 8 segments in one launch 537 us, 16 in two 316; in a kernel trace, with
+// its gaps, trans 34, V columns 215, combine 48, correction 37.  Where nothing is
+// forgotten (decays 1000 times weaker) it costs a combine of twice the length
+// and a launch: 224 + 242 + 49 + 140 us where the one launch takes 435 + 24 +
+// 141.  The combine's 3 us a segment did not move with its next segment's loads
+// requested ahead of the products, nor with the strip read at once.
 #include "kda_common.h"
 #include "kda_launch.h"
 
@@ -390,7 +392,8 @@ int64_t long_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t
 
 // Segments of the split form: twice P (or the power of two times P) while the
 // V columns fit one round of workgroups and a segment keeps kSplitSegment
-// tokens; none (0) where P cannot be doubled: its one launch holds both kinds
+// tokens (us in one launch / split at H=16 d=128: T=8192, segments of 512, 168 /
+// 166, T=4096, 256, 97 / 126; T=16384, 1024, 288 / 217); none (0) where P cannot be doubled: its one launch holds both kinds
 // of columns side by side.
 static int64_t split_segments(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P) {
     constexpr int64_t kSplitSegment = 1024;

@@ -101,7 +101,7 @@ def _common(kind, q, k, v, g, beta, state, chunk_size, state_dtype, state_out=No
         segments = long_segments(*q.shape, v.shape[-1], v.dtype)
     try:
         return _native.host().core(kind == "recurrent", q, k, v, g, beta, state, chunk_size, state_dtype, state_out,
-                                   *gate, *epilogue, segments)
+                                   *gate, *epilogue, segments, segments > 1 and _transitions_first(q.shape[1], segments))
     except TypeError:       # an argument of no type a common call has
         return None
 
@@ -255,7 +255,9 @@ def _forward(kind, q, k, v, g, beta, state, chunk_size, state_dtype, state_out=N
                 segments = long_segments(B, T, H, K, V, qk_dtype)
         if segments > 1:
             # the form whose transition columns end when they are zero, where there is one
-            size, fwd = int(lib.kda_chunkwise_split_workspace_size(B, T, H, K, V, segments)), lib.kda_chunkwise_split_fwd
+            size, fwd = 0, lib.kda_chunkwise_split_fwd
+            if _transitions_first(T, segments):
+                size = int(lib.kda_chunkwise_split_workspace_size(B, T, H, K, V, segments))
             if size == 0:
                 size, fwd = int(lib.kda_chunkwise_long_workspace_size(B, T, H, K, V, segments)), \
                     lib.kda_chunkwise_long_fwd
@@ -301,6 +303,20 @@ def ckpt_record(K: int, V: int) -> int:
 LONG_MIN_SEGMENT = 1024    # shortest segment worth the three-pass split (kda_chunkwise_long_fwd)
 FEW_CHAIN_MIN_SEGMENT = 256   # shortest segment of the few-chain form
 CU_COUNT = 256
+SPLIT_MIN_SEGMENT = 2048   # shortest segment of kda_chunkwise_split_fwd
+
+
+def _transitions_first(T, segments) -> bool:
+    """Whether a sequence split into ``segments`` runs as kda_chunkwise_split_fwd
+    where that has a form, in at least twice as many.  It gains where a segment
+    forgets its initial state exactly and costs a combine of twice the length and
+    a launch (about 55 us) where it does not, which only the kernels know; so it is
+    for segments long enough that the cost is small.  us in one launch / split, fp16
+    d=128, decays of the training distribution and 1000 times weaker: H=16 T=32768,
+    segments of 2048, 534 / 317 and 559 / 629; T=16384, 1024, 288 / 217 and 295 /
+    350; H=8 T=32768, 1024, 308 / 269 and 313 / 391; H=16 T=8192, 512, 168 / 166
+    and 170 / 226."""
+    return T // (2 * segments) >= SPLIT_MIN_SEGMENT
 
 
 def long_segments(B, T, H, K, V, dtype) -> int:

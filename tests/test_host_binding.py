@@ -279,3 +279,30 @@ def test_an_output_among_the_rows_of_an_input_is_the_general_paths(stand_in):
         x = torch.rand(4, 1, 64).half()
         assert mod.linear(x, w, rows, buf[4:8]) is None and mod.linear(x, w, rows, None) is not None
         assert mod.linear(x, w[:16], None, x.view(-1)[64:128].view(4, 1, 16)) is None
+
+
+@pytest.mark.parametrize("T,segments,first", [(32768, 8, True), (16384, 8, False), (32768, 16, False), (32704, 8, False),
+                                              (65536, 8, True)])
+def test_the_split_form_is_for_long_segments(stand_in, kda, monkeypatch, T, segments, first):
+    """Transition columns before V columns only in segments of at least 2048
+    tokens, from the native side and from the general path."""
+    assert kda._transitions_first(T, segments) is first
+    seen = []
+
+    class Host:
+        @staticmethod
+        def core(*a):
+            seen.append(a[-2:])
+    q = torch.empty(1, T, 2, 128, device="meta")
+    monkeypatch.setattr(kda._native, "host", lambda: Host)
+    monkeypatch.setattr(kda, "long_segments", lambda *a: segments)
+    kda._common("chunkwise", q, q, q, q, q[..., 0], None, 64, None, split=True)
+    assert seen == [(segments, first)]
+    calls = []
+    entry = {n: (lambda *a, n=n: calls.append(n) or 0) for n in ("kda_chunkwise_split_fwd", "kda_chunkwise_long_fwd")}
+    mod = stand_in(**entry, kda_chunkwise_split_workspace_size=lambda *a: 256)
+    args, _ = inputs(torch.float16, device="cpu")
+    one = [x[:1].repeat(1, 4, *[1] * (x.dim() - 2)) for x in args]
+    with torch.no_grad():
+        assert mod.core(False, *one, None, 64, None, None, None, None, None, None, 0.0, 2, first) is not None
+    assert calls == ["kda_chunkwise_split_fwd" if first else "kda_chunkwise_long_fwd"]
