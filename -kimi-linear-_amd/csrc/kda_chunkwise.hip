@@ -1137,8 +1137,9 @@ struct Kern {
     }
 
     // TOUT: a chunk's outputs in fp32, the V columns' to oz ([B, T, H, V]),
-    // the transition columns' to c ([B, T, H, K]); the choice is uniform over
-    // the workgroup and taken by selecting the base, not by a branch.
+    // the transition columns' to c ([B, T, H, K]); the choice is wave-uniform
+    // (kToutTrans, kToutV: the workgroup's) and taken by selecting the base, not
+    // by a branch.
     __device__ void store_fp32_chunk(const f4 (&O)[CG][CB], int blk, int64_t colw) const {
         const bool tr = vzero, on = TOUT != kToutV || blk < nz;
         float* base = tr ? lo.c : lo.oz;
@@ -1452,6 +1453,7 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
                                                                    const kda_gate_args gate,
                                                                    const kda_out_epilogue epi, const long_out lout) {
     static_assert(TOUT == 0 || TRANS, "fp32 outputs belong to the transition pass");
+    static_assert(TOUT < kToutTrans || 16 * NC * CG == K, "a head's transition columns are one workgroup's");
     using KN = Kern<K, NC, TQ, GATED, CG, EPI, TRANS, TOUT, CKPT>;
     constexpr int KT = KN::KT, VT = KN::VT, CH = KN::CH;
     static_assert(K % 32 == 0 && K <= 128, "chunkwise supports K in {32, 64, 128}");
@@ -1475,7 +1477,7 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
     // the tiles of a head in this launch, and the first of them
     const int nvt = static_cast<int>((TOUT == kToutTrans ? K : (TOUT == kToutV ? V : VS)) / VT);
     const int first = TOUT == kToutTrans ? static_cast<int>(V / VT) : 0;
-    const int tile = bid % nvt, vt = first + tile;
+    const int vt = first + bid % nvt;
     bid /= nvt;
     kn.h = bid % H;
     kn.b = bid / H;
@@ -1499,13 +1501,7 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
     if constexpr (TOUT != 0) kn.lo = lout;
     const int nss = (ncc + NCH - 1) / NCH;               // supersteps
     if constexpr (TOUT == kToutV) {
-        int n = 0;
-        const int nt = K / static_cast<int>(trans_tile(K, V));
-        for (int i = 0; i < nt; ++i) {
-            const int x = lout.n[(kn.b * H + kn.h) * nt + i];
-            n = x > n ? x : n;
-        }
-        kn.nz = __builtin_amdgcn_readfirstlane(CB * n);
+        kn.nz = __builtin_amdgcn_readfirstlane(CB * lout.n[kn.b * H + kn.h]);
     }
 
     const bool consumer = wave < NC;
@@ -1662,7 +1658,7 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
         }
         if constexpr (TOUT == kToutTrans) {
             if (threadIdx.x == 0)
-                lout.n[(kn.b * H + kn.h) * (K / VT) + tile] = NCH * done < ncc ? NCH * done : ncc;
+                lout.n[kn.b * H + kn.h] = NCH * done < ncc ? NCH * done : ncc;
         }
         // a null state_out (the output pass of a split long sequence) keeps no final state
         if (a.state_out != nullptr) {
@@ -1720,8 +1716,8 @@ int launch_knq(const kda_fwd_args& a, hipStream_t stream, float* ckpt, const kda
 
 // The first pass of a split long sequence: 64-column tiles over the V state
 // columns and the K transition columns (128-column tiles when they would
-// outnumber the CUs).  With outputs in two launches (lout->part), tiles of
-// trans_tile() columns over one kind.
+// outnumber the CUs).  With outputs in two launches (lout->part), tiles of K
+// columns over one kind.
 template <int K, typename TQ>
 int launch_trans(const kda_fwd_args& a, hipStream_t stream, const long_out* lout) {
     const kda_gate_args none{nullptr, nullptr};
@@ -1734,14 +1730,9 @@ int launch_trans(const kda_fwd_args& a, hipStream_t stream, const long_out* lout
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
     if (lout != nullptr && lout->part != long_out::kBoth) {
-        const bool trans = lout->part == long_out::kTrans;
-        if constexpr (K == 128) {
-            if (trans_tile(K, a.V) == 128)
-                return trans ? go(I2{}, std::integral_constant<int, kToutTrans>{})
-                             : go(I2{}, std::integral_constant<int, kToutV>{});
-        }
-        return trans ? go(I1{}, std::integral_constant<int, kToutTrans>{})
-                     : go(I1{}, std::integral_constant<int, kToutV>{});
+        using Cols = std::integral_constant<int, K / 64>;
+        return lout->part == long_out::kTrans ? go(Cols{}, std::integral_constant<int, kToutTrans>{})
+                                              : go(Cols{}, std::integral_constant<int, kToutV>{});
     }
     const bool wide = a.B * a.H * ((a.V + K) / 64) > 256 && (a.V + K) % 128 == 0;
     if (lout != nullptr) {

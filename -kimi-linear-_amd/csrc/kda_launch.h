@@ -34,10 +34,10 @@ int chunkwise_launch(const kda_fwd_args& a, hipStream_t stream, float* ckpt = nu
 // the state from zero and the transition, state_out [B, H, K, V + K] fp32;
 // with lout, also the outputs in fp32: oz [B, T, H, V] from the zero state and
 // c [B, T, H, K] those of the transition columns (the coefficients of the
-// initial state).  In two launches (kTrans, kV) the transition columns' 64- or
-// 128-column tiles write only the n[(b, h), tile] 32-token chunks in which
-// they may not be zero, and the V columns' outputs after those chunks go to o
-// [B, T, H, V] instead of oz.
+// initial state).  In two launches (kTrans, kV; V a multiple of K), of K columns
+// a workgroup, the transition columns write only the n[(b, h)] 32-token chunks
+// in which they may not be zero, and the V columns' outputs after those chunks
+// go to o [B, T, H, V] instead of oz.
 struct long_out {
     float* oz;
     float* c;
@@ -45,8 +45,6 @@ struct long_out {
     int part;
     static constexpr int kBoth = 0, kTrans = 1, kV = 2;
 };
-// columns of a transition tile with lout
-__host__ __device__ constexpr int64_t trans_tile(int64_t K, int64_t V) { return K == 128 && V % 128 == 0 ? 128 : 64; }
 bool chunkwise_trans_supported(const kda_fwd_args& a);
 int chunkwise_trans_launch(const kda_fwd_args& a, hipStream_t stream, const long_out* lout = nullptr);
 // The chunkwise forward with the layer's output epilogue (kda_chunkwise_fused_fwd).

@@ -167,10 +167,10 @@ constexpr int kCorrectTokens = 256;   // tokens per correction workgroup
 // segment that starts from zero (no initial state) takes oz as it is.  Rows
 // past the segment's end are outside the descriptors' ranges (read as zero,
 // stores dropped).  oz, cf: [B T, H, V] and [B T, H, K] fp32; sstart:
-// [B P, H, K, V] fp32; o: [B T, H, V] in the output dtype.  nch: [B P, H, K /
-// tile], the 32-token chunks of the segment whose coefficients of a tile of
-// channels were written (zero after them, and the outputs in o instead of
-// oz), or null: all; nonfinite: of the combine.
+// [B P, H, K, V] fp32; o: [B T, H, V] in the output dtype.  nch: [B P, H], the
+// 32-token chunks of the segment whose coefficients were written (zero after
+// them, and the outputs in o instead of oz), or null: all; nonfinite: of the
+// combine.
 template <int K>
 struct CorrectSmem {
     uint16_t hi[2][16][K + 8];
@@ -179,7 +179,7 @@ struct CorrectSmem {
 template <int K, typename TO>
 __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, const float* cf, const float* sstart,
                                                             TO* o, int64_t T, int64_t H, int64_t V, int64_t P,
-                                                            int zero_first, const int* nch, int tile,
+                                                            int zero_first, const int* nch,
                                                             const uint32_t* nonfinite) {
     __shared__ CorrectSmem<K> sm;
     const int t = threadIdx.x, lane = t & 63, ln = lane & 15, lg = lane >> 4;
@@ -196,24 +196,18 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
     const int64_t c0 = 16 * w;
     const int64_t t0 = tb * kCorrectTokens;
     const int64_t row0 = bp * Ts + t0;              // flat token index b T + p Ts + t0
-    // rows of this workgroup's tokens with coefficients, per channel tile
-    // (one or two); and whether S_start is not finite (a word a strip)
+    // rows of this workgroup's tokens with coefficients, whose V outputs are in
+    // oz; and whether S_start is not finite (a word a strip)
     const int64_t left = Ts - t0 < kCorrectTokens ? Ts - t0 : kCorrectTokens;
-    int n0 = static_cast<int>(left), n1 = n0;
+    int rows = static_cast<int>(left);
     uint32_t odd = 0;
     if (nch != nullptr) {
-        const int* nc = nch + (bp * H + h) * (K / tile);
-        auto with_c = [&](int i) {
-            const int64_t r = 32 * static_cast<int64_t>(nc[i]) - t0;
-            return static_cast<int>(r < 0 ? 0 : (r < left ? r : left));
-        };
-        n0 = with_c(0);
-        n1 = K / tile > 1 ? with_c(1) : n0;
+        const int64_t r = 32 * static_cast<int64_t>(nch[bp * H + h]) - t0;
+        rows = static_cast<int>(r < 0 ? 0 : (r < left ? r : left));
         constexpr int kWords = combine_threads(K) / 64 / 4;     // a strip's bytes
         for (int i = 0; i < static_cast<int>(V / kCombineCols) * kWords; ++i)
             odd |= nonfinite[(bp * H + h) * (V / kCombineCols) * kWords + i];
     }
-    const int rows = n0 > n1 ? n0 : n1;             // whose V outputs are in oz
     if (rows == 0 && !odd) return;                  // the others are final
     const int64_t hk = H * K, hv = H * V;
     const auto rc = make_rsrc(cf + row0 * hk + h * K, rows ? static_cast<uint32_t>(((rows - 1) * hk + K) * 4) : 0u);
@@ -269,10 +263,9 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
         for (int m = 0; m < 2; ++m) {
             const int i = t + nthr * m;
             const int r = i / (K / 4), c4 = i % (K / 4);
-            // a slot past the step's pieces, or past the coefficients of its
-            // channels, reads past the range: no memory access, zeros
-            const int nr = 4 * c4 < tile ? n0 : n1;
-            const int off = i < NP && tt + r < nr ? static_cast<int>(((tt + r) * hk + 4 * c4) * 4) : 0x7ffffff0;
+            // a slot past the step's pieces, or past the coefficients, reads past
+            // the range: no memory access, zeros
+            const int off = i < NP && tt + r < rows ? static_cast<int>(((tt + r) * hk + 4 * c4) * 4) : 0x7ffffff0;
             fc[m] = __builtin_bit_cast(w4, __builtin_amdgcn_raw_buffer_load_b128(rc, off, 0, 0));
         }
     };
@@ -390,6 +383,7 @@ int64_t long_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t
     return segment_bytes(B, T, H, K, V, P, long_correct_form(B, H, K, V, P));
 }
 
+// (V + K a multiple of 128 makes V a multiple of K, the columns of a workgroup.)
 // Segments of the split form: twice P (or the power of two times P) while the
 // V columns fit one round of workgroups and a segment keeps kSplitSegment
 // tokens (us in one launch / split at H=16 d=128: T=8192, segments of 512, 168 /
@@ -398,7 +392,7 @@ int64_t long_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t
 static int64_t split_segments(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P) {
     constexpr int64_t kSplitSegment = 1024;
     if ((K != 64 && K != 128) || T % P != 0 || !long_correct_form(B, H, K, V, P)) return 0;
-    const int64_t cus = cu_count(), tiles = B * H * (V / trans_tile(K, V)), P0 = P;
+    const int64_t cus = cu_count(), tiles = B * H * (V / K), P0 = P;
     while (2 * P * tiles <= cus && T % (2 * P) == 0 && T / (2 * P) >= kSplitSegment) P *= 2;
     return P > P0 ? P : 0;
 }
@@ -407,7 +401,7 @@ int64_t split_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_
     P = split_segments(B, T, H, K, V, P);
     if (P == 0) return 0;
     // and the chunk counts and the combine's bytes
-    return segment_bytes(B, T, H, K, V, P, true) + 4 * B * P * H * (K / trans_tile(K, V) + V / kCombineCols * (K / 64));
+    return segment_bytes(B, T, H, K, V, P, true) + 4 * B * P * H * (1 + V / kCombineCols * (K / 64));
 }
 
 // The three kernels (ends: transition columns may end early).
@@ -421,13 +415,12 @@ static int run_segments(const kda_fwd_args& a, int64_t P, bool correct, bool end
         !split_strides(s.v_stride, B, T, P) || !split_strides(s.g_stride, B, T, P) ||
         !split_strides(s.beta_stride, B, T, P))
         return KDA_ERR_UNSUPPORTED;
-    const int tile = static_cast<int>(trans_tile(K, V));
     float* seg = static_cast<float*>(workspace);
     float* sstart = seg + B * P * H * K * (V + K);
     float* oz = sstart + B * P * H * K * V;
     float* cf = oz + B * T * H * V;
     int* nch = ends ? reinterpret_cast<int*>(cf + B * T * H * K) : nullptr;
-    uint32_t* nonfinite = ends ? reinterpret_cast<uint32_t*>(nch + B * P * H * (K / tile)) : nullptr;
+    uint32_t* nonfinite = ends ? reinterpret_cast<uint32_t*>(nch + B * P * H) : nullptr;
 
     // 1. per chain: the state from zero and the transition (and in the
     // few-chain form the outputs from zero and the coefficients c)
@@ -463,7 +456,7 @@ static int run_segments(const kda_fwd_args& a, int64_t P, bool correct, bool end
         const int zero_first = a.state_in == nullptr ? 1 : 0;
 #define KDA_CORRECT(KK, TO)                                                                                    \
     hipLaunchKernelGGL((long_correct_kernel<KK, TO>), grid, block, 0, stream, oz, cf, sstart,                   \
-                       static_cast<TO*>(a.o), T, H, V, P, zero_first, nch, tile, nonfinite)
+                       static_cast<TO*>(a.o), T, H, V, P, zero_first, nch, nonfinite)
         if (a.qkv_dtype == KDA_DTYPE_F16) {
             if (K == 64) KDA_CORRECT(64, _Float16); else KDA_CORRECT(128, _Float16);
         } else {
