@@ -211,9 +211,9 @@ __device__ __forceinline__ void load_rows(Rows8& v, const T* p, int64_t stride, 
     }
 }
 
-// Grid (N / 64 * K / 128, splits); out: fp32 [splits, N, K], or one split's dw itself.
-template <typename T, typename OT>
-__global__ __launch_bounds__(256) void wgrad_kernel(kda_linear_wgrad_args a, OT* out, int64_t per) {
+// Grid (N / 64 * K / 128, splits); out: fp32 [splits, N, K].
+template <typename T>
+__global__ __launch_bounds__(256) void wgrad_kernel(kda_linear_wgrad_args a, float* out, int64_t per) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ln = lane & 15, lg = lane >> 4;
     const int64_t nt = a.N / kWgN;
@@ -294,10 +294,11 @@ __global__ __launch_bounds__(256) void wgrad_sum_kernel(const float* part, T* dw
     store4(dw + e, s);
 }
 
-// One workgroup a CU, each with at least two steps a wave.
+// One workgroup a CU, each with at least two steps a wave; two or more, with at
+// most 64 tiles and at least 16 steps.
 int64_t wgrad_splits(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = (N / kWgN) * (K / kWgK), steps = (M + 31) / 32;
-    return max(int64_t{1}, min(256 / tiles, steps / 8));
+    return min(256 / tiles, steps / 8);
 }
 
 template <typename T>
@@ -305,12 +306,8 @@ int launch_wgrad(const kda_linear_wgrad_args& a, hipStream_t stream) {
     const int64_t splits = wgrad_splits(a.M, a.N, a.K), steps = (a.M + 31) / 32;
     const int64_t per = (steps + splits - 1) / splits;
     const dim3 grid(static_cast<unsigned>((a.N / kWgN) * (a.K / kWgK)), static_cast<unsigned>(splits));
-    if (splits == 1) {
-        wgrad_kernel<T, T><<<grid, 256, 0, stream>>>(a, static_cast<T*>(a.dw), per);
-        return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
-    }
     float* part = static_cast<float*>(a.workspace);
-    wgrad_kernel<T, float><<<grid, 256, 0, stream>>>(a, part, per);
+    wgrad_kernel<T><<<grid, 256, 0, stream>>>(a, part, per);
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
     const int64_t n = a.N * a.K;
     wgrad_sum_kernel<T><<<static_cast<unsigned>((n / 4 + 255) / 256), 256, 0, stream>>>(part, static_cast<T*>(a.dw), n,
