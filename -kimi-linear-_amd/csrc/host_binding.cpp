@@ -135,11 +135,21 @@ struct Plain {
 };
 
 void* stream_of(const at::Device& dev) {
-    py::object s = py::reinterpret_steal<py::object>(
-        PyObject_CallFunction(raw_stream, "i", static_cast<int>(dev.index())));
+    const py::int_ index(static_cast<int>(dev.index()));
+    py::object s = py::reinterpret_steal<py::object>(PyObject_CallOneArg(raw_stream, index.ptr()));
     if (!s) throw py::error_already_set();
     return reinterpret_cast<void*>(s.cast<uintptr_t>());
 }
+
+// The interpreter lock given up for a scope (without the bookkeeping of
+// py::gil_scoped_release, which a decode step's call of 6 us would notice).
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+    Unlocked() = default;
+    Unlocked(const Unlocked&) = delete;
+    Unlocked& operator=(const Unlocked&) = delete;
+};
 
 // f(stream), f the allocations and the C ABI call of one entry, on dev and its
 // current stream.  Without the interpreter lock: an allocation or a launch into
@@ -147,7 +157,7 @@ void* stream_of(const at::Device& dev) {
 template <typename F>
 int run(const at::Device& dev, F&& f) {
     void* stream = stream_of(dev);
-    const py::gil_scoped_release unlocked;
+    const Unlocked unlocked;
     const c10::DeviceGuard guard(dev);
     return f(stream);
 }
@@ -545,10 +555,15 @@ PYBIND11_MODULE(_kda_host, m) {
     m.def("abi_version", [] { return KDA_ABI_VERSION; });
     m.attr("torch_version") = KDA_TORCH_VERSION;    // it was compiled against; its C++ interface is not stable
     m.def("bind", &bind);
-    m.def("core", &core, py::arg("recurrent"), py::arg("q"), py::arg("k"), py::arg("v"), py::arg("g"), py::arg("beta"),
-          py::arg("state"), py::arg("chunk_size"), py::arg("state_dtype"), py::arg("state_out"), py::arg("a_log"),
-          py::arg("dt_bias"), py::arg("og"), py::arg("weight"), py::arg("eps"), py::arg("segments"),
-          py::arg("transitions_first") = true);
+    m.def("core", [](bool recurrent, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g,
+                     const Tensor& beta, const OptTensor& state, int64_t chunk_size,
+                     const std::optional<at::ScalarType>& state_dtype, const OptTensor& state_out,
+                     const OptTensor& a_log, const OptTensor& dt_bias, const OptTensor& og, const OptTensor& weight,
+                     double eps, int64_t segments) {
+        return core(recurrent, q, k, v, g, beta, state, chunk_size, state_dtype, state_out, a_log, dt_bias, og, weight,
+                    eps, segments, true);
+    });
+    m.def("core", &core);
     m.def("prep", &prep);
     m.def("output", &output);
     m.def("linear", &linear);

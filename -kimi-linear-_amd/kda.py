@@ -100,8 +100,9 @@ def _common(kind, q, k, v, g, beta, state, chunk_size, state_dtype, state_out=No
     if split and isinstance(q, torch.Tensor) and isinstance(v, torch.Tensor) and q.dim() == 4 and v.dim() == 4:
         segments = long_segments(*q.shape, v.shape[-1], v.dtype)
     try:
+        form = (segments, _transitions_first(q.shape[1], segments)) if segments > 1 else (1,)
         return _native.host().core(kind == "recurrent", q, k, v, g, beta, state, chunk_size, state_dtype, state_out,
-                                   *gate, *epilogue, segments, segments > 1 and _transitions_first(q.shape[1], segments))
+                                   *gate, *epilogue, *form)
     except TypeError:       # an argument of no type a common call has
         return None
 
