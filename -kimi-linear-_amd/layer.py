@@ -170,22 +170,20 @@ def _plain_weight(mod, *inputs):
     without a bias, hooks or a forward of its own, with no torch function mode
     or tensor subclass that takes part in ``F.linear``; else None."""
     if (type(mod) is not nn.Linear or mod.bias is not None or mod._forward_hooks or mod._forward_pre_hooks
-            or "forward" in mod.__dict__ or nn.modules.module._has_any_global_hook()
-            or has_torch_function((mod.weight, *inputs))):
+            or "forward" in mod.__dict__ or nn.modules.module._has_any_global_hook()):
         return None
-    return mod.weight
+    w = mod.weight
+    return None if has_torch_function((w, *inputs)) else w
 
 
-def _few_rows(x, n: int) -> bool:
-    """Whether ``kda_linear_fwd`` is the faster product for x [B, T, K] and n
-    outputs, by measurement over K 256 to 4096 and n 512 to 12576 (us, library /
+def _few_rows(rows: int, k: int, n: int) -> bool:
+    """Whether ``kda_linear_fwd`` is the faster product of x [rows, k] for n outputs, by measurement over K 256 to 4096 and n 512 to 12576 (us, library /
     kernel, fp16).  More than 8192 outputs are more workgroups than the chip
     holds: K = 2048, n = 12576 10.7 / 11.8 at one row, 512 4.9 at K = 512 (8.6).
     Beyond K = 2048 only the reads of W count that fill the chip at once: K =
     2304, 4 rows, n = 4096 6.7 / 5.8, n = 6416 7.9 / 8.1, n = 512 4.8 / 4.8; 16
     rows, n = 2048 6.4 / 6.5.  Steps of 32 that do not divide over four waves
     leave one a workgroup: K = 1568, n = 2048 5.8 / 6.3, n = 4096 8.4 / 6.8."""
-    rows, k = x.shape[0] * x.shape[1], x.shape[2]
     if rows > 64 or k % 32 != 0:
         return False
     one_wave = k % 128 != 0 or k < 512
@@ -201,8 +199,9 @@ def _few_rows(x, n: int) -> bool:
 def _project(mod, x, residual=None, out=None):
     """``mod(x)``, plus ``residual``, into ``out``: in the few-row kernel
     (``kda_linear_fwd``) where it applies, else as written."""
-    w = _plain_weight(mod, x) if x.shape[0] * x.shape[1] <= 64 else None
-    if w is not None and not _few_rows(x, w.shape[0]):
+    B, T, k = x.shape
+    w = _plain_weight(mod, x) if B * T <= 64 else None
+    if w is not None and not _few_rows(B * T, k, w.shape[0]):
         w = None
     y = _native.host().linear(x, w, residual, out) if w is not None else None
     if y is not None:
@@ -349,7 +348,11 @@ class KimiDeltaAttention(nn.Module):
     def _unmodified(self, *methods):
         """Whether these methods are the ones written here, not a subclass's, the
         instance's or a later replacement: only then may a call go by them."""
-        return all(getattr(type(self), n) is _METHODS[n] and n not in self.__dict__ for n in methods)
+        cls, own = type(self), self.__dict__
+        for n in methods:
+            if getattr(cls, n) is not _METHODS[n] or n in own:
+                return False
+        return True
 
     def _projections(self, x, conv_cache=None, use_cache=False, conv_out=None, gates=False):
         """q, k, v, the gate's up-projection gk ``[B, T, H, K]``, the beta logits
@@ -375,20 +378,25 @@ class KimiDeltaAttention(nn.Module):
         convs = (self.conv_q.conv, self.conv_k.conv, self.conv_v.conv)
         H, K, V = self.num_heads, self.head_dim, self.value_head_dim
         w, b = self._input_weight()
-        few = x.shape[0] * x.shape[1] <= 64 and not has_torch_function((x,))
-        y = _native.host().linear(x, w, None, None) if few and b is None and _few_rows(x, w.shape[0]) else None
+        B, T, d = x.shape
+        rows = B * T
+        few = rows <= 64 and not has_torch_function((x,))
+        y = None
+        if few and b is None and _few_rows(rows, d, w.shape[0]):
+            y = _native.host().linear(x, w, None, None)
         if y is None:
             y = torch.nn.functional.linear(x, w, b)
+        (gk_down, gk_up), (og_down, og_up) = self.gk_proj, self.og_proj
         q_in, k_in, v_in, beta_logit, gk_low, og_low = torch.split(
-            y, (H * K, H * K, H * V, H, self.gk_proj[0].out_features, self.og_proj[0].out_features), dim=-1)
+            y, (H * K, H * K, H * V, H, gk_down.out_features, og_down.out_features), dim=-1)
         gk = gate = None
         if few and output_gate:       # both up-projections in one launch
-            w_gk, w_og = _plain_weight(self.gk_proj[1]), _plain_weight(self.og_proj[1])
-            if (w_gk is not None and w_og is not None and _few_rows(gk_low, w_gk.shape[0])
-                    and _few_rows(og_low, w_og.shape[0])):
+            w_gk, w_og = _plain_weight(gk_up), _plain_weight(og_up)
+            if (w_gk is not None and w_og is not None and _few_rows(rows, gk_down.out_features, w_gk.shape[0])
+                    and _few_rows(rows, og_down.out_features, w_og.shape[0])):
                 gk, gate = _native.host().linear2(gk_low, w_gk, og_low, w_og) or (None, None)
         if gk is None:
-            gk = self.gk_proj[1](gk_low)
+            gk = gk_up(gk_low)
         gate_in = (gk, *self._gate_params(), beta_logit) if gates else (None, None, None, None)
         q, k, v, g, beta, new_conv = kda_prep(
             q_in, k_in, v_in,
@@ -399,7 +407,7 @@ class KimiDeltaAttention(nn.Module):
             want_hist=use_cache and conv_out is None)
         if gates:
             return q, k, v, g, beta, new_conv, og_low, gate
-        return q, k, v, gk.view(x.shape[0], x.shape[1], H, K), beta_logit, new_conv, og_low, gate
+        return q, k, v, gk.view(B, T, H, K), beta_logit, new_conv, og_low, gate
 
     def _core_inputs(self, x, **kw):
         """:meth:`_inputs`, through :meth:`_projections` if that or :meth:`_output` has been replaced."""
