@@ -1671,8 +1671,8 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
             }
 #pragma unroll
             for (int g = 0; g < CG; ++g)
-                store_state<KT, kIntState>(S[g], a.state_out, a.state_out_dtype, sbase + (4 * kn.lg) * VS + colw + 16 * g + kn.ln,
-                                VS);
+                store_state<KT, kIntState>(S[g], a.state_out, a.state_out_dtype,
+                                           sbase + (4 * kn.lg) * VS + colw + 16 * g + kn.ln, VS);
         }
     } else {
         const int p = wave - NC;

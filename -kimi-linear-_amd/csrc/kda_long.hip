@@ -387,8 +387,8 @@ int64_t long_workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t K, int64_t
 // Segments of the split form: twice P (or the power of two times P) while the
 // V columns fit one round of workgroups and a segment keeps kSplitSegment
 // tokens (us in one launch / split at H=16 d=128: T=8192, segments of 512, 168 /
-// 166, T=4096, 256, 97 / 126; T=16384, 1024, 288 / 217); none (0) where P cannot be doubled: its one launch holds both kinds
-// of columns side by side.
+// 166, T=4096, 256, 97 / 126; T=16384, 1024, 288 / 217); none (0) where P cannot
+// be doubled: its one launch holds both kinds of columns side by side.
 static int64_t split_segments(int64_t B, int64_t T, int64_t H, int64_t K, int64_t V, int64_t P) {
     constexpr int64_t kSplitSegment = 1024;
     if ((K != 64 && K != 128) || T % P != 0 || !long_correct_form(B, H, K, V, P)) return 0;

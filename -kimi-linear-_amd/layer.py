@@ -177,9 +177,10 @@ def _plain_weight(mod, *inputs):
 
 
 def _few_rows(rows: int, k: int, n: int) -> bool:
-    """Whether ``kda_linear_fwd`` is the faster product of x [rows, k] for n outputs, by measurement over K 256 to 4096 and n 512 to 12576 (us, library /
-    kernel, fp16).  More than 8192 outputs are more workgroups than the chip
-    holds: K = 2048, n = 12576 10.7 / 11.8 at one row, 512 4.9 at K = 512 (8.6).
+    """Whether ``kda_linear_fwd`` is the faster product of x [rows, k] for n
+    outputs, by measurement over k 128 and 256 to 4096 and n 512 to 12576 (us,
+    library / kernel, fp16).  More than 8192 outputs are more workgroups than the
+    chip holds: n = 12576 at one row, K = 2048 10.7 / 11.8, K = 512 8.6 / 4.9.
     Beyond K = 2048 only the reads of W count that fill the chip at once: K =
     2304, 4 rows, n = 4096 6.7 / 5.8, n = 6416 7.9 / 8.1, n = 512 4.8 / 4.8; 16
     rows, n = 2048 6.4 / 6.5.  Steps of 32 that do not divide over four waves
