@@ -251,7 +251,8 @@ class KimiDeltaAttention(nn.Module):
         self.fuse_output = None    # output epilogue in the chunk kernel: True, False, None = by shape
 
     def _input_mods(self):
-        return (self.in_proj_q, self.in_proj_k, self.in_proj_v, self.beta_proj, self.gk_proj[0], self.og_proj[0])
+        return (self.in_proj_q, self.in_proj_k, self.in_proj_v, self.beta_proj, next(iter(self.gk_proj)),
+                next(iter(self.og_proj)))
 
     def _input_weight(self):
         """The six projections of x -- q, k, v, beta and the down-projections
@@ -387,7 +388,7 @@ class KimiDeltaAttention(nn.Module):
             y = _native.host().linear(x, w, None, None)
         if y is None:
             y = torch.nn.functional.linear(x, w, b)
-        (gk_down, gk_up), (og_down, og_up) = self.gk_proj, self.og_proj
+        (gk_down, gk_up, *_), (og_down, og_up, *_) = self.gk_proj, self.og_proj
         q_in, k_in, v_in, beta_logit, gk_low, og_low = torch.split(
             y, (H * K, H * K, H * V, H, gk_down.out_features, og_down.out_features), dim=-1)
         gk = gate = None

@@ -95,3 +95,19 @@ def test_few_row_projections_where_they_are_faster(kda_pkg, rows, k, n, own):
     assert layer._few_rows(rows, k, n) is own
     if own:       # nothing that the kernel refuses
         assert k % 32 == 0 and (rows <= 16 or k <= (1024 if rows <= 32 else 512))
+
+
+def test_gate_projections_may_hold_further_modules(kda_pkg, monkeypatch):
+    """The gates' projections are the first and second module of theirs, whatever follows."""
+    import importlib
+    layer = importlib.import_module("kimi_linear_amd.layer")
+    monkeypatch.setattr(layer, "kda_prep", lambda *a, **kw: (None,) * 6)
+    m = kda_pkg.KimiDeltaAttention(kda_pkg.linear_attn_config(hidden_size=64, num_heads=1, head_dim=64,
+                                                              value_head_dim=64))
+    x = torch.randn(1, 5, 64)
+    with torch.no_grad():
+        want = m._projections(x)
+        for proj in (m.gk_proj, m.og_proj):
+            proj.append(torch.nn.ReLU())
+        got = m._projections(x)
+    assert torch.equal(got[3], want[3]) and torch.equal(got[6], want[6])
