@@ -169,11 +169,12 @@ def _plain_weight(mod, *inputs):
     """The weight of a module that is just x W^T: an ``nn.Linear`` as torch has it,
     without a bias, hooks or a forward of its own, with no torch function mode
     or tensor subclass that takes part in ``F.linear``; else None."""
-    if (type(mod) is not nn.Linear or mod.bias is not None or mod._forward_hooks or mod._forward_pre_hooks
+    if (type(mod) is not nn.Linear or mod._forward_hooks or mod._forward_pre_hooks
             or "forward" in mod.__dict__ or nn.modules.module._has_any_global_hook()):
         return None
-    w = mod.weight
-    return None if has_torch_function((w, *inputs)) else w
+    own = mod._parameters       # (the module's attribute lookup takes longer; a name set otherwise is not here)
+    w = own.get("weight")
+    return None if w is None or own.get("bias", mod) is not None or has_torch_function((w, *inputs)) else w
 
 
 def _few_rows(rows: int, k: int, n: int) -> bool:
