@@ -531,7 +531,7 @@ class KimiDeltaAttention(nn.Module):
         split = (not fused and not (use_cache and T == 1) and body > 0 and (B == 1 or body == T)
                  and long_segments(B, body, self.num_heads, self.head_dim, self.value_head_dim, x.dtype) > 1)
         q, k, v, g, beta, new_conv, *og = self._core_inputs(x, conv_cache=conv_cache, use_cache=use_cache, gates=split)
-        gate = self._gate_params()      # unless split, g and beta above are gk and the beta logits
+        gate = None if split else self._gate_params()       # then g and beta above are gk and the beta logits
         if fused:
             # one chunkwise body and no tail: the output epilogue runs on the
             # chunk kernel's tiles and its result is the o_proj input
