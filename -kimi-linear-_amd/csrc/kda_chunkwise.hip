@@ -1670,9 +1670,11 @@ __global__ __launch_bounds__(64 * (NC + NB)) void chunkwise_kernel(const kda_fwd
                     for (int t = 0; t < KT; ++t) S[g][t] *= kn.isig;
             }
 #pragma unroll
-            for (int g = 0; g < CG; ++g)
-                store_state<KT, kIntState>(S[g], a.state_out, a.state_out_dtype,
-                                           sbase + (4 * kn.lg) * VS + colw + 16 * g + kn.ln, VS);
+            for (int g = 0; g < CG; ++g) {
+                const int64_t off = sbase + (4 * kn.lg) * VS + colw + 16 * g + kn.ln;
+                if constexpr (TRANS) store_state_t<KT, kIntState>(S[g], static_cast<float*>(a.state_out), off, VS);
+                else store_state<KT, kIntState>(S[g], a.state_out, a.state_out_dtype, off, VS);
+            }
         }
     } else {
         const int p = wave - NC;

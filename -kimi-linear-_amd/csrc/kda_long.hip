@@ -33,11 +33,13 @@
 // then it takes those tokens too, with c = 0).  Each of the two launches has
 // the chip to itself, so a segment is half as long.  B=1 T=32768 H=16 K=V=128
 // fp16: 8 segments in one launch 537 us, 16 in two 316; in a kernel trace, with
-// its gaps, trans 34, V columns 215, combine 48, correction 37.  Where nothing is
+// its gaps, trans 34, V columns 210, combine 46, correction 39.  Where nothing is
 // forgotten (decays 1000 times weaker) it costs a combine of twice the length
 // and a launch: 224 + 242 + 49 + 140 us where the one launch takes 435 + 24 +
 // 141.  The combine's 3 us a segment did not move with its next segment's loads
 // requested ahead of the products, nor with the strip read at once.
+#include <type_traits>
+
 #include "kda_common.h"
 #include "kda_launch.h"
 
@@ -65,9 +67,11 @@ constexpr int kCombinePad = 20;    // LDS row of the state strip: conflict-free 
 // load of the row covers u = 0 .. 3) against S[16 U + 4 lg + u][ln].
 // seg: [B P, H, K, V + K] fp32 (columns [0, V) S_loc, [V, V + K) Phi);
 // sstart: [B P, H, K, V] fp32; s0 (nullable, any dtype) and sout: [B, H, K, V].
-// nonfinite (nullable): [B P, H, V / 16, waves], whether S_start[p]'s part is
-// not finite (a byte a wave).
-template <int K>
+// ENDS: also nonfinite [B P, H, V / 16, waves], whether S_start[p]'s part is not
+// finite (a byte a wave), for the split form.  (Off where the transition columns
+// never end: B=1 T=8192 H=4 K=V=64, 32 segments, 27.7 us with it, 26.4 without,
+// the correction 10.3 and 9.9.)
+template <int K, bool ENDS>
 __global__ __launch_bounds__(combine_threads(K)) void long_combine_kernel(const float* seg, float* sstart,
                                                                        const void* s0, int s0_dtype, void* sout,
                                                                        int sout_dtype, int64_t B, int64_t H,
@@ -105,18 +109,19 @@ __global__ __launch_bounds__(combine_threads(K)) void long_combine_kernel(const 
     if (P > 0) fetch(0);
     for (int64_t p = 0; p < P; ++p) {
         const int64_t bp = b * P + p;
-        bool odd = false;
+        [[maybe_unused]] bool odd = false;
 #pragma unroll
         for (int m = 0; m < EPT; ++m) {
             const int e = t + kCombineThreads * m, r = e / kCombineCols, j = e % kCombineCols;
             const float x = S[r][j];
             sstart[((bp * H + h) * K + r) * V + c0 + j] = x;
-            odd = odd || !(fabsf(x) <= 3.4028235e38f);
+            if constexpr (ENDS) odd = odd || !(fabsf(x) <= 3.4028235e38f);
         }
-        // one byte a wave: its part of the strip holds an infinity or a NaN
-        const bool any_odd = __any(odd);
-        if (nonfinite != nullptr && lane == 0)
-            nonfinite[((bp * H + h) * nct + c0 / kCombineCols) * kCombineWaves + w] = any_odd;
+        if constexpr (ENDS) {
+            // one byte a wave: its part of the strip holds an infinity or a NaN
+            const bool any_odd = __any(odd);
+            if (lane == 0) nonfinite[((bp * H + h) * nct + c0 / kCombineCols) * kCombineWaves + w] = any_odd;
+        }
         f4 acc = sl;
 #pragma unroll
         for (int U = 0; U < K / 16; ++U)
@@ -167,16 +172,16 @@ constexpr int kCorrectTokens = 256;   // tokens per correction workgroup
 // segment that starts from zero (no initial state) takes oz as it is.  Rows
 // past the segment's end are outside the descriptors' ranges (read as zero,
 // stores dropped).  oz, cf: [B T, H, V] and [B T, H, K] fp32; sstart:
-// [B P, H, K, V] fp32; o: [B T, H, V] in the output dtype.  nch: [B P, H], the
-// 32-token chunks of the segment whose coefficients were written (zero after
-// them, and the outputs in o instead of oz), or null: all; nonfinite: of the
-// combine.
+// [B P, H, K, V] fp32; o: [B T, H, V] in the output dtype.  ENDS: nch [B P, H],
+// the 32-token chunks of the segment whose coefficients were written (zero after
+// them, and the outputs in o instead of oz), and nonfinite of the combine;
+// otherwise all of them were.
 template <int K>
 struct CorrectSmem {
     uint16_t hi[2][16][K + 8];
     uint16_t lo[2][16][K + 8];
 };
-template <int K, typename TO>
+template <int K, typename TO, bool ENDS>
 __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, const float* cf, const float* sstart,
                                                             TO* o, int64_t T, int64_t H, int64_t V, int64_t P,
                                                             int zero_first, const int* nch,
@@ -200,18 +205,19 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
     // oz; and whether S_start is not finite (a word a strip)
     const int64_t left = Ts - t0 < kCorrectTokens ? Ts - t0 : kCorrectTokens;
     int rows = static_cast<int>(left);
-    uint32_t odd = 0;
-    if (nch != nullptr) {
+    [[maybe_unused]] bool odd = false;
+    if constexpr (ENDS) {
         const int64_t r = 32 * static_cast<int64_t>(nch[bp * H + h]) - t0;
         rows = static_cast<int>(r < 0 ? 0 : (r < left ? r : left));
         constexpr int kWords = combine_threads(K) / 64 / 4;     // a strip's bytes
         for (int i = 0; i < static_cast<int>(V / kCombineCols) * kWords; ++i)
-            odd |= nonfinite[(bp * H + h) * (V / kCombineCols) * kWords + i];
+            odd = odd || nonfinite[(bp * H + h) * (V / kCombineCols) * kWords + i] != 0;
+        if (rows == 0 && !odd) return;              // the others are final
     }
-    if (rows == 0 && !odd) return;                  // the others are final
     const int64_t hk = H * K, hv = H * V;
-    const auto rc = make_rsrc(cf + row0 * hk + h * K, rows ? static_cast<uint32_t>(((rows - 1) * hk + K) * 4) : 0u);
-    const auto rz = make_rsrc(oz + row0 * hv + h * V, rows ? static_cast<uint32_t>(((rows - 1) * hv + V) * 4) : 0u);
+    const bool some = !ENDS || rows != 0;
+    const auto rc = make_rsrc(cf + row0 * hk + h * K, some ? static_cast<uint32_t>(((rows - 1) * hk + K) * 4) : 0u);
+    const auto rz = make_rsrc(oz + row0 * hv + h * V, some ? static_cast<uint32_t>(((rows - 1) * hv + V) * 4) : 0u);
     const auto ro = make_rsrc(o + row0 * hv + h * V,
                               static_cast<uint32_t>(((left - 1) * hv + V) * static_cast<int64_t>(sizeof(TO))));
     auto store_out = [&](const f4& y, int orow) {
@@ -263,9 +269,9 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
         for (int m = 0; m < 2; ++m) {
             const int i = t + nthr * m;
             const int r = i / (K / 4), c4 = i % (K / 4);
-            // a slot past the step's pieces, or past the coefficients, reads past
-            // the range: no memory access, zeros
-            const int off = i < NP && tt + r < rows ? static_cast<int>(((tt + r) * hk + 4 * c4) * 4) : 0x7ffffff0;
+            // a slot past the step's pieces reads past the range, as do rows past
+            // the last: no memory access, zeros
+            const int off = i < NP ? static_cast<int>(((tt + r) * hk + 4 * c4) * 4) : 0x7ffffff0;
             fc[m] = __builtin_bit_cast(w4, __builtin_amdgcn_raw_buffer_load_b128(rc, off, 0, 0));
         }
     };
@@ -327,7 +333,7 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
         z = zn;
         buf ^= 1;
     }
-    if (odd) {
+    if (ENDS && odd) {
         // the tokens after them: o + 0 S_start, a NaN in the columns of S_start
         // that hold an infinity or a NaN
         f4 nan = {0.f, 0.f, 0.f, 0.f};
@@ -441,12 +447,15 @@ static int run_segments(const kda_fwd_args& a, int64_t P, bool correct, bool end
     const dim3 cgrid(static_cast<unsigned>(B * H * (V / kCombineCols)));
     const dim3 cblock(static_cast<unsigned>(combine_threads(static_cast<int>(K))));
     auto* bad = reinterpret_cast<uint8_t*>(nonfinite);
-    if (K == 64)
-        hipLaunchKernelGGL((long_combine_kernel<64>), cgrid, cblock, 0, stream, seg, sstart, a.state_in,
-                           a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P, bad);
-    else
-        hipLaunchKernelGGL((long_combine_kernel<128>), cgrid, cblock, 0, stream, seg, sstart, a.state_in,
-                           a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P, bad);
+#define KDA_COMBINE(KK, ENDS)                                                                                  \
+    hipLaunchKernelGGL((long_combine_kernel<KK, ENDS>), cgrid, cblock, 0, stream, seg, sstart, a.state_in,      \
+                       a.state_in_dtype, a.state_out, a.state_out_dtype, B, H, V, P, bad)
+    if (K == 64) {
+        if (ends) KDA_COMBINE(64, true); else KDA_COMBINE(64, false);
+    } else {
+        if (ends) KDA_COMBINE(128, true); else KDA_COMBINE(128, false);
+    }
+#undef KDA_COMBINE
     if (hipGetLastError() != hipSuccess) return KDA_ERR_LAUNCH;
 
     if (correct) {
@@ -454,14 +463,19 @@ static int run_segments(const kda_fwd_args& a, int64_t P, bool correct, bool end
         const int64_t nblk = (T / P + kCorrectTokens - 1) / kCorrectTokens;
         const dim3 grid(static_cast<unsigned>(B * P * nblk * H)), block(static_cast<unsigned>(4 * V));
         const int zero_first = a.state_in == nullptr ? 1 : 0;
-#define KDA_CORRECT(KK, TO)                                                                                    \
-    hipLaunchKernelGGL((long_correct_kernel<KK, TO>), grid, block, 0, stream, oz, cf, sstart,                   \
+#define KDA_CORRECT(KK, TO, ENDS)                                                                              \
+    hipLaunchKernelGGL((long_correct_kernel<KK, TO, ENDS>), grid, block, 0, stream, oz, cf, sstart,             \
                        static_cast<TO*>(a.o), T, H, V, P, zero_first, nch, nonfinite)
-        if (a.qkv_dtype == KDA_DTYPE_F16) {
-            if (K == 64) KDA_CORRECT(64, _Float16); else KDA_CORRECT(128, _Float16);
-        } else {
-            if (K == 64) KDA_CORRECT(64, bf16_t); else KDA_CORRECT(128, bf16_t);
-        }
+        const auto go = [&](auto to, auto e) {
+            using TO = decltype(to);
+            constexpr bool ENDS = decltype(e)::value;
+            if (K == 64) KDA_CORRECT(64, TO, ENDS); else KDA_CORRECT(128, TO, ENDS);
+        };
+        const bool f16 = a.qkv_dtype == KDA_DTYPE_F16;
+        if (ends && f16) go(_Float16{}, std::true_type{});
+        else if (ends) go(bf16_t{}, std::true_type{});
+        else if (f16) go(_Float16{}, std::false_type{});
+        else go(bf16_t{}, std::false_type{});
 #undef KDA_CORRECT
         return hipGetLastError() == hipSuccess ? KDA_OK : KDA_ERR_LAUNCH;
     }
