@@ -33,7 +33,7 @@
 // then it takes those tokens too, with c = 0).  Each of the two launches has
 // the chip to itself, so a segment is half as long.  B=1 T=32768 H=16 K=V=128
 // fp16: 8 segments in one launch 537 us, 16 in two 316; in a kernel trace, with
-// its gaps, trans 34, V columns 210, combine 46, correction 39.  Where nothing is
+// its gaps, trans 34, V columns 210, combine 46, correction 36.  Where nothing is
 // forgotten (decays 1000 times weaker) it costs a combine of twice the length
 // and a launch: 224 + 242 + 49 + 140 us where the one launch takes 435 + 24 +
 // 141.  The combine's 3 us a segment did not move with its next segment's loads
@@ -210,8 +210,8 @@ __global__ __launch_bounds__(1024) void long_correct_kernel(const float* oz, con
         const int64_t r = 32 * static_cast<int64_t>(nch[bp * H + h]) - t0;
         rows = static_cast<int>(r < 0 ? 0 : (r < left ? r : left));
         constexpr int kWords = combine_threads(K) / 64 / 4;     // a strip's bytes
-        for (int i = 0; i < static_cast<int>(V / kCombineCols) * kWords; ++i)
-            odd = odd || nonfinite[(bp * H + h) * (V / kCombineCols) * kWords + i] != 0;
+        const int64_t words = V / kCombineCols * kWords;        // at most 32
+        odd = __any(lane < words && nonfinite[(bp * H + h) * words + lane] != 0);
         if (rows == 0 && !odd) return;              // the others are final
     }
     const int64_t hk = H * K, hv = H * V;
