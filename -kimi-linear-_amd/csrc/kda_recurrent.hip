@@ -651,6 +651,23 @@ int launch_seq(const kda_fwd_args& a, hipStream_t stream, const kda_gate_args& g
     return launch_seq_c<K, 1>(a, stream, gate, ckpt);
 }
 
+// Spans of smaller states (cols = B H V) whose tokens are faster one at a time:
+// 2 tokens of many columns, whose chains already fill the chip; up to four of more
+// workgroups of 32 columns than run side by side (V no multiple of 64); and K =
+// 256, whose span kernel holds 8 tokens a group.  us, one at a time / span kernel,
+// fp16: T=2 K=V=128, 8192 columns 6.6 / 6.2, 16384 7.4 / 8.2, 32768 8.9 / 10.5;
+// K=V=64, 16384 5.8 / 5.9, 24576 6.1 / 6.6, T=3 7.5 / 7.0; K=V=32, 24576 5.6 /
+// 5.6, 32768 5.7 / 6.3; K=64 V=32, 32768, T=2 6.4 / 9.4, T=4 9.3 / 10.0, T=6 12.1
+// / 10.7, at 24576 T=3 7.5 / 7.1; K=256 V=64, 8192, T=2 8.0 / 8.8, T=3 10.0 /
+// 9.2, 16384, T=4 13.7 / 13.2 (fp32 13.5 / 14.2), T=6 17.3 / 14.2, 24576, T=6
+// 21.9 / 24.9.
+template <int K>
+bool one_by_one(int64_t T, int64_t V, int64_t cols) {
+    if (K == 256) return cols > 16384 || (cols > 8192 && T <= 4) || (cols > 4096 && T == 2);
+    if (T == 2) return cols > (K == 128 ? 8192 : 16384);
+    return K == 64 && V % 64 != 0 && cols > 24576 && T <= 4;
+}
+
 template <int K>
 int launch_k(const kda_fwd_args& a, hipStream_t stream, const kda_gate_args& gate, float* ckpt) {
     // A single token, and 2 to 7 tokens of a state large enough to be bound by
@@ -658,7 +675,7 @@ int launch_k(const kda_fwd_args& a, hipStream_t stream, const kda_gate_args& gat
     // in the span kernel, T=4 33 / 40, T=8 41 / 41; B=16: T=2 11.5 / 11.2, T=4
     // 17 / 12), run one token at a time over wide column tiles.
     const int64_t cols = a.B * a.H * a.V;
-    const bool wide = cols > 64 * 512;
+    const bool wide = cols > 64 * 512 || one_by_one<K>(a.T, a.V, cols);
     if (ckpt != nullptr || (a.T > 1 && (a.T >= 8 || !wide))) return launch_seq<K>(a, stream, gate, ckpt);
     // K <= 128: one wave a workgroup, of 64 columns (K = 128: 32 rows x 4
     // columns a lane, 2 waves a SIMD: the 2048 waves of a B=64 H=16 V=128 step

@@ -63,6 +63,12 @@ def check(tag, o, s, ref, dtype):
     (5, 9, 16, 128, 256, torch.bfloat16),    # 1280, K = 128
     (40, 8, 8, 64, 128, torch.float16),      # a state above the wide bound, at T = 8
     (40, 7, 8, 64, 128, torch.float16),      # and just below it (the per-token kernel)
+    (257, 2, 1, 64, 64, torch.float32),      # smaller states whose tokens are faster one at a time
+    (65, 2, 1, 128, 128, torch.float16),
+    (65, 2, 1, 256, 64, torch.float32),
+    (129, 4, 1, 256, 64, torch.bfloat16),
+    (129, 7, 1, 256, 128, torch.float32),
+    (769, 4, 1, 64, 32, torch.float16),
 ])
 def test_span_matches_float64(kda_pkg, B, T, H, K, V, dtype):
     inp, dev = inputs(B, T, H, K, V, dtype)
