@@ -658,14 +658,15 @@ int launch_seq(const kda_fwd_args& a, hipStream_t stream, const kda_gate_args& g
 // fp16: T=2 K=V=128, 8192 columns 6.6 / 6.2, 16384 7.4 / 8.2, 32768 8.9 / 10.5;
 // K=V=64, 16384 5.8 / 5.9, 24576 6.1 / 6.6, T=3 7.5 / 7.0; K=V=32, 24576 5.6 /
 // 5.6, 32768 5.7 / 6.3; K=64 V=32, 32768, T=2 6.4 / 9.4, T=4 9.3 / 10.0, T=6 12.1
-// / 10.7, at 24576 T=3 7.5 / 7.1; K=256 V=64, 8192, T=2 8.0 / 8.8, T=3 10.0 /
+// / 10.7, at 24576 T=3 7.5 / 7.1; K=128 V=32, 16384, T=3 9.2 / 8.5, 24576, T=3
+// 10.3 / 12.5, T=4 12.3 / 12.9, T=6 16.4 / 14.0; K=256 V=64, 8192, T=2 8.0 / 8.8, T=3 10.0 /
 // 9.2, 16384, T=4 13.7 / 13.2 (fp32 13.5 / 14.2), T=6 17.3 / 14.2, 24576, T=6
 // 21.9 / 24.9.
 template <int K>
 bool one_by_one(int64_t T, int64_t V, int64_t cols) {
     if (K == 256) return cols > 16384 || (cols > 8192 && T <= 4) || (cols > 4096 && T == 2);
     if (T == 2) return cols > (K == 128 ? 8192 : 16384);
-    return K == 64 && V % 64 != 0 && cols > 24576 && T <= 4;
+    return K >= 64 && V % 64 != 0 && cols > (K == 128 ? 16384 : 24576) && T <= 4;
 }
 
 template <int K>

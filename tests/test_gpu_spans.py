@@ -69,6 +69,7 @@ def check(tag, o, s, ref, dtype):
     (129, 4, 1, 256, 64, torch.bfloat16),
     (129, 7, 1, 256, 128, torch.float32),
     (769, 4, 1, 64, 32, torch.float16),
+    (1025, 3, 1, 128, 16, torch.float32),
 ])
 def test_span_matches_float64(kda_pkg, B, T, H, K, V, dtype):
     inp, dev = inputs(B, T, H, K, V, dtype)
